@@ -271,6 +271,56 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
                           float q_scale, void *stream);
 
 /*
+ * fp32 matrix product C[M,N] on the bf16 matrix cores, each operand as the sum of three bf16 numbers (all of fp32's
+ * 24 bits), fp32 sums.  For the projections and feed-forward layers around the operators
+ * (language_modeling/src/utils/cuda_fast_weight_layer.py:108,163, utils/model_utils.py:45-50), which the
+ * reference leaves to its BLAS.
+ *   FWP_MM_NT: C = A B^T, A [M,K], B [N,K]      FWP_MM_NN: C = A B, A [M,K], B [K,N]
+ *   FWP_MM_TN: C = A^T B, A [K,M], B [K,N]      row-major, rows lda, ldb, ldc floats apart
+ * epi (NULL: none): C = relu(C + bias) + residual where gate > 0, 0 elsewhere, each part optional; residual and
+ * gate are laid out like C.  colsum (FWP_MM_TN): [M], the sums of A's columns (a bias gradient).
+ * workspace: fwp_matmul_workspace(M, N, K) floats, or NULL (a product with few tiles and a long K then runs on fewer CUs).
+ */
+enum { FWP_MM_NT = 0, FWP_MM_NN = 1, FWP_MM_TN = 2 };
+typedef struct fwp_mm_epilogue {
+    const float *bias, *residual, *gate;
+    float *colsum;
+    int relu;
+} fwp_mm_epilogue;
+long long fwp_matmul_workspace(int M, int N, int K);
+int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C,
+               long long ldc, int M, int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream);
+
+/*
+ * Per-row negative log-likelihood under softmax(x W^T + bias) (language_modeling/src/model_main.py:1333-1361 without
+ * clusters): x [rows,dim], W [vocab,dim], bias [vocab], target [rows] (negative: the row is ignored), loss [rows].
+ * Saved for backward, both or none: logits [rows,vocab], lse [rows].  workspace: fwp_nll_workspace(rows, vocab) floats.
+ */
+long long fwp_nll_workspace(int rows, int vocab);
+int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits,
+                float *loss, float *lse, float *workspace, int rows, int vocab, int dim, void *stream);
+
+/* Its adjoint: gloss [rows] to gx [rows,dim], gW [vocab,dim], gbias [vocab] (each may be NULL; gbias comes with gW).
+ * workspace: the larger of fwp_matmul_workspace(rows, dim, vocab) and fwp_matmul_workspace(vocab, dim, rows). */
+int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
+                const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows,
+                int vocab, int dim, void *stream);
+
+/*
+ * LayerNorm of the layers (utils/model_utils.py:52-66, cuda_fast_weight_layer.py:168-176): y = (x - mean) rstd gamma +
+ * beta over rows of `cols` floats (a multiple of 4 up to 1024).  stats [rows,2] (mean, rstd) may be NULL.
+ */
+int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats,
+                       int rows, int cols, float eps, void *stream);
+
+/* Its adjoint; gx = the gradient of x (+ add, when given: the gradient that reaches x by another way).
+ * workspace: fwp_layer_norm_workspace(rows, cols) floats. */
+long long fwp_layer_norm_workspace(int rows, int cols);
+int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma,
+                       const float *add, float *gx, float *ggamma, float *gbeta, float *workspace,
+                       int rows, int cols, void *stream);
+
+/*
  * Recurrent Delta Net forward.  Replaces rec_update_fwm_tanh_forward
  * (algorithmic/rec_update_fwm_tanh/rec_update_fwm_tanh.cu:349-444, kernel :25-345).
  *   qx,kx,vx [N,H,L,D] and bx [N,H,L,1] are pre-activation

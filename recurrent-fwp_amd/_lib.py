@@ -26,11 +26,17 @@ class OutView(ctypes.Structure):
                 ("sL", ctypes.c_int64)]
 
 
+class Epilogue(ctypes.Structure):
+    """struct fwp_mm_epilogue: what a matrix product does to its result (device addresses, None: not wanted)."""
+    _fields_ = [("bias", ctypes.c_void_p), ("residual", ctypes.c_void_p), ("gate", ctypes.c_void_p),
+                ("colsum", ctypes.c_void_p), ("relu", ctypes.c_int)]
+
+
 class FwpError(RuntimeError):
     pass
 
 
-_P, _I, _V = ctypes.c_void_p, ctypes.c_int, View
+_P, _I, _V, _L = ctypes.c_void_p, ctypes.c_int, View, ctypes.c_longlong
 _VP = ctypes.POINTER(View)          # host array of views (one per gate)
 _SIGNATURES = {
     "fwp_delta_fwd": [_V] * 4 + [_P] * 4 + [_I] * 6 + [_P],
@@ -48,7 +54,17 @@ _SIGNATURES = {
     "fwp_rec_bwd": [_P] * 6 + [_V] + [_P] * 14 + [_I] * 5 + [_P],
     "fwp_rec_bwd_static": [_P] * 6 + [_V] + [_P] * 13 + [_I] * 5 + [_P],
 }
-EXPORTS = sorted(list(_SIGNATURES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",
+# The language model's kernels, which the C++ blocks call; bound here for tests where the library has them (the
+# stand-in library of the host tests does not).
+_MODEL_SIGNATURES = {
+    "fwp_matmul": [_I, _P, _L, _P, _L, _P, _L] + [_I] * 3 + [_P] * 3,
+    "fwp_nll_fwd": [_P] * 8 + [_I] * 3 + [_P],
+    "fwp_nll_bwd": [_P] * 10 + [_I] * 3 + [_P],
+    "fwp_layer_norm_fwd": [_P] * 5 + [_I] * 2 + [ctypes.c_float, _P],
+    "fwp_layer_norm_bwd": [_P] * 9 + [_I] * 2 + [_P],
+}
+_WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
+EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",
                                        "fwp_delta_ckpt_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
 KIND_LDS, KIND_SCAN, KIND_CHUNKED, KIND_SPLIT, KIND_PHASE, KIND_STEP = 0, 1, 2, 3, 4, 5
 CFG_DELTA_KERNELS, DELTA_AUTO, DELTA_SCAN, DELTA_CHUNKED, DELTA_SPLIT, DELTA_PHASE = 0, 0, 1, 2, 3, 4
@@ -78,6 +94,13 @@ def lib():
         handle.fwp_check_device.restype = ctypes.c_int
         handle.fwp_delta_ckpt_floats.argtypes = [ctypes.c_int] * 6
         handle.fwp_delta_ckpt_floats.restype = ctypes.c_longlong
+        for name, argtypes in _MODEL_SIGNATURES.items():
+            if hasattr(handle, name):
+                getattr(handle, name).argtypes = argtypes
+        for name, n in _WORKSPACES.items():
+            if hasattr(handle, name):
+                getattr(handle, name).argtypes = [ctypes.c_int] * n
+                getattr(handle, name).restype = ctypes.c_longlong
         handle.fwp_delta_kind.argtypes = [_I] + [_V] * 4 + [_I] * 5
         handle.fwp_delta_kind.restype = ctypes.c_int
         handle.fwp_delta_fwd_kind.argtypes = [_V] * 4 + [OutView] + [_I] * 6

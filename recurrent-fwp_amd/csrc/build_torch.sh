@@ -17,7 +17,7 @@ g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden \
     -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -DTORCH_EXTENSION_NAME=_fwp_torch -DTORCH_API_INCLUDE_EXTENSION_H \
     -D_GLIBCXX_USE_CXX11_ABI="$CXX11" \
     ${TORCH_INC//,/ } -I"$PY_INC" -I/opt/rocm/include -I"$root/include" \
-    "$here"/fwp_torch.cpp \
+    "$here"/fwp_torch.cpp "$here"/fwp_torch_blocks.cpp \
     -L"$TORCH_LIB" -ltorch -ltorch_cpu -ltorch_python -lc10 -lc10_hip \
     -L"$pkg" -lfwp_hip -Wl,-rpath,'$ORIGIN' \
     -o "$pkg/_fwp_torch.so" "$@"

@@ -387,6 +387,68 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
     return deltanet_prep_bwd(qkvb, gq, gk, gv, gbeta, gqkvb, T, B, H, D, q_scale, (hipStream_t)stream);
 }
 
+long long fwp_matmul_workspace(int M, int N, int K) {
+    return M < 1 || N < 1 || K < 1 ? FWP_E_SHAPE : matmul_workspace(M, N, K);
+}
+
+// rows further apart than this could leave the 32-bit offsets within a tile
+static bool pitch_ok(long long ld, long long least) { return ld >= least && ld <= (1 << 21); }
+
+int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C, long long ldc,
+               int M, int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream) {
+    if (!A || !B || !C) return FWP_E_NULL;
+    if (M < 1 || N < 1 || K < 1 || layout < FWP_MM_NT || layout > FWP_MM_TN) return FWP_E_SHAPE;
+    if (!pitch_ok(lda, layout == FWP_MM_TN ? M : K) || !pitch_ok(ldb, layout == FWP_MM_NT ? K : N) || ldc < N)
+        return FWP_E_SHAPE;
+    const fwp_mm_epilogue none = {};
+    return matmul(layout, A, lda, B, ldb, C, ldc, M, N, K, epi ? *epi : none, workspace, nullptr, (hipStream_t)stream);
+}
+
+long long fwp_nll_workspace(int rows, int vocab) {
+    return rows < 1 || vocab < 1 ? FWP_E_SHAPE : nll_workspace(rows, vocab);
+}
+
+int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                float *lse, float *workspace, int rows, int vocab, int dim, void *stream) {
+    if (!x || !W || !target || !loss || !workspace || (logits == nullptr) != (lse == nullptr)) return FWP_E_NULL;
+    if (rows < 1 || vocab < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1)) return FWP_E_SHAPE;
+    return nll_fwd(x, W, bias, target, logits, loss, lse, workspace, rows, vocab, dim, (hipStream_t)stream);
+}
+
+int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
+                const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
+                void *stream) {
+    if (!x || !W || !logits || !lse || !target || !gloss || (gbias && !gW)) return FWP_E_NULL;
+    if (rows < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1)) return FWP_E_SHAPE;
+    const NllView nll = {lse, gloss, target};
+    fwp_mm_epilogue epi = {};
+    if (gx)
+        if (int rc = matmul(FWP_MM_NN, logits, vocab, W, dim, gx, dim, rows, dim, vocab, epi, workspace, &nll,
+                            (hipStream_t)stream))
+            return rc;
+    if (!gW) return 0;
+    epi.colsum = gbias;
+    return matmul(FWP_MM_TN, logits, vocab, x, dim, gW, dim, vocab, dim, rows, epi, workspace, &nll, (hipStream_t)stream);
+}
+
+int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows,
+                       int cols, float eps, void *stream) {
+    if (!x || !gamma || !beta || !y) return FWP_E_NULL;
+    if (rows < 1 || !layer_norm_supported(cols)) return FWP_E_SHAPE;
+    return layer_norm_fwd(x, gamma, beta, y, stats, rows, cols, eps, (hipStream_t)stream);
+}
+
+long long fwp_layer_norm_workspace(int rows, int cols) {
+    return rows < 1 || cols < 1 ? FWP_E_SHAPE : layer_norm_workspace(rows, cols);
+}
+
+int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, const float *add,
+                       float *gx, float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream) {
+    if (!gy || !x || !stats || !gamma || !gx || !ggamma || !gbeta || !workspace) return FWP_E_NULL;
+    if (rows < 1 || !layer_norm_supported(cols)) return FWP_E_SHAPE;
+    return layer_norm_bwd(gy, x, stats, gamma, add, gx, ggamma, gbeta, workspace, rows, cols, (hipStream_t)stream);
+}
+
 int fwp_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float *Rq,
                 const float *Rk, const float *Rv, const float *rb, float *W, float *h, float *out,
                 float *q_act, float *k_act, float *beta_act, float *vdiff, float *ckpt, int N,

@@ -185,6 +185,27 @@ int deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *be
 int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,
                       const float *gbeta, float *gqkvb, int T, int B, int H, int D, float q_scale, hipStream_t s);
 
+// fp32 matrix products on the bf16 matrix cores (fwp_matmul); `nll`: A holds logits and stands for the gradient of
+// the loss that nll_fwd computed from them.
+struct NllView {
+    const float *lse, *gloss;
+    const int64_t *target;
+};
+int64_t matmul_workspace(int M, int N, int K);
+int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
+           int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s);
+int64_t nll_workspace(int rows, int vocab);
+int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+            float *lse, float *workspace, int rows, int vocab, int dim, hipStream_t s);
+
+// LayerNorm over rows of up to 1024 floats (a multiple of 4) and its adjoint.
+bool layer_norm_supported(int cols);
+int64_t layer_norm_workspace(int rows, int cols);
+int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows, int cols,
+                   float eps, hipStream_t s);
+int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, const float *add, float *gx,
+                   float *ggamma, float *gbeta, float *workspace, int rows, int cols, hipStream_t s);
+
 // Largest dynamic LDS allocation the LDS-state kernels ask for (bytes).
 constexpr size_t kMaxLds = 160 * 1024 - 1024;
 

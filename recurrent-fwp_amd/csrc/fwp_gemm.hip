@@ -1,0 +1,499 @@
+// fp32 matrix products of the language model's layers on the bf16 matrix cores.
+//
+// An fp32 number is the sum of three bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest:
+// 3 x 8 significant bits and their signs hold all 24), so a product of two fp32 numbers is the sum of nine bf16
+// products.  Six of them are formed, h h', h m', m h', m m', h l', l h'; the three left out are below
+// 2^-26 |x x'|, a quarter of the rounding of an fp32 product.  Sums are fp32, six roundings per 32 terms where a
+// chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm): 2.2e-7 at K = 256,
+// 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling, no overflow but that of the operands (an
+// infinite operand gives NaN where an fp32 product gives infinity or NaN).
+//
+// v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
+// the 32x32x16 form 1.8), i.e. 350 TFLOP/s of such fp32 products, where the fp32 matrix instructions make 155.
+// The operands are split on their way from global memory to LDS, in the registers of the thread that loads
+// them: 11 vector instructions per two numbers, 45 % of the matrix instructions' time in a 128 x 128 tile, and
+// issued beside them by the other workgroups of the CU.  LDS holds 16-byte units of 8 consecutive k of one row,
+// [plane][k / 8][row], so that a fragment is one ds_read_b128 of consecutive addresses; an operand that is
+// contiguous along its rows instead of along k is transposed in registers on the way.
+#include "fwp_common.hpp"
+#include "fwp_mfma.hpp"
+
+namespace fwp {
+namespace {
+
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+__device__ v2f llvm_raw_buffer_load_v2f32(v4i rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
+
+constexpr int kBK = 32;          // k per LDS tile
+constexpr int kPad = 2;          // units after a k-chunk's rows: the chunks of a row start 32 bytes apart in the banks
+constexpr int kThreads = 256;
+constexpr unsigned kOut = 0x80000000u;      // an offset beyond every buffer: reads as zero
+
+__device__ __forceinline__ unsigned pack2(float a, float b) {
+    const bf2 r = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(unsigned, r);
+}
+__device__ __forceinline__ float low_f(unsigned u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float high_f(unsigned u) { return __uint_as_float(u & 0xffff0000u); }
+
+__device__ __forceinline__ v4i buffer_of(const float *base, int64_t floats) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)((a >> 32) & 0xffff), (int)(uint32_t)(floats * 4), 0x00020000};
+}
+
+template <int ROWS>
+struct Planes {
+    v4u u[3][kBK / 8][ROWS + kPad];
+};
+
+// What turns stored logits into the gradient of the loss as an operand is loaded:
+// (exp(logit - lse[token]) - [vocabulary entry == target[token]]) * gloss[token], 0 for a negative target
+struct NllArgs {
+    const float *lse, *gloss;
+    const int64_t *target;
+};
+
+__device__ __forceinline__ float nll_grad(float logit, float lse, float g, bool hit) {
+    return (__expf(logit - lse) - (hit ? 1.f : 0.f)) * g;
+}
+
+// One operand's share of the loads and LDS writes of a thread.  KC: rows are contiguous along k; a task is 8
+// consecutive k of one row (two 16-byte loads, one unit per plane).  Otherwise contiguous along the rows; a
+// task is VEC consecutive rows x 8 k (8 loads, VEC units per plane).
+// NLL: the operand is the loss gradient, formed from the logits; tokens are the rows (KC) or k.
+template <bool KC, int ROWS, bool NLL>
+struct Operand {
+    static constexpr int kChunks = kBK / 8;
+    static constexpr int VEC = KC ? 1 : ROWS * kChunks / kThreads;          // 2 at 128 rows, 1 at 64
+    static constexpr int kTasks = KC ? ROWS * kChunks / kThreads : 1;
+    static_assert(KC ? kTasks >= 1 : (VEC == 1 || VEC == 2), "a whole number of tasks per thread");
+    float x[kTasks][8 * VEC];
+    unsigned off[kTasks];
+    float lse[NLL && KC ? kTasks : 1], gl[NLL && KC ? kTasks : 1];
+    int hit[NLL && KC ? kTasks : 1];
+
+    static __device__ __forceinline__ int row_of(int t) { return KC ? t / kChunks : (t % (ROWS / VEC)) * VEC; }
+    static __device__ __forceinline__ int chunk_of(int t) { return KC ? t % kChunks : t / (ROWS / VEC); }
+
+    __device__ __forceinline__ void init(int tid, int64_t ld, int row0, int rows, const NllArgs &nll) {
+#pragma unroll
+        for (int i = 0; i < kTasks; i++) {
+            const int r = row_of(tid + i * kThreads), c = chunk_of(tid + i * kThreads);
+            off[i] = (unsigned)(KC ? r * ld + 8 * c : 8 * c * ld + r) * 4;
+            if constexpr (NLL && KC) {
+                const int t = min(row0 + r, rows - 1);
+                lse[i] = nll.lse[t];
+                hit[i] = (int)nll.target[t];
+                gl[i] = hit[i] >= 0 ? nll.gloss[t] : 0.f;
+            }
+        }
+    }
+    // P: the tile's first row at k = 0, `left` rows from there, k0 .. min(k0 + kBK, K)
+    __device__ __forceinline__ void load(const float *P, int64_t ld, int left, int tid, int k0, int K) {
+        if constexpr (KC) {
+            const v4i rs = buffer_of(P + k0, (int64_t)(min(left, ROWS) - 1) * ld + (K - k0));
+#pragma unroll
+            for (int i = 0; i < kTasks; i++) {
+                const int k = k0 + 8 * chunk_of(tid + i * kThreads);
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)(k < K ? off[i] : kOut), 0, 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)(k + 4 < K ? off[i] + 16 : kOut), 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[i][j] = a[j], x[i][4 + j] = b[j];
+            }
+        } else {
+            const v4i rs = buffer_of(P + (int64_t)k0 * ld, (int64_t)(min(K - k0, kBK) - 1) * ld + left);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if constexpr (VEC == 1) {
+                    x[0][j] = llvm_raw_buffer_load_f32(rs, (int)off[0], (int)(j * ld * 4), 0);
+                } else {
+                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)off[0], (int)(j * ld * 4), 0);
+                    x[0][j] = a[0], x[0][8 + j] = a[1];
+                }
+            }
+        }
+    }
+    // What load() brought: zeros beyond K (a row contiguous along k runs on into the next row there), and the
+    // loss gradient in place of the logits
+    __device__ __forceinline__ void finish(int tid, int row0, int k0, int K, const NllArgs &nll) {
+        if constexpr (KC) {
+            const bool tail = k0 + kBK > K;
+#pragma unroll
+            for (int i = 0; i < kTasks; i++) {
+                const int k = k0 + 8 * chunk_of(tid + i * kThreads);
+                if constexpr (NLL)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) x[i][j] = nll_grad(x[i][j], lse[i], gl[i], hit[i] == k + j);
+                if (tail)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) x[i][j] = k + j < K ? x[i][j] : 0.f;
+            }
+        } else if constexpr (NLL) {
+            const int k = k0 + 8 * chunk_of(tid), r = row0 + row_of(tid);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int t = min(k + j, K - 1), h = (int)nll.target[t];
+                const float l = nll.lse[t], g = k + j < K && h >= 0 ? nll.gloss[t] : 0.f;
+#pragma unroll
+                for (int c = 0; c < VEC; c++) x[0][8 * c + j] = nll_grad(x[0][8 * c + j], l, g, h == r + c);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(Planes<ROWS> &L, int tid) const {
+#pragma unroll
+        for (int i = 0; i < kTasks; i++)
+#pragma unroll
+            for (int c = 0; c < VEC; c++) {
+                v4u h, m, l;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float a = x[i][8 * c + 2 * j], b = x[i][8 * c + 2 * j + 1];
+                    h[j] = pack2(a, b);
+                    const float ra = a - low_f(h[j]), rb = b - high_f(h[j]);
+                    m[j] = pack2(ra, rb);
+                    l[j] = pack2(ra - low_f(m[j]), rb - high_f(m[j]));
+                }
+                const int r = row_of(tid + i * kThreads) + c, ch = chunk_of(tid + i * kThreads);
+                L.u[0][ch][r] = h;
+                L.u[1][ch][r] = m;
+                L.u[2][ch][r] = l;
+            }
+    }
+};
+
+struct GemmArgs {
+    const float *A, *B;
+    float *C;                    // the result, or (several k ranges) one M x N partial result per range
+    int64_t lda, ldb, ldc;
+    int M, N, K;
+    int ks;                      // k per range (a multiple of kBK)
+    int tm, tn;                  // tiles
+    float *colsum;               // sums over k of A's rows, per range [M] (A contiguous along its rows), or NULL
+    fwp_mm_epilogue epi;         // applied here when there is one range
+    NllArgs nll;
+    // per tile of columns and row: the largest logit and the sum of exp(logit - largest); logits of the targets
+    float *part_max, *part_sum, *hit;
+};
+
+enum { kPlain = 0, kLse = 1, kGrad = 2 };
+
+__device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_t at, int n) {
+    if (e.bias) x += e.bias[n];
+    if (e.relu) x = fmaxf(x, 0.f);
+    if (e.residual) x += e.residual[at];
+    if (e.gate) x = e.gate[at] > 0.f ? x : 0.f;
+    return x;
+}
+
+template <int X>
+__device__ __forceinline__ float row16_max(float x) {      // over the 16 lanes of a DPP row
+    return fmaxf(x, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true)));
+}
+template <int X>
+__device__ __forceinline__ float row16_add(float x) {
+    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true));
+}
+
+// BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
+template <bool AKC, bool BKC, int BM, int BN, int MODE>
+__global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
+    constexpr int WM = BM / 2, WN = BN / 2, MT = WM / 16, NT = WN / 16;
+    __shared__ Planes<BM> La;
+    __shared__ Planes<BN> Lb;
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int wm = (wave % 2) * WM, wn = (wave / 2) * WN;
+    // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
+    // rows of A, through that XCD's L2)
+    const int total = g.tm * g.tn, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
+    const int id = xcd * each + min(xcd, rest) + blockIdx.x / 8;
+    const int m0 = (id / g.tn) * BM, n0 = (id % g.tn) * BN;
+    const int kb = blockIdx.y * g.ks, ke = min(g.K, kb + g.ks);
+    Operand<AKC, BM, MODE == kGrad> a;
+    Operand<BKC, BN, false> b;
+    a.init(tid, g.lda, m0, g.M, g.nll);
+    b.init(tid, g.ldb, n0, g.N, g.nll);
+    const float *Ap = AKC ? g.A + (int64_t)m0 * g.lda : g.A + m0;
+    const float *Bp = BKC ? g.B + (int64_t)n0 * g.ldb : g.B + n0;
+    const int ml = g.M - m0, nl = g.N - n0;
+    constexpr int CV = AKC ? 1 : Operand<AKC, BM, MODE == kGrad>::VEC;
+    float csum[CV];
+#pragma unroll
+    for (int c = 0; c < CV; c++) csum[c] = 0.f;
+    const bool sums = !AKC && g.colsum && n0 == 0;
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    const int lr = lane % 16, lc = lane / 16;
+    a.load(Ap, g.lda, ml, tid, kb, ke);
+    b.load(Bp, g.ldb, nl, tid, kb, ke);
+    for (int k0 = kb; k0 < ke; k0 += kBK) {
+        a.finish(tid, m0, k0, ke, g.nll);
+        b.finish(tid, n0, k0, ke, g.nll);
+        if constexpr (!AKC) {
+            if (sums)
+#pragma unroll
+                for (int c = 0; c < CV; c++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) csum[c] += a.x[0][8 * c + j];
+        }
+        a.store(La, tid);
+        b.store(Lb, tid);
+        lds_barrier();
+        if (k0 + kBK < ke) {
+            a.load(Ap, g.lda, ml, tid, k0 + kBK, ke);
+            b.load(Bp, g.ldb, nl, tid, k0 + kBK, ke);
+        }
+        bf8 fa[3][MT], fb[3][NT];
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+#pragma unroll
+            for (int i = 0; i < MT; i++) fa[p][i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lr]);
+#pragma unroll
+            for (int j = 0; j < NT; j++) fb[p][j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lr]);
+        }
+        // the small products first
+        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int q = 0; q < 6; q++)
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[PA[q]][i], fb[PB[q]][j], acc[i][j], 0, 0, 0);
+        lds_barrier();
+    }
+
+    // acc[i][j][r] = C[m0 + wm + 16 i + 4 lc + r][n0 + wn + 16 j + lr]
+    if constexpr (!AKC) {
+        if (sums) {      // the threads of a row pair's four k-chunks
+            float *s = reinterpret_cast<float *>(&La);
+            using Op = Operand<AKC, BM, MODE == kGrad>;
+#pragma unroll
+            for (int c = 0; c < CV; c++) s[Op::chunk_of(tid) * BM + Op::row_of(tid) + c] = csum[c];
+            __syncthreads();
+            for (int r = tid; r < min(BM, ml); r += kThreads)
+                g.colsum[(int64_t)blockIdx.y * g.M + m0 + r] = (s[r] + s[BM + r]) + (s[2 * BM + r] + s[3 * BM + r]);
+        }
+    }
+    if constexpr (MODE == kLse) {
+        float *sm = reinterpret_cast<float *>(&La), *ss = sm + 2 * BM;      // [column half][row]
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int row = wm + 16 * i + 4 * lc + r, m = m0 + row;
+                const int want = (int)g.nll.target[min(m, g.M - 1)];
+                float mx = -INFINITY;
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const int n = n0 + wn + 16 * j + lr;
+                    if (n < g.N && g.epi.bias) acc[i][j][r] += g.epi.bias[n];
+                    if (n >= g.N) acc[i][j][r] = -INFINITY;
+                    if (m < g.M && n == want) g.hit[m] = acc[i][j][r];
+                    mx = fmaxf(mx, acc[i][j][r]);
+                }
+                mx = row16_max<1>(row16_max<2>(row16_max<4>(row16_max<8>(mx))));
+                float s = 0.f;
+#pragma unroll
+                for (int j = 0; j < NT; j++) s += mx == -INFINITY ? 0.f : __expf(acc[i][j][r] - mx);
+                s = row16_add<1>(row16_add<2>(row16_add<4>(row16_add<8>(s))));
+                if (lr == 0) {
+                    sm[(wave / 2) * BM + row] = mx;
+                    ss[(wave / 2) * BM + row] = s;
+                }
+            }
+        __syncthreads();
+        for (int row = tid; row < min(BM, ml); row += kThreads) {
+            const float m1 = sm[row], m2 = sm[BM + row], mx = fmaxf(m1, m2);
+            const float s = ss[row] * __expf(m1 - mx) + (m2 == -INFINITY ? 0.f : ss[BM + row] * __expf(m2 - mx));
+            const int64_t at = (int64_t)(id % g.tn) * g.M + m0 + row;
+            g.part_max[at] = mx;
+            g.part_sum[at] = s;
+        }
+        if (!g.C) return;
+    }
+    float *C = g.C + (int64_t)blockIdx.y * g.M * g.ldc;
+    const bool one = gridDim.y == 1 && MODE != kLse;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const int n = n0 + wn + 16 * j + lr;
+            if (n >= g.N) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = m0 + wm + 16 * i + 4 * lc + r;
+                if (m >= g.M) continue;
+                const int64_t at = (int64_t)m * g.ldc + n;
+                C[at] = one ? apply(g.epi, acc[i][j][r], at, n) : acc[i][j][r];
+            }
+        }
+}
+
+// C[M,N] = the sum of `ranges` partial results, with the epilogue; four threads share four neighbouring
+// elements, a quarter of the ranges each, and add up in a fixed order.
+__global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restrict__ part, float *__restrict__ C,
+                                                          int64_t total, int N, int ranges, fwp_mm_epilogue epi) {
+    __shared__ float4 s[4][64];
+    const int e = threadIdx.x % 64, q = threadIdx.x / 64;
+    const int64_t at = ((int64_t)blockIdx.x * 64 + e) * 4;
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (at < total)
+        for (int r = q; r < ranges; r += 4) {
+            const float4 y = *reinterpret_cast<const float4 *>(part + r * total + at);
+            x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
+        }
+    s[q][e] = x;
+    __syncthreads();
+    if (q || at >= total) return;
+    for (int o = 1; o < 4; o++) {
+        const float4 y = s[o][e];
+        x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
+    }
+    const int n = (int)(at % N);
+    float4 y;
+    y.x = apply(epi, x.x, at, n), y.y = apply(epi, x.y, at + 1, n + 1);
+    y.z = apply(epi, x.z, at + 2, n + 2), y.w = apply(epi, x.w, at + 3, n + 3);
+    *reinterpret_cast<float4 *>(C + at) = y;
+}
+
+__global__ __launch_bounds__(kThreads) void k_sum_ranges(const float *__restrict__ part, float *__restrict__ out, int n,
+                                                         int ranges) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= n) return;
+    float x = 0.f;
+    for (int r = 0; r < ranges; r++) x += part[(int64_t)r * n + i];
+    out[i] = x;
+}
+
+struct Plan {
+    bool wide;           // 128 x 128 tiles, else 64 x 64
+    int tm, tn, ranges, ks;
+};
+
+// 128 x 128 tiles where they fill the chip (two workgroups on each of 256 CUs) or where k can be cut into ranges
+// until they do; the partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k.
+// Without ranges to cut, fewer tiles than CUs: 64 x 64.
+Plan plan_of(int M, int N, int K, bool may_cut) {
+    Plan p;
+    const auto tiles = [&](int b) { return (int64_t)((M + b - 1) / b) * ((N + b - 1) / b); };
+    p.wide = tiles(128) >= 256 || (may_cut && tiles(128) * (K / 256) >= 256);
+    const int b = p.wide ? 128 : 64;
+    p.tm = (M + b - 1) / b;
+    p.tn = (N + b - 1) / b;
+    int64_t ranges = 1;
+    if (may_cut) {
+        ranges = 512 / (tiles(b));
+        if (ranges > K / 256) ranges = K / 256;
+        if (ranges < 1) ranges = 1;
+    }
+    p.ks = (int)((K + ranges - 1) / ranges + kBK - 1) / kBK * kBK;
+    p.ranges = (K + p.ks - 1) / p.ks;
+    return p;
+}
+
+template <bool AKC, bool BKC, int MODE>
+void launch(const GemmArgs &g, const Plan &p, hipStream_t s) {
+    const dim3 grid((unsigned)(p.tm * p.tn), (unsigned)p.ranges);
+    if (p.wide) hipLaunchKernelGGL((k_gemm<AKC, BKC, 128, 128, MODE>), grid, dim3(kThreads), 0, s, g);
+    else hipLaunchKernelGGL((k_gemm<AKC, BKC, 64, 64, MODE>), grid, dim3(kThreads), 0, s, g);
+}
+
+bool may_cut(int N, const float *C, int64_t ldc) {
+    return ldc == N && N % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+}
+
+}  // namespace
+
+int64_t matmul_workspace(int M, int N, int K) {
+    const Plan p = plan_of(M, N, K, N % 4 == 0);
+    return p.ranges > 1 ? (int64_t)p.ranges * ((int64_t)M * N + M) : 0;
+}
+
+int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
+           int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s) {
+    GemmArgs g{};
+    g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
+    if (nll) g.nll = NllArgs{nll->lse, nll->gloss, nll->target};
+    const Plan p = plan_of(M, N, K, workspace && may_cut(N, C, ldc));
+    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
+    const bool cut = p.ranges > 1;
+    g.C = cut ? workspace : C;
+    g.ldc = cut ? N : ldc;
+    float *const col = cut ? workspace + (int64_t)p.ranges * M * N : epi.colsum;
+    g.colsum = layout == FWP_MM_TN && epi.colsum ? col : nullptr;
+    if (layout == FWP_MM_NT) launch<true, true, kPlain>(g, p, s);
+    else if (layout == FWP_MM_NN && !nll) launch<true, false, kPlain>(g, p, s);
+    else if (layout == FWP_MM_NN) launch<true, false, kGrad>(g, p, s);
+    else if (!nll) launch<false, false, kPlain>(g, p, s);
+    else launch<false, false, kGrad>(g, p, s);
+    if (cut) {
+        const int64_t total = (int64_t)M * N;
+        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((total / 4 + 63) / 64)), dim3(kThreads), 0, s, workspace, C, total,
+                           N, p.ranges, epi);
+        if (g.colsum)
+            hipLaunchKernelGGL(k_sum_ranges, dim3((M + kThreads - 1) / kThreads), dim3(kThreads), 0, s, col, epi.colsum, M,
+                               p.ranges);
+    }
+    return (int)hipGetLastError();
+}
+
+namespace {
+
+// loss = lse - logit of the target (0 for a negative target), lse from the tiles' maxima and sums; four threads
+// share a row, a quarter of the tiles each
+__global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part_max, const float *__restrict__ part_sum,
+                                                  const float *__restrict__ hit, const int64_t *__restrict__ target,
+                                                  float *__restrict__ loss, float *__restrict__ lse, int rows, int vocab,
+                                                  int tiles) {
+    __shared__ float sm[4][64], ss[4][64];
+    const int e = threadIdx.x % 64, q = threadIdx.x / 64, m = blockIdx.x * 64 + e;
+    float mx = -INFINITY, s = 0.f;
+    if (m < rows)
+        for (int t = q; t < tiles; t += 4) {
+            const float x = part_max[(int64_t)t * rows + m], y = part_sum[(int64_t)t * rows + m], big = fmaxf(mx, x);
+            s = (mx == -INFINITY ? 0.f : s * __expf(mx - big)) + y * __expf(x - big);
+            mx = big;
+        }
+    sm[q][e] = mx;
+    ss[q][e] = s;
+    __syncthreads();
+    if (q || m >= rows) return;
+    for (int o = 1; o < 4; o++) {
+        const float x = sm[o][e], big = fmaxf(mx, x);
+        s = s * __expf(mx - big) + (x == -INFINITY ? 0.f : ss[o][e] * __expf(x - big));
+        mx = big;
+    }
+    const float l = mx + __logf(s);
+    const int64_t want = target[m];
+    if (lse) lse[m] = l;
+    loss[m] = want < 0 ? 0.f : want < vocab ? l - hit[m] : NAN;
+}
+
+}  // namespace
+
+int64_t nll_workspace(int rows, int vocab) { return (int64_t)((vocab + 63) / 64) * rows * 2 + rows; }
+
+int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+            float *lse, float *workspace, int rows, int vocab, int dim, hipStream_t s) {
+    GemmArgs g{};
+    g.A = x, g.B = W, g.lda = dim, g.ldb = dim, g.M = rows, g.N = vocab, g.K = dim, g.C = logits, g.ldc = vocab;
+    g.epi.bias = bias;
+    g.nll.target = target;
+    const Plan p = plan_of(rows, vocab, dim, false);
+    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
+    g.part_max = workspace;
+    g.part_sum = workspace + (int64_t)p.tn * rows;
+    g.hit = g.part_sum + (int64_t)p.tn * rows;
+    launch<true, true, kLse>(g, p, s);
+    hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, target, loss, lse,
+                       rows, vocab, p.tn);
+    return (int)hipGetLastError();
+}
+
+}  // namespace fwp

@@ -1,0 +1,305 @@
+// The Delta-Net language model's blocks as C++ autograd functions over the C ABI: the feed-forward block, the
+// Delta-Net layer's projections around the delta rule, LayerNorm, and the softmax's negative log-likelihood
+// (reference: language_modeling/src/utils/model_utils.py:34-67, cuda_fast_weight_layer.py:57-188,
+// model_main.py:1333-1361).  Biases, ReLU and its mask, residual additions and bias gradients happen inside the
+// matrix products (fwp_matmul's epilogue), so a block is its products and nothing else.  Host code only.
+//
+// A backward pass that is itself to be differentiated (create_graph) recomputes the block from PyTorch's own
+// operators and differentiates that.
+#include "fwp_torch.hpp"
+
+#include <optional>
+#include <tuple>
+#include <vector>
+
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+at::Tensor given(const std::optional<at::Tensor> &t) { return t.has_value() ? *t : at::Tensor(); }
+
+float *ptr(const at::Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
+
+// fp32, contiguous, 16-byte aligned
+at::Tensor plain(const at::Tensor &t) {
+    if (t.scalar_type() != at::kFloat) fail("fp32 tensors only");
+    if (!t.is_contiguous()) return t.contiguous();
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
+}
+
+// C = op(A) op(B) with an epilogue, shaped `shape` (M x N elements)
+at::Tensor matmul(int layout, const at::Tensor &A, const at::Tensor &B, int64_t M, int64_t N, int64_t K, at::IntArrayRef shape,
+                  const fwp_mm_epilogue &epi = {}) {
+    at::Tensor C = at::empty(shape, A.options()), work;
+    const int64_t n = fwp_matmul_workspace((int)M, (int)N, (int)K);
+    if (n > 0) work = at::empty({n}, A.options());
+    check(fwp_matmul(layout, ptr(A), layout == FWP_MM_TN ? M : K, ptr(B), layout == FWP_MM_NT ? K : N, ptr(C), N, (int)M,
+                     (int)N, (int)K, &epi, ptr(work), stream_of(A)),
+          "fwp_matmul");
+    return C;
+}
+
+// Gradients of the weights of y = x W^T + bias from g = dy: g^T x, and the columns of g summed
+at::Tensor weight_grad(const at::Tensor &g, const at::Tensor &x, int64_t rows, int64_t out, int64_t in, float *colsum) {
+    fwp_mm_epilogue e{};
+    e.colsum = colsum;
+    return matmul(FWP_MM_TN, g, x, out, in, rows, {out, in}, e);
+}
+
+at::Tensor bias_like(int64_t n, const at::Tensor &x, bool want) { return want ? at::empty({n}, x.options()) : at::Tensor(); }
+
+variable_list differentiate(const at::Tensor &y, const variable_list &inputs, const at::Tensor &g) {
+    variable_list used, res(inputs.size());
+    for (const at::Tensor &t : inputs)
+        if (t.defined() && t.requires_grad()) used.push_back(t);
+    if (used.empty()) return res;
+    const variable_list grads = torch::autograd::grad({y}, used, {g}, std::nullopt, /*create_graph=*/true, /*allow_unused=*/true);
+    for (size_t i = 0, j = 0; i < inputs.size(); i++)
+        if (inputs[i].defined() && inputs[i].requires_grad()) res[i] = grads[j++];
+    return res;
+}
+
+// ------------------------------------------------------------------ y = x W^T (+ bias) (relu)
+
+struct LinearFn : torch::autograd::Function<LinearFn> {
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &W,
+                              const std::optional<at::Tensor> &bias_in, bool relu) {
+        const at::Tensor bias = given(bias_in);
+        require_device(x_in);
+        same_device(x_in, {W, bias});
+        const int64_t in = W.size(1), out = W.size(0), rows = x_in.numel() / in;
+        const at::Tensor x = plain(x_in);
+        std::vector<int64_t> shape = x.sizes().vec();
+        shape.back() = out;
+        LaunchGuard guard(x);
+        fwp_mm_epilogue e{};
+        e.bias = ptr(bias);
+        e.relu = relu;
+        const at::Tensor y = matmul(FWP_MM_NT, x, W, rows, out, in, shape, e);
+        if (ctx) {
+            ctx->save_for_backward({x_in, W, bias, relu ? y : at::Tensor()});
+            ctx->set_materialize_grads(false);
+        }
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &W = saved[1], &bias = saved[2], &y = saved[3];
+        if (!grads[0].defined()) return variable_list(4);
+        if (at::GradMode::is_enabled()) {
+            at::Tensor z = at::linear(saved[0], W, bias.defined() ? std::optional<at::Tensor>(bias) : std::nullopt);
+            variable_list res = differentiate(y.defined() ? at::relu(z) : z, {saved[0], W, bias}, grads[0]);
+            res.resize(4);
+            return res;
+        }
+        const at::Tensor x = plain(saved[0]);
+        at::Tensor g = plain(grads[0]);
+        if (y.defined()) g = at::threshold_backward(g, y, 0);
+        const int64_t in = W.size(1), out = W.size(0), rows = x.numel() / in;
+        LaunchGuard guard(x);
+        variable_list res(4);
+        if (ctx->needs_input_grad(0)) res[0] = matmul(FWP_MM_NN, g, W, rows, in, out, saved[0].sizes());
+        const bool want_bias = bias.defined() && ctx->needs_input_grad(2);
+        res[2] = bias_like(out, x, want_bias);
+        if (ctx->needs_input_grad(1) || want_bias) res[1] = weight_grad(g, x, rows, out, in, ptr(res[2]));
+        return res;
+    }
+};
+
+// ------------------------------------------------------------------ s = relu(x W1^T + b1) W2^T + b2 (+ residual)
+
+struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
+    // residual: undefined, or added; `same`: it is x (its gradient then joins x's inside the last product)
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &W1, const at::Tensor &b1,
+                              const at::Tensor &W2, const at::Tensor &b2, const std::optional<at::Tensor> &residual_in,
+                              bool same) {
+        const at::Tensor residual = given(residual_in);
+        require_device(x_in);
+        same_device(x_in, {W1, b1, W2, b2, residual});
+        const int64_t d = W1.size(1), inner = W1.size(0), rows = x_in.numel() / d;
+        const at::Tensor x = plain(x_in), res = same ? x : residual.defined() ? plain(residual) : residual;
+        LaunchGuard guard(x);
+        fwp_mm_epilogue e{};
+        e.bias = ptr(b1);
+        e.relu = 1;
+        const at::Tensor hid = matmul(FWP_MM_NT, x, W1, rows, inner, d, {rows, inner}, e);
+        e = {};
+        e.bias = ptr(b2);
+        e.residual = ptr(res);
+        const at::Tensor s = matmul(FWP_MM_NT, hid, W2, rows, d, inner, x_in.sizes(), e);
+        if (ctx) {
+            ctx->save_for_backward({x_in, W1, b1, W2, b2, hid});
+            ctx->saved_data["same"] = same;
+            ctx->saved_data["residual"] = residual.defined();
+            ctx->set_materialize_grads(false);
+        }
+        return s;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        variable_list res(7);
+        if (!grads[0].defined()) return res;
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &W1 = saved[1], &b1 = saved[2], &W2 = saved[3], &b2 = saved[4], &hid = saved[5];
+        const bool same = ctx->saved_data["same"].toBool();
+        if (ctx->saved_data["residual"].toBool() && !same) res[5] = grads[0];
+        if (at::GradMode::is_enabled()) {
+            at::Tensor s = at::linear(at::relu(at::linear(saved[0], W1, b1)), W2, b2);
+            const variable_list g = differentiate(same ? s + saved[0] : s, {saved[0], W1, b1, W2, b2}, grads[0]);
+            std::copy(g.begin(), g.end(), res.begin());
+            return res;
+        }
+        const at::Tensor x = plain(saved[0]), g = plain(grads[0]);
+        const int64_t d = W1.size(1), inner = W1.size(0), rows = x.numel() / d;
+        LaunchGuard guard(x);
+        res[4] = bias_like(d, x, ctx->needs_input_grad(4));
+        if (ctx->needs_input_grad(3) || res[4].defined()) res[3] = weight_grad(g, hid, rows, d, inner, ptr(res[4]));
+        if (!(ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(2))) return res;
+        fwp_mm_epilogue e{};
+        e.gate = ptr(hid);      // the ReLU's gradient: where the activation is positive
+        const at::Tensor gh = matmul(FWP_MM_NN, g, W2, rows, inner, d, {rows, inner}, e);
+        res[2] = bias_like(inner, x, ctx->needs_input_grad(2));
+        if (ctx->needs_input_grad(1) || res[2].defined()) res[1] = weight_grad(gh, x, rows, inner, d, ptr(res[2]));
+        if (ctx->needs_input_grad(0)) {
+            e = {};
+            e.residual = same ? ptr(g) : nullptr;
+            res[0] = matmul(FWP_MM_NN, gh, W1, rows, d, inner, saved[0].sizes(), e);
+        }
+        return res;
+    }
+};
+
+// ------------------------------------------------------------------ s = (x +) o_net(delta rule(qkvb_net(x)))
+
+struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
+    // x [T,B,d]; Wqkvb [H (3D+1), d]; Wo [d, H D]; state [B,H,D,D] in/out
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &Wqkvb, const at::Tensor &Wo,
+                              const at::Tensor &state, int64_t H, int64_t D, double scale, bool residual) {
+        require_device(x_in);
+        same_device(x_in, {Wqkvb, Wo, state});
+        require(x_in.dim() == 3, "expected [len, bsz, d_model]");
+        const int64_t T = x_in.size(0), B = x_in.size(1), d = x_in.size(2), rows = T * B, width = H * (3 * D + 1);
+        require(Wqkvb.size(0) == width && Wqkvb.size(1) == d && Wo.size(1) == H * D && same_shape(state, {B, H, D, D}),
+                "projections and state do not fit the heads");
+        require_state(state, "W");
+        const at::Tensor x = plain(x_in);
+        const auto opts = x.options();
+        LaunchGuard guard(x);
+        void *const s = stream_of(x);
+        const at::Tensor qkvb = matmul(FWP_MM_NT, x, Wqkvb, rows, width, d, {T, B, width});
+        Parts parts({rows * H * D, rows * H * D, rows * H * D, rows * H}, opts);
+        const at::Tensor q = parts.take(B, H, T, D), k = parts.take(B, H, T, D), v = parts.take(B, H, T, D),
+                         beta = parts.take(B, H, T, 1);
+        check(fwp_deltanet_prep_fwd(ptr(qkvb), ptr(q), ptr(k), ptr(v), ptr(beta), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
+              "fwp_deltanet_prep_fwd");
+        const at::Tensor out = at::empty({T, B, H, D}, opts);
+        const fwp_out_view ov = {ptr(out), H * D, D, B * H * D};
+        const int chunk = fwp_query(FWP_Q_DEFAULT_CHUNK);
+        at::Tensor saved;
+        float *vdiff = nullptr, *ckpt = nullptr;
+        if (ctx) {
+            const int64_t n_vdiff = rows * H * D, n_ckpt = fwp_delta_ckpt_floats((int)B, (int)H, (int)T, (int)D, (int)D, chunk);
+            if (n_ckpt < 0) fail("invalid dimensions");
+            saved = at::empty({n_vdiff + n_ckpt}, opts);
+            vdiff = ptr(saved);
+            ckpt = vdiff + n_vdiff;
+        }
+        check(fwp_delta_fwd_strided(view_of(q), view_of(k), view_of(v), view_of(beta), ptr(state), ov, vdiff, ckpt, (int)B,
+                                    (int)H, (int)T, (int)D, (int)D, chunk, s),
+              "fwp_delta_fwd_strided");
+        fwp_mm_epilogue e{};
+        e.residual = residual ? ptr(x) : nullptr;
+        const at::Tensor y = matmul(FWP_MM_NT, out, Wo, rows, d, H * D, x_in.sizes(), e);
+        if (ctx) {
+            ctx->save_for_backward({x_in, Wqkvb, Wo, qkvb, q, k, beta, saved, out});
+            ctx->saved_data["scale"] = scale;
+            ctx->saved_data["residual"] = residual;
+            ctx->set_materialize_grads(false);
+        }
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        variable_list res(8);
+        if (!grads[0].defined()) return res;
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor x = plain(saved[0]), g = plain(grads[0]), &Wqkvb = saved[1], &Wo = saved[2], &qkvb = saved[3],
+                         &q = saved[4], &k = saved[5], &beta = saved[6], &buf = saved[7], &out = saved[8];
+        const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3), rows = T * B, d = Wqkvb.size(1),
+                      width = Wqkvb.size(0);
+        const auto opts = x.options();
+        LaunchGuard guard(x);
+        void *const s = stream_of(x);
+        // create_graph: the projections' products from PyTorch's operators (the delta rule's own gradients, as from
+        // fast_weight_delta, carry no graph)
+        const bool graph = at::GradMode::is_enabled();
+        if (ctx->needs_input_grad(2))
+            res[2] = graph ? at::matmul(grads[0].reshape({rows, d}).t(), out.reshape({rows, H * D}))
+                           : weight_grad(g, out, rows, d, H * D, nullptr);
+        const at::Tensor go = matmul(FWP_MM_NN, g, Wo, rows, H * D, d, {T, B, H, D});
+        Parts parts({rows * H * D, rows * H * D, rows * H * D, rows * H}, opts);
+        const at::Tensor gq = parts.take(B, H, T, D), gk = parts.take(B, H, T, D), gv = parts.take(B, H, T, D),
+                         gb = parts.take(B, H, T, 1);
+        const float *vdiff = ptr(buf), *ckpt = vdiff + rows * H * D;
+        const fwp_view gov = {ptr(go), H * D, D, B * H * D};
+        check(fwp_delta_bwd(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), (int)B,
+                            (int)H, (int)T, (int)D, (int)D, fwp_query(FWP_Q_DEFAULT_CHUNK), s),
+              "fwp_delta_bwd");
+        const at::Tensor gp = at::empty_like(qkvb);
+        check(fwp_deltanet_prep_bwd(ptr(qkvb), ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(gp), (int)T, (int)B, (int)H, (int)D,
+                                    (float)ctx->saved_data["scale"].toDouble(), s),
+              "fwp_deltanet_prep_bwd");
+        if (ctx->needs_input_grad(1))
+            res[1] = graph ? at::matmul(gp.reshape({rows, width}).t(), saved[0].reshape({rows, d}))
+                           : weight_grad(gp, x, rows, width, d, nullptr);
+        if (ctx->needs_input_grad(0) && graph) {
+            res[0] = at::matmul(gp, Wqkvb);
+            if (ctx->saved_data["residual"].toBool()) res[0] = res[0] + grads[0];
+        } else if (ctx->needs_input_grad(0)) {
+            fwp_mm_epilogue e{};
+            e.residual = ctx->saved_data["residual"].toBool() ? ptr(g) : nullptr;
+            res[0] = matmul(FWP_MM_NN, gp, Wqkvb, rows, d, width, saved[0].sizes(), e);
+        }
+        return res;
+    }
+};
+
+bool records(std::initializer_list<const at::Tensor *> ts) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const at::Tensor *t : ts)
+        if (t->defined() && t->requires_grad()) return true;
+    return false;
+}
+
+at::Tensor linear(const at::Tensor &x, const at::Tensor &W, const std::optional<at::Tensor> &bias_, bool relu) {
+    const at::Tensor bias = given(bias_);
+    if (records({&x, &W, &bias})) return LinearFn::apply(x, W, bias_, relu);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return LinearFn::forward(nullptr, x, W, bias_, relu);
+}
+
+at::Tensor feed_forward(const at::Tensor &x, const at::Tensor &W1, const at::Tensor &b1, const at::Tensor &W2, const at::Tensor &b2,
+                        const std::optional<at::Tensor> &residual_) {
+    const at::Tensor residual = given(residual_);
+    const bool same = residual.defined() && residual.is_same(x);
+    if (records({&x, &W1, &b1, &W2, &b2, &residual}))
+        return FeedForwardFn::apply(x, W1, b1, W2, b2, same ? std::nullopt : residual_, same);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return FeedForwardFn::forward(nullptr, x, W1, b1, W2, b2, residual_, same);
+}
+
+at::Tensor delta_block(const at::Tensor &x, const at::Tensor &Wqkvb, const at::Tensor &Wo, const at::Tensor &state, int64_t n_head,
+                       int64_t d_head, double scale, bool residual) {
+    if (records({&x, &Wqkvb, &Wo})) return DeltaBlockFn::apply(x, Wqkvb, Wo, state, n_head, d_head, scale, residual);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return DeltaBlockFn::forward(nullptr, x, Wqkvb, Wo, state, n_head, d_head, scale, residual);
+}
+
+}  // namespace
+
+void bind_blocks(py::module_ &m) {
+    m.def("linear", &linear, py::arg("x"), py::arg("W"), py::arg("bias") = py::none(), py::arg("relu") = false,
+          "x W^T (+ bias) (relu)");
+    m.def("feed_forward", &feed_forward, py::arg("x"), py::arg("W1"), py::arg("b1"), py::arg("W2"), py::arg("b2"),
+          py::arg("residual") = py::none(), "relu(x W1^T + b1) W2^T + b2 (+ residual)");
+    m.def("delta_block", &delta_block, "the Delta-Net layer between its input and its LayerNorm; the state is updated in place");
+}

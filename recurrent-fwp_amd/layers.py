@@ -1,17 +1,46 @@
 """The caller of ``fast_weight_delta`` in language modelling: the Delta-Net layer and the
 feed-forward block that follows it, with the module and parameter names of the reference
 (language_modeling/src/utils/cuda_fast_weight_layer.py:57-188, utils/model_utils.py:15-67)
-so a reference state_dict loads unchanged.  The fast-weight operator and, on the GPU, the
-elementwise lines in front of it are HIP kernels; the rest is stock PyTorch.  A caller may pass
-another operator (tests do, to compare against a step-by-step loop); the layer then also takes
-the stock-PyTorch form of those lines.
+so a reference state_dict loads unchanged.  On the GPU, in fp32, a layer is HIP kernels throughout: the
+fast-weight operator, the elementwise lines in front of it, and the matrix products with their biases,
+ReLU and residual additions (``_fwp_torch``'s blocks).  Everything else - other data types, autocast, the CPU,
+sub-modules that were replaced or carry hooks - runs on stock PyTorch around the operator.  A caller may
+pass another operator (tests do, to compare against a step-by-step loop); the layer then also takes
+the stock-PyTorch form.
 """
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
-from .fast_weight import fast_weight_delta
+from .fast_weight import _fwp_torch, fast_weight_delta
+
+
+def _untouched(m, cls):
+    """Is this sub-module exactly a ``cls`` (not a replacement) that nothing is hooked to?"""
+    return type(m) is cls and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
+def _blocks(x, *params):
+    """The C++ blocks (csrc/fwp_torch_blocks.cpp) if they apply to this input and these parameters: fp32 on the
+    GPU, outside autocast, tracing and functional transforms."""
+    if _fwp_torch is None or not x.is_cuda or x.numel() == 0:
+        return None
+    for t in (x, *params):
+        if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter):
+            return None
+    if not all(p.is_contiguous() for p in params):
+        return None
+    if (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch.nn.modules.module._has_any_global_hook() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None):
+        return None
+    return _fwp_torch
+
+
+def _drops(m):
+    """Does this dropout module change anything now?"""
+    return m.training and m.p > 0
 
 
 class PositionalEmbedding(nn.Module):
@@ -44,10 +73,24 @@ class PositionwiseFF(nn.Module):
             nn.Linear(d_inner, d_model), nn.Dropout(dropout))
         self.layer_norm = nn.LayerNorm(d_model)
 
+    def _core(self, x, residual):
+        """``residual + CoreNet(x)``"""
+        net = self.CoreNet
+        if (_untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
+                and _untouched(net[2], nn.Dropout) and _untouched(net[3], nn.Linear) and _untouched(net[4], nn.Dropout)
+                and net[0].bias is not None and net[3].bias is not None):
+            blocks = _blocks(x, net[0].weight, net[0].bias, net[3].weight, net[3].bias)
+            if blocks is not None and not (_drops(net[2]) or _drops(net[4])):
+                return blocks.feed_forward(x, net[0].weight, net[0].bias, net[3].weight, net[3].bias, residual)
+            if blocks is not None:
+                hid = net[2](blocks.linear(x, net[0].weight, net[0].bias, True))
+                return residual + net[4](blocks.linear(hid, net[3].weight, net[3].bias))
+        return residual + net(x)
+
     def forward(self, inp):
         if self.pre_lnorm:
-            return inp + self.CoreNet(self.layer_norm(inp))
-        return self.layer_norm(inp + self.CoreNet(inp))
+            return self._core(self.layer_norm(inp), inp)
+        return self.layer_norm(self._core(inp, inp))
 
 
 def sum_normalised_elu(x):
@@ -129,6 +172,15 @@ class DeltaNetLayer(nn.Module):
         self.pre_lnorm = pre_lnorm
         self.fast_weight_op = fast_weight_op or fast_weight_delta
 
+    def _state(self, mems, carry_over_fast_weight, bsz, h, dtype):
+        """The state the operator starts from and overwrites: zeros, or a copy of what was carried over."""
+        if mems is None:
+            return torch.zeros(bsz, self.n_head, self.d_head, self.d_head, device=h.device, dtype=dtype)
+        if not carry_over_fast_weight:
+            raise ValueError("mems are only meaningful with carry_over_fast_weight=True")
+        # the last batch of an epoch may be smaller than the carried state
+        return mems[0][:bsz].clone()
+
     def forward(self, h, attn_mask=None, mems=None, carry_over_fast_weight=False):
         slen, bsz, _ = h.shape
         H, D = self.n_head, self.d_head
@@ -136,8 +188,22 @@ class DeltaNetLayer(nn.Module):
         # The reference's pre-LN branch adds the normalised input back (it rebinds h, :100-104).
         residual = x
 
-        qkvb = self.qkvb_net(x)
         hip_op = self.fast_weight_op is fast_weight_delta
+        blocks = None
+        if (hip_op and D in (16, 32, 64) and _untouched(self.qkvb_net, nn.Linear) and _untouched(self.o_net, nn.Linear)
+                and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)):
+            blocks = _blocks(x, self.qkvb_net.weight, self.o_net.weight)
+        if blocks is not None:
+            W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32)
+            drops = _drops(self.drop)
+            out = blocks.delta_block(x, self.qkvb_net.weight, self.o_net.weight, W, H, D, self.scale, not drops)
+            if drops:
+                out = residual + self.drop(out)
+            if not self.pre_lnorm:
+                out = self.layer_norm(out)
+            return (out, (W.detach(), None)) if carry_over_fast_weight else out
+
+        qkvb = self.qkvb_net(x)
         fused = hip_op and DeltaNetPrep.supported(qkvb, D)
         if fused:
             # one fused kernel each way; q carries the 1/sqrt(D) of the read-out (the operator is
@@ -152,14 +218,7 @@ class DeltaNetLayer(nn.Module):
             # half or bf16 activations (autocast): the operator and its state are fp32, as the
             # reference's kernel and its torch.zeros state are
             q, k, v, beta = q.float(), k.float(), v.float(), beta.float()
-        if mems is None:
-            W = torch.zeros(bsz, H, D, D, device=h.device, dtype=torch.float32 if hip_op else q.dtype)
-        else:
-            if not carry_over_fast_weight:
-                raise ValueError("mems are only meaningful with carry_over_fast_weight=True")
-            # The last batch of an epoch may be smaller than the carried state.  The
-            # operator overwrites its state argument, so it gets storage of its own.
-            W = mems[0][:bsz].clone()
+        W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32 if hip_op else q.dtype)
 
         if fused:
             out = fast_weight_delta(q, k, v, beta, W, True)          # [bsz, H, slen, D] over [slen, bsz, H, D] storage

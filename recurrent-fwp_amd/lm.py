@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import DeltaNetDecoderLayer, PositionalEmbedding
+from .layers import DeltaNetDecoderLayer, PositionalEmbedding, _blocks, _untouched
 
 
 class _WordEmbedding(nn.Module):
@@ -36,7 +36,10 @@ class _TiedSoftmaxLoss(nn.Module):
         self.out_layers = nn.ModuleList([nn.Linear(d_model, n_token)])
 
     def forward(self, hidden, target):
-        return F.cross_entropy(self.out_layers[0](hidden), target, reduction="none")
+        out = self.out_layers[0]
+        blocks = _blocks(hidden, out.weight, out.bias) if _untouched(out, nn.Linear) and out.bias is not None else None
+        logits = out(hidden) if blocks is None else blocks.linear(hidden, out.weight, out.bias)
+        return F.cross_entropy(logits, target, reduction="none")
 
 
 class DeltaNetLM(nn.Module):

@@ -1,0 +1,87 @@
+"""The layers on the C++ blocks against themselves in float64 on stock PyTorch: dropout in and out, LayerNorm
+before and after, hooks and second derivatives (which take stock PyTorch), products in every order."""
+import pytest
+import torch
+
+from oracle.torch_loop import delta_loop
+
+pytestmark = pytest.mark.gpu
+
+
+def loop_op(q, k, v, beta, W):
+    out, W_end = delta_loop(q, k, v, beta, W.clone())
+    W.copy_(W_end.detach())
+    return out
+
+
+def close(name, got, want, scale=1.0):
+    """A few dozen fp32 roundings of values of the size of `want`."""
+    got, want = got.detach(), want.detach()
+    err, size = (got.double() - want).abs().max(), want.abs().max()
+    assert float(err) <= 64 * 2.0 ** -24 * float(size) * scale, f"{name}: {float(err):.2e} of {float(size):.2e}"
+
+
+def both(make, x, seed=0):
+    """The module in fp32 and in float64 with the same parameters, and their input."""
+    torch.manual_seed(seed)
+    ours, ref = make(None).cuda(), make(loop_op).cuda().double()
+    with torch.no_grad():
+        for p in ours.parameters():
+            p.normal_(0.0, 0.2)
+    ref.load_state_dict(ours.state_dict())
+    return ours, ref, x.clone().requires_grad_(), x.double().requires_grad_()
+
+
+@pytest.mark.parametrize("drop", [0.0, 1e-9])       # 1e-9: the path with dropout, nothing dropped
+@pytest.mark.parametrize("pre", [False, True])
+def test_feed_forward_block(fwp, pre, drop):
+    x = torch.randn(37, 3, 64, generator=torch.Generator().manual_seed(1)).cuda()
+    ours, ref, a, b = both(lambda op: fwp.PositionwiseFF(64, 200, drop, pre), x)
+    y, want = ours(a), ref(b)
+    close("y", y, want)
+    g = torch.randn_like(x)
+    grads = torch.autograd.grad(y, [a, *ours.parameters()], g)
+    wants = torch.autograd.grad(want, [b, *ref.parameters()], g.double())
+    for i, (got, w) in enumerate(zip(grads, wants)):
+        close(i, got, w, 4)
+
+
+@pytest.mark.parametrize("drop", [0.0, 1e-9])
+@pytest.mark.parametrize("pre,D", [(False, 16), (True, 32), (False, 64)])
+def test_delta_block(fwp, pre, D, drop):
+    x = torch.randn(50, 3, 96, generator=torch.Generator().manual_seed(1)).cuda()
+    ours, ref, a, b = both(lambda op: fwp.DeltaNetLayer(2, 96, D, dropout=drop, pre_lnorm=pre, fast_weight_op=op), x)
+    W0 = torch.randn(3, 2, D, D, generator=torch.Generator().manual_seed(2)).cuda() * 0.1
+    y, (W, _) = ours(a, mems=(W0, None), carry_over_fast_weight=True)
+    want, (W_want, _) = ref(b, mems=(W0.double(), None), carry_over_fast_weight=True)
+    close("y", y, want)
+    close("W", W, W_want)
+    g = torch.randn_like(x)
+    grads = torch.autograd.grad(y, [a, *ours.parameters()], g)
+    wants = torch.autograd.grad(want, [b, *ref.parameters()], g.double())
+    for i, (got, w) in enumerate(zip(grads, wants)):
+        close(i, got, w, 16)
+    # frozen weights, an input that wants nothing
+    for p in ours.parameters():
+        p.requires_grad_(False)
+    ours.o_net.weight.requires_grad_(True)
+    y, _ = ours(x, mems=(W0, None), carry_over_fast_weight=True)
+    got, = torch.autograd.grad(y, [ours.o_net.weight], g)
+    assert torch.equal(got, grads[1 + [n for n, _ in ours.named_parameters()].index("o_net.weight")])
+
+
+def test_second_derivatives_and_hooks_take_stock_operators(fwp):
+    x = torch.randn(9, 2, 32, generator=torch.Generator().manual_seed(1)).cuda()
+    ours, ref, a, b = both(lambda op: fwp.PositionwiseFF(32, 64, 0.0), x)
+    seconds = []
+    for m, z in ((ours, a), (ref, b)):
+        g, = torch.autograd.grad(m(z).square().sum(), [z], create_graph=True)
+        seconds.append(torch.autograd.grad(g.square().sum(), [z, *m.parameters()], allow_unused=True))
+    for i, (got, want) in enumerate(zip(*seconds)):
+        assert (got is None) == (want is None)
+        if got is not None:
+            close(i, got, want, 64)
+    seen = []
+    ours.CoreNet[1].register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    ours(a)
+    assert seen == [(9, 2, 64)]

@@ -1,0 +1,130 @@
+"""The language model's matrix products, negative log-likelihood and LayerNorm kernels through the C ABI, against
+float64.  Tolerance of a product: every one of the six roundings per 32 terms, and the split of an operand into
+three bf16 numbers, is at most 2^-24 of the sum of the terms' magnitudes."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+NT, NN, TN = 0, 1, 2
+
+
+def bound(K, mag):
+    return (6 * (K // 32 + 2)) * EPS * mag + 1e-30
+
+
+def randn(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).cuda()
+
+
+def matmul(L, layout, A, B, cut=True, **epi):
+    K = A.shape[0] if layout == TN else A.shape[1]
+    M = A.shape[1] if layout == TN else A.shape[0]
+    N = B.shape[0] if layout == NT else B.shape[1]
+    C = torch.full((M, N), float("nan"), device="cuda")
+    e = L.Epilogue(*(epi[n].data_ptr() if n in epi else None for n in ("bias", "residual", "gate", "colsum")),
+                   int(epi.get("relu", 0)))
+    work = torch.empty(max(1, L.lib().fwp_matmul_workspace(M, N, K)), device="cuda") if cut else None
+    rc = L.lib().fwp_matmul(layout, A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), C.data_ptr(), N, M, N, K,
+                            ctypes.byref(e), work.data_ptr() if cut else None, L.stream_of(A))
+    assert rc == 0, L.strerror(rc)
+    return C
+
+
+# the edges of the 64 and 128 tiles and of the 32-wide steps of k; few tiles and a long k (cut into ranges)
+SHAPES = [(1, 1, 1), (3, 5, 7), (64, 64, 32), (65, 63, 33), (128, 128, 256), (130, 776, 256), (257, 36, 1000),
+          (2048, 2049, 40), (16, 256, 4096), (776, 256, 3001), (200, 260, 8192)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("layout", [NT, NN, TN])
+def test_products(fwp, layout, M, N, K):
+    A = randn(*((K, M) if layout == TN else (M, K)), seed=1)
+    B = randn(*((N, K) if layout == NT else (K, N)), seed=2)
+    a, b = A.double(), B.double()
+    a, b = (a.t() if layout == TN else a), (b.t() if layout == NT else b)
+    want, mag = a @ b, a.abs() @ b.abs()
+    for cut in (True, False):
+        got = matmul(fwp._lib, layout, A, B, cut)
+        assert bool(((got.double() - want).abs() <= bound(K, mag)).all())
+    # operands of any size: fp32's exponents, no scaling
+    got = matmul(fwp._lib, layout, A * 1e-30, B * 1e25)
+    assert bool(((got.double() / 1e-5 - want).abs() <= 2 * bound(K, mag)).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 776, 256), (64, 256, 4096)])      # one range of k, several
+def test_epilogues_and_column_sums(fwp, M, N, K):
+    A, B = randn(M, K, seed=1), randn(N, K, seed=2)
+    bias, residual, gate = randn(N, seed=3) * 30, randn(M, N, seed=4) * 30, randn(M, N, seed=5)
+    raw, mag = A.double() @ B.double().t(), A.double().abs() @ B.double().abs().t()
+    got = matmul(fwp._lib, NT, A, B, bias=bias, relu=1, residual=residual, gate=gate)
+    want = torch.where(gate > 0, torch.relu(raw + bias.double()) + residual.double(), 0.0)
+    assert bool(((got.double() - want).abs() <= bound(K, mag + 400)).all())
+    # TN: the columns of A summed over k
+    G, X = randn(K, M, seed=6), randn(K, N, seed=7)
+    colsum = torch.full((M,), float("nan"), device="cuda")
+    got = matmul(fwp._lib, TN, G, X, colsum=colsum)
+    assert bool(((got.double() - G.double().t() @ X.double()).abs() <= bound(K, G.double().abs().t() @ X.double().abs())).all())
+    assert bool(((colsum.double() - G.double().sum(0)).abs() <= K * EPS * G.double().abs().sum(0)).all())
+
+
+@pytest.mark.parametrize("rows,vocab,dim", [(1, 5, 4), (70, 211, 64), (64, 64, 36), (300, 4099, 128), (520, 33000, 256)])
+def test_negative_log_likelihood(fwp, rows, vocab, dim):
+    L = fwp._lib
+    x, W, b = randn(rows, dim, seed=1), randn(vocab, dim, seed=2) * 0.3, randn(vocab, seed=3)
+    target = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
+    target[rows // 2] = -100 if rows > 1 else target[0]          # ignored
+    gloss = randn(rows, seed=5)
+    logits, loss, lse = (torch.full(s, float("nan"), device="cuda") for s in ((rows, vocab), (rows,), (rows,)))
+    work = torch.empty(L.lib().fwp_nll_workspace(rows, vocab), device="cuda")
+    ptrs = [t.data_ptr() for t in (x, W, b, target)]
+    assert L.lib().fwp_nll_fwd(*ptrs, logits.data_ptr(), loss.data_ptr(), lse.data_ptr(), work.data_ptr(), rows, vocab,
+                               dim, L.stream_of(x)) == 0
+    only = torch.empty_like(loss)
+    assert L.lib().fwp_nll_fwd(*ptrs, None, only.data_ptr(), None, work.data_ptr(), rows, vocab, dim, L.stream_of(x)) == 0
+    assert torch.equal(only, loss)
+    xd, Wd, bd = (t.double().requires_grad_() for t in (x, W, b))
+    want = torch.nn.functional.cross_entropy(xd @ Wd.t() + bd, target, reduction="none")
+    # the logits' rounding, and the hardware exponential's and logarithm's (2^-21 of the largest)
+    err = bound(dim, x.double().abs() @ W.double().abs().t() + bd.abs()).max() + 2.0 ** -20
+    assert float((loss.double() - want.detach()).abs().max()) <= float(err)
+    gx, gW, gb = torch.full_like(x, float("nan")), torch.full_like(W, float("nan")), torch.full_like(b, float("nan"))
+    n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
+    work = torch.empty(n, device="cuda")
+    assert L.lib().fwp_nll_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), lse.data_ptr(), target.data_ptr(),
+                               gloss.data_ptr(), gx.data_ptr(), gW.data_ptr(), gb.data_ptr(), work.data_ptr(), rows, vocab,
+                               dim, L.stream_of(x)) == 0
+    wants = torch.autograd.grad(want, (xd, Wd, bd), gloss.double())
+    # a probability is off by its logit's error, relatively: 2 err of the gradient's magnitude
+    p = torch.softmax((xd @ Wd.t() + bd).detach(), -1)
+    d = (p + torch.nn.functional.one_hot(target.clamp_min(0), vocab)) * gloss.double().abs()[:, None]
+    mags = (d @ Wd.detach().abs(), d.t() @ xd.detach().abs(), d.sum(0))
+    for name, got, w, mag in zip("xWb", (gx, gW, gb), wants, mags):
+        assert bool(((got.double() - w).abs() <= (2 * float(err) + bound(max(rows, vocab), 1.0)) * mag + 1e-12).all()), name
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (5, 36), (3000, 128), (2500, 256), (9, 260), (70, 1024)])
+def test_layer_norm(fwp, rows, cols):
+    L = fwp._lib
+    x, g, b, gy, add = (randn(*s, seed=i) for i, s in enumerate(((rows, cols), (cols,), (cols,), (rows, cols), (rows, cols))))
+    x = 3 * x + 1
+    xd, gd, bd = (t.double().requires_grad_() for t in (x, g, b))
+    want = torch.nn.functional.layer_norm(xd, (cols,), gd, bd, 1e-5)
+    wants = torch.autograd.grad(want, (xd, gd, bd), gy.double())
+    y, stats = torch.full_like(x, float("nan")), torch.empty(rows, 2, device="cuda")
+    assert L.lib().fwp_layer_norm_fwd(x.data_ptr(), g.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr(), rows, cols,
+                                      1e-5, L.stream_of(x)) == 0
+    # cols roundings in a sum, a few more around it, of values whose scale is that of the row
+    tol = (cols / 8 + 16) * EPS
+    rms = xd.detach().abs().max() / xd.detach().std(-1, keepdim=True, correction=0).clamp_min(1e-2)
+    assert bool(((y.double() - want).abs() <= tol * rms * (gd.abs() + 1) * 4 + 1e-6).all())
+    gx, gg, gb = torch.full_like(x, float("nan")), torch.empty_like(g), torch.empty_like(b)
+    work = torch.empty(L.lib().fwp_layer_norm_workspace(rows, cols), device="cuda")
+    assert L.lib().fwp_layer_norm_bwd(gy.data_ptr(), x.data_ptr(), stats.data_ptr(), g.data_ptr(), add.data_ptr(),
+                                      gx.data_ptr(), gg.data_ptr(), gb.data_ptr(), work.data_ptr(), rows, cols,
+                                      L.stream_of(x)) == 0
+    for name, got, w in zip(("x", "gamma", "beta"), (gx, gg, gb), (wants[0] + add.double(), *wants[1:])):
+        scale = float(w.abs().max()) + float(gy.abs().max())
+        assert float((got.double() - w).abs().max()) <= (rows / 8 + cols / 8 + 64) * EPS * scale * float(rms.max()), name
