@@ -313,12 +313,10 @@ int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float
 int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats,
                        int rows, int cols, float eps, void *stream);
 
-/* Its adjoint; gx = the gradient of x (+ add, when given: the gradient that reaches x by another way).
- * workspace: fwp_layer_norm_workspace(rows, cols) floats. */
+/* Its adjoint.  workspace: fwp_layer_norm_workspace(rows, cols) floats. */
 long long fwp_layer_norm_workspace(int rows, int cols);
-int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma,
-                       const float *add, float *gx, float *ggamma, float *gbeta, float *workspace,
-                       int rows, int cols, void *stream);
+int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
+                       float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream);
 
 /*
  * Recurrent Delta Net forward.  Replaces rec_update_fwm_tanh_forward

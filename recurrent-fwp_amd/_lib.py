@@ -61,7 +61,7 @@ _MODEL_SIGNATURES = {
     "fwp_nll_fwd": [_P] * 8 + [_I] * 3 + [_P],
     "fwp_nll_bwd": [_P] * 10 + [_I] * 3 + [_P],
     "fwp_layer_norm_fwd": [_P] * 5 + [_I] * 2 + [ctypes.c_float, _P],
-    "fwp_layer_norm_bwd": [_P] * 9 + [_I] * 2 + [_P],
+    "fwp_layer_norm_bwd": [_P] * 8 + [_I] * 2 + [_P],
 }
 _WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
 EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",

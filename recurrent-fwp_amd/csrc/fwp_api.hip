@@ -442,11 +442,11 @@ long long fwp_layer_norm_workspace(int rows, int cols) {
     return rows < 1 || cols < 1 ? FWP_E_SHAPE : layer_norm_workspace(rows, cols);
 }
 
-int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, const float *add,
-                       float *gx, float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream) {
+int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
+                       float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream) {
     if (!gy || !x || !stats || !gamma || !gx || !ggamma || !gbeta || !workspace) return FWP_E_NULL;
     if (rows < 1 || !layer_norm_supported(cols)) return FWP_E_SHAPE;
-    return layer_norm_bwd(gy, x, stats, gamma, add, gx, ggamma, gbeta, workspace, rows, cols, (hipStream_t)stream);
+    return layer_norm_bwd(gy, x, stats, gamma, gx, ggamma, gbeta, workspace, rows, cols, (hipStream_t)stream);
 }
 
 int fwp_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float *Rq,

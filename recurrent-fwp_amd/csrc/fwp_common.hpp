@@ -203,7 +203,7 @@ bool layer_norm_supported(int cols);
 int64_t layer_norm_workspace(int rows, int cols);
 int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows, int cols,
                    float eps, hipStream_t s);
-int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, const float *add, float *gx,
+int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
                    float *ggamma, float *gbeta, float *workspace, int rows, int cols, hipStream_t s);
 
 // Largest dynamic LDS allocation the LDS-state kernels ask for (bytes).

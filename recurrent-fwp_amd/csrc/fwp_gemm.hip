@@ -19,13 +19,15 @@
 #include "fwp_mfma.hpp"
 
 namespace fwp {
+
+typedef float v2f __attribute__((ext_vector_type(2)));
+__device__ v2f llvm_raw_buffer_load_v2f32(v4i rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
+
 namespace {
 
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
-__device__ v2f llvm_raw_buffer_load_v2f32(v4i rsrc, int voffset, int soffset, int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
 
 constexpr int kBK = 32;          // k per LDS tile
 constexpr int kPad = 2;          // units after a k-chunk's rows: the chunks of a row start 32 bytes apart in the banks

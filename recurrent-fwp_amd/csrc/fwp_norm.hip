@@ -60,11 +60,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_fwd(const float *__restric
     if (stats && lane == 0) *reinterpret_cast<float2 *>(stats + 2 * (int64_t)row) = make_float2(mean, rstd);
 }
 
-// gx = rstd (g - mean(g) - xh mean(g xh)) (+ add),  g = gy gamma, xh = (x - mean) rstd
+// gx = rstd (g - mean(g) - xh mean(g xh)),  g = gy gamma, xh = (x - mean) rstd
 template <int V>
 __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restrict__ gy, const float *__restrict__ x,
                                                           const float *__restrict__ stats, const float *__restrict__ gamma,
-                                                          const float *__restrict__ add, float *__restrict__ gx,
+                                                          float *__restrict__ gx,
                                                           float *__restrict__ part, int rows, int cols) {
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
     float4 gam[V], sg[V], sb[V];
@@ -98,10 +98,6 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restric
             if (c >= cols) continue;
             float4 o = make_float4(st.y * (g[i].x - s - xh[i].x * t), st.y * (g[i].y - s - xh[i].y * t),
                                    st.y * (g[i].z - s - xh[i].z * t), st.y * (g[i].w - s - xh[i].w * t));
-            if (add) {
-                const float4 r = load4(add + at + c, true);
-                o.x += r.x, o.y += r.y, o.z += r.z, o.w += r.w;
-            }
             *reinterpret_cast<float4 *>(gx + at + c) = o;
         }
     }
@@ -154,13 +150,13 @@ int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float 
     return (int)hipGetLastError();
 }
 
-int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, const float *add, float *gx,
+int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
                    float *ggamma, float *gbeta, float *workspace, int rows, int cols, hipStream_t s) {
     const int blocks = blocks_of(rows), v = (cols + 255) / 256;
     const dim3 grid(blocks), block(64 * kWaves);
-    if (v == 1) hipLaunchKernelGGL(k_norm_bwd<1>, grid, block, 0, s, gy, x, stats, gamma, add, gx, workspace, rows, cols);
-    else if (v == 2) hipLaunchKernelGGL(k_norm_bwd<2>, grid, block, 0, s, gy, x, stats, gamma, add, gx, workspace, rows, cols);
-    else hipLaunchKernelGGL(k_norm_bwd<4>, grid, block, 0, s, gy, x, stats, gamma, add, gx, workspace, rows, cols);
+    if (v == 1) hipLaunchKernelGGL(k_norm_bwd<1>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
+    else if (v == 2) hipLaunchKernelGGL(k_norm_bwd<2>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
+    else hipLaunchKernelGGL(k_norm_bwd<4>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
     hipLaunchKernelGGL(k_norm_params, dim3((2 * cols + 15) / 16), dim3(256), 0, s, workspace, ggamma, gbeta, blocks, cols);
     return (int)hipGetLastError();
 }

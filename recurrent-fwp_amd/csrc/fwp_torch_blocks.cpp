@@ -263,6 +263,109 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
     }
 };
 
+// ------------------------------------------------------------------ LayerNorm over the last axis
+
+struct LayerNormFn : torch::autograd::Function<LayerNormFn> {
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
+        require_device(x_in);
+        same_device(x_in, {gamma, beta});
+        const at::Tensor x = plain(x_in), g = plain(gamma), b = plain(beta);
+        const int64_t cols = gamma.numel(), rows = x.numel() / cols;
+        LaunchGuard guard(x);
+        at::Tensor y = at::empty(x.sizes(), x.options()), stats;
+        if (ctx) stats = at::empty({rows, 2}, x.options());
+        check(fwp_layer_norm_fwd(ptr(x), ptr(g), ptr(b), ptr(y), ptr(stats), (int)rows, (int)cols, (float)eps, stream_of(x)),
+              "fwp_layer_norm_fwd");
+        if (ctx) {
+            ctx->save_for_backward({x_in, gamma, beta, stats});
+            ctx->saved_data["eps"] = eps;
+            ctx->set_materialize_grads(false);
+        }
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        variable_list res(4);
+        if (!grads[0].defined()) return res;
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &gamma = saved[1], &stats = saved[3];
+        if (at::GradMode::is_enabled()) {
+            res = differentiate(at::layer_norm(saved[0], gamma.sizes(), gamma, saved[2], ctx->saved_data["eps"].toDouble()),
+                                {saved[0], gamma, saved[2]}, grads[0]);
+            res.resize(4);
+            return res;
+        }
+        const at::Tensor x = plain(saved[0]), g = plain(gamma), gy = plain(grads[0]);
+        const int64_t cols = gamma.numel(), rows = x.numel() / cols;
+        LaunchGuard guard(x);
+        res[0] = at::empty(x.sizes(), x.options());
+        res[1] = at::empty({cols}, x.options());
+        res[2] = at::empty({cols}, x.options());
+        const at::Tensor work = at::empty({fwp_layer_norm_workspace((int)rows, (int)cols)}, x.options());
+        check(fwp_layer_norm_bwd(ptr(gy), ptr(x), ptr(stats), ptr(g), ptr(res[0]), ptr(res[1]), ptr(res[2]), ptr(work), (int)rows,
+                                 (int)cols, stream_of(x)),
+              "fwp_layer_norm_bwd");
+        return res;
+    }
+};
+
+// ------------------------------------------------------------------ negative log-likelihood under softmax(x W^T + bias)
+
+struct NllFn : torch::autograd::Function<NllFn> {
+    // x [rows, dim], target [rows] int64
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &W, const at::Tensor &bias,
+                              const at::Tensor &target_in) {
+        require_device(x_in);
+        same_device(x_in, {W, bias, target_in});
+        require(x_in.dim() == 2 && target_in.dim() == 1 && target_in.size(0) == x_in.size(0) && target_in.scalar_type() == at::kLong,
+                "hidden [rows, d_model] and int64 targets [rows]");
+        const at::Tensor x = plain(x_in), target = target_in.contiguous();
+        const int64_t rows = x.size(0), dim = x.size(1), vocab = W.size(0);
+        LaunchGuard guard(x);
+        at::Tensor loss = at::empty({rows}, x.options()), logits, lse;
+        if (ctx) {
+            logits = at::empty({rows, vocab}, x.options());
+            lse = at::empty({rows}, x.options());
+        }
+        const at::Tensor work = at::empty({fwp_nll_workspace((int)rows, (int)vocab)}, x.options());
+        check(fwp_nll_fwd(ptr(x), ptr(W), ptr(bias), target.data_ptr<int64_t>(), ptr(logits), ptr(loss), ptr(lse), ptr(work),
+                          (int)rows, (int)vocab, (int)dim, stream_of(x)),
+              "fwp_nll_fwd");
+        if (ctx) {
+            ctx->save_for_backward({x_in, W, bias, target, logits, lse});
+            ctx->set_materialize_grads(false);
+        }
+        return loss;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        variable_list res(4);
+        if (!grads[0].defined()) return res;
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &W = saved[1], &bias = saved[2], &target = saved[3], &logits = saved[4], &lse = saved[5];
+        if (at::GradMode::is_enabled()) {
+            res = differentiate(at::cross_entropy_loss(at::linear(saved[0], W, bias), target, {}, at::Reduction::None),
+                                {saved[0], W, bias}, grads[0]);
+            res.resize(4);
+            return res;
+        }
+        const at::Tensor x = plain(saved[0]), g = plain(grads[0]);
+        const int64_t rows = x.size(0), dim = x.size(1), vocab = W.size(0);
+        LaunchGuard guard(x);
+        if (ctx->needs_input_grad(0)) res[0] = at::empty({rows, dim}, x.options());
+        if (ctx->needs_input_grad(1) || ctx->needs_input_grad(2)) {
+            res[1] = at::empty({vocab, dim}, x.options());
+            res[2] = at::empty({vocab}, x.options());
+        }
+        at::Tensor work;
+        const int64_t n = std::max(fwp_matmul_workspace((int)rows, (int)dim, (int)vocab),
+                                   fwp_matmul_workspace((int)vocab, (int)dim, (int)rows));
+        if (n > 0) work = at::empty({n}, x.options());
+        check(fwp_nll_bwd(ptr(x), ptr(W), ptr(logits), ptr(lse), target.data_ptr<int64_t>(), ptr(g), ptr(res[0]), ptr(res[1]),
+                          ptr(res[2]), ptr(work), (int)rows, (int)vocab, (int)dim, stream_of(x)),
+              "fwp_nll_bwd");
+        return res;
+    }
+};
+
 bool records(std::initializer_list<const at::Tensor *> ts) {
     if (!at::GradMode::is_enabled()) return false;
     for (const at::Tensor *t : ts)
@@ -294,6 +397,18 @@ at::Tensor delta_block(const at::Tensor &x, const at::Tensor &Wqkvb, const at::T
     return DeltaBlockFn::forward(nullptr, x, Wqkvb, Wo, state, n_head, d_head, scale, residual);
 }
 
+at::Tensor layer_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
+    if (records({&x, &gamma, &beta})) return LayerNormFn::apply(x, gamma, beta, eps);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return LayerNormFn::forward(nullptr, x, gamma, beta, eps);
+}
+
+at::Tensor nll(const at::Tensor &x, const at::Tensor &W, const at::Tensor &bias, const at::Tensor &target) {
+    if (records({&x, &W, &bias})) return NllFn::apply(x, W, bias, target);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return NllFn::forward(nullptr, x, W, bias, target);
+}
+
 }  // namespace
 
 void bind_blocks(py::module_ &m) {
@@ -301,5 +416,7 @@ void bind_blocks(py::module_ &m) {
           "x W^T (+ bias) (relu)");
     m.def("feed_forward", &feed_forward, py::arg("x"), py::arg("W1"), py::arg("b1"), py::arg("W2"), py::arg("b2"),
           py::arg("residual") = py::none(), "relu(x W1^T + b1) W2^T + b2 (+ residual)");
+    m.def("layer_norm", &layer_norm, "LayerNorm over the last axis (a multiple of 4 up to 1024)");
+    m.def("nll", &nll, "per-row negative log-likelihood of the targets under softmax(x W^T + bias); a negative target counts 0");
     m.def("delta_block", &delta_block, "the Delta-Net layer between its input and its LayerNorm; the state is updated in place");
 }

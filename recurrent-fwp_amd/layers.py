@@ -43,6 +43,16 @@ def _drops(m):
     return m.training and m.p > 0
 
 
+def _layer_norm(m, x):
+    """``m(x)`` for a LayerNorm over the last axis."""
+    if _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:
+        d = m.normalized_shape[0]
+        blocks = _blocks(x, m.weight, m.bias) if d % 4 == 0 and d <= 1024 and x.shape[-1] == d else None
+        if blocks is not None:
+            return blocks.layer_norm(x, m.weight, m.bias, m.eps)
+    return m(x)
+
+
 class PositionalEmbedding(nn.Module):
     """Sinusoidal embedding of a position sequence: ``[sin | cos]`` halves, shape
     ``[len, 1, demb]`` (or ``[len, bsz, demb]``).  utils/model_utils.py:15-31."""
@@ -89,8 +99,8 @@ class PositionwiseFF(nn.Module):
 
     def forward(self, inp):
         if self.pre_lnorm:
-            return self._core(self.layer_norm(inp), inp)
-        return self.layer_norm(self._core(inp, inp))
+            return self._core(_layer_norm(self.layer_norm, inp), inp)
+        return _layer_norm(self.layer_norm, self._core(inp, inp))
 
 
 def sum_normalised_elu(x):
@@ -184,7 +194,7 @@ class DeltaNetLayer(nn.Module):
     def forward(self, h, attn_mask=None, mems=None, carry_over_fast_weight=False):
         slen, bsz, _ = h.shape
         H, D = self.n_head, self.d_head
-        x = self.layer_norm(h) if self.pre_lnorm else h
+        x = _layer_norm(self.layer_norm, h) if self.pre_lnorm else h
         # The reference's pre-LN branch adds the normalised input back (it rebinds h, :100-104).
         residual = x
 
@@ -200,7 +210,7 @@ class DeltaNetLayer(nn.Module):
             if drops:
                 out = residual + self.drop(out)
             if not self.pre_lnorm:
-                out = self.layer_norm(out)
+                out = _layer_norm(self.layer_norm, out)
             return (out, (W.detach(), None)) if carry_over_fast_weight else out
 
         qkvb = self.qkvb_net(x)

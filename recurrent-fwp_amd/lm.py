@@ -38,8 +38,9 @@ class _TiedSoftmaxLoss(nn.Module):
     def forward(self, hidden, target):
         out = self.out_layers[0]
         blocks = _blocks(hidden, out.weight, out.bias) if _untouched(out, nn.Linear) and out.bias is not None else None
-        logits = out(hidden) if blocks is None else blocks.linear(hidden, out.weight, out.bias)
-        return F.cross_entropy(logits, target, reduction="none")
+        if blocks is not None and target.dtype is torch.int64 and target.device == hidden.device:
+            return blocks.nll(hidden, out.weight, out.bias, target)
+        return F.cross_entropy(out(hidden), target, reduction="none")
 
 
 class DeltaNetLM(nn.Module):

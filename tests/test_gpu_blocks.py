@@ -85,3 +85,26 @@ def test_second_derivatives_and_hooks_take_stock_operators(fwp):
     ours.CoreNet[1].register_forward_hook(lambda m, i, o: seen.append(o.shape))
     ours(a)
     assert seen == [(9, 2, 64)]
+
+
+@pytest.mark.parametrize("pre", [False, True])
+def test_language_model_with_ignored_targets(fwp, pre):
+    """Losses and every gradient of a two-layer model, some targets ignored, frozen embedding included."""
+    cfg = dict(n_token=309, n_layer=2, n_head=3, d_model=48, d_head=16, d_inner=100, pre_lnorm=pre, tie_weight=False)
+    torch.manual_seed(0)
+    ours = fwp.DeltaNetLM(init_std=0.3, **cfg).cuda()
+    ref = fwp.DeltaNetLM(fast_weight_op=loop_op, init_std=0.3, **cfg).cuda().double()
+    ref.load_state_dict(ours.state_dict())
+    g = torch.Generator().manual_seed(1)
+    data, target = (torch.randint(0, 309, (45, 3), generator=g).cuda() for _ in range(2))
+    target[5:9, 1] = -100
+    (loss,), (want,) = ours(data, target), ref(data, target)
+    close("loss", loss, want)
+    assert bool((loss[5:9, 1] == 0).all())
+    with torch.no_grad():
+        assert torch.equal(ours(data, target)[0], loss)
+    w = torch.randn(45, 3, generator=g).cuda()
+    (loss * w).sum().backward()
+    (want * w.double()).sum().backward()
+    for (name, a), (_, b) in zip(ours.named_parameters(), ref.named_parameters()):
+        close(name, a.grad, b.grad, 16)
