@@ -46,6 +46,10 @@ __device__ __forceinline__ v4i buffer_of(const float *base, int64_t floats) {
     return v4i{(int)(uint32_t)a, (int)(uint32_t)((a >> 32) & 0xffff), (int)(uint32_t)(floats * 4), 0x00020000};
 }
 
+__device__ __forceinline__ float lane_of(float x, int lane) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane));
+}
+
 template <int ROWS>
 struct Planes {
     v4u u[3][kBK / 8][ROWS + kPad];
@@ -74,8 +78,10 @@ struct Operand {
     static_assert(KC ? kTasks >= 1 : (VEC == 1 || VEC == 2), "a whole number of tasks per thread");
     float x[kTasks][8 * VEC];
     unsigned off[kTasks];
-    float lse[NLL && KC ? kTasks : 1], gl[NLL && KC ? kTasks : 1];
-    int hit[NLL && KC ? kTasks : 1];
+    // the tokens' values for the loss gradient: of this task's row (KC), or of the wave's k-chunk, token j in
+    // the lanes with lane % 8 == j
+    float lse[NLL ? kTasks : 1], gl[NLL ? kTasks : 1];
+    int hit[NLL ? kTasks : 1];
 
     static __device__ __forceinline__ int row_of(int t) { return KC ? t / kChunks : (t % (ROWS / VEC)) * VEC; }
     static __device__ __forceinline__ int chunk_of(int t) { return KC ? t % kChunks : t / (ROWS / VEC); }
@@ -94,7 +100,7 @@ struct Operand {
         }
     }
     // P: the tile's first row at k = 0, `left` rows from there, k0 .. min(k0 + kBK, K)
-    __device__ __forceinline__ void load(const float *P, int64_t ld, int left, int tid, int k0, int K) {
+    __device__ __forceinline__ void load(const float *P, int64_t ld, int left, int tid, int k0, int K, const NllArgs &nll) {
         if constexpr (KC) {
             const v4i rs = buffer_of(P + k0, (int64_t)(min(left, ROWS) - 1) * ld + (K - k0));
 #pragma unroll
@@ -106,6 +112,12 @@ struct Operand {
                 for (int j = 0; j < 4; j++) x[i][j] = a[j], x[i][4 + j] = b[j];
             }
         } else {
+            if constexpr (NLL) {
+                const int t = min(k0 + 8 * chunk_of(tid) + tid % 8, K - 1);
+                lse[0] = nll.lse[t];
+                gl[0] = nll.gloss[t];
+                hit[0] = (int)nll.target[t];
+            }
             const v4i rs = buffer_of(P + (int64_t)k0 * ld, (int64_t)(min(K - k0, kBK) - 1) * ld + left);
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -134,13 +146,15 @@ struct Operand {
                     for (int j = 0; j < 8; j++) x[i][j] = k + j < K ? x[i][j] : 0.f;
             }
         } else if constexpr (NLL) {
+            static_assert(ROWS / VEC == 64, "a k-chunk per wave");
             const int k = k0 + 8 * chunk_of(tid), r = row0 + row_of(tid);
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const int t = min(k + j, K - 1), h = (int)nll.target[t];
-                const float l = nll.lse[t], g = k + j < K && h >= 0 ? nll.gloss[t] : 0.f;
+                const float l = lane_of(lse[0], j), g = lane_of(gl[0], j);
+                const int h = __builtin_amdgcn_readlane(hit[0], j);
+                const float w = k + j < K && h >= 0 ? g : 0.f;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) x[0][8 * c + j] = nll_grad(x[0][8 * c + j], l, g, h == r + c);
+                for (int c = 0; c < VEC; c++) x[0][8 * c + j] = nll_grad(x[0][8 * c + j], l, w, h == r + c);
             }
         }
     }
@@ -172,6 +186,7 @@ struct GemmArgs {
     int64_t lda, ldb, ldc;
     int M, N, K;
     int ks;                      // k per range (a multiple of kBK)
+    int vec;                     // C, residual and gate can be accessed 16 bytes at a time
     int tm, tn;                  // tiles
     float *colsum;               // sums over k of A's rows, per range [M] (A contiguous along its rows), or NULL
     fwp_mm_epilogue epi;         // applied here when there is one range
@@ -182,8 +197,8 @@ struct GemmArgs {
 
 enum { kPlain = 0, kLse = 1, kGrad = 2 };
 
-__device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_t at, int n) {
-    if (e.bias) x += e.bias[n];
+// everything but the bias
+__device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_t at) {
     if (e.relu) x = fmaxf(x, 0.f);
     if (e.residual) x += e.residual[at];
     if (e.gate) x = e.gate[at] > 0.f ? x : 0.f;
@@ -191,12 +206,38 @@ __device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_
 }
 
 template <int X>
-__device__ __forceinline__ float row16_max(float x) {      // over the 16 lanes of a DPP row
-    return fmaxf(x, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true)));
+__device__ __forceinline__ float rotated(float x) {      // within the 16 lanes of a DPP row
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true));
 }
-template <int X>
-__device__ __forceinline__ float row16_add(float x) {
-    return x + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true));
+
+// LDS accesses of one wave execute in order; this keeps the compiler from moving them across.
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+// The largest of a row's logits and the sum of exp(logit - largest): four logits per lane, LANES (8 or 16) lanes per row.
+template <int LANES>
+__device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, float *out, int at, int pitch) {
+    if (n + 3 >= N) {
+        v.x = n < N ? v.x : -INFINITY, v.y = n + 1 < N ? v.y : -INFINITY;
+        v.z = n + 2 < N ? v.z : -INFINITY, v.w = -INFINITY;
+    }
+    float m = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w));
+    if constexpr (LANES == 16) {
+        m = fmaxf(m, rotated<8>(m));
+        m = fmaxf(m, rotated<4>(m)), m = fmaxf(m, rotated<2>(m)), m = fmaxf(m, rotated<1>(m));
+    } else {
+#pragma unroll
+        for (int o = 4; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    }
+    const float z = m == -INFINITY ? 0.f : m;
+    float s = (__expf(v.x - z) + __expf(v.y - z)) + (__expf(v.z - z) + __expf(v.w - z));
+    if constexpr (LANES == 16) {
+        s += rotated<8>(s);
+        s += rotated<4>(s), s += rotated<2>(s), s += rotated<1>(s);
+    } else {
+#pragma unroll
+        for (int o = 4; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    }
+    if (lane % LANES == 0) out[at] = m, out[at + pitch] = s;
 }
 
 // BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
@@ -231,8 +272,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
     const int lr = lane % 16, lc = lane / 16;
-    a.load(Ap, g.lda, ml, tid, kb, ke);
-    b.load(Bp, g.ldb, nl, tid, kb, ke);
+    a.load(Ap, g.lda, ml, tid, kb, ke, g.nll);
+    b.load(Bp, g.ldb, nl, tid, kb, ke, g.nll);
     for (int k0 = kb; k0 < ke; k0 += kBK) {
         a.finish(tid, m0, k0, ke, g.nll);
         b.finish(tid, n0, k0, ke, g.nll);
@@ -247,26 +288,32 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
         b.store(Lb, tid);
         lds_barrier();
         if (k0 + kBK < ke) {
-            a.load(Ap, g.lda, ml, tid, k0 + kBK, ke);
-            b.load(Bp, g.ldb, nl, tid, k0 + kBK, ke);
+            a.load(Ap, g.lda, ml, tid, k0 + kBK, ke, g.nll);
+            b.load(Bp, g.ldb, nl, tid, k0 + kBK, ke, g.nll);
         }
-        bf8 fa[3][MT], fb[3][NT];
+        // the products in an order in which three fragment sets are live at a time (six in the order of their size:
+        // 178 registers instead of 162, two workgroups on a CU instead of three)
+        bf8 a1[MT], a2[MT], b1[NT], b2[NT];
+        const auto read_a = [&](bf8 *d, int p) {
 #pragma unroll
-        for (int p = 0; p < 3; p++) {
+            for (int i = 0; i < MT; i++) d[i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lr]);
+        };
+        const auto read_b = [&](bf8 *d, int p) {
 #pragma unroll
-            for (int i = 0; i < MT; i++) fa[p][i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lr]);
-#pragma unroll
-            for (int j = 0; j < NT; j++) fb[p][j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lr]);
-        }
-        // the small products first
-        constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-        for (int q = 0; q < 6; q++)
+            for (int j = 0; j < NT; j++) d[j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lr]);
+        };
+        const auto products = [&](const bf8 *x, const bf8 *y) {
 #pragma unroll
             for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int j = 0; j < NT; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[PA[q]][i], fb[PB[q]][j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
+        };
+        read_a(a1, 2), read_b(b1, 0), products(a1, b1);      // l h'
+        read_a(a2, 1), products(a2, b1);                     // m h'
+        read_b(b2, 1), products(a2, b2);                     // m m'
+        read_a(a1, 0), products(a1, b2);                     // h m'
+        products(a1, b1);                                    // h h'
+        read_b(b2, 2), products(a1, b2);                     // h l'
         lds_barrier();
     }
 
@@ -282,74 +329,109 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
                 g.colsum[(int64_t)blockIdx.y * g.M + m0 + r] = (s[r] + s[BM + r]) + (s[2 * BM + r] + s[3 * BM + r]);
         }
     }
-    if constexpr (MODE == kLse) {
-        float *sm = reinterpret_cast<float *>(&La), *ss = sm + 2 * BM;      // [column half][row]
+    // A wave turns its rows round through LDS (its own: no barrier), 16 at a time, so that they leave, and the
+    // residual and the gate arrive, 16 bytes per lane: 4-byte accesses in the MFMA layout, 64-byte pieces of rows, cost
+    // 112 us where this costs 90 at 32768 x 1024, K = 256.
+    constexpr int kPitch = WN + 4;
+    static_assert(4 * 16 * kPitch <= (int)(sizeof(La) / 4), "four waves' strips fit the first operand's planes");
+    float *const strip = reinterpret_cast<float *>(&La) + wave * 16 * kPitch;
+    constexpr int kLanes = WN / 4, kRows = 64 / kLanes;      // lanes per row, rows per access
+    const int c4 = (lane % kLanes) * 4, n = n0 + wn + c4;
+    const bool vec = g.vec && n + 3 < g.N;
+    if constexpr (!AKC) __syncthreads();      // the column sums' reads of the same memory
+    float bias[4];
 #pragma unroll
-        for (int i = 0; i < MT; i++)
+    for (int e = 0; e < 4; e++) bias[e] = g.epi.bias && n + e < g.N && (gridDim.y == 1) ? g.epi.bias[n + e] : 0.f;
+    float *const C = g.C + (int64_t)blockIdx.y * g.M * g.ldc;
+    const bool one = gridDim.y == 1;
+    float *const sums_of = reinterpret_cast<float *>(&Lb);       // kLse: [2][column half][row]
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = wm + 16 * i + 4 * lc + r, m = m0 + row;
-                const int want = (int)g.nll.target[min(m, g.M - 1)];
-                float mx = -INFINITY;
+    for (int i = 0; i < MT; i++) {
 #pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    const int n = n0 + wn + 16 * j + lr;
-                    if (n < g.N && g.epi.bias) acc[i][j][r] += g.epi.bias[n];
-                    if (n >= g.N) acc[i][j][r] = -INFINITY;
-                    if (m < g.M && n == want) g.hit[m] = acc[i][j][r];
-                    mx = fmaxf(mx, acc[i][j][r]);
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) strip[(4 * lc + r) * kPitch + 16 * j + lr] = acc[i][j][r];
+        wave_lds_order();
+#pragma unroll
+        for (int q = 0; q < 16 / kRows; q++) {
+            const int row = kRows * q + lane / kLanes, m = m0 + wm + 16 * i + row;
+            float4 v = *reinterpret_cast<const float4 *>(strip + row * kPitch + c4);
+            v.x += bias[0], v.y += bias[1], v.z += bias[2], v.w += bias[3];
+            if constexpr (MODE == kLse) {
+                lse_of_row<kLanes>(v, n, g.N, lane, sums_of, (wave / 2) * BM + wm + 16 * i + row, 2 * BM);
+                if (g.hit && m < g.M) {
+                    const int at = (int)g.nll.target[m] - n;
+                    if (at >= 0 && at < 4 && n + at < g.N) g.hit[m] = at == 0 ? v.x : at == 1 ? v.y : at == 2 ? v.z : v.w;
                 }
-                mx = row16_max<1>(row16_max<2>(row16_max<4>(row16_max<8>(mx))));
-                float s = 0.f;
-#pragma unroll
-                for (int j = 0; j < NT; j++) s += mx == -INFINITY ? 0.f : __expf(acc[i][j][r] - mx);
-                s = row16_add<1>(row16_add<2>(row16_add<4>(row16_add<8>(s))));
-                if (lr == 0) {
-                    sm[(wave / 2) * BM + row] = mx;
-                    ss[(wave / 2) * BM + row] = s;
-                }
+                if (!g.C) continue;
             }
+            if (m >= g.M) continue;
+            const int64_t at = (int64_t)m * g.ldc + n;
+            if (vec) {
+                if (one) {
+                    if (g.epi.relu) v = make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f));
+                    if (g.epi.residual) {
+                        const float4 y = *reinterpret_cast<const float4 *>(g.epi.residual + at);
+                        v.x += y.x, v.y += y.y, v.z += y.z, v.w += y.w;
+                    }
+                    if (g.epi.gate) {
+                        const float4 y = *reinterpret_cast<const float4 *>(g.epi.gate + at);
+                        v = make_float4(y.x > 0.f ? v.x : 0.f, y.y > 0.f ? v.y : 0.f, y.z > 0.f ? v.z : 0.f, y.w > 0.f ? v.w : 0.f);
+                    }
+                }
+                *reinterpret_cast<float4 *>(C + at) = v;
+            } else {
+                const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < g.N) C[at + e] = one ? apply(g.epi, w[e], at + e) : w[e];
+            }
+        }
+        wave_lds_order();
+    }
+    if constexpr (MODE == kLse) {
         __syncthreads();
         for (int row = tid; row < min(BM, ml); row += kThreads) {
-            const float m1 = sm[row], m2 = sm[BM + row], mx = fmaxf(m1, m2);
-            const float s = ss[row] * __expf(m1 - mx) + (m2 == -INFINITY ? 0.f : ss[BM + row] * __expf(m2 - mx));
+            // the tile's first half of columns holds at least one; the second may hold none
+            const float m1 = sums_of[row], m2 = sums_of[BM + row], mx = fmaxf(m1, m2);
+            const float s2 = m2 == -INFINITY ? 0.f : sums_of[3 * BM + row] * __expf(m2 - mx);
             const int64_t at = (int64_t)(id % g.tn) * g.M + m0 + row;
             g.part_max[at] = mx;
-            g.part_sum[at] = s;
+            g.part_sum[at] = sums_of[2 * BM + row] * __expf(m1 - mx) + s2;
         }
-        if (!g.C) return;
     }
-    float *C = g.C + (int64_t)blockIdx.y * g.M * g.ldc;
-    const bool one = gridDim.y == 1 && MODE != kLse;
-#pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const int n = n0 + wn + 16 * j + lr;
-            if (n >= g.N) continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm + 16 * i + 4 * lc + r;
-                if (m >= g.M) continue;
-                const int64_t at = (int64_t)m * g.ldc + n;
-                C[at] = one ? apply(g.epi, acc[i][j][r], at, n) : acc[i][j][r];
-            }
-        }
 }
 
 // C[M,N] = the sum of `ranges` partial results, with the epilogue; four threads share four neighbouring
-// elements, a quarter of the ranges each, and add up in a fixed order.
+// elements, a quarter of the ranges each, and add up in a fixed order.  The workgroups behind them do the same for the
+// column sums of A ([ranges][M] behind the partial results).
 __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restrict__ part, float *__restrict__ C,
-                                                          int64_t total, int N, int ranges, fwp_mm_epilogue epi) {
+                                                          int64_t total, int M, int N, int ranges, fwp_mm_epilogue epi) {
     __shared__ float4 s[4][64];
     const int e = threadIdx.x % 64, q = threadIdx.x / 64;
+    const int64_t blocks = (total / 4 + 63) / 64;
+    if (blockIdx.x >= blocks) {
+        const float *const col = part + ranges * total;
+        const int m = (int)(blockIdx.x - blocks) * 64 + e;
+        float x = 0.f;
+        if (m < M) {
+#pragma unroll 4
+            for (int r = q; r < ranges; r += 4) x += col[(int64_t)r * M + m];
+        }
+        s[q][e].x = x;
+        __syncthreads();
+        if (q == 0 && m < M) epi.colsum[m] = (s[0][e].x + s[1][e].x) + (s[2][e].x + s[3][e].x);
+        return;
+    }
     const int64_t at = ((int64_t)blockIdx.x * 64 + e) * 4;
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (at < total)
+    if (at < total) {
+#pragma unroll 4
         for (int r = q; r < ranges; r += 4) {
             const float4 y = *reinterpret_cast<const float4 *>(part + r * total + at);
             x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
         }
+    }
     s[q][e] = x;
     __syncthreads();
     if (q || at >= total) return;
@@ -357,20 +439,12 @@ __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restric
         const float4 y = s[o][e];
         x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
     }
-    const int n = (int)(at % N);
-    float4 y;
-    y.x = apply(epi, x.x, at, n), y.y = apply(epi, x.y, at + 1, n + 1);
-    y.z = apply(epi, x.z, at + 2, n + 2), y.w = apply(epi, x.w, at + 3, n + 3);
+    if (epi.bias) {
+        const float *b = epi.bias + (int)(at % N);
+        x.x += b[0], x.y += b[1], x.z += b[2], x.w += b[3];
+    }
+    const float4 y = make_float4(apply(epi, x.x, at), apply(epi, x.y, at + 1), apply(epi, x.z, at + 2), apply(epi, x.w, at + 3));
     *reinterpret_cast<float4 *>(C + at) = y;
-}
-
-__global__ __launch_bounds__(kThreads) void k_sum_ranges(const float *__restrict__ part, float *__restrict__ out, int n,
-                                                         int ranges) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    float x = 0.f;
-    for (int r = 0; r < ranges; r++) x += part[(int64_t)r * n + i];
-    out[i] = x;
 }
 
 struct Plan {
@@ -406,8 +480,10 @@ void launch(const GemmArgs &g, const Plan &p, hipStream_t s) {
     else hipLaunchKernelGGL((k_gemm<AKC, BKC, 64, 64, MODE>), grid, dim3(kThreads), 0, s, g);
 }
 
+bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 bool may_cut(int N, const float *C, int64_t ldc) {
-    return ldc == N && N % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+    return ldc == N && N % 4 == 0 && aligned(C);
 }
 
 }  // namespace
@@ -427,6 +503,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     const bool cut = p.ranges > 1;
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
+    g.vec = g.ldc % 4 == 0 && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
     float *const col = cut ? workspace + (int64_t)p.ranges * M * N : epi.colsum;
     g.colsum = layout == FWP_MM_TN && epi.colsum ? col : nullptr;
     if (layout == FWP_MM_NT) launch<true, true, kPlain>(g, p, s);
@@ -435,12 +512,8 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     else if (!nll) launch<false, false, kPlain>(g, p, s);
     else launch<false, false, kGrad>(g, p, s);
     if (cut) {
-        const int64_t total = (int64_t)M * N;
-        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((total / 4 + 63) / 64)), dim3(kThreads), 0, s, workspace, C, total,
-                           N, p.ranges, epi);
-        if (g.colsum)
-            hipLaunchKernelGGL(k_sum_ranges, dim3((M + kThreads - 1) / kThreads), dim3(kThreads), 0, s, col, epi.colsum, M,
-                               p.ranges);
+        const int64_t total = (int64_t)M * N, blocks = (total / 4 + 63) / 64 + (g.colsum ? (M + 63) / 64 : 0);
+        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)blocks), dim3(kThreads), 0, s, workspace, C, total, M, N, p.ranges, epi);
     }
     return (int)hipGetLastError();
 }
@@ -450,9 +523,9 @@ namespace {
 // loss = lse - logit of the target (0 for a negative target), lse from the tiles' maxima and sums; four threads
 // share a row, a quarter of the tiles each
 __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part_max, const float *__restrict__ part_sum,
-                                                  const float *__restrict__ hit, const int64_t *__restrict__ target,
-                                                  float *__restrict__ loss, float *__restrict__ lse, int rows, int vocab,
-                                                  int tiles) {
+                                                  const float *__restrict__ hit, const float *__restrict__ logits,
+                                                  const int64_t *__restrict__ target, float *__restrict__ loss, float *__restrict__ lse,
+                                                  int rows, int vocab, int tiles) {
     __shared__ float sm[4][64], ss[4][64];
     const int e = threadIdx.x % 64, q = threadIdx.x / 64, m = blockIdx.x * 64 + e;
     float mx = -INFINITY, s = 0.f;
@@ -474,7 +547,7 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
     const float l = mx + __logf(s);
     const int64_t want = target[m];
     if (lse) lse[m] = l;
-    loss[m] = want < 0 ? 0.f : want < vocab ? l - hit[m] : NAN;
+    loss[m] = want < 0 ? 0.f : want < vocab ? l - (logits ? logits[(int64_t)m * vocab + want] : hit[m]) : NAN;
 }
 
 }  // namespace
@@ -491,10 +564,11 @@ int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *ta
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
     g.part_max = workspace;
     g.part_sum = workspace + (int64_t)p.tn * rows;
-    g.hit = g.part_sum + (int64_t)p.tn * rows;
+    g.hit = logits ? nullptr : g.part_sum + (int64_t)p.tn * rows;
+    g.vec = vocab % 4 == 0 && aligned(logits);
     launch<true, true, kLse>(g, p, s);
-    hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, target, loss, lse,
-                       rows, vocab, p.tn);
+    hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, logits, target, loss,
+                       lse, rows, vocab, p.tn);
     return (int)hipGetLastError();
 }
 

@@ -124,8 +124,10 @@ __global__ __launch_bounds__(256) void k_norm_params(const float *__restrict__ p
     __shared__ float sh[16][17];
     const int c = threadIdx.x % 16, q = threadIdx.x / 16, col = blockIdx.x * 16 + c;
     float s = 0.f;
-    if (col < 2 * cols)
+    if (col < 2 * cols) {
+#pragma unroll 8
         for (int b = q; b < blocks; b += 16) s += part[(int64_t)b * 2 * cols + col];
+    }
     sh[q][c] = s;
     __syncthreads();
     if (q || col >= 2 * cols) return;
