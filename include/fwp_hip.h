@@ -319,6 +319,26 @@ int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, cons
                        float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream);
 
 /*
+ * Decoding: one token per sequence.  A product of up to 64 rows with a layer's weights,
+ *   out = relu(x W^T + bias) + residual   (each part optional), x [rows,K], W [N,K], residual and out [rows,N],
+ * with LayerNorm on x when gamma and beta are given (y, when given, receives the normalised rows).
+ * K must be a multiple of 64, and at most 1024 with LayerNorm.  All pointers 16-byte aligned.
+ */
+int fwp_rows_matmul(const float *x, const float *gamma, const float *beta, float eps, float *y, const float *W,
+                    const float *bias, const float *residual, int relu, float *out, int rows, int N, int K,
+                    void *stream);
+
+/* fwp_deltanet_prep_fwd and a single step of fwp_delta_fwd in one: qkvb [B,H,3D+1] to out [B,H,D] (q_scale as there), the
+ * state [B,H,D,D] read from `from` (NULL: zero) and written to `to` (which may be the same).  D in {16, 32, 64}. */
+int fwp_deltanet_step(const float *qkvb, const float *from, float *to, float *out, int B, int H, int D,
+                      float q_scale, void *stream);
+
+/* The model's input (language_modeling/src/model_main.py:836-898,1267-1303): out [T,B,d] = table[ids] * scale + the
+ * sinusoidal embedding of the positions T-1 .. 0 (at most `clamp` when that is positive); inv_freq [d/2], d even. */
+int fwp_embed(const float *table, const int64_t *ids, const float *inv_freq, float *out, int T, int B, int d,
+              long long n_token, float scale, float clamp, void *stream);
+
+/*
  * Recurrent Delta Net forward.  Replaces rec_update_fwm_tanh_forward
  * (algorithmic/rec_update_fwm_tanh/rec_update_fwm_tanh.cu:349-444, kernel :25-345).
  *   qx,kx,vx [N,H,L,D] and bx [N,H,L,1] are pre-activation

@@ -62,6 +62,9 @@ _MODEL_SIGNATURES = {
     "fwp_nll_bwd": [_P] * 10 + [_I] * 3 + [_P],
     "fwp_layer_norm_fwd": [_P] * 5 + [_I] * 2 + [ctypes.c_float, _P],
     "fwp_layer_norm_bwd": [_P] * 8 + [_I] * 2 + [_P],
+    "fwp_rows_matmul": [_P] * 3 + [ctypes.c_float] + [_P] * 4 + [_I, _P] + [_I] * 3 + [_P],
+    "fwp_deltanet_step": [_P] * 4 + [_I] * 3 + [ctypes.c_float, _P],
+    "fwp_embed": [_P] * 4 + [_I] * 3 + [_L, ctypes.c_float, ctypes.c_float, _P],
 }
 _WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
 EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",

@@ -449,6 +449,29 @@ int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, cons
     return layer_norm_bwd(gy, x, stats, gamma, gx, ggamma, gbeta, workspace, rows, cols, (hipStream_t)stream);
 }
 
+int fwp_rows_matmul(const float *x, const float *gamma, const float *beta, float eps, float *y, const float *W,
+                    const float *bias, const float *residual, int relu, float *out, int rows, int N, int K, void *stream) {
+    if (!x || !W || !out || (gamma == nullptr) != (beta == nullptr)) return FWP_E_NULL;
+    if (N < 1 || !rows_supported(rows, K, gamma != nullptr)) return FWP_E_SHAPE;
+    for (const void *p : {(const void *)x, (const void *)gamma, (const void *)beta, (const void *)y, (const void *)W})
+        if (!aligned16(p)) return FWP_E_SHAPE;
+    return rows_matmul(x, gamma, beta, eps, y, W, bias, residual, relu, out, rows, N, K, (hipStream_t)stream);
+}
+
+int fwp_deltanet_step(const float *qkvb, const float *from, float *to, float *out, int B, int H, int D, float q_scale,
+                      void *stream) {
+    if (!qkvb || !to || !out) return FWP_E_NULL;
+    if (B < 1 || H < 1 || !prep_supported(D) || !aligned16(from) || !aligned16(to) || !aligned16(out)) return FWP_E_SHAPE;
+    return layer_step(qkvb, from, to, out, B, H, D, q_scale, (hipStream_t)stream);
+}
+
+int fwp_embed(const float *table, const int64_t *ids, const float *inv_freq, float *out, int T, int B, int d,
+              long long n_token, float scale, float clamp, void *stream) {
+    if (!table || !ids || !inv_freq || !out) return FWP_E_NULL;
+    if (T < 1 || B < 1 || d < 2 || d % 2 || n_token < 1) return FWP_E_SHAPE;
+    return embed(table, ids, inv_freq, out, T, B, d, n_token, scale, clamp, (hipStream_t)stream);
+}
+
 int fwp_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float *Rq,
                 const float *Rk, const float *Rv, const float *rb, float *W, float *h, float *out,
                 float *q_act, float *k_act, float *beta_act, float *vdiff, float *ckpt, int N,

@@ -206,6 +206,14 @@ int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float 
 int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
                    float *ggamma, float *gbeta, float *workspace, int rows, int cols, hipStream_t s);
 
+// One token per sequence through the language model's layers (up to 64 rows), and its embedding.
+bool rows_supported(int rows, int K, bool norm);
+int rows_matmul(const float *x, const float *gamma, const float *beta, float eps, float *y, const float *W, const float *bias,
+                const float *residual, int relu, float *out, int rows, int N, int K, hipStream_t s);
+int layer_step(const float *qkvb, const float *from, float *to, float *out, int B, int H, int D, float q_scale, hipStream_t s);
+int embed(const float *table, const int64_t *ids, const float *inv_freq, float *out, int T, int B, int d, int64_t n_token,
+          float scale, float clamp, hipStream_t s);
+
 // Largest dynamic LDS allocation the LDS-state kernels ask for (bytes).
 constexpr size_t kMaxLds = 160 * 1024 - 1024;
 

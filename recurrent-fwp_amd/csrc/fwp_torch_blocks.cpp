@@ -8,6 +8,7 @@
 // operators and differentiates that.
 #include "fwp_torch.hpp"
 
+#include <cmath>
 #include <optional>
 #include <tuple>
 #include <vector>
@@ -76,7 +77,16 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
         fwp_mm_epilogue e{};
         e.bias = ptr(bias);
         e.relu = relu;
-        const at::Tensor y = matmul(FWP_MM_NT, x, W, rows, out, in, shape, e);
+        at::Tensor y;
+        if (rows <= 64 && in >= 64 && in % 64 == 0) {       // few rows: latency counts (fwp_decode.hip)
+            y = at::empty(shape, x.options());
+            const at::Tensor w = plain(W);
+            check(fwp_rows_matmul(ptr(x), nullptr, nullptr, 0.f, nullptr, ptr(w), ptr(bias), nullptr, relu, ptr(y), (int)rows, (int)out,
+                                  (int)in, stream_of(x)),
+                  "fwp_rows_matmul");
+        } else {
+            y = matmul(FWP_MM_NT, x, W, rows, out, in, shape, e);
+        }
         if (ctx) {
             ctx->save_for_backward({x_in, W, bias, relu ? y : at::Tensor()});
             ctx->set_materialize_grads(false);
@@ -366,6 +376,99 @@ struct NllFn : torch::autograd::Function<NllFn> {
     }
 };
 
+// ------------------------------------------------------------------ decoding
+
+// A layer's parameters: qkvb_net.weight, o_net.weight, dec_attn.layer_norm weight and bias, CoreNet.0 weight and
+// bias, CoreNet.3 weight and bias, pos_ff.layer_norm weight and bias.
+constexpr size_t kPerLayer = 10;
+
+// One token per sequence through the layers: x [1,B,d], states [B,H,D,D] per layer (empty: zeros) ->
+// (hidden [1,B,d], the states after the token).  Nothing is recorded.
+std::tuple<at::Tensor, std::vector<at::Tensor>> decode_layers(const at::Tensor &x_in, const std::vector<at::Tensor> &params,
+                                                              const std::vector<at::Tensor> &states, int64_t H, int64_t D,
+                                                              double eps, bool pre_norm) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    require_device(x_in);
+    const size_t layers = params.size() / kPerLayer;
+    require(params.size() == layers * kPerLayer && (states.empty() || states.size() == layers) && x_in.dim() == 3 && x_in.size(0) == 1,
+            "one token per sequence, ten parameters and one state per layer");
+    const at::Tensor x = plain(x_in);
+    const int64_t B = x.size(1), d = x.size(2), width = H * (3 * D + 1);
+    const auto opts = x.options();
+    LaunchGuard guard(x);
+    void *const s = stream_of(x);
+    int64_t inner_most = 0;
+    for (size_t l = 0; l < layers; l++) {
+        const at::Tensor *p = &params[kPerLayer * l];
+        const int64_t inner = p[4].size(0);
+        bool ok = same_shape(p[0], {width, d}) && same_shape(p[1], {d, H * D}) && same_shape(p[4], {inner, d}) &&
+                  same_shape(p[5], {inner}) && same_shape(p[6], {d, inner});
+        for (size_t i : {2, 3, 7, 8, 9}) ok = ok && same_shape(p[i], {d});
+        for (size_t i = 0; i < kPerLayer; i++) {
+            same_device(x, {p[i]});
+            ok = ok && p[i].scalar_type() == at::kFloat && p[i].is_contiguous() &&
+                 reinterpret_cast<uintptr_t>(p[i].data_ptr()) % 16 == 0;
+        }
+        if (!ok) fail("parameters must be contiguous fp32 tensors of the model's sizes");
+        inner_most = std::max(inner_most, inner);
+    }
+    // one buffer for everything in between; the states in another (the caller keeps them)
+    const int64_t rows_d = (B * d + 3) & ~int64_t(3);
+    const at::Tensor work = at::empty({B * width + 4 + B * H * D + 4 * rows_d + B * inner_most}, opts);
+    float *const a = ptr(work), *const b = a + rows_d, *const y = b + rows_d, *const h2 = y + rows_d, *const out = h2 + rows_d,
+                *const hid = out + B * H * D, *const qkvb = hid + B * inner_most;
+    const at::Tensor result = at::empty({1, B, d}, opts), after = at::empty({(int64_t)layers, B, H, D, D}, opts);
+    const float *const none = nullptr;
+    const auto product = [&](const float *in, const at::Tensor *g, const at::Tensor *be, float *norm, const at::Tensor &W,
+                             const at::Tensor *bias, const float *residual, int relu, float *to) {
+        check(fwp_rows_matmul(in, g ? ptr(*g) : none, be ? ptr(*be) : none, (float)eps, norm, ptr(W), bias ? ptr(*bias) : none, residual,
+                              relu, to, (int)B, (int)W.size(0), (int)W.size(1), s),
+              "fwp_rows_matmul");
+    };
+    const float *in = ptr(x);       // the layer's input, before the last layer's LayerNorm (post-norm)
+    for (size_t l = 0; l < layers; l++) {
+        const at::Tensor *p = &params[kPerLayer * l], *before = pre_norm ? p + 2 : l ? p - 2 : nullptr;
+        at::Tensor from;
+        if (!states.empty()) {
+            from = plain(states[l]);
+            same_device(x, {from});
+            require(same_shape(from, {B, H, D, D}), "a state does not fit [bsz, n_head, d_head, d_head]");
+        }
+        // post-norm: LN of the previous layer's sum on the way in, that is also the residual; pre-norm: this layer's
+        product(in, before, before ? before + 1 : nullptr, before ? y : nullptr, p[0], nullptr, none, 0, qkvb);
+        check(fwp_deltanet_step(qkvb, ptr(from), ptr(after) + l * B * H * D * D, out, (int)B, (int)H, (int)D,
+                                (float)(1.0 / std::sqrt((double)D)), s),
+              "fwp_deltanet_step");
+        product(out, nullptr, nullptr, nullptr, p[1], nullptr, before ? y : in, 0, a);
+        // feed-forward: post-norm adds the normalised rows back, pre-norm the rows themselves
+        const at::Tensor *norm = pre_norm ? p + 8 : p + 2;
+        product(a, norm, norm + 1, pre_norm ? nullptr : h2, p[4], &p[5], none, 1, hid);
+        float *const to = pre_norm && l + 1 == layers ? ptr(result) : b;
+        product(hid, nullptr, nullptr, nullptr, p[6], &p[7], pre_norm ? a : h2, 0, to);
+        in = to;
+    }
+    if (!pre_norm) {
+        const at::Tensor *p = &params[kPerLayer * (layers - 1)];
+        check(fwp_layer_norm_fwd(in, ptr(p[8]), ptr(p[9]), ptr(result), nullptr, (int)B, (int)d, (float)eps, s), "fwp_layer_norm_fwd");
+    }
+    return {result, after.unbind(0)};
+}
+
+// word embedding times scale plus the positions' sinusoids, for ids [T,B]; nothing is recorded
+at::Tensor embed(const at::Tensor &table, const at::Tensor &ids, const at::Tensor &inv_freq, double scale, double clamp) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    require_device(table);
+    same_device(table, {ids, inv_freq});
+    const int64_t T = ids.size(0), B = ids.size(1), d = table.size(1);
+    require(ids.scalar_type() == at::kLong && inv_freq.numel() * 2 == d, "int64 ids [len, bsz] and d_model/2 frequencies");
+    const at::Tensor t = plain(table), i = ids.contiguous(), f = plain(inv_freq), out = at::empty({T, B, d}, t.options());
+    LaunchGuard guard(t);
+    check(fwp_embed(ptr(t), i.data_ptr<int64_t>(), ptr(f), ptr(out), (int)T, (int)B, (int)d, t.size(0), (float)scale, (float)clamp,
+                    stream_of(t)),
+          "fwp_embed");
+    return out;
+}
+
 bool records(std::initializer_list<const at::Tensor *> ts) {
     if (!at::GradMode::is_enabled()) return false;
     for (const at::Tensor *t : ts)
@@ -416,6 +519,8 @@ void bind_blocks(py::module_ &m) {
           "x W^T (+ bias) (relu)");
     m.def("feed_forward", &feed_forward, py::arg("x"), py::arg("W1"), py::arg("b1"), py::arg("W2"), py::arg("b2"),
           py::arg("residual") = py::none(), "relu(x W1^T + b1) W2^T + b2 (+ residual)");
+    m.def("decode_layers", &decode_layers, "one token per sequence through the layers -> (hidden, states); records nothing");
+    m.def("embed", &embed, "the model's input from token ids; records nothing");
     m.def("layer_norm", &layer_norm, "LayerNorm over the last axis (a multiple of 4 up to 1024)");
     m.def("nll", &nll, "per-row negative log-likelihood of the targets under softmax(x W^T + bias); a negative target counts 0");
     m.def("delta_block", &delta_block, "the Delta-Net layer between its input and its LayerNorm; the state is updated in place");

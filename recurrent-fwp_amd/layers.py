@@ -43,6 +43,50 @@ def _drops(m):
     return m.training and m.p > 0
 
 
+class Linear(nn.Linear):
+    """``nn.Linear`` on the package's matrix products where they apply."""
+
+    def forward(self, x):
+        if self.bias is not None and x.dim() > 0 and x.shape[-1] == self.in_features:
+            blocks = _blocks(x, self.weight, self.bias)
+            if blocks is not None:
+                return blocks.linear(x, self.weight, self.bias)
+        return super().forward(x)
+
+
+def decode_parameters(layer):
+    """The parameters of a :class:`DeltaNetDecoderLayer` as ``decode_layers`` takes them, or ``None`` when the layer
+    is not what that function computes: a replaced or hooked sub-module, an active dropout, another operator."""
+    if not (_untouched(layer, DeltaNetDecoderLayer)):
+        return None
+    att, ff = layer._modules["dec_attn"], layer._modules["pos_ff"]
+    if not (_untouched(att, DeltaNetLayer) and _untouched(ff, PositionwiseFF)) or att.fast_weight_op is not fast_weight_delta:
+        return None
+    a, f = att._modules, ff._modules
+    net = f["CoreNet"]
+    if not (_untouched(net, nn.Sequential) and len(net._modules) == 5):
+        return None
+    lin1, relu, drop1, lin2, drop2 = net._modules.values()
+    norms = (a["layer_norm"], f["layer_norm"])
+    for m in (a["qkvb_net"], a["o_net"], lin1, lin2):
+        if not _untouched(m, nn.Linear):
+            return None
+    for m in (a["drop"], drop1, drop2):
+        if not _untouched(m, nn.Dropout) or _drops(m):
+            return None
+    for m in norms:
+        if not _untouched(m, nn.LayerNorm) or m.eps != norms[0].eps:
+            return None
+    if not _untouched(relu, nn.ReLU) or att.pre_lnorm != ff.pre_lnorm:
+        return None
+    if a["qkvb_net"]._parameters["bias"] is not None or a["o_net"]._parameters["bias"] is not None:
+        return None
+    params = [a["qkvb_net"]._parameters["weight"], a["o_net"]._parameters["weight"]]
+    for m in (norms[0], lin1, lin2, norms[1]):
+        params += [m._parameters["weight"], m._parameters["bias"]]
+    return None if any(p is None for p in params) else params
+
+
 def _layer_norm(m, x):
     """``m(x)`` for a LayerNorm over the last axis."""
     if _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:

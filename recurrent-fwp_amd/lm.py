@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import DeltaNetDecoderLayer, PositionalEmbedding, _blocks, _untouched
+from .layers import DeltaNetDecoderLayer, DeltaNetLayer, Linear, PositionalEmbedding, _blocks, _drops, _untouched, decode_parameters
 
 
 class _WordEmbedding(nn.Module):
@@ -33,11 +33,11 @@ class _TiedSoftmaxLoss(nn.Module):
 
     def __init__(self, n_token, d_model):
         super().__init__()
-        self.out_layers = nn.ModuleList([nn.Linear(d_model, n_token)])
+        self.out_layers = nn.ModuleList([Linear(d_model, n_token)])
 
     def forward(self, hidden, target):
         out = self.out_layers[0]
-        blocks = _blocks(hidden, out.weight, out.bias) if _untouched(out, nn.Linear) and out.bias is not None else None
+        blocks = _blocks(hidden, out.weight, out.bias) if _untouched(out, Linear) and out.bias is not None else None
         if blocks is not None and target.dtype is torch.int64 and target.device == hidden.device:
             return blocks.nll(hidden, out.weight, out.bias, target)
         return F.cross_entropy(out(hidden), target, reduction="none")
@@ -78,14 +78,61 @@ class DeltaNetLM(nn.Module):
                 nn.init.normal_(m.weight, 1.0, std)
                 nn.init.zeros_(m.bias)
 
+    def _embed(self, data):
+        """Word and position embedding of ``data`` where nothing is recorded for a backward pass, in one kernel; or ``None``."""
+        word, pos = self.word_emb, self.pos_emb
+        if torch.is_grad_enabled() or data.dim() != 2 or data.dtype is not torch.int64 or not data.is_cuda:
+            return None
+        if not (_untouched(word, _WordEmbedding) and _untouched(word.emb_layers[0], nn.Embedding) and _untouched(pos, PositionalEmbedding)):
+            return None
+        table = word.emb_layers[0]
+        if table.max_norm is not None or data.numel() == 0 or pos.inv_freq.dtype is not torch.float32:
+            return None
+        blocks = _blocks(table.weight, table.weight)
+        return None if blocks is None else blocks.embed(table.weight, data, pos.inv_freq, word.emb_scale, self.clamp_len)
+
+    def _decode(self, x, mems):
+        """One token per sequence through all layers in one call, where nothing is recorded: ``(hidden, states)`` or ``None``."""
+        if x.shape[0] != 1 or not 1 <= x.shape[1] <= 64 or torch.is_grad_enabled() or len(self.layers) == 0:
+            return None
+        if mems is not None and len(mems) < len(self.layers):
+            return None
+        att = self.layers[0].dec_attn
+        if not isinstance(att, DeltaNetLayer) or att.d_head not in (16, 32, 64) or self.d_model % 64 or self.d_model > 1024:
+            return None
+        params = []
+        for layer in self.layers:
+            p = decode_parameters(layer)
+            a = layer._modules.get("dec_attn")
+            if (p is None or a.n_head != att.n_head or a.d_head != att.d_head or a.pre_lnorm != att.pre_lnorm
+                    or a.layer_norm.eps != att.layer_norm.eps or p[4].shape[0] % 64):
+                return None
+            params += p
+        if (att.n_head * att.d_head) % 64:
+            return None
+        blocks = _blocks(x, *params)
+        if blocks is None:
+            return None
+        states = [] if mems is None else [m[0][:x.shape[1]] for m in mems[:len(self.layers)]]
+        return blocks.decode_layers(x, params, states, att.n_head, att.d_head, att.layer_norm.eps, att.pre_lnorm)
+
     def hidden(self, data, mems=None, carry_over_fast_weight=False):
-        qlen = data.shape[0]
-        emb = self.word_emb(data)
-        # Positions count down to zero at the newest token (model_main.py:1273-1280).
-        pos_seq = torch.arange(qlen - 1, -1, -1.0, device=emb.device, dtype=emb.dtype)
-        if self.clamp_len > 0:
-            pos_seq.clamp_(max=self.clamp_len)
-        out = self.drop(emb + self.pos_emb(pos_seq))
+        emb = self._embed(data)
+        if emb is None:
+            # Positions count down to zero at the newest token (model_main.py:1273-1280).
+            emb = self.word_emb(data)
+            pos_seq = torch.arange(data.shape[0] - 1, -1, -1.0, device=emb.device, dtype=emb.dtype)
+            if self.clamp_len > 0:
+                pos_seq.clamp_(max=self.clamp_len)
+            emb = emb + self.pos_emb(pos_seq)
+        elif not _drops(self.drop) and (carry_over_fast_weight or mems is None):
+            done = self._decode(emb, mems)
+            if done is not None:
+                hid, states = done
+                return self.drop(hid), ([(W, None) for W in states] if carry_over_fast_weight else None)
+        return self._through_layers(self.drop(emb), mems, carry_over_fast_weight)
+
+    def _through_layers(self, out, mems, carry_over_fast_weight):
         new_mems = []
         for i, layer in enumerate(self.layers):
             out = layer(out, mems=None if mems is None else mems[i],

@@ -102,9 +102,44 @@ def test_language_model_with_ignored_targets(fwp, pre):
     close("loss", loss, want)
     assert bool((loss[5:9, 1] == 0).all())
     with torch.no_grad():
-        assert torch.equal(ours(data, target)[0], loss)
+        close("loss without a graph", ours(data, target)[0], want)
     w = torch.randn(45, 3, generator=g).cuda()
     (loss * w).sum().backward()
     (want * w.double()).sum().backward()
     for (name, a), (_, b) in zip(ours.named_parameters(), ref.named_parameters()):
         close(name, a.grad, b.grad, 16)
+
+
+@pytest.mark.parametrize("B,D,dm,inner,pre", [(1, 16, 128, 64, False), (5, 32, 128, 192, True), (17, 32, 256, 2048, False),
+                                              (33, 64, 1024, 128, True), (64, 16, 64, 1088, False), (50, 16, 64, 64, True),
+                                              (65, 16, 128, 64, False)])       # 65: the layers one by one
+def test_decoding_one_token_at_a_time(fwp, B, D, dm, inner, pre):
+    """Hidden states, logits and carried states of three tokens, the first without a state, against float64."""
+    cfg = dict(n_token=150, n_layer=2, n_head=4, d_model=dm, d_head=D, d_inner=inner, pre_lnorm=pre)
+    torch.manual_seed(0)
+    ours = fwp.DeltaNetLM(init_std=0.2, **cfg).cuda()
+    ref = fwp.DeltaNetLM(fast_weight_op=loop_op, init_std=0.2, **cfg).cuda().double()
+    ref.load_state_dict(ours.state_dict())
+    toks = torch.randint(0, 150, (3, 1, B), generator=torch.Generator().manual_seed(1)).cuda()
+    mems = mems_ref = None
+    with torch.no_grad():
+        for t in toks:
+            hid, mems = ours.hidden(t, mems, carry_over_fast_weight=True)
+            want, mems_ref = ref.hidden(t, mems_ref, carry_over_fast_weight=True)
+            close("hidden", hid, want)
+            close("logits", ours.crit.out_layers[0](hid), ref.crit.out_layers[0](want))
+            for (W, _), (W_ref, _) in zip(mems, mems_ref):
+                close("state", W, W_ref)
+        assert torch.equal(ours.hidden(toks[0])[0], ours.hidden(toks[0], carry_over_fast_weight=True)[0])
+
+
+@pytest.mark.parametrize("T,clamp", [(1, -1), (300, -1), (70, 20)])
+def test_embedding_without_a_graph(fwp, T, clamp):
+    """The fused embedding against the lines it replaces (they run when a graph is recorded)."""
+    lm = fwp.DeltaNetLM(n_token=50, n_layer=1, n_head=2, d_model=36, d_head=16, d_inner=32, clamp_len=clamp).cuda()
+    lm.layers = torch.nn.ModuleList()
+    data = torch.randint(0, 50, (T, 3), generator=torch.Generator().manual_seed(1)).cuda()
+    want, _ = lm.hidden(data)
+    with torch.no_grad():
+        got, _ = lm.hidden(data)
+    assert float((got - want.detach()).abs().max()) <= 2.0 ** -22
