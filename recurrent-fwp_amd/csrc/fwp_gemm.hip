@@ -13,8 +13,14 @@
 // The operands are split on their way from global memory to LDS, in the registers of the thread that loads
 // them: 11 vector instructions per two numbers, 45 % of the matrix instructions' time in a 128 x 128 tile, and
 // issued beside them by the other workgroups of the CU.  LDS holds 16-byte units of 8 consecutive k of one row,
-// [plane][k / 8][row], so that a fragment is one ds_read_b128 of consecutive addresses; an operand that is
-// contiguous along its rows instead of along k is transposed in registers on the way.
+// [plane][k / 8][row], so that a fragment is one ds_read_b128; an operand that is contiguous along its rows
+// instead of along k is transposed in registers on the way.
+//
+// What bounds it: 32768 x 256, K = 1024 takes 93 us, 1.1 PFLOP/s of bf16 products.  Matrix instructions, fragment reads and
+// barriers alone take 67 us (1.56 PFLOP/s), the LDS writes 15 us more, the split 5-10 us, loads that miss the cache 5 us; the
+// clock falls to 1.8-1.9 GHz, so that cycles saved come back as time only in part.  Tried without gain: 256 x 128 tiles
+// (256 registers, spills: 113 us), fragments fetched a dozen matrix instructions ahead (97 us), remainders by
+// v_dot2_f32_bf16 (fewer instructions, 101 us, and it drops denormals).
 #include "fwp_common.hpp"
 #include "fwp_mfma.hpp"
 
@@ -30,7 +36,6 @@ typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kBK = 32;          // k per LDS tile
-constexpr int kPad = 2;          // units after a k-chunk's rows: the chunks of a row start 32 bytes apart in the banks
 constexpr int kThreads = 256;
 constexpr unsigned kOut = 0x80000000u;      // an offset beyond every buffer: reads as zero
 
@@ -52,8 +57,15 @@ __device__ __forceinline__ float lane_of(float x, int lane) {
 
 template <int ROWS>
 struct Planes {
-    v4u u[3][kBK / 8][ROWS + kPad];
+    v4u u[3][kBK / 8][ROWS];
 };
+
+// The place of a row's unit in its k-chunk, such that no access meets a bank twice: a read takes lanes 0-3, 12-15, 20-23
+// and 24-27 together (two chunks' rows: whole groups of four, whichever chunk), a write eight lanes, which hold two rows x
+// four chunks (operands contiguous along k) or every other of sixteen rows (the others).  With rows in order and the
+// chunks 32 bytes apart 420 of 1280 LDS cycles per tile step (x W^T), 770 of 1560 (g^T x) were conflicts; 32768 x 256,
+// K = 1024: 4.7e7 -> 4.3e7 cycles of busy CUs, 95.0 -> 92.9 us.
+__device__ __forceinline__ constexpr int unit_of(int row, int chunk) { return row ^ (2 * chunk) ^ ((row >> 3) & 1); }
 
 // What turns stored logits into the gradient of the loss as an operand is loaded:
 // (exp(logit - lse[token]) - [vocabulary entry == target[token]]) * gloss[token], 0 for a negative target
@@ -173,9 +185,10 @@ struct Operand {
                     l[j] = pack2(ra - low_f(m[j]), rb - high_f(m[j]));
                 }
                 const int r = row_of(tid + i * kThreads) + c, ch = chunk_of(tid + i * kThreads);
-                L.u[0][ch][r] = h;
-                L.u[1][ch][r] = m;
-                L.u[2][ch][r] = l;
+                const int at = unit_of(r, ch);
+                L.u[0][ch][at] = h;
+                L.u[1][ch][at] = m;
+                L.u[2][ch][at] = l;
             }
     }
 };
@@ -271,7 +284,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int lr = lane % 16, lc = lane / 16;
+    const int lr = lane % 16, lc = lane / 16, lu = unit_of(lr, lc);
     a.load(Ap, g.lda, ml, tid, kb, ke, g.nll);
     b.load(Bp, g.ldb, nl, tid, kb, ke, g.nll);
     for (int k0 = kb; k0 < ke; k0 += kBK) {
@@ -296,11 +309,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
         bf8 a1[MT], a2[MT], b1[NT], b2[NT];
         const auto read_a = [&](bf8 *d, int p) {
 #pragma unroll
-            for (int i = 0; i < MT; i++) d[i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lr]);
+            for (int i = 0; i < MT; i++) d[i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lu]);
         };
         const auto read_b = [&](bf8 *d, int p) {
 #pragma unroll
-            for (int j = 0; j < NT; j++) d[j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lr]);
+            for (int j = 0; j < NT; j++) d[j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lu]);
         };
         const auto products = [&](const bf8 *x, const bf8 *y) {
 #pragma unroll
