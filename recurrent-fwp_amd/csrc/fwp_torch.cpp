@@ -675,9 +675,7 @@ void set_error_class(py::object cls) {
 
 }  // namespace
 
-#ifndef FWP_HOST_STUB
 void bind_blocks(py::module_ &m);       // fwp_torch_blocks.cpp
-#endif
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     py::register_exception_translator([](std::exception_ptr p) {
@@ -702,8 +700,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("fast_lstm_v4", &fast_lstm_v4,
           "rnn_out, cell_out = fast_lstm_v4(Zi, Ki, Vi, bi, Wi, Zu, Ku, Vu, bu, Wu, Zo, Ko, Vo, bo, Wo, h0, c0): "
           "Delta LSTM; the W, h0 and c0 are updated in place");
-#ifndef FWP_HOST_STUB
     bind_blocks(m);
-#endif
     m.def("set_error_class", &set_error_class, "exception class raised for rejected calls");
 }

@@ -3,10 +3,14 @@
  * HOST pointers.  Nothing is launched; each call READS every element of its inputs through their views
  * and WRITES every element of its outputs and saved buffers (simple sums, so that results depend on the
  * inputs), which is what makes it useful under AddressSanitizer: a buffer of the wrong size, a view of
- * freed memory or a stride mistake in the host binding above it (csrc/fwp_torch.cpp built with
- * -DFWP_HOST_STUB) shows up as a report instead of passing unseen.  Test infrastructure only.
+ * freed memory or a stride mistake in the host binding above it (csrc/fwp_torch*.cpp built with
+ * -DFWP_HOST_STUB) shows up as a report instead of passing unseen.  The language model's products, LayerNorm, loss
+ * and embedding are computed, one element after the other, so that the blocks made of them can be compared
+ * with PyTorch's operators.  Test infrastructure only.
  */
+#include <math.h>
 #include <stddef.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include "fwp_hip.h"
@@ -281,4 +285,150 @@ int fwp_rec_bwd_static(const float *q_act, const float *k_act, const float *beta
     (void)stream;
     return rec_bwd(q_act, k_act, beta_act, vdiff, out, h_init, grad_out, Rq, Rk, Rv, rb, ckpt, gqx, gkx, gvx, gbx,
                    gRq, gRk, gRv, grb, NULL, N, H, L, D, chunk);
+}
+
+/* ---- the language model's kernels, computed */
+
+long long fwp_matmul_workspace(int M, int N, int K) { (void)M; (void)N; return K >= 64 ? 8 : 0; }
+int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C, long long ldc, int M,
+               int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream) {
+    (void)stream;
+    g_calls++;
+    const fwp_mm_epilogue none = {0}, e = epi ? *epi : none;
+    if (workspace) fill(workspace, fwp_matmul_workspace(M, N, K), 0);
+    for (int m = 0; m < M; m++)
+        for (int n = 0; n < N; n++) {
+            double s = 0;
+            for (int k = 0; k < K; k++)
+                s += (double)(layout == FWP_MM_TN ? A[k * lda + m] : A[m * lda + k]) *
+                     (layout == FWP_MM_NT ? B[n * ldb + k] : B[k * ldb + n]);
+            const long long at = m * ldc + n;
+            if (e.bias) s += e.bias[n];
+            if (e.relu) s = s < 0 ? 0 : s;
+            if (e.residual) s += e.residual[at];
+            if (e.gate && e.gate[at] <= 0) s = 0;
+            C[at] = (float)s;
+        }
+    if (layout == FWP_MM_TN && e.colsum)
+        for (int m = 0; m < M; m++) {
+            double s = 0;
+            for (int k = 0; k < K; k++) s += A[k * lda + m];
+            e.colsum[m] = (float)s;
+        }
+    return 0;
+}
+
+/* x's row normalised; the two statistics where wanted */
+static void norm_row(const float *x, const float *gamma, const float *beta, float *y, float *stats, int cols, double eps) {
+    double mean = 0, var = 0;
+    for (int c = 0; c < cols; c++) mean += x[c];
+    mean /= cols;
+    for (int c = 0; c < cols; c++) var += (x[c] - mean) * (x[c] - mean);
+    const double rstd = 1 / sqrt(var / cols + eps);
+    for (int c = 0; c < cols; c++) y[c] = (float)((x[c] - mean) * rstd * gamma[c] + beta[c]);
+    if (stats) stats[0] = (float)mean, stats[1] = (float)rstd;
+}
+int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows, int cols,
+                       float eps, void *stream) {
+    (void)stream;
+    g_calls++;
+    for (long long r = 0; r < rows; r++)
+        norm_row(x + r * cols, gamma, beta, y + r * cols, stats ? stats + 2 * r : NULL, cols, eps);
+    return 0;
+}
+long long fwp_layer_norm_workspace(int rows, int cols) { (void)rows; return 2 * cols; }
+int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
+                       float *ggamma, float *gbeta, float *workspace, int rows, int cols, void *stream) {
+    (void)stream;
+    g_calls++;
+    fill(workspace, fwp_layer_norm_workspace(rows, cols), 0);
+    memset(ggamma, 0, sizeof(float) * cols);
+    memset(gbeta, 0, sizeof(float) * cols);
+    for (long long r = 0; r < rows; r++) {
+        const float *d = gy + r * cols, *p = x + r * cols;
+        const double mean = stats[2 * r], rstd = stats[2 * r + 1];
+        double s = 0, t = 0;
+        for (int c = 0; c < cols; c++) {
+            const double h = (p[c] - mean) * rstd, g = (double)d[c] * gamma[c];
+            ggamma[c] += (float)(d[c] * h);
+            gbeta[c] += d[c];
+            s += g / cols, t += g * h / cols;
+        }
+        for (int c = 0; c < cols; c++)
+            gx[r * cols + c] = (float)(rstd * ((double)d[c] * gamma[c] - s - (p[c] - mean) * rstd * t));
+    }
+    return 0;
+}
+
+long long fwp_nll_workspace(int rows, int vocab) { (void)vocab; return rows; }
+int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                float *lse, float *workspace, int rows, int vocab, int dim, void *stream) {
+    (void)stream;
+    g_calls++;
+    fill(workspace, fwp_nll_workspace(rows, vocab), 0);
+    float *row = malloc(sizeof(float) * vocab);
+    for (long long r = 0; r < rows; r++) {
+        double s = 0;
+        for (long long v = 0; v < vocab; v++) {
+            double l = bias ? bias[v] : 0;
+            for (int k = 0; k < dim; k++) l += (double)x[r * dim + k] * W[v * dim + k];
+            row[v] = (float)l;
+            s += exp(l);
+        }
+        if (logits) memcpy(logits + r * vocab, row, sizeof(float) * vocab);
+        if (lse) lse[r] = (float)log(s);
+        loss[r] = target[r] < 0 ? 0 : (float)(log(s) - row[target[r]]);
+    }
+    free(row);
+    return 0;
+}
+int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
+                const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
+                void *stream) {
+    float *d = malloc(sizeof(float) * rows * vocab);
+    for (long long r = 0; r < rows; r++)
+        for (long long v = 0; v < vocab; v++)
+            d[r * vocab + v] = target[r] < 0 ? 0 : (float)((exp(logits[r * vocab + v] - lse[r]) - (v == target[r])) * gloss[r]);
+    const fwp_mm_epilogue epi = {NULL, NULL, NULL, gbias, 0};
+    if (gx) fwp_matmul(FWP_MM_NN, d, vocab, W, dim, gx, dim, rows, dim, vocab, NULL, workspace, stream);
+    if (gW) fwp_matmul(FWP_MM_TN, d, vocab, x, dim, gW, dim, vocab, dim, rows, &epi, workspace, stream);
+    free(d);
+    return 0;
+}
+
+int fwp_rows_matmul(const float *x, const float *gamma, const float *beta, float eps, float *y, const float *W,
+                    const float *bias, const float *residual, int relu, float *out, int rows, int N, int K, void *stream) {
+    float *z = malloc(sizeof(float) * rows * K);
+    for (long long r = 0; r < rows; r++)
+        if (gamma) norm_row(x + r * K, gamma, beta, z + r * K, NULL, K, eps);
+        else memcpy(z + r * K, x + r * K, sizeof(float) * K);
+    if (y) memcpy(y, z, sizeof(float) * rows * K);
+    const fwp_mm_epilogue epi = {bias, residual, NULL, NULL, relu};
+    fwp_matmul(FWP_MM_NT, z, K, W, K, out, N, rows, N, K, &epi, NULL, stream);
+    free(z);
+    return 0;
+}
+int fwp_deltanet_step(const float *qkvb, const float *from, float *to, float *out, int B, int H, int D, float q_scale,
+                      void *stream) {
+    (void)stream;
+    g_calls++;
+    const long long R = (long long)B * H, S = R * D * D;
+    const double s = sum_flat(qkvb, R * (3 * D + 1)) + q_scale;
+    for (long long i = 0; i < S; i++) to[i] = (from ? from[i] : 0) + 1.0f;
+    fill(out, R * D, s);
+    return 0;
+}
+int fwp_embed(const float *table, const int64_t *ids, const float *inv_freq, float *out, int T, int B, int d,
+              long long n_token, float scale, float clamp, void *stream) {
+    (void)stream;
+    g_calls++;
+    for (long long r = 0; r < (long long)T * B; r++)
+        for (int j = 0; j < d; j++) {
+            double pos = T - 1 - r / B;
+            if (clamp > 0 && pos > clamp) pos = clamp;
+            const double phase = pos * inv_freq[j % (d / 2)];
+            const float e = ids[r] >= 0 && ids[r] < n_token ? table[ids[r] * d + j] : NAN;
+            out[r * d + j] = (float)(e * scale + (j < d / 2 ? sin(phase) : cos(phase)));
+        }
+    return 0;
 }

@@ -41,3 +41,15 @@ def test_host_side_of_every_operator_against_the_stand_in_library(build, functio
     cmd = [sys.executable, os.path.join(STUB, "drive.py"), out] + (["python"] if functions == "python" else [])
     run = subprocess.run(cmd, env=env, capture_output=True, text=True, timeout=1500, cwd=out)
     assert run.returncode == 0 and "host stub drive ok" in run.stdout, run.stdout[-2000:] + run.stderr[-4000:]
+
+
+# the language model's blocks: tests/host_stub/drive_blocks.py says what each looks at
+BLOCK_CHECKS = ["results"]
+
+
+@pytest.mark.parametrize("check", BLOCK_CHECKS)
+def test_host_side_of_the_language_models_blocks(build, check):
+    out, env = build
+    run = subprocess.run([sys.executable, os.path.join(STUB, "drive_blocks.py"), out, check], env=env, capture_output=True,
+                         text=True, timeout=1500, cwd=out)
+    assert run.returncode == 0 and check + " ok" in run.stdout, run.stdout[-2000:] + run.stderr[-4000:]
