@@ -226,6 +226,11 @@ __device__ __forceinline__ float rotated(float x) {      // within the 16 lanes 
 // LDS accesses of one wave execute in order; this keeps the compiler from moving them across.
 __device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
 
+// What a sum of exp(logit - m) is multiplied with to become one of exp(logit - big).  A part of the vocabulary with no
+// logit but -infinity (masked words; columns beyond the last) has m = -infinity and the sum 0, or NaN if there
+// was one: it stays as it is (exp(-infinity + infinity) would make it NaN).
+__device__ __forceinline__ float to_max(float m, float big) { return m == -INFINITY ? 1.f : __expf(m - big); }
+
 // The largest of a row's logits and the sum of exp(logit - largest): four logits per lane, LANES (8 or 16) lanes per row.
 template <int LANES>
 __device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, float *out, int at, int pitch) {
@@ -405,12 +410,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     if constexpr (MODE == kLse) {
         __syncthreads();
         for (int row = tid; row < min(BM, ml); row += kThreads) {
-            // the tile's first half of columns holds at least one; the second may hold none
             const float m1 = sums_of[row], m2 = sums_of[BM + row], mx = fmaxf(m1, m2);
-            const float s2 = m2 == -INFINITY ? 0.f : sums_of[3 * BM + row] * __expf(m2 - mx);
             const int64_t at = (int64_t)(id % g.tn) * g.M + m0 + row;
             g.part_max[at] = mx;
-            g.part_sum[at] = sums_of[2 * BM + row] * __expf(m1 - mx) + s2;
+            g.part_sum[at] = sums_of[2 * BM + row] * to_max(m1, mx) + sums_of[3 * BM + row] * to_max(m2, mx);
         }
     }
 }
@@ -545,7 +548,7 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
     if (m < rows)
         for (int t = q; t < tiles; t += 4) {
             const float x = part_max[(int64_t)t * rows + m], y = part_sum[(int64_t)t * rows + m], big = fmaxf(mx, x);
-            s = (mx == -INFINITY ? 0.f : s * __expf(mx - big)) + y * __expf(x - big);
+            s = s * to_max(mx, big) + y * to_max(x, big);
             mx = big;
         }
     sm[q][e] = mx;
@@ -554,10 +557,10 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
     if (q || m >= rows) return;
     for (int o = 1; o < 4; o++) {
         const float x = sm[o][e], big = fmaxf(mx, x);
-        s = s * __expf(mx - big) + (x == -INFINITY ? 0.f : ss[o][e] * __expf(x - big));
+        s = s * to_max(mx, big) + ss[o][e] * to_max(x, big);
         mx = big;
     }
-    const float l = mx + __logf(s);
+    const float l = mx + __logf(s);      // NaN for a row of -infinities alone: mx + log 0 = -infinity, minus the target's
     const int64_t want = target[m];
     if (lse) lse[m] = l;
     loss[m] = want < 0 ? 0.f : want < vocab ? l - (logits ? logits[(int64_t)m * vocab + want] : hit[m]) : NAN;

@@ -105,6 +105,49 @@ def test_negative_log_likelihood(fwp, rows, vocab, dim):
         assert bool(((got.double() - w).abs() <= (2 * float(err) + bound(max(rows, vocab), 1.0)) * mag + 1e-12).all()), name
 
 
+def loss_and_gradients(L, x, W, b, target, gloss):
+    """The loss with and without a graph's buffers (they agree), and the gradients of x, W and b."""
+    rows, vocab, dim = x.shape[0], *W.shape
+    logits, loss, lse = (torch.full(s, float("nan"), device="cuda") for s in ((rows, vocab), (rows,), (rows,)))
+    work = torch.empty(L.lib().fwp_nll_workspace(rows, vocab), device="cuda")
+    ptrs = [t.data_ptr() for t in (x, W, b, target)]
+    assert L.lib().fwp_nll_fwd(*ptrs, logits.data_ptr(), loss.data_ptr(), lse.data_ptr(), work.data_ptr(), rows, vocab,
+                               dim, L.stream_of(x)) == 0
+    only = torch.empty_like(loss)
+    assert L.lib().fwp_nll_fwd(*ptrs, None, only.data_ptr(), None, work.data_ptr(), rows, vocab, dim, L.stream_of(x)) == 0
+    assert torch.equal(only, loss) or bool(loss.isnan().any())
+    gx, gW, gb = torch.full_like(x, float("nan")), torch.full_like(W, float("nan")), torch.full_like(b, float("nan"))
+    n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
+    work = torch.empty(n, device="cuda")
+    assert L.lib().fwp_nll_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), lse.data_ptr(), target.data_ptr(),
+                               gloss.data_ptr(), gx.data_ptr(), gW.data_ptr(), gb.data_ptr(), work.data_ptr(), rows, vocab,
+                               dim, L.stream_of(x)) == 0
+    return loss, gx, gW, gb
+
+
+def check_loss(L, x, W, b, target):
+    gloss = randn(x.shape[0], seed=5)
+    got = loss_and_gradients(L, x, W, b, target, gloss)
+    xd, Wd, bd = (t.double().requires_grad_() for t in (x, W, b))
+    want = torch.nn.functional.cross_entropy(xd @ Wd.t() + bd, target, reduction="none")
+    wants = (want.detach(), *torch.autograd.grad(want, (xd, Wd, bd), gloss.double()))
+    for name, g, w in zip(("loss", "x", "W", "bias"), got, wants):
+        # K = 64 products' roundings of logits of up to about 30, as errors of probabilities, over up to 64 tokens
+        assert float((g.double() - w).abs().max()) <= 2e-5 * (1 + float(w.abs().max())), name
+
+
+# 64-wide tiles (few tokens) and 128-wide ones; masked: the first tile, one in the middle, all but a few words
+@pytest.mark.parametrize("rows,vocab", [(70, 1000), (2048, 2200)])
+@pytest.mark.parametrize("masked", [(0, 128), (640, 768), (130, 520), (0, 960)])
+def test_loss_of_a_vocabulary_masked_in_part(fwp, rows, vocab, masked):
+    """A bias of -infinity takes words out: whole tiles of logits are -infinity."""
+    x, W, b = randn(rows, 64, seed=1), randn(vocab, 64, seed=2) * 0.3, randn(vocab, seed=3)
+    b[masked[0]:masked[1]] = -float("inf")
+    free = torch.nonzero(b.isfinite())[:, 0]
+    target = free[torch.randint(0, len(free), (rows,), generator=torch.Generator().manual_seed(4)).cuda()]
+    check_loss(fwp._lib, x, W, b, target)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 36), (3000, 128), (2500, 256), (9, 260), (70, 1024)])
 def test_layer_norm(fwp, rows, cols):
     L = fwp._lib
