@@ -164,9 +164,13 @@ struct Operand {
             for (int j = 0; j < 8; j++) {
                 const float l = lane_of(lse[0], j), g = lane_of(gl[0], j);
                 const int h = __builtin_amdgcn_readlane(hit[0], j);
-                const float w = k + j < K && h >= 0 ? g : 0.f;
+                const float w = h >= 0 ? g : 0.f;
 #pragma unroll
-                for (int c = 0; c < VEC; c++) x[0][8 * c + j] = nll_grad(x[0][8 * c + j], l, w, h == r + c);
+                for (int c = 0; c < VEC; c++) {
+                    // a token beyond K has the last one's values beside a logit of 0: its exponential may be infinite
+                    const float d = nll_grad(x[0][8 * c + j], l, w, h == r + c);
+                    x[0][8 * c + j] = k + j < K ? d : 0.f;
+                }
             }
         }
     }

@@ -148,6 +148,14 @@ def test_loss_of_a_vocabulary_masked_in_part(fwp, rows, vocab, masked):
     check_loss(fwp._lib, x, W, b, target)
 
 
+@pytest.mark.parametrize("rows", [1, 31, 33, 70])
+def test_loss_gradients_of_far_negative_logits(fwp, rows):
+    """A softmax does not mind a shift: logits around -100, token counts that do not fill the products' steps."""
+    x, W, b = randn(rows, 64, seed=1) * 0.1, randn(300, 64, seed=2) * 0.3, torch.full((300,), -100.0, device="cuda")
+    target = torch.randint(0, 300, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
+    check_loss(fwp._lib, x, W, b, target)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 36), (3000, 128), (2500, 256), (9, 260), (70, 1024)])
 def test_layer_norm(fwp, rows, cols):
     L = fwp._lib
