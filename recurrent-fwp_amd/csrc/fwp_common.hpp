@@ -13,6 +13,10 @@ constexpr int kTile = 16;
 constexpr int kChunkQuantum = 32;
 constexpr int kDefaultChunk = 64;
 
+// torch.relu and the gradient it lets through: NaN is neither cut off nor does it cut off (fmaxf(NaN, 0) is 0).
+__device__ __forceinline__ float relu(float x) { return x < 0.f ? 0.f : x; }
+__device__ __forceinline__ float gated(float gate, float x) { return gate <= 0.f ? 0.f : x; }
+
 __device__ __forceinline__ const float *row(const fwp_view &v, int n, int h, int t) {
     return v.ptr + (int64_t)n * v.sN + (int64_t)h * v.sH + (int64_t)t * v.sL;
 }

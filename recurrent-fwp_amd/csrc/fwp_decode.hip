@@ -139,7 +139,7 @@ __global__ __launch_bounds__(1024) void k_rows(RowsArgs a) {
         const int row = 16 * wave + 4 * g + r;
         if (row >= a.rows) continue;
         float o = v[r] + bias;
-        if (a.relu) o = fmaxf(o, 0.f);
+        if (a.relu) o = relu(o);
         a.out[(int64_t)row * a.N + col] = o + res[r];
     }
 }

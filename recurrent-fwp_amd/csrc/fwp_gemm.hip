@@ -216,9 +216,9 @@ enum { kPlain = 0, kLse = 1, kGrad = 2 };
 
 // everything but the bias
 __device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_t at) {
-    if (e.relu) x = fmaxf(x, 0.f);
+    if (e.relu) x = relu(x);
     if (e.residual) x += e.residual[at];
-    if (e.gate) x = e.gate[at] > 0.f ? x : 0.f;
+    if (e.gate) x = gated(e.gate[at], x);
     return x;
 }
 
@@ -391,14 +391,14 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
             const int64_t at = (int64_t)m * g.ldc + n;
             if (vec) {
                 if (one) {
-                    if (g.epi.relu) v = make_float4(fmaxf(v.x, 0.f), fmaxf(v.y, 0.f), fmaxf(v.z, 0.f), fmaxf(v.w, 0.f));
+                    if (g.epi.relu) v = make_float4(relu(v.x), relu(v.y), relu(v.z), relu(v.w));
                     if (g.epi.residual) {
                         const float4 y = *reinterpret_cast<const float4 *>(g.epi.residual + at);
                         v.x += y.x, v.y += y.y, v.z += y.z, v.w += y.w;
                     }
                     if (g.epi.gate) {
                         const float4 y = *reinterpret_cast<const float4 *>(g.epi.gate + at);
-                        v = make_float4(y.x > 0.f ? v.x : 0.f, y.y > 0.f ? v.y : 0.f, y.z > 0.f ? v.z : 0.f, y.w > 0.f ? v.w : 0.f);
+                        v = make_float4(gated(y.x, v.x), gated(y.y, v.y), gated(y.z, v.z), gated(y.w, v.w));
                     }
                 }
                 *reinterpret_cast<float4 *>(C + at) = v;

@@ -133,6 +133,49 @@ def test_decoding_one_token_at_a_time(fwp, B, D, dm, inner, pre):
         assert torch.equal(ours.hidden(toks[0])[0], ours.hidden(toks[0], carry_over_fast_weight=True)[0])
 
 
+def same_nans(name, got, want):
+    assert torch.equal(got.isnan(), want.isnan()), name
+    ok = ~want.isnan()
+    if bool(ok.any()):
+        close(name, got[ok], want[ok], 16)
+
+
+# tiles of whole 16-byte groups and others; a k in one range and in several
+@pytest.mark.parametrize("rows,d,inner", [(40, 64, 200), (40, 66, 201), (300, 512, 1024)])
+@pytest.mark.parametrize("where", ["W1", "b1", "x"])
+def test_nan_passes_the_feed_forward_blocks_relu(fwp, where, rows, d, inner):
+    """torch.relu(NaN) is NaN, and its gradient passes where the activation is NaN."""
+    x = torch.randn(rows, 1, d, generator=torch.Generator().manual_seed(1)).cuda()
+    ours, ref, a, b = both(lambda op: fwp.PositionwiseFF(d, inner, 0.0, True), x)
+    nan = float("nan")
+    with torch.no_grad():
+        for m, z in ((ours, a), (ref, b)):
+            {"W1": m.CoreNet[0].weight, "b1": m.CoreNet[0].bias[None], "x": z[0]}[where][0, 3] = nan
+    # without LayerNorm in between, which would spread a NaN of x over its row
+    ours.layer_norm, ref.layer_norm = torch.nn.Identity(), torch.nn.Identity()
+    y, want = ours(a), ref(b)
+    same_nans("y", y, want)
+    g = torch.randn_like(x)
+    grads = torch.autograd.grad(y, [a, *ours.parameters()], g)
+    wants = torch.autograd.grad(want, [b, *ref.parameters()], g.double())
+    for i, (got, w) in enumerate(zip(grads, wants)):
+        same_nans(i, got, w)
+
+
+@pytest.mark.parametrize("B", [3, 20, 40])
+def test_nan_passes_the_decoding_paths_relu(fwp, B):
+    cfg = dict(n_token=50, n_layer=1, n_head=4, d_model=64, d_head=16, d_inner=128)
+    torch.manual_seed(0)
+    ours = fwp.DeltaNetLM(init_std=0.2, **cfg).cuda()
+    ours.layers[0].pos_ff.CoreNet[0].bias.data[5] = float("nan")
+    with torch.no_grad():
+        hid, _ = ours.hidden(torch.zeros(1, B, dtype=torch.int64, device="cuda"))
+        assert bool(hid.isnan().all())
+        z = torch.randn(B, 1, 64, device="cuda")
+        lin = ours.layers[0].pos_ff.CoreNet[0]
+        same_nans("few rows", fwp._fwp_torch.linear(z, lin.weight, lin.bias, True), torch.relu(lin(z)).double())
+
+
 @pytest.mark.parametrize("T,clamp", [(1, -1), (300, -1), (70, 20)])
 def test_embedding_without_a_graph(fwp, T, clamp):
     """The fused embedding against the lines it replaces (they run when a graph is recorded)."""
