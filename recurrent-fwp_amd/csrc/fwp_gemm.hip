@@ -5,8 +5,9 @@
 // products.  Six of them are formed, h h', h m', m h', m m', h l', l h'; the three left out are below
 // 2^-26 |x x'|, a quarter of the rounding of an fp32 product.  Sums are fp32, six roundings per 32 terms where a
 // chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm): 2.2e-7 at K = 256,
-// 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling, no overflow but that of the operands (an
-// infinite operand gives NaN where an fp32 product gives infinity or NaN).
+// 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling.  An operand that no bf16 number
+// holds (infinity, NaN, the last 2^-9 below fp32's largest) leaves NaN or infinity in the sums; an element that is
+// not finite is formed again from its fp32 operands (plain_sum).
 //
 // v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
 // the 32x32x16 form 1.8), i.e. 350 TFLOP/s of such fp32 products, where the fp32 matrix instructions make 155.
@@ -262,6 +263,22 @@ __device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, flo
     if (lane % LANES == 0) out[at] = m, out[at + pitch] = s;
 }
 
+// The sum over k of one element in fp32 operations, for one that the bf16 products left infinite or NaN
+template <bool AKC, bool BKC, int MODE>
+__device__ float plain_sum(const GemmArgs &g, int m, int n, int kb, int ke) {
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k = kb; k < ke && sum == sum; k++) {      // up to the first NaN
+        float a = g.A[AKC ? (int64_t)m * g.lda + k : (int64_t)k * g.lda + m];
+        if constexpr (MODE == kGrad) {
+            const int token = AKC ? m : k, word = AKC ? k : m, hit = (int)g.nll.target[token];
+            a = nll_grad(a, g.nll.lse[token], hit >= 0 ? g.nll.gloss[token] : 0.f, hit == word);
+        }
+        sum = fmaf(a, g.B[BKC ? (int64_t)n * g.ldb + k : (int64_t)k * g.ldb + n], sum);
+    }
+    return sum;
+}
+
 // BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
 template <bool AKC, bool BKC, int BM, int BN, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
@@ -378,6 +395,13 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
         for (int q = 0; q < 16 / kRows; q++) {
             const int row = kRows * q + lane / kLanes, m = m0 + wm + 16 * i + row;
             float4 v = *reinterpret_cast<const float4 *>(strip + row * kPitch + c4);
+            if (m < g.M && !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) + fabsf(v.w) < INFINITY)) {
+                float *const p = strip + row * kPitch + c4;
+#pragma unroll 1
+                for (int e = 0; e < 4; e++)
+                    if (n + e < g.N && !(fabsf(p[e]) < INFINITY)) p[e] = plain_sum<AKC, BKC, MODE>(g, m, n + e, kb, ke);
+                v = *reinterpret_cast<const float4 *>(p);
+            }
             v.x += bias[0], v.y += bias[1], v.z += bias[2], v.w += bias[3];
             if constexpr (MODE == kLse) {
                 lse_of_row<kLanes>(v, n, g.N, lane, sums_of, (wave / 2) * BM + wm + 16 * i + row, 2 * BM);

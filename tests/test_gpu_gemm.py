@@ -156,6 +156,41 @@ def test_loss_gradients_of_far_negative_logits(fwp, rows):
     check_loss(fwp._lib, x, W, b, target)
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 66, 200), (300, 260, 1100), (40, 64, 2048), (2100, 2100, 40)])
+@pytest.mark.parametrize("layout", [NT, NN, TN])
+def test_products_of_infinities_and_the_largest_numbers(fwp, layout, M, N, K):
+    """Operands that bf16 cannot hold (infinities, NaN, numbers above its largest) meet the others as in fp32."""
+    A = randn(*((K, M) if layout == TN else (M, K)), seed=1)
+    B = randn(*((N, K) if layout == NT else (K, N)), seed=2)
+    a, b = (A.t() if layout == TN else A), (B.t() if layout == NT else B)
+    inf, big = float("inf"), 3.4e38            # rounds to infinity as a bf16 number
+    a[0, 3], a[1, K - 1], a[2, 0], a[3, 5], a[4, 7] = inf, -inf, float("nan"), big, -big
+    b[4, 0], b[K - 2, 1] = inf, float("nan")
+    b[3, 2], b[5], b[7] = 0.0, 0.01, -0.01     # infinity * 0; results that fp32 holds
+    want = a.double() @ b.double()
+    mag = a.double().abs() @ b.double().abs()
+    for cut in (True, False):
+        got = matmul(fwp._lib, layout, A, B, cut).double()
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert bool((got == want)[want.isinf()].all())
+        ok = want.isfinite()
+        assert bool(((got - want).abs() <= (bound(K, mag) + K * EPS * mag))[ok].all())      # K roundings in a row
+
+
+def test_loss_gradients_of_an_infinite_upstream_gradient(fwp):
+    x, W, b = randn(40, 64, seed=1), randn(300, 64, seed=2) * 0.1, randn(300, seed=3)
+    target = torch.randint(0, 300, (40,), generator=torch.Generator().manual_seed(4)).cuda()
+    gloss = randn(40, seed=5)
+    gloss[7] = float("inf")
+    _, *got = loss_and_gradients(fwp._lib, x, W, b, target, gloss)
+    xd, Wd, bd = (t.double().requires_grad_() for t in (x, W, b))
+    want = torch.nn.functional.cross_entropy(xd @ Wd.t() + bd, target, reduction="none")
+    for name, g, w in zip("xWb", got, torch.autograd.grad(want, (xd, Wd, bd), gloss.double())):
+        odd = ~w.isfinite()      # at the target PyTorch forms infinity - p infinity, NaN, and (p - 1) infinity is also right
+        assert torch.equal(~g.isfinite(), odd) and bool((g == w)[w.isinf()].all()), name
+        assert float((g.double() - w)[~odd].abs().max() if bool((~odd).any()) else 0.0) <= 2e-5 * 10, name
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 36), (3000, 128), (2500, 256), (9, 260), (70, 1024)])
 def test_layer_norm(fwp, rows, cols):
     L = fwp._lib
