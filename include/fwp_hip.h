@@ -306,6 +306,14 @@ int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float
                 const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows,
                 int vocab, int dim, void *stream);
 
+/* The same with two values saved per row, stats [rows,2] (8-byte aligned): the largest logit and 1 / the sum of exp(logit -
+ * largest).  A log-sum-exp rounds at the size of the largest logit; the probabilities from these two do not. */
+int fwp_nll_stats_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits,
+                      float *loss, float *stats, float *workspace, int rows, int vocab, int dim, void *stream);
+int fwp_nll_stats_bwd(const float *x, const float *W, const float *logits, const float *stats, const int64_t *target,
+                      const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows,
+                      int vocab, int dim, void *stream);
+
 /*
  * LayerNorm of the layers (utils/model_utils.py:52-66, cuda_fast_weight_layer.py:168-176): y = (x - mean) rstd gamma +
  * beta over rows of `cols` floats (a multiple of 4 up to 1024).  stats [rows,2] (mean, rstd) may be NULL.

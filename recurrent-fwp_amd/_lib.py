@@ -60,6 +60,8 @@ _MODEL_SIGNATURES = {
     "fwp_matmul": [_I, _P, _L, _P, _L, _P, _L] + [_I] * 3 + [_P] * 3,
     "fwp_nll_fwd": [_P] * 8 + [_I] * 3 + [_P],
     "fwp_nll_bwd": [_P] * 10 + [_I] * 3 + [_P],
+    "fwp_nll_stats_fwd": [_P] * 8 + [_I] * 3 + [_P],
+    "fwp_nll_stats_bwd": [_P] * 10 + [_I] * 3 + [_P],
     "fwp_layer_norm_fwd": [_P] * 5 + [_I] * 2 + [ctypes.c_float, _P],
     "fwp_layer_norm_bwd": [_P] * 8 + [_I] * 2 + [_P],
     "fwp_rows_matmul": [_P] * 3 + [ctypes.c_float] + [_P] * 4 + [_I, _P] + [_I] * 3 + [_P],

@@ -412,23 +412,38 @@ int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t
                 float *lse, float *workspace, int rows, int vocab, int dim, void *stream) {
     if (!x || !W || !target || !loss || !workspace || (logits == nullptr) != (lse == nullptr)) return FWP_E_NULL;
     if (rows < 1 || vocab < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1)) return FWP_E_SHAPE;
-    return nll_fwd(x, W, bias, target, logits, loss, lse, workspace, rows, vocab, dim, (hipStream_t)stream);
+    return nll_fwd(x, W, bias, target, logits, loss, lse, nullptr, workspace, rows, vocab, dim, (hipStream_t)stream);
+}
+
+int fwp_nll_stats_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                      float *stats, float *workspace, int rows, int vocab, int dim, void *stream) {
+    if (!x || !W || !target || !logits || !loss || !stats || !workspace) return FWP_E_NULL;
+    if (rows < 1 || vocab < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1) || reinterpret_cast<uintptr_t>(stats) % 8) return FWP_E_SHAPE;
+    return nll_fwd(x, W, bias, target, logits, loss, nullptr, stats, workspace, rows, vocab, dim, (hipStream_t)stream);
+}
+
+static int nll_bwd(const float *x, const float *W, const float *logits, const NllView &nll, float *gx, float *gW, float *gbias,
+                   float *workspace, int rows, int vocab, int dim, hipStream_t stream) {
+    if (!x || !W || !logits || !(nll.lse || nll.stats) || !nll.target || !nll.gloss || (gbias && !gW)) return FWP_E_NULL;
+    if (rows < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1) || reinterpret_cast<uintptr_t>(nll.stats) % 8) return FWP_E_SHAPE;
+    fwp_mm_epilogue epi = {};
+    if (gx)
+        if (int rc = matmul(FWP_MM_NN, logits, vocab, W, dim, gx, dim, rows, dim, vocab, epi, workspace, &nll, stream)) return rc;
+    if (!gW) return 0;
+    epi.colsum = gbias;
+    return matmul(FWP_MM_TN, logits, vocab, x, dim, gW, dim, vocab, dim, rows, epi, workspace, &nll, stream);
 }
 
 int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
                 const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
                 void *stream) {
-    if (!x || !W || !logits || !lse || !target || !gloss || (gbias && !gW)) return FWP_E_NULL;
-    if (rows < 1 || !pitch_ok(dim, 1) || !pitch_ok(vocab, 1)) return FWP_E_SHAPE;
-    const NllView nll = {lse, gloss, target};
-    fwp_mm_epilogue epi = {};
-    if (gx)
-        if (int rc = matmul(FWP_MM_NN, logits, vocab, W, dim, gx, dim, rows, dim, vocab, epi, workspace, &nll,
-                            (hipStream_t)stream))
-            return rc;
-    if (!gW) return 0;
-    epi.colsum = gbias;
-    return matmul(FWP_MM_TN, logits, vocab, x, dim, gW, dim, vocab, dim, rows, epi, workspace, &nll, (hipStream_t)stream);
+    return nll_bwd(x, W, logits, {lse, nullptr, gloss, target}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
+}
+
+int fwp_nll_stats_bwd(const float *x, const float *W, const float *logits, const float *stats, const int64_t *target,
+                      const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
+                      void *stream) {
+    return nll_bwd(x, W, logits, {nullptr, stats, gloss, target}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
 }
 
 int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows,

@@ -192,7 +192,7 @@ int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const
 // fp32 matrix products on the bf16 matrix cores (fwp_matmul); `nll`: A holds logits and stands for the gradient of
 // the loss that nll_fwd computed from them.
 struct NllView {
-    const float *lse, *gloss;
+    const float *lse, *stats, *gloss;      // lse [rows] or stats [rows,2], whichever nll_fwd wrote
     const int64_t *target;
 };
 int64_t matmul_workspace(int M, int N, int K);
@@ -200,7 +200,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
            int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s);
 int64_t nll_workspace(int rows, int vocab);
 int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
-            float *lse, float *workspace, int rows, int vocab, int dim, hipStream_t s);
+            float *lse, float *stats, float *workspace, int rows, int vocab, int dim, hipStream_t s);
 
 // LayerNorm over rows of up to 1024 floats (a multiple of 4) and its adjoint.
 bool layer_norm_supported(int cols);

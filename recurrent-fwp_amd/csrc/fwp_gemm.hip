@@ -69,14 +69,31 @@ struct Planes {
 __device__ __forceinline__ constexpr int unit_of(int row, int chunk) { return row ^ (2 * chunk) ^ ((row >> 3) & 1); }
 
 // What turns stored logits into the gradient of the loss as an operand is loaded:
-// (exp(logit - lse[token]) - [vocabulary entry == target[token]]) * gloss[token], 0 for a negative target
+// (exp(logit - shift) * scale - [vocabulary entry == target]) * gloss of the token, 0 for a negative target.
+// shift and scale: the largest logit and 1 / the sum of exp(logit - largest) (`stats`, exact where a token's probability
+// is near 1 and its logit large), or the log-sum-exp and 1 (`lse`).
 struct NllArgs {
-    const float *lse, *gloss;
+    const float *lse, *stats, *gloss;
     const int64_t *target;
 };
 
-__device__ __forceinline__ float nll_grad(float logit, float lse, float g, bool hit) {
-    return (__expf(logit - lse) - (hit ? 1.f : 0.f)) * g;
+struct NllToken {
+    float shift, scaled, g;      // scaled: scale * gloss
+    int hit;
+};
+
+__device__ __forceinline__ NllToken nll_token(const NllArgs &a, int token) {
+    NllToken t;
+    t.hit = (int)a.target[token];
+    t.g = t.hit >= 0 ? a.gloss[token] : 0.f;
+    const float2 s = a.stats ? reinterpret_cast<const float2 *>(a.stats)[token] : make_float2(a.lse[token], 1.f);
+    t.shift = s.x;
+    t.scaled = s.y * t.g;
+    return t;
+}
+
+__device__ __forceinline__ float nll_grad(float logit, float shift, float scaled, float g, bool hit) {
+    return fmaf(__expf(logit - shift), scaled, hit ? -g : 0.f);
 }
 
 // One operand's share of the loads and LDS writes of a thread.  KC: rows are contiguous along k; a task is 8
@@ -93,8 +110,7 @@ struct Operand {
     unsigned off[kTasks];
     // the tokens' values for the loss gradient: of this task's row (KC), or of the wave's k-chunk, token j in
     // the lanes with lane % 8 == j
-    float lse[NLL ? kTasks : 1], gl[NLL ? kTasks : 1];
-    int hit[NLL ? kTasks : 1];
+    NllToken token[NLL ? kTasks : 1];
 
     static __device__ __forceinline__ int row_of(int t) { return KC ? t / kChunks : (t % (ROWS / VEC)) * VEC; }
     static __device__ __forceinline__ int chunk_of(int t) { return KC ? t % kChunks : t / (ROWS / VEC); }
@@ -104,12 +120,7 @@ struct Operand {
         for (int i = 0; i < kTasks; i++) {
             const int r = row_of(tid + i * kThreads), c = chunk_of(tid + i * kThreads);
             off[i] = (unsigned)(KC ? r * ld + 8 * c : 8 * c * ld + r) * 4;
-            if constexpr (NLL && KC) {
-                const int t = min(row0 + r, rows - 1);
-                lse[i] = nll.lse[t];
-                hit[i] = (int)nll.target[t];
-                gl[i] = hit[i] >= 0 ? nll.gloss[t] : 0.f;
-            }
+            if constexpr (NLL && KC) token[i] = nll_token(nll, min(row0 + r, rows - 1));
         }
     }
     // P: the tile's first row at k = 0, `left` rows from there, k0 .. min(k0 + kBK, K)
@@ -125,12 +136,7 @@ struct Operand {
                 for (int j = 0; j < 4; j++) x[i][j] = a[j], x[i][4 + j] = b[j];
             }
         } else {
-            if constexpr (NLL) {
-                const int t = min(k0 + 8 * chunk_of(tid) + tid % 8, K - 1);
-                lse[0] = nll.lse[t];
-                gl[0] = nll.gloss[t];
-                hit[0] = (int)nll.target[t];
-            }
+            if constexpr (NLL) token[0] = nll_token(nll, min(k0 + 8 * chunk_of(tid) + tid % 8, K - 1));
             const v4i rs = buffer_of(P + (int64_t)k0 * ld, (int64_t)(min(K - k0, kBK) - 1) * ld + left);
 #pragma unroll
             for (int j = 0; j < 8; j++) {
@@ -153,7 +159,8 @@ struct Operand {
                 const int k = k0 + 8 * chunk_of(tid + i * kThreads);
                 if constexpr (NLL)
 #pragma unroll
-                    for (int j = 0; j < 8; j++) x[i][j] = nll_grad(x[i][j], lse[i], gl[i], hit[i] == k + j);
+                    for (int j = 0; j < 8; j++)
+                        x[i][j] = nll_grad(x[i][j], token[i].shift, token[i].scaled, token[i].g, token[i].hit == k + j);
                 if (tail)
 #pragma unroll
                     for (int j = 0; j < 8; j++) x[i][j] = k + j < K ? x[i][j] : 0.f;
@@ -163,13 +170,12 @@ struct Operand {
             const int k = k0 + 8 * chunk_of(tid), r = row0 + row_of(tid);
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const float l = lane_of(lse[0], j), g = lane_of(gl[0], j);
-                const int h = __builtin_amdgcn_readlane(hit[0], j);
-                const float w = h >= 0 ? g : 0.f;
+                const float shift = lane_of(token[0].shift, j), scaled = lane_of(token[0].scaled, j), g = lane_of(token[0].g, j);
+                const int h = __builtin_amdgcn_readlane(token[0].hit, j);
 #pragma unroll
                 for (int c = 0; c < VEC; c++) {
                     // a token beyond K has the last one's values beside a logit of 0: its exponential may be infinite
-                    const float d = nll_grad(x[0][8 * c + j], l, w, h == r + c);
+                    const float d = nll_grad(x[0][8 * c + j], shift, scaled, g, h == r + c);
                     x[0][8 * c + j] = k + j < K ? d : 0.f;
                 }
             }
@@ -271,8 +277,8 @@ __device__ float plain_sum(const GemmArgs &g, int m, int n, int kb, int ke) {
     for (int k = kb; k < ke && sum == sum; k++) {      // up to the first NaN
         float a = g.A[AKC ? (int64_t)m * g.lda + k : (int64_t)k * g.lda + m];
         if constexpr (MODE == kGrad) {
-            const int token = AKC ? m : k, word = AKC ? k : m, hit = (int)g.nll.target[token];
-            a = nll_grad(a, g.nll.lse[token], hit >= 0 ? g.nll.gloss[token] : 0.f, hit == word);
+            const NllToken t = nll_token(g.nll, AKC ? m : k);
+            a = nll_grad(a, t.shift, t.scaled, t.g, t.hit == (AKC ? k : m));
         }
         sum = fmaf(a, g.B[BKC ? (int64_t)n * g.ldb + k : (int64_t)k * g.ldb + n], sum);
     }
@@ -541,7 +547,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
            int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s) {
     GemmArgs g{};
     g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
-    if (nll) g.nll = NllArgs{nll->lse, nll->gloss, nll->target};
+    if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target};
     const Plan p = plan_of(M, N, K, workspace && may_cut(N, C, ldc));
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
     const bool cut = p.ranges > 1;
@@ -564,12 +570,13 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
 
 namespace {
 
-// loss = lse - logit of the target (0 for a negative target), lse from the tiles' maxima and sums; four threads
-// share a row, a quarter of the tiles each
+// loss = (largest logit - logit of the target) + log(sum of exp(logit - largest)) (0 for a negative target), from the
+// tiles' maxima and sums; four threads share a row, a quarter of the tiles each.  The difference comes first: added to
+// the logarithm first, a large logit would round it off (a loss of 1e-3 at a logit of 20 by half a percent).
 __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part_max, const float *__restrict__ part_sum,
                                                   const float *__restrict__ hit, const float *__restrict__ logits,
                                                   const int64_t *__restrict__ target, float *__restrict__ loss, float *__restrict__ lse,
-                                                  int rows, int vocab, int tiles) {
+                                                  float *__restrict__ stats, int rows, int vocab, int tiles) {
     __shared__ float sm[4][64], ss[4][64];
     const int e = threadIdx.x % 64, q = threadIdx.x / 64, m = blockIdx.x * 64 + e;
     float mx = -INFINITY, s = 0.f;
@@ -588,10 +595,12 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
         s = s * to_max(mx, big) + ss[o][e] * to_max(x, big);
         mx = big;
     }
-    const float l = mx + __logf(s);      // NaN for a row of -infinities alone: mx + log 0 = -infinity, minus the target's
+    const float l = __logf(s);
     const int64_t want = target[m];
-    if (lse) lse[m] = l;
-    loss[m] = want < 0 ? 0.f : want < vocab ? l - (logits ? logits[(int64_t)m * vocab + want] : hit[m]) : NAN;
+    if (lse) lse[m] = mx + l;
+    if (stats) *reinterpret_cast<float2 *>(stats + 2 * (int64_t)m) = make_float2(mx, 1.f / s);
+    // a row of -infinities alone: NaN
+    loss[m] = want < 0 ? 0.f : want < vocab ? (mx - (logits ? logits[(int64_t)m * vocab + want] : hit[m])) + l : NAN;
 }
 
 }  // namespace
@@ -599,7 +608,7 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
 int64_t nll_workspace(int rows, int vocab) { return (int64_t)((vocab + 63) / 64) * rows * 2 + rows; }
 
 int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
-            float *lse, float *workspace, int rows, int vocab, int dim, hipStream_t s) {
+            float *lse, float *stats, float *workspace, int rows, int vocab, int dim, hipStream_t s) {
     GemmArgs g{};
     g.A = x, g.B = W, g.lda = dim, g.ldb = dim, g.M = rows, g.N = vocab, g.K = dim, g.C = logits, g.ldc = vocab;
     g.epi.bias = bias;
@@ -612,7 +621,7 @@ int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *ta
     g.vec = vocab % 4 == 0 && aligned(logits);
     launch<true, true, kLse>(g, p, s);
     hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, logits, target, loss,
-                       lse, rows, vocab, p.tn);
+                       lse, stats, rows, vocab, p.tn);
     return (int)hipGetLastError();
 }
 

@@ -331,18 +331,21 @@ struct NllFn : torch::autograd::Function<NllFn> {
         const at::Tensor x = plain(x_in), target = target_in.contiguous();
         const int64_t rows = x.size(0), dim = x.size(1), vocab = W.size(0);
         LaunchGuard guard(x);
-        at::Tensor loss = at::empty({rows}, x.options()), logits, lse;
+        const at::Tensor loss = at::empty({rows}, x.options()),
+                         work = at::empty({fwp_nll_workspace((int)rows, (int)vocab)}, x.options());
+        at::Tensor logits, stats;
         if (ctx) {
             logits = at::empty({rows, vocab}, x.options());
-            lse = at::empty({rows}, x.options());
-        }
-        const at::Tensor work = at::empty({fwp_nll_workspace((int)rows, (int)vocab)}, x.options());
-        check(fwp_nll_fwd(ptr(x), ptr(W), ptr(bias), target.data_ptr<int64_t>(), ptr(logits), ptr(loss), ptr(lse), ptr(work),
-                          (int)rows, (int)vocab, (int)dim, stream_of(x)),
-              "fwp_nll_fwd");
-        if (ctx) {
-            ctx->save_for_backward({x_in, W, bias, target, logits, lse});
+            stats = at::empty({rows, 2}, x.options());
+            check(fwp_nll_stats_fwd(ptr(x), ptr(W), ptr(bias), target.data_ptr<int64_t>(), ptr(logits), ptr(loss), ptr(stats),
+                                    ptr(work), (int)rows, (int)vocab, (int)dim, stream_of(x)),
+                  "fwp_nll_stats_fwd");
+            ctx->save_for_backward({x_in, W, bias, target, logits, stats});
             ctx->set_materialize_grads(false);
+        } else {
+            check(fwp_nll_fwd(ptr(x), ptr(W), ptr(bias), target.data_ptr<int64_t>(), nullptr, ptr(loss), nullptr, ptr(work), (int)rows,
+                              (int)vocab, (int)dim, stream_of(x)),
+                  "fwp_nll_fwd");
         }
         return loss;
     }
@@ -350,7 +353,7 @@ struct NllFn : torch::autograd::Function<NllFn> {
         variable_list res(4);
         if (!grads[0].defined()) return res;
         const auto saved = ctx->get_saved_variables();
-        const at::Tensor &W = saved[1], &bias = saved[2], &target = saved[3], &logits = saved[4], &lse = saved[5];
+        const at::Tensor &W = saved[1], &bias = saved[2], &target = saved[3], &logits = saved[4], &stats = saved[5];
         if (at::GradMode::is_enabled()) {
             res = differentiate(at::cross_entropy_loss(at::linear(saved[0], W, bias), target, {}, at::Reduction::None),
                                 {saved[0], W, bias}, grads[0]);
@@ -369,9 +372,9 @@ struct NllFn : torch::autograd::Function<NllFn> {
         const int64_t n = std::max(fwp_matmul_workspace((int)rows, (int)dim, (int)vocab),
                                    fwp_matmul_workspace((int)vocab, (int)dim, (int)rows));
         if (n > 0) work = at::empty({n}, x.options());
-        check(fwp_nll_bwd(ptr(x), ptr(W), ptr(logits), ptr(lse), target.data_ptr<int64_t>(), ptr(g), ptr(res[0]), ptr(res[1]),
-                          ptr(res[2]), ptr(work), (int)rows, (int)vocab, (int)dim, stream_of(x)),
-              "fwp_nll_bwd");
+        check(fwp_nll_stats_bwd(ptr(x), ptr(W), ptr(logits), ptr(stats), target.data_ptr<int64_t>(), ptr(g), ptr(res[0]), ptr(res[1]),
+                                ptr(res[2]), ptr(work), (int)rows, (int)vocab, (int)dim, stream_of(x)),
+              "fwp_nll_stats_bwd");
         return res;
     }
 };

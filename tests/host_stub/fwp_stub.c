@@ -361,34 +361,46 @@ int fwp_layer_norm_bwd(const float *gy, const float *x, const float *stats, cons
 }
 
 long long fwp_nll_workspace(int rows, int vocab) { (void)vocab; return rows; }
-int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
-                float *lse, float *workspace, int rows, int vocab, int dim, void *stream) {
-    (void)stream;
+static int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                   float *lse, float *stats, float *workspace, int rows, int vocab, int dim) {
     g_calls++;
     fill(workspace, fwp_nll_workspace(rows, vocab), 0);
     float *row = malloc(sizeof(float) * vocab);
     for (long long r = 0; r < rows; r++) {
-        double s = 0;
+        double s = 0, mx = -INFINITY;
         for (long long v = 0; v < vocab; v++) {
             double l = bias ? bias[v] : 0;
             for (int k = 0; k < dim; k++) l += (double)x[r * dim + k] * W[v * dim + k];
             row[v] = (float)l;
-            s += exp(l);
+            mx = fmax(mx, row[v]);
         }
+        for (long long v = 0; v < vocab; v++) s += exp(row[v] - mx);
         if (logits) memcpy(logits + r * vocab, row, sizeof(float) * vocab);
-        if (lse) lse[r] = (float)log(s);
-        loss[r] = target[r] < 0 ? 0 : (float)(log(s) - row[target[r]]);
+        if (lse) lse[r] = (float)(mx + log(s));
+        if (stats) stats[2 * r] = (float)mx, stats[2 * r + 1] = (float)(1 / s);
+        loss[r] = target[r] < 0 ? 0 : (float)(mx - row[target[r]] + log(s));
     }
     free(row);
     return 0;
 }
-int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
-                const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
-                void *stream) {
+int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                float *lse, float *workspace, int rows, int vocab, int dim, void *stream) {
+    (void)stream;
+    return nll_fwd(x, W, bias, target, logits, loss, lse, NULL, workspace, rows, vocab, dim);
+}
+int fwp_nll_stats_fwd(const float *x, const float *W, const float *bias, const int64_t *target, float *logits, float *loss,
+                      float *stats, float *workspace, int rows, int vocab, int dim, void *stream) {
+    (void)stream;
+    return nll_fwd(x, W, bias, target, logits, loss, NULL, stats, workspace, rows, vocab, dim);
+}
+int fwp_nll_stats_bwd(const float *x, const float *W, const float *logits, const float *stats, const int64_t *target,
+                      const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
+                      void *stream) {
     float *d = malloc(sizeof(float) * rows * vocab);
     for (long long r = 0; r < rows; r++)
         for (long long v = 0; v < vocab; v++)
-            d[r * vocab + v] = target[r] < 0 ? 0 : (float)((exp(logits[r * vocab + v] - lse[r]) - (v == target[r])) * gloss[r]);
+            d[r * vocab + v] = target[r] < 0 ? 0 : (float)((exp(logits[r * vocab + v] - stats[2 * r]) * stats[2 * r + 1] -
+                                                            (v == target[r])) * gloss[r]);
     const fwp_mm_epilogue epi = {NULL, NULL, NULL, gbias, 0};
     if (gx) fwp_matmul(FWP_MM_NN, d, vocab, W, dim, gx, dim, rows, dim, vocab, NULL, workspace, stream);
     if (gW) fwp_matmul(FWP_MM_TN, d, vocab, x, dim, gW, dim, vocab, dim, rows, &epi, workspace, stream);

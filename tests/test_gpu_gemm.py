@@ -108,20 +108,20 @@ def test_negative_log_likelihood(fwp, rows, vocab, dim):
 def loss_and_gradients(L, x, W, b, target, gloss):
     """The loss with and without a graph's buffers (they agree), and the gradients of x, W and b."""
     rows, vocab, dim = x.shape[0], *W.shape
-    logits, loss, lse = (torch.full(s, float("nan"), device="cuda") for s in ((rows, vocab), (rows,), (rows,)))
+    logits, loss, stats = (torch.full(s, float("nan"), device="cuda") for s in ((rows, vocab), (rows,), (rows, 2)))
     work = torch.empty(L.lib().fwp_nll_workspace(rows, vocab), device="cuda")
     ptrs = [t.data_ptr() for t in (x, W, b, target)]
-    assert L.lib().fwp_nll_fwd(*ptrs, logits.data_ptr(), loss.data_ptr(), lse.data_ptr(), work.data_ptr(), rows, vocab,
-                               dim, L.stream_of(x)) == 0
+    assert L.lib().fwp_nll_stats_fwd(*ptrs, logits.data_ptr(), loss.data_ptr(), stats.data_ptr(), work.data_ptr(), rows, vocab,
+                                     dim, L.stream_of(x)) == 0
     only = torch.empty_like(loss)
     assert L.lib().fwp_nll_fwd(*ptrs, None, only.data_ptr(), None, work.data_ptr(), rows, vocab, dim, L.stream_of(x)) == 0
-    assert torch.equal(only, loss) or bool(loss.isnan().any())
+    assert torch.equal(only, loss)
     gx, gW, gb = torch.full_like(x, float("nan")), torch.full_like(W, float("nan")), torch.full_like(b, float("nan"))
     n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
-    work = torch.empty(n, device="cuda")
-    assert L.lib().fwp_nll_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), lse.data_ptr(), target.data_ptr(),
-                               gloss.data_ptr(), gx.data_ptr(), gW.data_ptr(), gb.data_ptr(), work.data_ptr(), rows, vocab,
-                               dim, L.stream_of(x)) == 0
+    work = torch.empty(max(1, n), device="cuda")
+    assert L.lib().fwp_nll_stats_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), stats.data_ptr(), target.data_ptr(),
+                                     gloss.data_ptr(), gx.data_ptr(), gW.data_ptr(), gb.data_ptr(), work.data_ptr(), rows, vocab,
+                                     dim, L.stream_of(x)) == 0
     return loss, gx, gW, gb
 
 
@@ -154,6 +154,29 @@ def test_loss_gradients_of_far_negative_logits(fwp, rows):
     x, W, b = randn(rows, 64, seed=1) * 0.1, randn(300, 64, seed=2) * 0.3, torch.full((300,), -100.0, device="cuda")
     target = torch.randint(0, 300, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
     check_loss(fwp._lib, x, W, b, target)
+
+
+@pytest.mark.parametrize("top", [1.0, 20.0, 200.0])
+@pytest.mark.parametrize("vocab", [130, 1000])
+def test_loss_of_confident_tokens(fwp, vocab, top):
+    """Exact logits (x is the identity, W has few bits), the target's far above the others: losses down to 1e-6."""
+    rows = 64
+    g = torch.Generator().manual_seed(1)
+    W = (torch.randint(-8, 9, (vocab, rows), generator=g) / 4.0 + (top - 18 * torch.rand(rows, generator=g)).round()).cuda()
+    target = torch.randint(0, vocab, (rows,), generator=g).cuda()
+    W[target, torch.arange(rows, device="cuda")] = top
+    gloss = randn(rows, seed=5)
+    loss, gx, gW, gb = loss_and_gradients(fwp._lib, torch.eye(rows, device="cuda"), W, torch.zeros(vocab, device="cuda"), target, gloss)
+    logits = W.t().double()
+    want = torch.nn.functional.cross_entropy(logits, target, reduction="none")
+    # a sum of about 20 roundings, at most, and its logarithm's; the difference of two logits is exact
+    assert bool(((loss.double() - want).abs() <= 32 * EPS * (1 + want)).all())
+    p = torch.softmax(logits, -1)
+    d = (p - torch.nn.functional.one_hot(target, vocab)) * gloss.double()[:, None]
+    # the exponential's argument is rounded twice on its way to a power of two; the target's p - 1 has its roundings at 1
+    hit = torch.nn.functional.one_hot(target, vocab)
+    tol = EPS * gloss.double().abs()[:, None] * (p * (32 + 2 * (logits.amax(-1, keepdim=True) - logits)) + 4 * hit)
+    assert bool(((gW.t().double() - d).abs() <= tol + 1e-12).all())
 
 
 @pytest.mark.parametrize("M,N,K", [(70, 66, 200), (300, 260, 1100), (40, 64, 2048), (2100, 2100, 40)])
