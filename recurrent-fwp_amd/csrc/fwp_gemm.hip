@@ -7,7 +7,8 @@
 // chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm): 2.2e-7 at K = 256,
 // 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling.  An operand that no bf16 number
 // holds (infinity, NaN, the last 2^-9 below fp32's largest) leaves NaN or infinity in the sums; an element that is
-// not finite is formed again from its fp32 operands (plain_sum).
+// not finite is formed again from its fp32 operands (plain_sum).  Parts below the smallest normal number count as zero, as
+// denormal operands do: an operand is exact to 2^-24 of itself or to 2^-126, whichever is more.
 //
 // v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
 // the 32x32x16 form 1.8), i.e. 350 TFLOP/s of such fp32 products, where the fp32 matrix instructions make 155.
@@ -68,6 +69,16 @@ struct Planes {
 // K = 1024: 4.7e7 -> 4.3e7 cycles of busy CUs, 95.0 -> 92.9 us.
 __device__ __forceinline__ constexpr int unit_of(int row, int chunk) { return row ^ (2 * chunk) ^ ((row >> 3) & 1); }
 
+// exp(x): 2^(x log2 e) by the hardware, x log2 e rounded to its nearest float and the rest of it as a factor: probabilities
+// are off by at most 4 roundings, down to e^-70 (with x log2 e alone by 60 there; PyTorch's, through the logarithm, by 69).  Arguments below -150 give
+// 0 as that one does (the rest of an infinity would be NaN); a NaN stays.
+__device__ __forceinline__ float exp_of(float x) {
+    constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
+    x = x < -150.f ? -150.f : x;
+    const float y = x * kLog2e, rest = fmaf(x, kLog2e, -y), e = __builtin_amdgcn_exp2f(y);
+    return fmaf(e, fmaf(rest, kLn2, x * (kLog2eRest * kLn2)), e);
+}
+
 // What turns stored logits into the gradient of the loss as an operand is loaded:
 // (exp(logit - shift) * scale - [vocabulary entry == target]) * gloss of the token, 0 for a negative target.
 // shift and scale: the largest logit and 1 / the sum of exp(logit - largest) (`stats`, exact where a token's probability
@@ -93,7 +104,7 @@ __device__ __forceinline__ NllToken nll_token(const NllArgs &a, int token) {
 }
 
 __device__ __forceinline__ float nll_grad(float logit, float shift, float scaled, float g, bool hit) {
-    return fmaf(__expf(logit - shift), scaled, hit ? -g : 0.f);
+    return fmaf(exp_of(logit - shift), scaled, hit ? -g : 0.f);
 }
 
 // One operand's share of the loads and LDS writes of a thread.  KC: rows are contiguous along k; a task is 8
@@ -240,7 +251,7 @@ __device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory")
 // What a sum of exp(logit - m) is multiplied with to become one of exp(logit - big).  A part of the vocabulary with no
 // logit but -infinity (masked words; columns beyond the last) has m = -infinity and the sum 0, or NaN if there
 // was one: it stays as it is (exp(-infinity + infinity) would make it NaN).
-__device__ __forceinline__ float to_max(float m, float big) { return m == -INFINITY ? 1.f : __expf(m - big); }
+__device__ __forceinline__ float to_max(float m, float big) { return m == -INFINITY ? 1.f : exp_of(m - big); }
 
 // The largest of a row's logits and the sum of exp(logit - largest): four logits per lane, LANES (8 or 16) lanes per row.
 template <int LANES>
@@ -258,7 +269,7 @@ __device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, flo
         for (int o = 4; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
     }
     const float z = m == -INFINITY ? 0.f : m;
-    float s = (__expf(v.x - z) + __expf(v.y - z)) + (__expf(v.z - z) + __expf(v.w - z));
+    float s = (exp_of(v.x - z) + exp_of(v.y - z)) + (exp_of(v.z - z) + exp_of(v.w - z));
     if constexpr (LANES == 16) {
         s += rotated<8>(s);
         s += rotated<4>(s), s += rotated<2>(s), s += rotated<1>(s);
@@ -595,7 +606,7 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
         s = s * to_max(mx, big) + ss[o][e] * to_max(x, big);
         mx = big;
     }
-    const float l = __logf(s);
+    const float l = logf(s);
     const int64_t want = target[m];
     if (lse) lse[m] = mx + l;
     if (stats) *reinterpret_cast<float2 *>(stats + 2 * (int64_t)m) = make_float2(mx, 1.f / s);

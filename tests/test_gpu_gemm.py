@@ -179,6 +179,24 @@ def test_loss_of_confident_tokens(fwp, vocab, top):
     assert bool(((gW.t().double() - d).abs() <= tol + 1e-12).all())
 
 
+@pytest.mark.parametrize("vocab", [130, 1000])
+def test_probabilities_far_below_the_largest(fwp, vocab):
+    """Exact logits down to 80 below the largest: the exponential's own error is a few roundings there too."""
+    rows, g = 64, torch.Generator().manual_seed(1)
+    W = (-torch.randint(0, 321, (vocab, rows), generator=g) / 4.0).cuda()
+    target = torch.randint(0, vocab, (rows,), generator=g).cuda()
+    gloss = randn(rows, seed=5)
+    loss, gx, gW, gb = loss_and_gradients(fwp._lib, torch.eye(rows, device="cuda"), W, torch.zeros(vocab, device="cuda"), target, gloss)
+    logits = W.t().double()
+    want = torch.nn.functional.cross_entropy(logits, target, reduction="none")
+    assert bool(((loss.double() - want).abs() <= 16 * EPS * (1 + want)).all())
+    p, hit = torch.softmax(logits, -1), torch.nn.functional.one_hot(target, vocab)
+    # the exponential 3 roundings, the sum and its inverse up to 16, two products; the target's p - 1 has its own at 1
+    # and an operand of the product loses what of its three parts is below the smallest normal number, 2^-126
+    tol = EPS * gloss.double().abs()[:, None] * (24 * p + 4 * hit) + 2.0 ** -125
+    assert bool(((gW.t().double() - (p - hit) * gloss.double()[:, None]).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 66, 200), (300, 260, 1100), (40, 64, 2048), (2100, 2100, 40)])
 @pytest.mark.parametrize("layout", [NT, NN, TN])
 def test_products_of_infinities_and_the_largest_numbers(fwp, layout, M, N, K):
