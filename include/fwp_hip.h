@@ -279,7 +279,7 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
  *   FWP_MM_TN: C = A^T B, A [K,M], B [K,N]      row-major, rows lda, ldb, ldc floats apart
  * epi (NULL: none): C = relu(C + bias) + residual, 0 where gate <= 0, each part optional (a NaN passes relu and gate, as in
  * PyTorch); residual and gate are laid out like C.  colsum (FWP_MM_TN): [M], the sums of A's columns (a bias gradient).
- * workspace: fwp_matmul_workspace(M, N, K) floats, or NULL (a product with few tiles and a long K then runs on fewer CUs).
+ * workspace: fwp_matmul_workspace(M, N, K) floats (16-byte aligned), or NULL (a product with few tiles and a long K then runs on fewer CUs).
  */
 enum { FWP_MM_NT = 0, FWP_MM_NN = 1, FWP_MM_TN = 2 };
 typedef struct fwp_mm_epilogue {

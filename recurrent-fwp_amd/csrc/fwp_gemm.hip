@@ -217,8 +217,8 @@ struct Operand {
 
 struct GemmArgs {
     const float *A, *B;
-    float *C;                    // the result, or (several k ranges) one M x N partial result per range
-    int64_t lda, ldb, ldc;
+    float *C;                    // the result, or (several k ranges) one M x N partial result per range, `part` floats apart
+    int64_t lda, ldb, ldc, part;
     int M, N, K;
     int ks;                      // k per range (a multiple of kBK)
     int vec;                     // C, residual and gate can be accessed 16 bytes at a time
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     float bias[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) bias[e] = g.epi.bias && n + e < g.N && (gridDim.y == 1) ? g.epi.bias[n + e] : 0.f;
-    float *const C = g.C + (int64_t)blockIdx.y * g.M * g.ldc;
+    float *const C = g.C + blockIdx.y * g.part;
     const bool one = gridDim.y == 1;
     float *const sums_of = reinterpret_cast<float *>(&Lb);       // kLse: [2][column half][row]
 #pragma unroll
@@ -463,16 +463,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     }
 }
 
-// C[M,N] = the sum of `ranges` partial results, with the epilogue; four threads share four neighbouring
-// elements, a quarter of the ranges each, and add up in a fixed order.  The workgroups behind them do the same for the
-// column sums of A ([ranges][M] behind the partial results).
+// C[M,N] = the sum of `ranges` partial results `stride` floats apart (whole 16-byte groups: the last may reach beyond M N),
+// with the epilogue; four threads share four neighbouring elements, a quarter of the ranges each, and add up in a
+// fixed order.  The workgroups behind them do the same for the column sums of A ([ranges][M] behind the partial results).
 __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restrict__ part, float *__restrict__ C,
-                                                          int64_t total, int M, int N, int ranges, fwp_mm_epilogue epi) {
+                                                          int64_t total, int64_t stride, int M, int N, int ranges,
+                                                          fwp_mm_epilogue epi) {
     __shared__ float4 s[4][64];
     const int e = threadIdx.x % 64, q = threadIdx.x / 64;
-    const int64_t blocks = (total / 4 + 63) / 64;
+    const int64_t blocks = (stride / 4 + 63) / 64;
     if (blockIdx.x >= blocks) {
-        const float *const col = part + ranges * total;
+        const float *const col = part + ranges * stride;
         const int m = (int)(blockIdx.x - blocks) * 64 + e;
         float x = 0.f;
         if (m < M) {
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restric
     if (at < total) {
 #pragma unroll 4
         for (int r = q; r < ranges; r += 4) {
-            const float4 y = *reinterpret_cast<const float4 *>(part + r * total + at);
+            const float4 y = *reinterpret_cast<const float4 *>(part + r * stride + at);
             x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
         }
     }
@@ -500,12 +501,17 @@ __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restric
         const float4 y = s[o][e];
         x.x += y.x, x.y += y.y, x.z += y.z, x.w += y.w;
     }
-    if (epi.bias) {
-        const float *b = epi.bias + (int)(at % N);
-        x.x += b[0], x.y += b[1], x.z += b[2], x.w += b[3];
+    float v[4] = {x.x, x.y, x.z, x.w};
+    const int n = (int)(at % N);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (at + i >= total) break;
+        if (epi.bias) v[i] += epi.bias[N % 4 ? (int)((at + i) % N) : n + i];
+        v[i] = apply(epi, v[i], at + i);
     }
-    const float4 y = make_float4(apply(epi, x.x, at), apply(epi, x.y, at + 1), apply(epi, x.z, at + 2), apply(epi, x.w, at + 3));
-    *reinterpret_cast<float4 *>(C + at) = y;
+    if (at + 3 < total) *reinterpret_cast<float4 *>(C + at) = make_float4(v[0], v[1], v[2], v[3]);
+    else
+        for (int i = 0; at + i < total; i++) C[at + i] = v[i];
 }
 
 struct Plan {
@@ -543,15 +549,14 @@ void launch(const GemmArgs &g, const Plan &p, hipStream_t s) {
 
 bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-bool may_cut(int N, const float *C, int64_t ldc) {
-    return ldc == N && N % 4 == 0 && aligned(C);
-}
+// a partial result, in whole 16-byte groups
+int64_t part_of(int M, int N) { return ((int64_t)M * N + 3) / 4 * 4; }
 
 }  // namespace
 
 int64_t matmul_workspace(int M, int N, int K) {
-    const Plan p = plan_of(M, N, K, N % 4 == 0);
-    return p.ranges > 1 ? (int64_t)p.ranges * ((int64_t)M * N + M) : 0;
+    const Plan p = plan_of(M, N, K, true);
+    return p.ranges > 1 ? p.ranges * (part_of(M, N) + M) : 0;
 }
 
 int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
@@ -559,13 +564,14 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     GemmArgs g{};
     g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
     if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target};
-    const Plan p = plan_of(M, N, K, workspace && may_cut(N, C, ldc));
+    const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace));
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
     const bool cut = p.ranges > 1;
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
+    g.part = part_of(M, N);
     g.vec = g.ldc % 4 == 0 && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
-    float *const col = cut ? workspace + (int64_t)p.ranges * M * N : epi.colsum;
+    float *const col = cut ? workspace + p.ranges * g.part : epi.colsum;
     g.colsum = layout == FWP_MM_TN && epi.colsum ? col : nullptr;
     if (layout == FWP_MM_NT) launch<true, true, kPlain>(g, p, s);
     else if (layout == FWP_MM_NN && !nll) launch<true, false, kPlain>(g, p, s);
@@ -573,8 +579,8 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     else if (!nll) launch<false, false, kPlain>(g, p, s);
     else launch<false, false, kGrad>(g, p, s);
     if (cut) {
-        const int64_t total = (int64_t)M * N, blocks = (total / 4 + 63) / 64 + (g.colsum ? (M + 63) / 64 : 0);
-        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)blocks), dim3(kThreads), 0, s, workspace, C, total, M, N, p.ranges, epi);
+        const int64_t total = (int64_t)M * N, blocks = (g.part / 4 + 63) / 64 + (g.colsum ? (M + 63) / 64 : 0);
+        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)blocks), dim3(kThreads), 0, s, workspace, C, total, g.part, M, N, p.ranges, epi);
     }
     return (int)hipGetLastError();
 }

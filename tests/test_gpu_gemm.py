@@ -197,6 +197,39 @@ def test_probabilities_far_below_the_largest(fwp, vocab):
     assert bool(((gW.t().double() - (p - hit) * gloss.double()[:, None]).abs() <= tol).all())
 
 
+def spread(t, by=0, first=0):
+    """The same values with rows `by` floats further apart, the first `first` floats into the storage; NaN around them."""
+    R, C = t.shape
+    buf = torch.full((R * (C + by) + first,), float("nan"), device="cuda")
+    out = buf[first:].view(R, C + by)[:, :C]
+    out.copy_(t)
+    return out
+
+
+# results whose rows are no whole 16-byte groups: k in several ranges, in one; wide tiles and small ones
+@pytest.mark.parametrize("M,N,K,cut", [(66, 201, 2400, True), (256, 1001, 700, True), (5, 3, 9000, True), (130, 775, 256, False),
+                                       (2100, 2101, 64, False)])
+@pytest.mark.parametrize("layout", [NT, NN, TN])
+def test_ragged_results_spread_and_unaligned_operands(fwp, layout, M, N, K, cut):
+    assert (fwp._lib.lib().fwp_matmul_workspace(M, N, K) > 0) == cut
+    A = randn(*((K, M) if layout == TN else (M, K)), seed=1)
+    B = randn(*((N, K) if layout == NT else (K, N)), seed=2)
+    bias, residual, gate = randn(N, seed=3) * 30, randn(M, N, seed=4) * 30, randn(M, N, seed=5)
+    a, b = A.double(), B.double()
+    a, b = (a.t() if layout == TN else a), (b.t() if layout == NT else b)
+    raw, mag = a @ b, a.abs() @ b.abs()
+    want = torch.where(gate > 0, torch.relu(raw + bias.double()) + residual.double(), 0.0)
+    for by, first in ((0, 0), (0, 1), (3, 2), (8, 4)):
+        x, y = spread(A, by, first), spread(B, by, first)
+        if layout == TN:
+            colsum = torch.full((M,), float("nan"), device="cuda")
+            got = matmul(fwp._lib, TN, x, y, colsum=colsum)
+            assert bool(((got.double() - raw).abs() <= bound(K, mag)).all())
+            assert bool(((colsum.double() - a.sum(1)).abs() <= K * EPS * a.abs().sum(1)).all())
+        got = matmul(fwp._lib, layout, x, y, bias=bias, relu=1, residual=residual, gate=gate)
+        assert bool(((got.double() - want).abs() <= bound(K, mag + 400)).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 66, 200), (300, 260, 1100), (40, 64, 2048), (2100, 2100, 40)])
 @pytest.mark.parametrize("layout", [NT, NN, TN])
 def test_products_of_infinities_and_the_largest_numbers(fwp, layout, M, N, K):
