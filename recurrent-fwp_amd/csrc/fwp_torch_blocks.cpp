@@ -29,6 +29,10 @@ at::Tensor plain(const at::Tensor &t) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 ? t.clone() : t;
 }
 
+// The kernels get addresses and sizes: every block compares its tensors' sizes before it hands them on.
+bool optional_of(const at::Tensor &t, int64_t n) { return !t.defined() || same_shape(t, {n}); }
+bool ends_in(const at::Tensor &x, int64_t n) { return x.dim() > 0 && x.size(-1) == n; }
+
 // C = op(A) op(B) with an epilogue, shaped `shape` (M x N elements)
 at::Tensor matmul(int layout, const at::Tensor &A, const at::Tensor &B, int64_t M, int64_t N, int64_t K, at::IntArrayRef shape,
                   const fwp_mm_epilogue &epi = {}) {
@@ -69,6 +73,8 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
         const at::Tensor bias = given(bias_in);
         require_device(x_in);
         same_device(x_in, {W, bias});
+        require(W.dim() == 2 && W.numel() > 0 && x_in.numel() > 0 && ends_in(x_in, W.size(1)) && optional_of(bias, W.size(0)),
+                "x, weight and bias do not fit one another");
         const int64_t in = W.size(1), out = W.size(0), rows = x_in.numel() / in;
         const at::Tensor x = plain(x_in);
         std::vector<int64_t> shape = x.sizes().vec();
@@ -127,6 +133,10 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
         const at::Tensor residual = given(residual_in);
         require_device(x_in);
         same_device(x_in, {W1, b1, W2, b2, residual});
+        require(W1.dim() == 2 && W1.numel() > 0 && x_in.numel() > 0 && ends_in(x_in, W1.size(1)) && same_shape(b1, {W1.size(0)}) &&
+                    same_shape(W2, {W1.size(1), W1.size(0)}) && same_shape(b2, {W1.size(1)}) &&
+                    (!residual.defined() || residual.sizes() == x_in.sizes()),
+                "x, weights, biases and residual do not fit one another");
         const int64_t d = W1.size(1), inner = W1.size(0), rows = x_in.numel() / d;
         const at::Tensor x = plain(x_in), res = same ? x : residual.defined() ? plain(residual) : residual;
         LaunchGuard guard(x);
@@ -189,7 +199,7 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
         same_device(x_in, {Wqkvb, Wo, state});
         require(x_in.dim() == 3, "expected [len, bsz, d_model]");
         const int64_t T = x_in.size(0), B = x_in.size(1), d = x_in.size(2), rows = T * B, width = H * (3 * D + 1);
-        require(Wqkvb.size(0) == width && Wqkvb.size(1) == d && Wo.size(1) == H * D && same_shape(state, {B, H, D, D}),
+        require(x_in.numel() > 0 && same_shape(Wqkvb, {width, d}) && same_shape(Wo, {d, H * D}) && same_shape(state, {B, H, D, D}),
                 "projections and state do not fit the heads");
         require_state(state, "W");
         const at::Tensor x = plain(x_in);
@@ -279,6 +289,8 @@ struct LayerNormFn : torch::autograd::Function<LayerNormFn> {
     static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
         require_device(x_in);
         same_device(x_in, {gamma, beta});
+        require(gamma.dim() == 1 && beta.sizes() == gamma.sizes() && x_in.numel() > 0 && ends_in(x_in, gamma.size(0)),
+                "rows, weight and bias do not fit one another");
         const at::Tensor x = plain(x_in), g = plain(gamma), b = plain(beta);
         const int64_t cols = gamma.numel(), rows = x.numel() / cols;
         LaunchGuard guard(x);
@@ -328,6 +340,8 @@ struct NllFn : torch::autograd::Function<NllFn> {
         same_device(x_in, {W, bias, target_in});
         require(x_in.dim() == 2 && target_in.dim() == 1 && target_in.size(0) == x_in.size(0) && target_in.scalar_type() == at::kLong,
                 "hidden [rows, d_model] and int64 targets [rows]");
+        require(x_in.numel() > 0 && W.dim() == 2 && W.numel() > 0 && W.size(1) == x_in.size(1) && same_shape(bias, {W.size(0)}),
+                "hidden, weight and bias do not fit one another");
         const at::Tensor x = plain(x_in), target = target_in.contiguous();
         const int64_t rows = x.size(0), dim = x.size(1), vocab = W.size(0);
         LaunchGuard guard(x);
@@ -462,6 +476,7 @@ at::Tensor embed(const at::Tensor &table, const at::Tensor &ids, const at::Tenso
     at::AutoDispatchBelowADInplaceOrView below;
     require_device(table);
     same_device(table, {ids, inv_freq});
+    require(table.dim() == 2 && ids.dim() == 2, "a table [n_token, d_model] and ids [len, bsz]");
     const int64_t T = ids.size(0), B = ids.size(1), d = table.size(1);
     require(ids.scalar_type() == at::kLong && inv_freq.numel() * 2 == d, "int64 ids [len, bsz] and d_model/2 frequencies");
     const at::Tensor t = plain(table), i = ids.contiguous(), f = plain(inv_freq), out = at::empty({T, B, d}, t.options());

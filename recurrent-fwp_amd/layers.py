@@ -24,10 +24,10 @@ def _untouched(m, cls):
 def _blocks(x, *params):
     """The C++ blocks (csrc/fwp_torch_blocks.cpp) if they apply to this input and these parameters: fp32 on the
     GPU, outside autocast, tracing and functional transforms."""
-    if _fwp_torch is None or not x.is_cuda or x.numel() == 0:
+    if _fwp_torch is None or not x.is_cuda:
         return None
     for t in (x, *params):
-        if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter):
+        if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter) or t.numel() == 0:
             return None
     if not all(p.is_contiguous() for p in params):
         return None
@@ -47,7 +47,8 @@ class Linear(nn.Linear):
     """``nn.Linear`` on the package's matrix products where they apply."""
 
     def forward(self, x):
-        if self.bias is not None and x.dim() > 0 and x.shape[-1] == self.in_features:
+        if (self.bias is not None and x.dim() > 0 and self.weight.shape[1:] == x.shape[-1:]
+                and self.bias.shape == self.weight.shape[:1]):
             blocks = _blocks(x, self.weight, self.bias)
             if blocks is not None:
                 return blocks.linear(x, self.weight, self.bias)
@@ -91,7 +92,8 @@ def _layer_norm(m, x):
     """``m(x)`` for a LayerNorm over the last axis."""
     if _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:
         d = m.normalized_shape[0]
-        blocks = _blocks(x, m.weight, m.bias) if d % 4 == 0 and d <= 1024 and x.shape[-1] == d else None
+        fits = m.weight.shape == (d,) and m.bias.shape == (d,) and x.shape[-1] == d
+        blocks = _blocks(x, m.weight, m.bias) if d % 4 == 0 and d <= 1024 and fits else None
         if blocks is not None:
             return blocks.layer_norm(x, m.weight, m.bias, m.eps)
     return m(x)
@@ -133,12 +135,15 @@ class PositionwiseFF(nn.Module):
         if (_untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
                 and _untouched(net[2], nn.Dropout) and _untouched(net[3], nn.Linear) and _untouched(net[4], nn.Dropout)
                 and net[0].bias is not None and net[3].bias is not None):
-            blocks = _blocks(x, net[0].weight, net[0].bias, net[3].weight, net[3].bias)
+            W1, b1, W2, b2 = net[0].weight, net[0].bias, net[3].weight, net[3].bias
+            d, inner = x.shape[-1], b1.numel()
+            fits = W1.shape == (inner, d) and b1.shape == (inner,) and W2.shape == (d, inner) and b2.shape == (d,)
+            blocks = _blocks(x, W1, b1, W2, b2) if fits else None
             if blocks is not None and not (_drops(net[2]) or _drops(net[4])):
-                return blocks.feed_forward(x, net[0].weight, net[0].bias, net[3].weight, net[3].bias, residual)
+                return blocks.feed_forward(x, W1, b1, W2, b2, residual)
             if blocks is not None:
-                hid = net[2](blocks.linear(x, net[0].weight, net[0].bias, True))
-                return residual + net[4](blocks.linear(hid, net[3].weight, net[3].bias))
+                hid = net[2](blocks.linear(x, W1, b1, True))
+                return residual + net[4](blocks.linear(hid, W2, b2))
         return residual + net(x)
 
     def forward(self, inp):
@@ -245,7 +250,8 @@ class DeltaNetLayer(nn.Module):
         hip_op = self.fast_weight_op is fast_weight_delta
         blocks = None
         if (hip_op and D in (16, 32, 64) and _untouched(self.qkvb_net, nn.Linear) and _untouched(self.o_net, nn.Linear)
-                and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)):
+                and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)
+                and self.qkvb_net.weight.shape == (H * (3 * D + 1), x.shape[-1]) and self.o_net.weight.shape == (x.shape[-1], H * D)):
             blocks = _blocks(x, self.qkvb_net.weight, self.o_net.weight)
         if blocks is not None:
             W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32)

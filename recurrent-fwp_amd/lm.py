@@ -37,9 +37,12 @@ class _TiedSoftmaxLoss(nn.Module):
 
     def forward(self, hidden, target):
         out = self.out_layers[0]
-        blocks = _blocks(hidden, out.weight, out.bias) if _untouched(out, Linear) and out.bias is not None else None
-        if blocks is not None and target.dtype is torch.int64 and target.device == hidden.device:
-            return blocks.nll(hidden, out.weight, out.bias, target)
+        if (_untouched(out, Linear) and out.bias is not None and target.dtype is torch.int64 and target.device == hidden.device
+                and hidden.dim() == 2 and target.shape == hidden.shape[:1]
+                and out.weight.shape[1:] == hidden.shape[1:] and out.bias.shape == out.weight.shape[:1]):
+            blocks = _blocks(hidden, out.weight, out.bias)
+            if blocks is not None:
+                return blocks.nll(hidden, out.weight, out.bias, target)
         return F.cross_entropy(out(hidden), target, reduction="none")
 
 

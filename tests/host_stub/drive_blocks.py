@@ -2,6 +2,9 @@
 the same computation by PyTorch's operators in float64: the stand-in library computes the products, LayerNorm and the
 loss, so what is compared is what the blocks make of them.  Run as a script (python drive_blocks.py BUILD_DIR CHECK),
 normally by tests/test_binding_host.py.  Prints 'CHECK ok' at the end."""
+import importlib
+import inspect
+import os
 import sys
 
 import torch
@@ -84,6 +87,111 @@ def results(m):
     phase = torch.arange(3.0, -1, -1).clamp_max(2)[:, None] * freq
     want = W[ids] * 8.0 + torch.cat((phase.sin(), phase.cos()), -1)[:, None]
     close(m.embed(W, ids, freq, 8.0, 2.0), want, "embedding")
+
+
+def refused(f, *args):
+    for grad in (True, False):
+        with torch.set_grad_enabled(grad):
+            try:
+                f(*args)
+            except (RuntimeError, AssertionError):
+                continue
+        raise AssertionError(("accepted", f, [tuple(t.shape) for t in args if torch.is_tensor(t)]))
+
+
+def misfits(m):
+    """Operands whose sizes do not fit one another raise before a kernel gets their addresses."""
+    x, W, b, W2, b2 = rnd(6, 64, grad=True), rnd(128, 64, grad=True), rnd(128), rnd(64, 128), rnd(64)
+    for bad in ((rnd(6, 60), W, b), (rnd(6, 128), W, b), (x, W, rnd(127)), (x, W, rnd(129)), (x, rnd(128), None), (rnd(()), W, None)):
+        refused(m.linear, *bad)
+    refused(m.feed_forward, rnd(6, 32), W, b, W2, b2)
+    refused(m.feed_forward, x, W, b, rnd(64, 96), b2)           # 8192 of 6144 floats
+    refused(m.feed_forward, x, W, b, rnd(64, 130), b2)
+    refused(m.feed_forward, x, W, rnd(120), W2, b2)
+    refused(m.feed_forward, x, W, b, W2, rnd(60))
+    refused(m.feed_forward, x, W, b, W2, b2, rnd(1, 64))
+    refused(m.feed_forward, x, W, b, rnd(1, 128), rnd(1))
+    target = torch.zeros(6, dtype=torch.int64)
+    for bad in ((x, rnd(100, 32), rnd(100)), (x, rnd(100, 64), rnd(90)), (x, rnd(100, 65), rnd(100)), (x, rnd(100, 64), rnd(101))):
+        refused(m.nll, *bad, target)
+    refused(m.nll, x, rnd(100, 64), rnd(100), target[:5])
+    refused(m.nll, rnd(2, 3, 64), rnd(100, 64), rnd(100), target)
+    for bad in ((rnd(6, 24), rnd(24), rnd(20)), (rnd(6, 24), rnd(20), rnd(20)), (rnd(6, 24), rnd(28), rnd(24)), (rnd(6, 24), rnd(2, 12), rnd(24))):
+        refused(m.layer_norm, *bad, 1e-5)
+    y, Wqkvb, Wo, state = rnd(5, 2, 48, grad=True), rnd(3 * 49, 48), rnd(48, 48), torch.zeros(2, 3, 16, 16)
+    m.delta_block(y, Wqkvb, Wo, state, 3, 16, 0.25, True)
+    for bad in ((y, Wqkvb, rnd(40, 48), state), (y, Wqkvb, rnd(50, 48), state), (y, Wqkvb, rnd(48, 32), state), (y, rnd(146, 48), Wo, state),
+                (y, rnd(3 * 49, 40), Wo, state), (y, Wqkvb, Wo, torch.zeros(1, 3, 16, 16)), (rnd(10, 48), Wqkvb, Wo, state)):
+        refused(m.delta_block, *bad, 3, 16, 0.25, True)
+    refused(m.embed, rnd(24, 64), torch.zeros(4, 3, dtype=torch.int64), rnd(30), 8.0, 0.0)
+    refused(m.embed, rnd(24, 64), torch.zeros(4, dtype=torch.int64), rnd(32), 8.0, 0.0)
+    refused(m.embed, rnd(64), torch.zeros(4, 3, dtype=torch.int64), rnd(32), 8.0, 0.0)
+
+
+class Recorded:
+    """The blocks, with the names of those that were called."""
+
+    def __init__(self, m):
+        self.m, self.calls = m, []
+
+    def __getattr__(self, name):
+        f = getattr(self.m, name)
+
+        def call(*args):
+            self.calls.append(name)
+            return f(*args)
+        return call
+
+    def of(self, f, *args):
+        """The blocks that f(*args) goes through, and its result (an exception among them)."""
+        self.calls.clear()
+        try:
+            res = f(*args)
+        except Exception as e:
+            res = e
+        return list(self.calls), res
+
+
+def package(m):
+    """The package with its layers on the host build's blocks: host tensors count as the GPU's."""
+    sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
+    pkg = importlib.import_module("recurrent-fwp_amd")
+    layers, lm, rec = pkg.layers, pkg.lm, Recorded(m)
+    layers._fwp_torch = rec
+    exec(inspect.getsource(layers._blocks).replace("x.is_cuda", "True").replace("t.is_cuda", "True"), layers.__dict__)
+    lm._blocks = layers._blocks
+    return pkg, rec
+
+
+def misfitting_modules(m):
+    """Modules whose parameters do not fit one another do what they do on stock PyTorch."""
+    pkg, rec = package(m)
+    nn, x = torch.nn, rnd(5, 2, 24)
+    ff = pkg.PositionwiseFF(24, 40, 0.0)
+    assert rec.of(ff, x)[0] == ["feed_forward", "layer_norm"]
+    ff.CoreNet[3] = nn.Linear(40, 1)                       # added to the input by broadcasting
+    calls, y = rec.of(ff._core, x, x)
+    assert calls == [] and torch.equal(y, x + ff.CoreNet(x))
+    ff.CoreNet[3] = nn.Linear(36, 24)
+    calls, e = rec.of(ff, x)
+    assert calls == [] and type(e) is RuntimeError, e
+    ff = pkg.PositionwiseFF(24, 40, 0.0)
+    for bad in (rnd(5, 2, 20), rnd(5, 2, 48)):
+        calls, e = rec.of(ff, bad)
+        assert calls == [] and type(e) is RuntimeError, e
+    crit, target = pkg.lm._TiedSoftmaxLoss(100, 24), torch.zeros(6, dtype=torch.int64)
+    assert rec.of(crit, rnd(6, 24), target)[0] == ["nll"]
+    for hidden, t in ((rnd(6, 20), target), (rnd(6, 30), target), (rnd(6, 24), target[:5])):
+        calls, e = rec.of(crit, hidden, t)
+        assert calls in ([], ["linear"]) and type(e) in (RuntimeError, ValueError), e
+    calls, y = rec.of(crit, rnd(24), target[0])            # one token without a batch
+    assert calls == ["linear"] and y.shape == ()
+    crit.out_layers[0].weight = nn.Parameter(rnd(120, 24))  # a vocabulary that grew without its bias
+    calls, e = rec.of(crit, rnd(6, 24), target)
+    assert calls == [] and type(e) is RuntimeError, e
+    lin = pkg.layers.Linear(24, 0)
+    calls, y = rec.of(lin, x)
+    assert calls == [] and y.shape == (5, 2, 0)
 
 
 def main():
