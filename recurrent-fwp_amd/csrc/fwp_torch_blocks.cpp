@@ -191,6 +191,45 @@ struct FeedForwardFn : torch::autograd::Function<FeedForwardFn> {
 
 // ------------------------------------------------------------------ s = (x +) o_net(delta rule(qkvb_net(x)))
 
+// The gradient of the projection qkvb from that of the delta rule's read-out, go [T,B,H,D]
+at::Tensor projection_grad(const at::Tensor &go, const at::Tensor &qkvb, const at::Tensor &q, const at::Tensor &k, const at::Tensor &beta,
+                           const at::Tensor &buf, double scale) {
+    const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3), rows = T * B;
+    void *const s = stream_of(go);
+    Parts parts({rows * H * D, rows * H * D, rows * H * D, rows * H}, go.options());
+    const at::Tensor gq = parts.take(B, H, T, D), gk = parts.take(B, H, T, D), gv = parts.take(B, H, T, D), gb = parts.take(B, H, T, 1);
+    const float *vdiff = ptr(buf), *ckpt = vdiff + rows * H * D;
+    const fwp_view gov = {ptr(go), H * D, D, B * H * D};
+    check(fwp_delta_bwd(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), (int)B, (int)H, (int)T,
+                        (int)D, (int)D, fwp_query(FWP_Q_DEFAULT_CHUNK), s),
+          "fwp_delta_bwd");
+    const at::Tensor gp = at::empty_like(qkvb);
+    check(fwp_deltanet_prep_bwd(ptr(qkvb), ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(gp), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
+          "fwp_deltanet_prep_bwd");
+    return gp;
+}
+
+// The read-out [T,B,H,D] that a DeltaBlockFn's forward pass left, as a function of its x and Wqkvb again: with create_graph the
+// gradient of Wo is a product with it.
+struct DeltaReadOutFn : torch::autograd::Function<DeltaReadOutFn> {
+    static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x, const at::Tensor &Wqkvb, const at::Tensor &qkvb, const at::Tensor &q,
+                              const at::Tensor &k, const at::Tensor &beta, const at::Tensor &buf, const at::Tensor &out, double scale) {
+        ctx->save_for_backward({x, Wqkvb, qkvb, q, k, beta, buf});
+        ctx->saved_data["scale"] = scale;
+        return out.detach();
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &x = saved[0], &Wqkvb = saved[1], go = plain(grads[0]);
+        LaunchGuard guard(go);
+        const at::Tensor gp = projection_grad(go, saved[2], saved[3], saved[4], saved[5], saved[6], ctx->saved_data["scale"].toDouble());
+        variable_list res(9);
+        if (ctx->needs_input_grad(0)) res[0] = at::matmul(gp, Wqkvb);
+        if (ctx->needs_input_grad(1)) res[1] = at::matmul(gp.flatten(0, 1).t(), x.reshape({-1, x.size(2)}));
+        return res;
+    }
+};
+
 struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
     // x [T,B,d]; Wqkvb [H (3D+1), d]; Wo [d, H D]; state [B,H,D,D] in/out
     static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &Wqkvb, const at::Tensor &Wo,
@@ -246,28 +285,17 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
                          &q = saved[4], &k = saved[5], &beta = saved[6], &buf = saved[7], &out = saved[8];
         const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3), rows = T * B, d = Wqkvb.size(1),
                       width = Wqkvb.size(0);
-        const auto opts = x.options();
         LaunchGuard guard(x);
-        void *const s = stream_of(x);
         // create_graph: the projections' products from PyTorch's operators (the delta rule's own gradients, as from
         // fast_weight_delta, carry no graph)
         const bool graph = at::GradMode::is_enabled();
         if (ctx->needs_input_grad(2))
-            res[2] = graph ? at::matmul(grads[0].reshape({rows, d}).t(), out.reshape({rows, H * D}))
+            res[2] = graph ? at::matmul(grads[0].reshape({rows, d}).t(),
+                                        DeltaReadOutFn::apply(saved[0], Wqkvb, qkvb, q, k, beta, buf, out, ctx->saved_data["scale"].toDouble())
+                                            .reshape({rows, H * D}))
                            : weight_grad(g, out, rows, d, H * D, nullptr);
         const at::Tensor go = matmul(FWP_MM_NN, g, Wo, rows, H * D, d, {T, B, H, D});
-        Parts parts({rows * H * D, rows * H * D, rows * H * D, rows * H}, opts);
-        const at::Tensor gq = parts.take(B, H, T, D), gk = parts.take(B, H, T, D), gv = parts.take(B, H, T, D),
-                         gb = parts.take(B, H, T, 1);
-        const float *vdiff = ptr(buf), *ckpt = vdiff + rows * H * D;
-        const fwp_view gov = {ptr(go), H * D, D, B * H * D};
-        check(fwp_delta_bwd(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), (int)B,
-                            (int)H, (int)T, (int)D, (int)D, fwp_query(FWP_Q_DEFAULT_CHUNK), s),
-              "fwp_delta_bwd");
-        const at::Tensor gp = at::empty_like(qkvb);
-        check(fwp_deltanet_prep_bwd(ptr(qkvb), ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(gp), (int)T, (int)B, (int)H, (int)D,
-                                    (float)ctx->saved_data["scale"].toDouble(), s),
-              "fwp_deltanet_prep_bwd");
+        const at::Tensor gp = projection_grad(go, qkvb, q, k, beta, buf, ctx->saved_data["scale"].toDouble());
         if (ctx->needs_input_grad(1))
             res[1] = graph ? at::matmul(gp.reshape({rows, width}).t(), saved[0].reshape({rows, d}))
                            : weight_grad(gp, x, rows, width, d, nullptr);

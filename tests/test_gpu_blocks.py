@@ -88,6 +88,39 @@ def test_second_derivatives_and_hooks_take_stock_operators(fwp):
 
 
 @pytest.mark.parametrize("pre", [False, True])
+@pytest.mark.parametrize("power", [1, 2])
+def test_second_derivatives_of_the_delta_block(fwp, pre, power):
+    """Through the gradients of every parameter and of the input, as from the layer's general path (a hook on the dropout
+    sends it there): the delta rule's own gradients are constants there, what they are multiplied with is not."""
+    x, c = torch.randn(2, 20, 2, 48, generator=torch.Generator().manual_seed(1)).cuda()      # c: a sum over LayerNorm is constant
+    seconds = []
+    for general in (False, True):
+        torch.manual_seed(0)
+        m = fwp.DeltaNetLayer(3, 48, 16, pre_lnorm=pre).cuda()
+        if general:
+            m.drop.register_forward_hook(lambda *a: None)
+        z = x.clone().requires_grad_()
+        firsts = torch.autograd.grad(((c * m(z)) ** power).sum(), [z, *m.parameters()], create_graph=True)
+        # one by one: what each first derivative depends on
+        g = torch.Generator().manual_seed(2)
+        for (name, _), first in zip([("x", z), *m.named_parameters()], firsts):
+            w = torch.randn(first.shape, generator=g).cuda()
+            if first.requires_grad:
+                got = torch.autograd.grad((first * w).sum(), [z, *m.parameters()], allow_unused=True, retain_graph=True)
+            else:
+                got = [None] * len(firsts)
+            seconds += [(general, name, i, t) for i, t in enumerate(got)]
+    half = len(seconds) // 2
+    for (_, name, i, got), (_, _, _, want) in zip(seconds[:half], seconds[half:]):
+        zero = torch.zeros(1, device="cuda")      # no dependence and a gradient of zeros are the same
+        got, want = zero if got is None else got, zero if want is None else want.double()
+        if got.numel() == 1 or want.numel() == 1:
+            assert float(got.abs().max()) == float(want.abs().max()) == 0, (name, i)
+        else:
+            close((name, i), got, want, 64)
+
+
+@pytest.mark.parametrize("pre", [False, True])
 def test_language_model_with_ignored_targets(fwp, pre):
     """Losses and every gradient of a two-layer model, some targets ignored, frozen embedding included."""
     cfg = dict(n_token=309, n_layer=2, n_head=3, d_model=48, d_head=16, d_inner=100, pre_lnorm=pre, tie_weight=False)
