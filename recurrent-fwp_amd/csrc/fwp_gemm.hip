@@ -6,8 +6,8 @@
 // 2^-26 |x x'|, a quarter of the rounding of an fp32 product.  Sums are fp32, six roundings per 32 terms where a
 // chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm): 2.2e-7 at K = 256,
 // 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling.  An operand that no bf16 number
-// holds (infinity, NaN, the last 2^-9 below fp32's largest) leaves NaN or infinity in the sums; an element that is
-// not finite is formed again from its fp32 operands (plain_sum).  Parts below the smallest normal number count as zero, as
+// holds (infinity, NaN, the last 2^-9 below fp32's largest) leaves NaN or infinity in the sums: a tile
+// with an element that is not finite is formed again on the fp32 matrix instructions (three times the tile's time).  Parts below the smallest normal number count as zero, as
 // denormal operands do: an operand is exact to 2^-24 of itself or to 2^-126, whichever is more.
 //
 // v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
@@ -213,6 +213,19 @@ struct Operand {
                 L.u[2][ch][at] = l;
             }
     }
+    // fp32 as it is: 16-byte units of 4 consecutive k of one row, [k / 4][row], in the same memory
+    static __device__ __forceinline__ v4f *plain(Planes<ROWS> &L) { return reinterpret_cast<v4f *>(&L); }
+    __device__ __forceinline__ void store_plain(Planes<ROWS> &L, int tid) const {
+#pragma unroll
+        for (int i = 0; i < kTasks; i++)
+#pragma unroll
+            for (int c = 0; c < VEC; c++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    const float *const y = x[i] + 8 * c + 4 * j;
+                    plain(L)[(2 * chunk_of(tid + i * kThreads) + j) * ROWS + row_of(tid + i * kThreads) + c] = v4f{y[0], y[1], y[2], y[3]};
+                }
+    }
 };
 
 struct GemmArgs {
@@ -280,28 +293,13 @@ __device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, flo
     if (lane % LANES == 0) out[at] = m, out[at + pitch] = s;
 }
 
-// The sum over k of one element in fp32 operations, for one that the bf16 products left infinite or NaN
-template <bool AKC, bool BKC, int MODE>
-__device__ float plain_sum(const GemmArgs &g, int m, int n, int kb, int ke) {
-    float sum = 0.f;
-#pragma unroll 1
-    for (int k = kb; k < ke && sum == sum; k++) {      // up to the first NaN
-        float a = g.A[AKC ? (int64_t)m * g.lda + k : (int64_t)k * g.lda + m];
-        if constexpr (MODE == kGrad) {
-            const NllToken t = nll_token(g.nll, AKC ? m : k);
-            a = nll_grad(a, t.shift, t.scaled, t.g, t.hit == (AKC ? k : m));
-        }
-        sum = fmaf(a, g.B[BKC ? (int64_t)n * g.ldb + k : (int64_t)k * g.ldb + n], sum);
-    }
-    return sum;
-}
-
 // BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
 template <bool AKC, bool BKC, int BM, int BN, int MODE>
-__global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
+__global__ __launch_bounds__(kThreads, 3) void k_gemm(GemmArgs g) {
     constexpr int WM = BM / 2, WN = BN / 2, MT = WM / 16, NT = WN / 16;
     __shared__ Planes<BM> La;
     __shared__ Planes<BN> Lb;
+    __shared__ int odd_waves[4];
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int wm = (wave % 2) * WM, wn = (wave / 2) * WN;
     // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
@@ -373,6 +371,49 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
         lds_barrier();
     }
 
+    // An element that is not finite (0 times it is NaN): the tile once more from the fp32 operands
+    float odd = 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) odd = fmaf(acc[i][j][r], 0.f, odd);
+    const bool wave_odd = __any(odd != 0.f);
+    if (lane == 0) odd_waves[wave] = wave_odd;
+    __syncthreads();
+    if (odd_waves[0] | odd_waves[1] | odd_waves[2] | odd_waves[3]) {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int k0 = kb; k0 < ke; k0 += kBK) {
+            a.load(Ap, g.lda, ml, tid, k0, ke, g.nll);
+            b.load(Bp, g.ldb, nl, tid, k0, ke, g.nll);
+            a.finish(tid, m0, k0, ke, g.nll);
+            b.finish(tid, n0, k0, ke, g.nll);
+            a.store_plain(La, tid);
+            b.store_plain(Lb, tid);
+            __syncthreads();
+            // lane (lc, lr) holds four consecutive k of row lr; register r of both operands is an instruction's four k
+#pragma unroll 1
+            for (int s = 0; s < kBK / 4; s += 4) {
+                v4f y[NT];
+#pragma unroll
+                for (int j = 0; j < NT; j++) y[j] = b.plain(Lb)[(s + lc) * BN + wn + 16 * j + lr];
+#pragma unroll
+                for (int i = 0; i < MT; i++) {
+                    const v4f x = a.plain(La)[(s + lc) * BM + wm + 16 * i + lr];
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[j][r], acc[i][j], 0, 0, 0);
+                }
+            }
+            __syncthreads();
+        }
+    }
+
     // acc[i][j][r] = C[m0 + wm + 16 i + 4 lc + r][n0 + wn + 16 j + lr]
     if constexpr (!AKC) {
         if (sums) {      // the threads of a row pair's four k-chunks
@@ -412,13 +453,6 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
         for (int q = 0; q < 16 / kRows; q++) {
             const int row = kRows * q + lane / kLanes, m = m0 + wm + 16 * i + row;
             float4 v = *reinterpret_cast<const float4 *>(strip + row * kPitch + c4);
-            if (m < g.M && !(fabsf(v.x) + fabsf(v.y) + fabsf(v.z) + fabsf(v.w) < INFINITY)) {
-                float *const p = strip + row * kPitch + c4;
-#pragma unroll 1
-                for (int e = 0; e < 4; e++)
-                    if (n + e < g.N && !(fabsf(p[e]) < INFINITY)) p[e] = plain_sum<AKC, BKC, MODE>(g, m, n + e, kb, ke);
-                v = *reinterpret_cast<const float4 *>(p);
-            }
             v.x += bias[0], v.y += bias[1], v.z += bias[2], v.w += bias[3];
             if constexpr (MODE == kLse) {
                 lse_of_row<kLanes>(v, n, g.N, lane, sums_of, (wave / 2) * BM + wm + 16 * i + row, 2 * BM);
