@@ -98,7 +98,7 @@ class DeltaNetLM(nn.Module):
         """One token per sequence through all layers in one call, where nothing is recorded: ``(hidden, states)`` or ``None``."""
         if x.shape[0] != 1 or not 1 <= x.shape[1] <= 64 or torch.is_grad_enabled() or len(self.layers) == 0:
             return None
-        if mems is not None and len(mems) < len(self.layers):
+        if mems is not None and (len(mems) < len(self.layers) or any(m is None for m in mems)):
             return None
         att = self.layers[0].dec_attn
         if not isinstance(att, DeltaNetLayer) or att.d_head not in (16, 32, 64) or self.d_model % 64 or self.d_model > 1024:

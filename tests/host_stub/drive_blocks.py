@@ -194,6 +194,34 @@ def misfitting_modules(m):
     assert calls == [] and y.shape == (5, 2, 0)
 
 
+def language_model(pkg, rec, **more):
+    """A small model that decodes on the host build: its input, and the first state of every layer."""
+    pkg.lm.DeltaNetLM._embed = lambda self, data: self.word_emb(data).detach() if not torch.is_grad_enabled() else None
+    lm = pkg.DeltaNetLM(**{**dict(n_token=50, n_layer=3, n_head=4, d_model=64, d_head=16, d_inner=64), **more})
+    toks = torch.randint(0, 50, (1, 3))
+    with torch.no_grad():
+        calls, (hid, mems) = rec.of(lambda: lm.hidden(toks, None, carry_over_fast_weight=True))
+    assert calls == ["decode_layers"] and len(mems) == 3
+    return lm, toks, mems
+
+
+def decode(rec, lm, toks, mems):
+    with torch.no_grad():
+        calls, res = rec.of(lambda: lm.hidden(toks, mems, carry_over_fast_weight=True))
+    if isinstance(res, Exception):
+        raise res
+    return calls, res
+
+
+def states_left_out(m):
+    """None in the place of a layer's state is no state, as for the layers one by one."""
+    pkg, rec = package(m)
+    lm, toks, mems = language_model(pkg, rec)
+    for given in ([None] * 3, [mems[0], None, mems[2]]):
+        calls, (hid, new) = decode(rec, lm, toks, given)
+        assert "decode_layers" not in calls and calls.count("delta_block") == 3 and len(new) == 3
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
