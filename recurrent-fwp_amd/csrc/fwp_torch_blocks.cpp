@@ -428,8 +428,9 @@ struct NllFn : torch::autograd::Function<NllFn> {
 constexpr size_t kPerLayer = 10;
 
 // One token per sequence through the layers: x [1,B,d], states [B,H,D,D] per layer (empty: zeros) ->
-// (hidden [1,B,d], the states after the token).  Nothing is recorded.
-std::tuple<at::Tensor, std::vector<at::Tensor>> decode_layers(const at::Tensor &x_in, const std::vector<at::Tensor> &params,
+// (hidden [1,B,d], the states after the token), or nothing for parameters that fwp_rows_matmul does not take (the layers
+// one by one do).  Nothing is recorded.
+std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(const at::Tensor &x_in, const std::vector<at::Tensor> &params,
                                                               const std::vector<at::Tensor> &states, int64_t H, int64_t D,
                                                               double eps, bool pre_norm) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -445,16 +446,15 @@ std::tuple<at::Tensor, std::vector<at::Tensor>> decode_layers(const at::Tensor &
     int64_t inner_most = 0;
     for (size_t l = 0; l < layers; l++) {
         const at::Tensor *p = &params[kPerLayer * l];
-        const int64_t inner = p[4].size(0);
-        bool ok = same_shape(p[0], {width, d}) && same_shape(p[1], {d, H * D}) && same_shape(p[4], {inner, d}) &&
+        const int64_t inner = p[4].dim() == 2 ? p[4].size(0) : 0;
+        bool ok = inner > 0 && inner % 64 == 0 && same_shape(p[0], {width, d}) && same_shape(p[1], {d, H * D}) && same_shape(p[4], {inner, d}) &&
                   same_shape(p[5], {inner}) && same_shape(p[6], {d, inner});
         for (size_t i : {2, 3, 7, 8, 9}) ok = ok && same_shape(p[i], {d});
         for (size_t i = 0; i < kPerLayer; i++) {
-            same_device(x, {p[i]});
-            ok = ok && p[i].scalar_type() == at::kFloat && p[i].is_contiguous() &&
+            ok = ok && p[i].device() == x.device() && p[i].scalar_type() == at::kFloat && p[i].is_contiguous() &&
                  reinterpret_cast<uintptr_t>(p[i].data_ptr()) % 16 == 0;
         }
-        if (!ok) fail("parameters must be contiguous fp32 tensors of the model's sizes");
+        if (!ok) return std::nullopt;
         inner_most = std::max(inner_most, inner);
     }
     // one buffer for everything in between; the states in another (the caller keeps them)
@@ -496,7 +496,7 @@ std::tuple<at::Tensor, std::vector<at::Tensor>> decode_layers(const at::Tensor &
         const at::Tensor *p = &params[kPerLayer * (layers - 1)];
         check(fwp_layer_norm_fwd(in, ptr(p[8]), ptr(p[9]), ptr(result), nullptr, (int)B, (int)d, (float)eps, s), "fwp_layer_norm_fwd");
     }
-    return {result, after.unbind(0)};
+    return std::make_tuple(result, after.unbind(0));
 }
 
 // word embedding times scale plus the positions' sinusoids, for ids [T,B]; nothing is recorded

@@ -55,24 +55,30 @@ class Linear(nn.Linear):
         return super().forward(x)
 
 
+def _own(m, name):
+    """A parameter of a module, or the plain tensor in its place (a replica's, a flattened parameter's), or ``None``."""
+    p = m._parameters.get(name)
+    return p if p is not None else m.__dict__.get(name)
+
+
 def decode_parameters(layer):
     """The parameters of a :class:`DeltaNetDecoderLayer` as ``decode_layers`` takes them, or ``None`` when the layer
     is not what that function computes: a replaced or hooked sub-module, an active dropout, another operator."""
     if not (_untouched(layer, DeltaNetDecoderLayer)):
         return None
-    att, ff = layer._modules["dec_attn"], layer._modules["pos_ff"]
+    att, ff = layer._modules.get("dec_attn"), layer._modules.get("pos_ff")
     if not (_untouched(att, DeltaNetLayer) and _untouched(ff, PositionwiseFF)) or att.fast_weight_op is not fast_weight_delta:
         return None
     a, f = att._modules, ff._modules
-    net = f["CoreNet"]
+    net = f.get("CoreNet")
     if not (_untouched(net, nn.Sequential) and len(net._modules) == 5):
         return None
     lin1, relu, drop1, lin2, drop2 = net._modules.values()
-    norms = (a["layer_norm"], f["layer_norm"])
-    for m in (a["qkvb_net"], a["o_net"], lin1, lin2):
+    norms, projections = (a.get("layer_norm"), f.get("layer_norm")), (a.get("qkvb_net"), a.get("o_net"))
+    for m in (*projections, lin1, lin2):
         if not _untouched(m, nn.Linear):
             return None
-    for m in (a["drop"], drop1, drop2):
+    for m in (a.get("drop"), drop1, drop2):
         if not _untouched(m, nn.Dropout) or _drops(m):
             return None
     for m in norms:
@@ -80,11 +86,11 @@ def decode_parameters(layer):
             return None
     if not _untouched(relu, nn.ReLU) or att.pre_lnorm != ff.pre_lnorm:
         return None
-    if a["qkvb_net"]._parameters["bias"] is not None or a["o_net"]._parameters["bias"] is not None:
+    if any(_own(m, "bias") is not None for m in projections):
         return None
-    params = [a["qkvb_net"]._parameters["weight"], a["o_net"]._parameters["weight"]]
+    params = [_own(m, "weight") for m in projections]
     for m in (norms[0], lin1, lin2, norms[1]):
-        params += [m._parameters["weight"], m._parameters["bias"]]
+        params += [_own(m, "weight"), _own(m, "bias")]
     return None if any(p is None for p in params) else params
 
 

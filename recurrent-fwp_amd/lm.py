@@ -100,7 +100,7 @@ class DeltaNetLM(nn.Module):
             return None
         if mems is not None and (len(mems) < len(self.layers) or any(m is None for m in mems)):
             return None
-        att = self.layers[0].dec_attn
+        att = self.layers[0]._modules.get("dec_attn")
         if not isinstance(att, DeltaNetLayer) or att.d_head not in (16, 32, 64) or self.d_model % 64 or self.d_model > 1024:
             return None
         params = []
@@ -108,7 +108,7 @@ class DeltaNetLM(nn.Module):
             p = decode_parameters(layer)
             a = layer._modules.get("dec_attn")
             if (p is None or a.n_head != att.n_head or a.d_head != att.d_head or a.pre_lnorm != att.pre_lnorm
-                    or a.layer_norm.eps != att.layer_norm.eps or p[4].shape[0] % 64):
+                    or a.layer_norm.eps != att.layer_norm.eps):
                 return None
             params += p
         if (att.n_head * att.d_head) % 64:

@@ -222,6 +222,37 @@ def states_left_out(m):
         assert "decode_layers" not in calls and calls.count("delta_block") == 3 and len(new) == 3
 
 
+def unusual_parameters(m):
+    """Weights that are plain attributes (replicas, flattened parameters) or off a 16-byte boundary, modules left out."""
+    pkg, rec = package(m)
+    nn = torch.nn
+    lm, toks, mems = language_model(pkg, rec)
+    want = decode(rec, lm, toks, mems)[1][0]
+    for lin in (lm.layers[1].dec_attn.qkvb_net, lm.layers[1].pos_ff.CoreNet[0], lm.layers[2].pos_ff.layer_norm):
+        w = lin.weight.detach().clone()
+        del lin.weight
+        lin.weight = w
+        calls, (hid, _) = decode(rec, lm, toks, mems)
+        assert calls == ["decode_layers"] and torch.equal(hid, want)
+    lin = lm.layers[1].pos_ff.CoreNet[3]
+    lin.weight = nn.Parameter(unaligned(lin.weight))
+    calls, _ = decode(rec, lm, toks, mems)
+    assert calls.count("delta_block") == 3 and calls.count("feed_forward") == 3, calls
+    lin.weight = nn.Parameter(lin.weight.detach().clone())
+    assert decode(rec, lm, toks, mems)[0] == ["decode_layers"]
+    lm.layers[1].pos_ff.CoreNet[0].bias = None
+    calls, _ = decode(rec, lm, toks, mems)
+    assert "decode_layers" not in calls and calls.count("delta_block") == 3
+
+    class Other(nn.Module):             # a layer of another kind, first
+        def forward(self, x, mems=None, carry_over_fast_weight=False):
+            return x, mems
+    lm, toks, mems = language_model(pkg, rec)
+    lm.layers[0] = Other()
+    calls, _ = decode(rec, lm, toks, mems)
+    assert "decode_layers" not in calls and calls.count("delta_block") == 2
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
