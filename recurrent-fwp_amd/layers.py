@@ -17,8 +17,9 @@ from .fast_weight import _fwp_torch, fast_weight_delta
 
 
 def _untouched(m, cls):
-    """Is this sub-module exactly a ``cls`` (not a replacement) that nothing is hooked to?"""
-    return type(m) is cls and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+    """Is this sub-module exactly a ``cls`` (not a replacement) with its class's ``forward``, that nothing is hooked to?"""
+    return type(m) is cls and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                                   or "forward" in m.__dict__)
 
 
 def _blocks(x, *params):

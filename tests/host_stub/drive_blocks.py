@@ -153,11 +153,13 @@ class Recorded:
 
 
 def package(m):
-    """The package with its layers on the host build's blocks: host tensors count as the GPU's."""
+    """The package with its layers on the host build's blocks: host tensors count as the GPU's, and the operator that
+    stands in for fast_weight_delta in a layer's general path returns its values."""
     sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
     pkg = importlib.import_module("recurrent-fwp_amd")
     layers, lm, rec = pkg.layers, pkg.lm, Recorded(m)
     layers._fwp_torch = rec
+    layers.fast_weight_delta = lambda q, k, v, beta, W, *more: v
     exec(inspect.getsource(layers._blocks).replace("x.is_cuda", "True").replace("t.is_cuda", "True"), layers.__dict__)
     lm._blocks = layers._blocks
     return pkg, rec
@@ -251,6 +253,37 @@ def unusual_parameters(m):
     lm.layers[0] = Other()
     calls, _ = decode(rec, lm, toks, mems)
     assert "decode_layers" not in calls and calls.count("delta_block") == 2
+
+
+def wrapped_modules(m):
+    """A sub-module whose forward was replaced on the instance (adapters, instrumentation) is called."""
+    pkg, rec = package(m)
+
+    def wrap(mod):
+        inner, seen = mod.forward, []
+
+        def forward(*args, **kwargs):
+            seen.append(1)
+            return inner(*args, **kwargs)
+        mod.forward = forward
+        return seen
+
+    x = rnd(5, 2, 24)
+    for pick in (lambda f: f.CoreNet, lambda f: f.CoreNet[0], lambda f: f.CoreNet[1], lambda f: f.CoreNet[4], lambda f: f.layer_norm):
+        ff = pkg.PositionwiseFF(24, 40, 0.0)
+        seen = wrap(pick(ff))
+        ff(x)
+        assert seen == [1]
+    crit = pkg.lm._TiedSoftmaxLoss(30, 24)
+    seen = wrap(crit.out_layers[0])
+    crit(rnd(6, 24), torch.zeros(6, dtype=torch.int64))
+    assert seen == [1]
+    for pick in (lambda l: l, lambda l: l.dec_attn, lambda l: l.pos_ff, lambda l: l.pos_ff.CoreNet[3], lambda l: l.pos_ff.layer_norm,
+                 lambda l: l.dec_attn.drop, lambda l: l.dec_attn.layer_norm):
+        lm, toks, mems = language_model(pkg, rec)
+        seen = wrap(pick(lm.layers[1]))
+        decode(rec, lm, toks, mems)
+        assert seen == [1], pick
 
 
 def main():
