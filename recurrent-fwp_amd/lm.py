@@ -128,11 +128,11 @@ class DeltaNetLM(nn.Module):
             if self.clamp_len > 0:
                 pos_seq.clamp_(max=self.clamp_len)
             emb = emb + self.pos_emb(pos_seq)
-        elif not _drops(self.drop) and (carry_over_fast_weight or mems is None):
+        elif _untouched(self.drop, nn.Dropout) and not _drops(self.drop) and (carry_over_fast_weight or mems is None):
             done = self._decode(emb, mems)
             if done is not None:
                 hid, states = done
-                return self.drop(hid), ([(W, None) for W in states] if carry_over_fast_weight else None)
+                return hid, ([(W, None) for W in states] if carry_over_fast_weight else None)
         return self._through_layers(self.drop(emb), mems, carry_over_fast_weight)
 
     def _through_layers(self, out, mems, carry_over_fast_weight):

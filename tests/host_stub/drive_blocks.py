@@ -286,6 +286,31 @@ def wrapped_modules(m):
         assert seen == [1], pick
 
 
+def replaced_dropouts(m):
+    """The model's dropout replaced or hooked: it runs on the embedding and on the last hidden state, in both modes."""
+    pkg, rec = package(m)
+    nn = torch.nn
+
+    class Half(nn.Module):
+        def forward(self, x):
+            return 0.5 * x
+    for training in (True, False):
+        lm, toks, mems = language_model(pkg, rec)
+        lm.train(training)
+        lm.drop = nn.Identity()
+        decode(rec, lm, toks, mems)
+        seen = []
+        lm.drop = nn.Dropout(0.0)
+        lm.drop.register_forward_hook(lambda *a: seen.append(1))
+        decode(rec, lm, toks, mems)
+        assert seen == [1, 1]
+        lm.drop = Half()
+        calls, (hid, _) = decode(rec, lm, toks, mems)
+        with torch.no_grad():
+            want = lm._through_layers(0.5 * lm._embed(toks), mems, True)[0]
+        assert "decode_layers" not in calls and torch.equal(hid, want)
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
