@@ -8,7 +8,6 @@
 // operators and differentiates that.
 #include "fwp_torch.hpp"
 
-#include <cmath>
 #include <optional>
 #include <tuple>
 #include <vector>
@@ -432,7 +431,7 @@ constexpr size_t kPerLayer = 10;
 // one by one do).  Nothing is recorded.
 std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(const at::Tensor &x_in, const std::vector<at::Tensor> &params,
                                                               const std::vector<at::Tensor> &states, int64_t H, int64_t D,
-                                                              double eps, bool pre_norm) {
+                                                              double eps, bool pre_norm, double scale) {
     at::AutoDispatchBelowADInplaceOrView below;
     require_device(x_in);
     const size_t layers = params.size() / kPerLayer;
@@ -482,7 +481,7 @@ std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(con
         // post-norm: LN of the previous layer's sum on the way in, that is also the residual; pre-norm: this layer's
         product(in, before, before ? before + 1 : nullptr, before ? y : nullptr, p[0], nullptr, none, 0, qkvb);
         check(fwp_deltanet_step(qkvb, ptr(from), ptr(after) + l * B * H * D * D, out, (int)B, (int)H, (int)D,
-                                (float)(1.0 / std::sqrt((double)D)), s),
+                                (float)scale, s),
               "fwp_deltanet_step");
         product(out, nullptr, nullptr, nullptr, p[1], nullptr, before ? y : in, 0, a);
         // feed-forward: post-norm adds the normalised rows back, pre-norm the rows themselves

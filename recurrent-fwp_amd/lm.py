@@ -103,12 +103,15 @@ class DeltaNetLM(nn.Module):
         att = self.layers[0]._modules.get("dec_attn")
         if not isinstance(att, DeltaNetLayer) or att.d_head not in (16, 32, 64) or self.d_model % 64 or self.d_model > 1024:
             return None
+        if type(att.scale) is not float:
+            return None
         params = []
         for layer in self.layers:
             p = decode_parameters(layer)
             a = layer._modules.get("dec_attn")
             if (p is None or a.n_head != att.n_head or a.d_head != att.d_head or a.pre_lnorm != att.pre_lnorm
-                    or a.layer_norm.eps != att.layer_norm.eps):
+                    or a.layer_norm.eps != att.layer_norm.eps
+                    or type(a.scale) is not float or a.scale != att.scale):
                 return None
             params += p
         if (att.n_head * att.d_head) % 64:
@@ -117,7 +120,8 @@ class DeltaNetLM(nn.Module):
         if blocks is None:
             return None
         states = [] if mems is None else [m[0][:x.shape[1]] for m in mems[:len(self.layers)]]
-        return blocks.decode_layers(x, params, states, att.n_head, att.d_head, att.layer_norm.eps, att.pre_lnorm)
+        return blocks.decode_layers(x, params, states, att.n_head, att.d_head, att.layer_norm.eps, att.pre_lnorm,
+                                    att.scale)
 
     def hidden(self, data, mems=None, carry_over_fast_weight=False):
         emb = self._embed(data)

@@ -311,6 +311,20 @@ def replaced_dropouts(m):
         assert "decode_layers" not in calls and torch.equal(hid, want)
 
 
+def own_scales(m):
+    """A layer's read-out scale is its attribute, when all layers decode in one call too."""
+    pkg, rec = package(m)
+    lm, toks, mems = language_model(pkg, rec)
+    hidden = decode(rec, lm, toks, mems)[1][0]
+    for layer in lm.layers:
+        layer.dec_attn.scale = 0.5
+    calls, (hid, _) = decode(rec, lm, toks, mems)
+    assert calls == ["decode_layers"] and not torch.equal(hid, hidden)
+    for other in (0.125, torch.tensor(0.5)):
+        lm.layers[1].dec_attn.scale = other
+        assert decode(rec, lm, toks, mems)[0].count("delta_block") == 3
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
