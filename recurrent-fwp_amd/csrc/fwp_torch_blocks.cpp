@@ -10,6 +10,7 @@
 
 #include <optional>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 namespace {
@@ -456,12 +457,13 @@ std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(con
         if (!ok) return std::nullopt;
         inner_most = std::max(inner_most, inner);
     }
-    // one buffer for everything in between; the states in another (the caller keeps them)
+    // one buffer for everything in between; the states, which the caller keeps or drops one by one, on their own
     const int64_t rows_d = (B * d + 3) & ~int64_t(3);
     const at::Tensor work = at::empty({B * width + 4 + B * H * D + 4 * rows_d + B * inner_most}, opts);
     float *const a = ptr(work), *const b = a + rows_d, *const y = b + rows_d, *const h2 = y + rows_d, *const out = h2 + rows_d,
                 *const hid = out + B * H * D, *const qkvb = hid + B * inner_most;
-    const at::Tensor result = at::empty({1, B, d}, opts), after = at::empty({(int64_t)layers, B, H, D, D}, opts);
+    const at::Tensor result = at::empty({1, B, d}, opts);
+    std::vector<at::Tensor> after(layers);
     const float *const none = nullptr;
     const auto product = [&](const float *in, const at::Tensor *g, const at::Tensor *be, float *norm, const at::Tensor &W,
                              const at::Tensor *bias, const float *residual, int relu, float *to) {
@@ -478,9 +480,10 @@ std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(con
             same_device(x, {from});
             require(same_shape(from, {B, H, D, D}), "a state does not fit [bsz, n_head, d_head, d_head]");
         }
+        after[l] = at::empty({B, H, D, D}, opts);
         // post-norm: LN of the previous layer's sum on the way in, that is also the residual; pre-norm: this layer's
         product(in, before, before ? before + 1 : nullptr, before ? y : nullptr, p[0], nullptr, none, 0, qkvb);
-        check(fwp_deltanet_step(qkvb, ptr(from), ptr(after) + l * B * H * D * D, out, (int)B, (int)H, (int)D,
+        check(fwp_deltanet_step(qkvb, ptr(from), ptr(after[l]), out, (int)B, (int)H, (int)D,
                                 (float)scale, s),
               "fwp_deltanet_step");
         product(out, nullptr, nullptr, nullptr, p[1], nullptr, before ? y : in, 0, a);
@@ -495,7 +498,7 @@ std::optional<std::tuple<at::Tensor, std::vector<at::Tensor>>> decode_layers(con
         const at::Tensor *p = &params[kPerLayer * (layers - 1)];
         check(fwp_layer_norm_fwd(in, ptr(p[8]), ptr(p[9]), ptr(result), nullptr, (int)B, (int)d, (float)eps, s), "fwp_layer_norm_fwd");
     }
-    return std::make_tuple(result, after.unbind(0));
+    return std::make_tuple(result, std::move(after));
 }
 
 // word embedding times scale plus the positions' sinusoids, for ids [T,B]; nothing is recorded

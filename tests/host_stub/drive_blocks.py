@@ -325,6 +325,14 @@ def own_scales(m):
         assert decode(rec, lm, toks, mems)[0].count("delta_block") == 3
 
 
+def states_of_their_own(m):
+    """A layer's carried state has its own memory: keeping one keeps no other."""
+    pkg, rec = package(m)
+    lm, toks, mems = language_model(pkg, rec)
+    for W, _ in mems:
+        assert W.untyped_storage().nbytes() == W.numel() * 4 and W.is_contiguous()
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
