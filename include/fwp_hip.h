@@ -293,7 +293,8 @@ int fwp_matmul(int layout, const float *A, long long lda, const float *B, long l
 
 /*
  * Per-row negative log-likelihood under softmax(x W^T + bias) (language_modeling/src/model_main.py:1333-1361 without
- * clusters): x [rows,dim], W [vocab,dim], bias [vocab], target [rows] (negative: the row is ignored), loss [rows].
+ * clusters): x [rows,dim], W [vocab,dim], bias [vocab], target [rows] (-100: the row is ignored; another
+ * number that is no word: NaN, in the gradients too), loss [rows].
  * Saved for backward, both or none: logits [rows,vocab], lse [rows].  workspace: fwp_nll_workspace(rows, vocab) floats.
  */
 long long fwp_nll_workspace(int rows, int vocab);

@@ -437,13 +437,13 @@ static int nll_bwd(const float *x, const float *W, const float *logits, const Nl
 int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
                 const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
                 void *stream) {
-    return nll_bwd(x, W, logits, {lse, nullptr, gloss, target}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
+    return nll_bwd(x, W, logits, {lse, nullptr, gloss, target, vocab}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
 }
 
 int fwp_nll_stats_bwd(const float *x, const float *W, const float *logits, const float *stats, const int64_t *target,
                       const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows, int vocab, int dim,
                       void *stream) {
-    return nll_bwd(x, W, logits, {nullptr, stats, gloss, target}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
+    return nll_bwd(x, W, logits, {nullptr, stats, gloss, target, vocab}, gx, gW, gbias, workspace, rows, vocab, dim, (hipStream_t)stream);
 }
 
 int fwp_layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows,

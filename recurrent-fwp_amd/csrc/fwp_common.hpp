@@ -194,6 +194,7 @@ int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const
 struct NllView {
     const float *lse, *stats, *gloss;      // lse [rows] or stats [rows,2], whichever nll_fwd wrote
     const int64_t *target;
+    int vocab;
 };
 int64_t matmul_workspace(int M, int N, int K);
 int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,

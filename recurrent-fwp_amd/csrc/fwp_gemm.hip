@@ -80,13 +80,17 @@ __device__ __forceinline__ float exp_of(float x) {
 }
 
 // What turns stored logits into the gradient of the loss as an operand is loaded:
-// (exp(logit - shift) * scale - [vocabulary entry == target]) * gloss of the token, 0 for a negative target.
+// (exp(logit - shift) * scale - [vocabulary entry == target]) * gloss of the token, 0 for an ignored target, NaN for one that
+// is no word.
 // shift and scale: the largest logit and 1 / the sum of exp(logit - largest) (`stats`, exact where a token's probability
 // is near 1 and its logit large), or the log-sum-exp and 1 (`lse`).
 struct NllArgs {
     const float *lse, *stats, *gloss;
     const int64_t *target;
+    int vocab;
 };
+
+constexpr int64_t kIgnored = -100;      // torch.nn.functional.cross_entropy's ignore_index
 
 struct NllToken {
     float shift, scaled, g;      // scaled: scale * gloss
@@ -95,8 +99,9 @@ struct NllToken {
 
 __device__ __forceinline__ NllToken nll_token(const NllArgs &a, int token) {
     NllToken t;
-    t.hit = (int)a.target[token];
-    t.g = t.hit >= 0 ? a.gloss[token] : 0.f;
+    const int64_t want = a.target[token];
+    t.hit = (int)want;
+    t.g = want == kIgnored ? 0.f : want >= 0 && want < a.vocab ? a.gloss[token] : NAN;
     const float2 s = a.stats ? reinterpret_cast<const float2 *>(a.stats)[token] : make_float2(a.lse[token], 1.f);
     t.shift = s.x;
     t.scaled = s.y * t.g;
@@ -597,7 +602,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
            int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s) {
     GemmArgs g{};
     g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
-    if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target};
+    if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target, nll->vocab};
     const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace));
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
     const bool cut = p.ranges > 1;
@@ -621,8 +626,8 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
 
 namespace {
 
-// loss = (largest logit - logit of the target) + log(sum of exp(logit - largest)) (0 for a negative target), from the
-// tiles' maxima and sums; four threads share a row, a quarter of the tiles each.  The difference comes first: added to
+// loss = (largest logit - logit of the target) + log(sum of exp(logit - largest)) (0 for an ignored target, NaN for one
+// that is no word), from the tiles' maxima and sums; four threads share a row, a quarter of the tiles each.  The difference comes first: added to
 // the logarithm first, a large logit would round it off (a loss of 1e-3 at a logit of 20 by half a percent).
 __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part_max, const float *__restrict__ part_sum,
                                                   const float *__restrict__ hit, const float *__restrict__ logits,
@@ -651,7 +656,7 @@ __global__ __launch_bounds__(kThreads) void k_nll(const float *__restrict__ part
     if (lse) lse[m] = mx + l;
     if (stats) *reinterpret_cast<float2 *>(stats + 2 * (int64_t)m) = make_float2(mx, 1.f / s);
     // a row of -infinities alone: NaN
-    loss[m] = want < 0 ? 0.f : want < vocab ? (mx - (logits ? logits[(int64_t)m * vocab + want] : hit[m])) + l : NAN;
+    loss[m] = want == kIgnored ? 0.f : want >= 0 && want < vocab ? (mx - (logits ? logits[(int64_t)m * vocab + want] : hit[m])) + l : NAN;
 }
 
 }  // namespace

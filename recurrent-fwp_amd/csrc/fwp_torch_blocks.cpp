@@ -570,6 +570,6 @@ void bind_blocks(py::module_ &m) {
     m.def("decode_layers", &decode_layers, "one token per sequence through the layers -> (hidden, states); records nothing");
     m.def("embed", &embed, "the model's input from token ids; records nothing");
     m.def("layer_norm", &layer_norm, "LayerNorm over the last axis (a multiple of 4 up to 1024)");
-    m.def("nll", &nll, "per-row negative log-likelihood of the targets under softmax(x W^T + bias); a negative target counts 0");
+    m.def("nll", &nll, "per-row negative log-likelihood of the targets under softmax(x W^T + bias); a target of -100 counts 0");
     m.def("delta_block", &delta_block, "the Delta-Net layer between its input and its LayerNorm; the state is updated in place");
 }

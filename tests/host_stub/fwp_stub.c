@@ -378,7 +378,7 @@ static int nll_fwd(const float *x, const float *W, const float *bias, const int6
         if (logits) memcpy(logits + r * vocab, row, sizeof(float) * vocab);
         if (lse) lse[r] = (float)(mx + log(s));
         if (stats) stats[2 * r] = (float)mx, stats[2 * r + 1] = (float)(1 / s);
-        loss[r] = target[r] < 0 ? 0 : (float)(mx - row[target[r]] + log(s));
+        loss[r] = target[r] == -100 ? 0 : target[r] < 0 || target[r] >= vocab ? NAN : (float)(mx - row[target[r]] + log(s));
     }
     free(row);
     return 0;
@@ -399,7 +399,7 @@ int fwp_nll_stats_bwd(const float *x, const float *W, const float *logits, const
     float *d = malloc(sizeof(float) * rows * vocab);
     for (long long r = 0; r < rows; r++)
         for (long long v = 0; v < vocab; v++)
-            d[r * vocab + v] = target[r] < 0 ? 0 : (float)((exp(logits[r * vocab + v] - stats[2 * r]) * stats[2 * r + 1] -
+            d[r * vocab + v] = target[r] == -100 ? 0 : target[r] < 0 || target[r] >= vocab ? NAN : (float)((exp(logits[r * vocab + v] - stats[2 * r]) * stats[2 * r + 1] -
                                                             (v == target[r])) * gloss[r]);
     const fwp_mm_epilogue epi = {NULL, NULL, NULL, gbias, 0};
     if (gx) fwp_matmul(FWP_MM_NN, d, vocab, W, dim, gx, dim, rows, dim, vocab, NULL, workspace, stream);

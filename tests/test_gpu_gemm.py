@@ -115,7 +115,7 @@ def loss_and_gradients(L, x, W, b, target, gloss):
                                      dim, L.stream_of(x)) == 0
     only = torch.empty_like(loss)
     assert L.lib().fwp_nll_fwd(*ptrs, None, only.data_ptr(), None, work.data_ptr(), rows, vocab, dim, L.stream_of(x)) == 0
-    assert torch.equal(only, loss)
+    assert torch.equal(only.nan_to_num(-1.0), loss.nan_to_num(-1.0))
     gx, gW, gb = torch.full_like(x, float("nan")), torch.full_like(W, float("nan")), torch.full_like(b, float("nan"))
     n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
     work = torch.empty(max(1, n), device="cuda")
@@ -228,6 +228,21 @@ def test_ragged_results_spread_and_unaligned_operands(fwp, layout, M, N, K, cut)
             assert bool(((colsum.double() - a.sum(1)).abs() <= K * EPS * a.abs().sum(1)).all())
         got = matmul(fwp._lib, layout, x, y, bias=bias, relu=1, residual=residual, gate=gate)
         assert bool(((got.double() - want).abs() <= bound(K, mag + 400)).all())
+
+
+@pytest.mark.parametrize("rows", [40, 2100])
+@pytest.mark.parametrize("odd", [-1, -99, -101, 300, 2 ** 32 + 5, -2 ** 40])
+def test_a_target_that_is_no_word(fwp, odd, rows):
+    """-100 is ignored; any other number outside the vocabulary shows as NaN in its loss and in the gradients."""
+    x, W, b = randn(rows, 64, seed=1), randn(300, 64, seed=2) * 0.1, randn(300, seed=3)
+    target = torch.randint(0, 300, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
+    target[3] = -100
+    check_loss(fwp._lib, x, W, b, target)
+    target[7] = odd
+    loss, gx, gW, gb = loss_and_gradients(fwp._lib, x, W, b, target, randn(rows, seed=5))
+    assert torch.nonzero(loss.isnan()).flatten().tolist() == [7] and float(loss[3]) == 0
+    assert torch.nonzero(gx.isnan().any(1)).flatten().tolist() == [7]
+    assert bool(gW.isnan().all()) and bool(gb.isnan().all())
 
 
 @pytest.mark.parametrize("M,N,K", [(70, 66, 200), (300, 260, 1100), (40, 64, 2048), (2100, 2100, 40)])
