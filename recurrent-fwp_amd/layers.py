@@ -30,7 +30,8 @@ def _blocks(x, *params):
     for t in (x, *params):
         if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter) or t.numel() == 0:
             return None
-    if not all(p.is_contiguous() for p in params):
+    # the kernels' offsets reach rows of 2^21 floats, their launches 2^24 rows
+    if x.dim() == 0 or x.numel() > x.shape[-1] << 24 or not all(p.is_contiguous() and max(p.shape, default=0) <= 1 << 21 for p in params):
         return None
     if (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing()
             or torch.nn.modules.module._has_any_global_hook() or torch.autograd.forward_ad._current_level >= 0

@@ -89,7 +89,8 @@ class DeltaNetLM(nn.Module):
         if not (_untouched(word, _WordEmbedding) and _untouched(word.emb_layers[0], nn.Embedding) and _untouched(pos, PositionalEmbedding)):
             return None
         table = word.emb_layers[0]
-        if table.max_norm is not None or data.numel() == 0 or pos.inv_freq.dtype is not torch.float32:
+        if (table.max_norm is not None or data.numel() == 0 or pos.inv_freq.dtype is not torch.float32
+                or data.numel() * table.weight.shape[-1] >= 1 << 32):      # a thread per number
             return None
         blocks = _blocks(table.weight, table.weight)
         return None if blocks is None else blocks.embed(table.weight, data, pos.inv_freq, word.emb_scale, self.clamp_len)

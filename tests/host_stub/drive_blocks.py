@@ -333,6 +333,23 @@ def states_of_their_own(m):
         assert W.untyped_storage().nbytes() == W.numel() * 4 and W.is_contiguous()
 
 
+def beyond_the_kernels(m):
+    """Matrices wider than the kernels' offsets reach (2^21) and inputs of more rows than a launch takes go to PyTorch."""
+    pkg, rec = package(m)
+    crit, wide = pkg.lm._TiedSoftmaxLoss(5, 2), 2 ** 21 + 1
+    crit.out_layers[0] = pkg.layers.Linear(2, wide)
+    with torch.no_grad():
+        calls, loss = rec.of(crit, rnd(3, 2), torch.zeros(3, dtype=torch.int64))
+        assert calls == [] and loss.shape == (3,)
+        calls, y = rec.of(pkg.layers.Linear(wide, 2), rnd(1, wide))
+        assert calls == [] and y.shape == (1, 2)
+        ff = pkg.PositionwiseFF(2, wide, 0.0)
+        calls, y = rec.of(ff, rnd(1, 2))
+        assert calls == [] and y.shape == (1, 2)
+    x = torch.empty(1, 1).expand(2 ** 24 + 1, 4)           # no memory behind it
+    assert pkg.layers._blocks(x, rnd(4, 4)) is None and pkg.layers._blocks(x[:2 ** 24], rnd(4, 4)) is not None
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
