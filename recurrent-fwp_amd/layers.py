@@ -11,6 +11,7 @@ the stock-PyTorch form.
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from . import _lib
 from .fast_weight import _fwp_torch, fast_weight_delta
@@ -22,10 +23,22 @@ def _untouched(m, cls):
                                    or "forward" in m.__dict__)
 
 
+def _eager(x):
+    """Is ``x`` an ordinary tensor of an ordinary call, not a stand-in for one or a traced one?"""
+    return type(x) in (torch.Tensor, nn.Parameter) and not (torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
+def _watched():
+    """Does a mode see the operators that are called?  (A default device is such a mode, but changes none of them.)"""
+    if torch._C._len_torch_dispatch_stack():
+        return True
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
+
+
 def _blocks(x, *params):
     """The C++ blocks (csrc/fwp_torch_blocks.cpp) if they apply to this input and these parameters: fp32 on the
-    GPU, outside autocast, tracing and functional transforms."""
-    if _fwp_torch is None or not x.is_cuda:
+    GPU, outside autocast, tracing, modes and functional transforms."""
+    if _fwp_torch is None or not _eager(x) or not x.is_cuda:
         return None
     for t in (x, *params):
         if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter) or t.numel() == 0:
@@ -33,9 +46,8 @@ def _blocks(x, *params):
     # the kernels' offsets reach rows of 2^21 floats, their launches 2^24 rows
     if x.dim() == 0 or x.numel() > x.shape[-1] << 24 or not all(p.is_contiguous() and max(p.shape, default=0) <= 1 << 21 for p in params):
         return None
-    if (torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing()
-            or torch.nn.modules.module._has_any_global_hook() or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None):
+    if (torch.is_autocast_enabled() or _watched() or torch.nn.modules.module._has_any_global_hook()
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None):
         return None
     return _fwp_torch
 
@@ -49,12 +61,18 @@ class Linear(nn.Linear):
     """``nn.Linear`` on the package's matrix products where they apply."""
 
     def forward(self, x):
-        if (self.bias is not None and x.dim() > 0 and self.weight.shape[1:] == x.shape[-1:]
+        if torch.jit.is_scripting():
+            return F.linear(x, self.weight, self.bias)
+        else:
+            return self._forward(x)
+
+    def _forward(self, x):
+        if (_eager(x) and self.bias is not None and x.dim() > 0 and self.weight.shape[1:] == x.shape[-1:]
                 and self.bias.shape == self.weight.shape[:1]):
             blocks = _blocks(x, self.weight, self.bias)
             if blocks is not None:
                 return blocks.linear(x, self.weight, self.bias)
-        return super().forward(x)
+        return F.linear(x, self.weight, self.bias)
 
 
 def _own(m, name):
@@ -98,7 +116,7 @@ def decode_parameters(layer):
 
 def _layer_norm(m, x):
     """``m(x)`` for a LayerNorm over the last axis."""
-    if _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:
+    if _eager(x) and _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:
         d = m.normalized_shape[0]
         fits = m.weight.shape == (d,) and m.bias.shape == (d,) and x.shape[-1] == d
         blocks = _blocks(x, m.weight, m.bias) if d % 4 == 0 and d <= 1024 and fits else None
@@ -140,7 +158,7 @@ class PositionwiseFF(nn.Module):
     def _core(self, x, residual):
         """``residual + CoreNet(x)``"""
         net = self.CoreNet
-        if (_untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
+        if (_eager(x) and _untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
                 and _untouched(net[2], nn.Dropout) and _untouched(net[3], nn.Linear) and _untouched(net[4], nn.Dropout)
                 and net[0].bias is not None and net[3].bias is not None):
             W1, b1, W2, b2 = net[0].weight, net[0].bias, net[3].weight, net[3].bias
@@ -155,6 +173,13 @@ class PositionwiseFF(nn.Module):
         return residual + net(x)
 
     def forward(self, inp):
+        if torch.jit.is_scripting():
+            out = inp + self.CoreNet(self.layer_norm(inp) if self.pre_lnorm else inp)
+            return out if self.pre_lnorm else self.layer_norm(out)
+        else:
+            return self._forward(inp)
+
+    def _forward(self, inp):
         if self.pre_lnorm:
             return self._core(_layer_norm(self.layer_norm, inp), inp)
         return _layer_norm(self.layer_norm, self._core(inp, inp))

@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import DeltaNetDecoderLayer, DeltaNetLayer, Linear, PositionalEmbedding, _blocks, _drops, _untouched, decode_parameters
+from .layers import DeltaNetDecoderLayer, DeltaNetLayer, Linear, PositionalEmbedding, _blocks, _drops, _eager, _untouched, decode_parameters
 
 
 class _WordEmbedding(nn.Module):
@@ -36,8 +36,14 @@ class _TiedSoftmaxLoss(nn.Module):
         self.out_layers = nn.ModuleList([Linear(d_model, n_token)])
 
     def forward(self, hidden, target):
+        if torch.jit.is_scripting():
+            return F.cross_entropy(self.out_layers[0](hidden), target, reduction="none")
+        else:
+            return self._forward(hidden, target)
+
+    def _forward(self, hidden, target):
         out = self.out_layers[0]
-        if (_untouched(out, Linear) and out.bias is not None and target.dtype is torch.int64 and target.device == hidden.device
+        if (_eager(hidden) and _eager(target) and _untouched(out, Linear) and out.bias is not None and target.dtype is torch.int64 and target.device == hidden.device
                 and hidden.dim() == 2 and target.shape == hidden.shape[:1]
                 and out.weight.shape[1:] == hidden.shape[1:] and out.bias.shape == out.weight.shape[:1]):
             blocks = _blocks(hidden, out.weight, out.bias)

@@ -350,6 +350,38 @@ def beyond_the_kernels(m):
     assert pkg.layers._blocks(x, rnd(4, 4)) is None and pkg.layers._blocks(x[:2 ** 24], rnd(4, 4)) is not None
 
 
+def traced_and_watched(m):
+    """Tracers, the script compiler and modes that watch the operators see PyTorch's; a default device changes nothing."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    pkg, rec = package(m)
+    x, target = rnd(6, 24), torch.randint(0, 30, (6,))
+
+    class Watch(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, f, types, args=(), kwargs=None):
+            return f(*args, **(kwargs or {}))
+
+    class WatchFunctions(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, f, types, args=(), kwargs=None):
+            return f(*args, **(kwargs or {}))
+
+    for mod, args in ((pkg.PositionwiseFF(24, 40, 0.0), (x,)), (pkg.PositionwiseFF(24, 40, 0.0, True), (x,)),
+                      (pkg.layers.Linear(24, 9), (x,)), (pkg.lm._TiedSoftmaxLoss(30, 24), (x, target))):
+        with torch.no_grad():
+            calls, want = rec.of(mod, *args)
+            assert calls
+            with torch.device("cpu"):
+                assert rec.of(mod, *args)[0] == calls
+            others = (torch.fx.symbolic_trace(mod), torch.jit.script(mod), torch.jit.trace(mod, args),
+                      make_fx(lambda *a: mod(*a))(*args), torch.compile(mod, backend="eager", fullgraph=True))
+            for other in others:
+                calls, y = rec.of(other, *args)
+                assert calls in ([], ["linear"]) and torch.allclose(y, want, atol=1e-5), (type(mod), other, y)
+            for mode in (Watch, WatchFunctions):
+                with mode():
+                    calls, y = rec.of(mod, *args)
+                assert calls == [] and torch.allclose(y, want, atol=1e-5)
+
+
 def main():
     m, check = load(sys.argv[1]), sys.argv[2]
     torch.manual_seed(0)
