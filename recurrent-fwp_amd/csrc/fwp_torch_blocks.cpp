@@ -560,9 +560,93 @@ at::Tensor nll(const at::Tensor &x, const at::Tensor &W, const at::Tensor &bias,
     return NllFn::forward(nullptr, x, W, bias, target);
 }
 
+// ------------------------------------------------------------------ does a block apply?
+
+// One call per block instead of a dozen attributes looked up from Python, which costs as much as a small layer's kernels.
+// The two Python types, held for good from bind_blocks on.
+PyObject *g_tensor_type, *g_parameter_type;
+
+// An ordinary tensor or parameter (no subclass, no tracer's stand-in), or nothing
+const at::Tensor *ordinary(py::handle h) {
+    const PyObject *const type = reinterpret_cast<PyObject *>(Py_TYPE(h.ptr()));
+    return type == g_tensor_type || type == g_parameter_type ? &THPVariable_Unpack(h.ptr()) : nullptr;
+}
+
+bool on_gpu(const at::Tensor &t) {
+#ifdef FWP_HOST_STUB
+    return true;
+#else
+    return t.is_cuda();
+#endif
+}
+
+// fp32 on the GPU, with something in it
+const at::Tensor *fp32(py::handle h) {
+    const at::Tensor *const t = ordinary(h);
+    return t && t->scalar_type() == at::kFloat && t->numel() > 0 && on_gpu(*t) ? t : nullptr;
+}
+
+// The kernels' offsets reach rows of 2^21 floats, their launches 2^24 rows.
+const at::Tensor *input(py::handle h) {
+    const at::Tensor *const t = fp32(h);
+    return t && t->dim() > 0 && t->numel() / t->size(-1) <= (int64_t(1) << 24) ? t : nullptr;
+}
+const at::Tensor *parameter(py::handle h) {
+    const at::Tensor *const t = fp32(h);
+    if (!t || !t->is_contiguous()) return nullptr;
+    for (const int64_t n : t->sizes())
+        if (n > (int64_t(1) << 21)) return nullptr;
+    return t;
+}
+
+bool takes_all(py::handle x_, const py::list &params) {
+    if (!input(x_)) return false;
+    for (py::handle p : params)
+        if (!parameter(p)) return false;
+    return true;
+}
+
+bool takes_linear(py::handle x_, py::handle W_, py::handle b_) {
+    const at::Tensor *const x = input(x_), *const W = parameter(W_), *const b = parameter(b_);
+    return x && W && b && W->dim() == 2 && x->size(-1) == W->size(1) && same_shape(*b, {W->size(0)});
+}
+
+bool takes_feed_forward(py::handle x_, py::handle W1_, py::handle b1_, py::handle W2_, py::handle b2_) {
+    const at::Tensor *const x = input(x_), *const W1 = parameter(W1_), *const b1 = parameter(b1_), *const W2 = parameter(W2_),
+                     *const b2 = parameter(b2_);
+    if (!(x && W1 && b1 && W2 && b2)) return false;
+    const int64_t d = x->size(-1), inner = b1->numel();
+    return same_shape(*W1, {inner, d}) && same_shape(*b1, {inner}) && same_shape(*W2, {d, inner}) && same_shape(*b2, {d});
+}
+
+bool takes_layer_norm(py::handle x_, py::handle g_, py::handle b_, int64_t d) {
+    const at::Tensor *const x = input(x_), *const g = parameter(g_), *const b = parameter(b_);
+    return x && g && b && d % 4 == 0 && d <= 1024 && x->size(-1) == d && same_shape(*g, {d}) && same_shape(*b, {d});
+}
+
+bool takes_delta_block(py::handle x_, py::handle Wqkvb_, py::handle Wo_, int64_t H, int64_t D) {
+    const at::Tensor *const x = input(x_), *const Wqkvb = parameter(Wqkvb_), *const Wo = parameter(Wo_);
+    return x && Wqkvb && Wo && (D == 16 || D == 32 || D == 64) && same_shape(*Wqkvb, {H * (3 * D + 1), x->size(-1)}) &&
+           same_shape(*Wo, {x->size(-1), H * D});
+}
+
+bool takes_nll(py::handle x_, py::handle W_, py::handle b_, py::handle target_) {
+    const at::Tensor *const x = input(x_), *const W = parameter(W_), *const b = parameter(b_), *const target = ordinary(target_);
+    return x && W && b && target && x->dim() == 2 && W->dim() == 2 && x->size(1) == W->size(1) && same_shape(*b, {W->size(0)}) &&
+           target->scalar_type() == at::kLong && target->device() == x->device() && same_shape(*target, {x->size(0)});
+}
+
 }  // namespace
 
 void bind_blocks(py::module_ &m) {
+    g_tensor_type = py::object(py::module_::import("torch").attr("Tensor")).release().ptr();
+    g_parameter_type = py::object(py::module_::import("torch.nn").attr("Parameter")).release().ptr();
+    m.def("takes_all", &takes_all, "may an input and parameters of any sizes go to the kernels?");
+    m.def("takes_linear", &takes_linear, "does linear apply?");
+    m.def("takes_feed_forward", &takes_feed_forward, "does feed_forward apply?");
+    m.def("takes_layer_norm", &takes_layer_norm, "does layer_norm apply?");
+    m.def("takes_delta_block", &takes_delta_block, "does delta_block apply?");
+    m.def("takes_nll", &takes_nll, "does nll apply?");
     m.def("linear", &linear, py::arg("x"), py::arg("W"), py::arg("bias") = py::none(), py::arg("relu") = false,
           "x W^T (+ bias) (relu)");
     m.def("feed_forward", &feed_forward, py::arg("x"), py::arg("W1"), py::arg("b1"), py::arg("W2"), py::arg("b2"),

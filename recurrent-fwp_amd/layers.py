@@ -23,11 +23,6 @@ def _untouched(m, cls):
                                    or "forward" in m.__dict__)
 
 
-def _eager(x):
-    """Is ``x`` an ordinary tensor of an ordinary call, not a stand-in for one or a traced one?"""
-    return type(x) in (torch.Tensor, nn.Parameter) and not (torch.jit.is_tracing() or torch.compiler.is_compiling())
-
-
 def _watched():
     """Does a mode see the operators that are called?  (A default device is such a mode, but changes none of them.)"""
     if torch._C._len_torch_dispatch_stack():
@@ -35,16 +30,11 @@ def _watched():
     return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(torch._C._len_torch_function_stack()))
 
 
-def _blocks(x, *params):
-    """The C++ blocks (csrc/fwp_torch_blocks.cpp) if they apply to this input and these parameters: fp32 on the
-    GPU, outside autocast, tracing, modes and functional transforms."""
-    if _fwp_torch is None or not _eager(x) or not x.is_cuda:
-        return None
-    for t in (x, *params):
-        if t.dtype is not torch.float32 or not t.is_cuda or type(t) not in (torch.Tensor, nn.Parameter) or t.numel() == 0:
-            return None
-    # the kernels' offsets reach rows of 2^21 floats, their launches 2^24 rows
-    if x.dim() == 0 or x.numel() > x.shape[-1] << 24 or not all(p.is_contiguous() and max(p.shape, default=0) <= 1 << 21 for p in params):
+def _blocks(takes, *args):
+    """The C++ blocks (csrc/fwp_torch_blocks.cpp) if they apply, else ``None``.  Their function ``takes`` says so of the
+    tensors: ordinary ones, fp32, on the GPU, of sizes that fit one another; here: a call outside autocast, tracing, modes and
+    functional transforms."""
+    if _fwp_torch is None or torch.compiler.is_compiling() or torch.jit.is_tracing() or not getattr(_fwp_torch, takes)(*args):
         return None
     if (torch.is_autocast_enabled() or _watched() or torch.nn.modules.module._has_any_global_hook()
             or torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None):
@@ -67,11 +57,9 @@ class Linear(nn.Linear):
             return self._forward(x)
 
     def _forward(self, x):
-        if (_eager(x) and self.bias is not None and x.dim() > 0 and self.weight.shape[1:] == x.shape[-1:]
-                and self.bias.shape == self.weight.shape[:1]):
-            blocks = _blocks(x, self.weight, self.bias)
-            if blocks is not None:
-                return blocks.linear(x, self.weight, self.bias)
+        blocks = _blocks("takes_linear", x, self.weight, self.bias)
+        if blocks is not None:
+            return blocks.linear(x, self.weight, self.bias)
         return F.linear(x, self.weight, self.bias)
 
 
@@ -116,10 +104,8 @@ def decode_parameters(layer):
 
 def _layer_norm(m, x):
     """``m(x)`` for a LayerNorm over the last axis."""
-    if _eager(x) and _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1 and m.weight is not None and m.bias is not None:
-        d = m.normalized_shape[0]
-        fits = m.weight.shape == (d,) and m.bias.shape == (d,) and x.shape[-1] == d
-        blocks = _blocks(x, m.weight, m.bias) if d % 4 == 0 and d <= 1024 and fits else None
+    if _untouched(m, nn.LayerNorm) and len(m.normalized_shape) == 1:
+        blocks = _blocks("takes_layer_norm", x, m.weight, m.bias, m.normalized_shape[0])
         if blocks is not None:
             return blocks.layer_norm(x, m.weight, m.bias, m.eps)
     return m(x)
@@ -158,13 +144,10 @@ class PositionwiseFF(nn.Module):
     def _core(self, x, residual):
         """``residual + CoreNet(x)``"""
         net = self.CoreNet
-        if (_eager(x) and _untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
-                and _untouched(net[2], nn.Dropout) and _untouched(net[3], nn.Linear) and _untouched(net[4], nn.Dropout)
-                and net[0].bias is not None and net[3].bias is not None):
+        if (_untouched(net, nn.Sequential) and len(net) == 5 and _untouched(net[0], nn.Linear) and _untouched(net[1], nn.ReLU)
+                and _untouched(net[2], nn.Dropout) and _untouched(net[3], nn.Linear) and _untouched(net[4], nn.Dropout)):
             W1, b1, W2, b2 = net[0].weight, net[0].bias, net[3].weight, net[3].bias
-            d, inner = x.shape[-1], b1.numel()
-            fits = W1.shape == (inner, d) and b1.shape == (inner,) and W2.shape == (d, inner) and b2.shape == (d,)
-            blocks = _blocks(x, W1, b1, W2, b2) if fits else None
+            blocks = _blocks("takes_feed_forward", x, W1, b1, W2, b2)
             if blocks is not None and not (_drops(net[2]) or _drops(net[4])):
                 return blocks.feed_forward(x, W1, b1, W2, b2, residual)
             if blocks is not None:
@@ -282,10 +265,9 @@ class DeltaNetLayer(nn.Module):
 
         hip_op = self.fast_weight_op is fast_weight_delta
         blocks = None
-        if (hip_op and D in (16, 32, 64) and _untouched(self.qkvb_net, nn.Linear) and _untouched(self.o_net, nn.Linear)
-                and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)
-                and self.qkvb_net.weight.shape == (H * (3 * D + 1), x.shape[-1]) and self.o_net.weight.shape == (x.shape[-1], H * D)):
-            blocks = _blocks(x, self.qkvb_net.weight, self.o_net.weight)
+        if (hip_op and _untouched(self.qkvb_net, nn.Linear) and _untouched(self.o_net, nn.Linear)
+                and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)):
+            blocks = _blocks("takes_delta_block", x, self.qkvb_net.weight, self.o_net.weight, H, D)
         if blocks is not None:
             W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32)
             drops = _drops(self.drop)

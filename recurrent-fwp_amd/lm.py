@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from .layers import DeltaNetDecoderLayer, DeltaNetLayer, Linear, PositionalEmbedding, _blocks, _drops, _eager, _untouched, decode_parameters
+from .layers import DeltaNetDecoderLayer, DeltaNetLayer, Linear, PositionalEmbedding, _blocks, _drops, _untouched, decode_parameters
 
 
 class _WordEmbedding(nn.Module):
@@ -43,10 +43,8 @@ class _TiedSoftmaxLoss(nn.Module):
 
     def _forward(self, hidden, target):
         out = self.out_layers[0]
-        if (_eager(hidden) and _eager(target) and _untouched(out, Linear) and out.bias is not None and target.dtype is torch.int64 and target.device == hidden.device
-                and hidden.dim() == 2 and target.shape == hidden.shape[:1]
-                and out.weight.shape[1:] == hidden.shape[1:] and out.bias.shape == out.weight.shape[:1]):
-            blocks = _blocks(hidden, out.weight, out.bias)
+        if _untouched(out, Linear):
+            blocks = _blocks("takes_nll", hidden, out.weight, out.bias, target)
             if blocks is not None:
                 return blocks.nll(hidden, out.weight, out.bias, target)
         return F.cross_entropy(out(hidden), target, reduction="none")
@@ -98,7 +96,7 @@ class DeltaNetLM(nn.Module):
         if (table.max_norm is not None or data.numel() == 0 or pos.inv_freq.dtype is not torch.float32
                 or data.numel() * table.weight.shape[-1] >= 1 << 32):      # a thread per number
             return None
-        blocks = _blocks(table.weight, table.weight)
+        blocks = _blocks("takes_all", table.weight, [table.weight])
         return None if blocks is None else blocks.embed(table.weight, data, pos.inv_freq, word.emb_scale, self.clamp_len)
 
     def _decode(self, x, mems):
@@ -123,7 +121,7 @@ class DeltaNetLM(nn.Module):
             params += p
         if (att.n_head * att.d_head) % 64:
             return None
-        blocks = _blocks(x, *params)
+        blocks = _blocks("takes_all", x, params)
         if blocks is None:
             return None
         states = [] if mems is None else [m[0][:x.shape[1]] for m in mems[:len(self.layers)]]
