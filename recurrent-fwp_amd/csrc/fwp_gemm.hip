@@ -4,11 +4,14 @@
 // 3 x 8 significant bits and their signs hold all 24), so a product of two fp32 numbers is the sum of nine bf16
 // products.  Six of them are formed, h h', h m', m h', m m', h l', l h'; the three left out are below
 // 2^-26 |x x'|, a quarter of the rounding of an fp32 product.  Sums are fp32, six roundings per 32 terms where a
-// chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm): 2.2e-7 at K = 256,
-// 5e-7 at K = 1024.  bf16 has fp32's exponents: no scaling.  An operand that no bf16 number
-// holds (infinity, NaN, the last 2^-9 below fp32's largest) leaves NaN or infinity in the sums: a tile
-// with an element that is not finite is formed again on the fp32 matrix instructions (three times the tile's time).  Parts below the smallest normal number count as zero, as
-// denormal operands do: an operand is exact to 2^-24 of itself or to 2^-126, whichever is more.
+// chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm), with hipBLASLt's fp32 products of
+// the same operands behind it: 32768 x 1024, K = 256 2.4e-7 (2.9e-7); 32768 x 256, K = 1024 4.9e-7 (5.7e-7); 32768 x 256,
+// K = 32768 3.04e-6 (3.24e-6); 1024 x 256, K = 32768 in ranges 5.7e-7 (2.0e-6).
+//
+// bf16 has fp32's exponents: no scaling.  An operand that no bf16 number holds (infinity, NaN, the last 2^-9 below
+// fp32's largest) leaves NaN or infinity in the sums: a tile with an element that is not finite is formed again on the fp32
+// matrix instructions, which takes another one to one and a half times its time.  Parts of an operand below the
+// smallest normal number count as zero: it is exact to 2^-24 of itself or to 2^-126, whichever is more.
 //
 // v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
 // the 32x32x16 form 1.8), i.e. 350 TFLOP/s of such fp32 products, where the fp32 matrix instructions make 155.
@@ -18,7 +21,7 @@
 // [plane][k / 8][row], so that a fragment is one ds_read_b128; an operand that is contiguous along its rows
 // instead of along k is transposed in registers on the way.
 //
-// What bounds it: 32768 x 256, K = 1024 takes 93 us, 1.1 PFLOP/s of bf16 products.  Matrix instructions, fragment reads and
+// What bounds it: 32768 x 256, K = 1024 takes 89-93 us, 1.1 PFLOP/s of bf16 products.  Matrix instructions, fragment reads and
 // barriers alone take 67 us (1.56 PFLOP/s), the LDS writes 15 us more, the split 5-10 us, loads that miss the cache 5 us; the
 // clock falls to 1.8-1.9 GHz, so that cycles saved come back as time only in part.  Tried without gain: 256 x 128 tiles
 // (256 registers, spills: 113 us), fragments fetched a dozen matrix instructions ahead (97 us), remainders by
@@ -298,6 +301,9 @@ __device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, flo
     if (lane % LANES == 0) out[at] = m, out[at + pitch] = s;
 }
 
+// Three waves per SIMD, three workgroups on a CU: the products with the loss's gradient are held to 168 registers for it
+// (174 without the bound; one is spilled, outside the loop).
+//
 // BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
 template <bool AKC, bool BKC, int BM, int BN, int MODE>
 __global__ __launch_bounds__(kThreads, 3) void k_gemm(GemmArgs g) {
