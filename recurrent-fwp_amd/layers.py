@@ -289,9 +289,9 @@ class DeltaNetLayer(nn.Module):
             q, k, v, beta = (t.permute(1, 2, 0, 3) for t in qkvb.split((D, D, D, 1), dim=-1))
             q, k, beta = sum_normalised_elu(q), sum_normalised_elu(k), torch.sigmoid(beta)
 
-        if hip_op and q.dtype != torch.float32:
-            # half or bf16 activations (autocast): the operator and its state are fp32, as the
-            # reference's kernel and its torch.zeros state are
+        if hip_op:
+            # half or bf16 activations (autocast, which makes some of them fp32): the operator and its state are fp32, as
+            # the reference's kernel and its torch.zeros state are
             q, k, v, beta = q.float(), k.float(), v.float(), beta.float()
         W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32 if hip_op else q.dtype)
 

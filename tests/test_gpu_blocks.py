@@ -120,6 +120,24 @@ def test_second_derivatives_of_the_delta_block(fwp, pre, power):
             close((name, i), got, want, 64)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_decoder_layer_under_autocast(fwp, dtype):
+    """PyTorch's products in the lower precision around the fp32 operator."""
+    x = torch.randn(20, 2, 64, generator=torch.Generator().manual_seed(1)).cuda().requires_grad_()
+    torch.manual_seed(0)
+    layer = fwp.DeltaNetDecoderLayer(2, 64, 32, 128).cuda()
+    w = torch.randn_like(x)
+    want = layer(x)
+    wants = torch.autograd.grad((want * w).sum(), [x, *layer.parameters()])
+    with torch.autocast("cuda", dtype=dtype):
+        y = layer(x)
+    grads = torch.autograd.grad((y * w).sum(), [x, *layer.parameters()])
+    # four products of bf16's 8 bits in a row.  In the 2-norm: an activation that rounding takes across the ReLU's zero
+    # changes single elements of a gradient by a token's whole share (one of 40 tokens here, up to 2 ** -3 of the largest).
+    for got, ref in zip((y, *grads), (want, *wants)):
+        assert got.dtype is torch.float32 and float((got - ref).norm()) <= 16 * 2.0 ** -8 * float(ref.norm())
+
+
 @pytest.mark.parametrize("pre", [False, True])
 def test_language_model_with_ignored_targets(fwp, pre):
     """Losses and every gradient of a two-layer model, some targets ignored, frozen embedding included."""
