@@ -1,33 +1,36 @@
-// fp32 matrix products of the language model's layers on the bf16 matrix cores.
+// fp32 matrix products of the language model's layers on the 16-bit matrix cores, each operand split into a few 16-bit
+// numbers, their products summed in fp32.
 //
-// An fp32 number is the sum of three bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest:
-// 3 x 8 significant bits and their signs hold all 24), so a product of two fp32 numbers is the sum of nine bf16
-// products.  Six of them are formed, h h', h m', m h', m m', h l', l h'; the three left out are below
-// 2^-26 |x x'|, a quarter of the rounding of an fp32 product.  Sums are fp32, six roundings per 32 terms where a
-// chain of fp32 multiply-adds has 32.  Measured against float64 (N(0,1) operands, 2-norm), with hipBLASLt's fp32 products of
-// the same operands behind it: 32768 x 1024, K = 256 2.4e-7 (2.9e-7); 32768 x 256, K = 1024 4.9e-7 (5.7e-7); 32768 x 256,
-// K = 32768 3.04e-6 (3.24e-6); 1024 x 256, K = 32768 in ranges 5.7e-7 (2.0e-6).
+// Half2 (K >= 128): x s = h + m, h = fp16(x s), m = fp16(x s - h), three products m h', h m', h h'.  s is a power of two for each row
+// of an operand (the rows of C, the columns of C).  h and m hold x to the last or the last but one of its 24 bits; m m' is below
+// 2^-22 |x x'|.  That is 7e-8 of a product, at random, where a sum's roundings, three per 32 terms, make more: relative error
+// against float64 (N(0,1) operands, 2-norm; in brackets Bf16x3, then hipBLASLt's fp32): K = 128 1.39e-7 (1.61e-7), 32768 x 1024, K = 256
+// 1.87e-7 (2.36e-7, 2.9e-7); 32768 x 256, K = 1024 3.6e-7 (4.9e-7, 5.7e-7); 1024 x 256, K = 32768 in ranges 3.9e-7 (5.75e-7, 2.0e-6).
+// fp16 has few exponents: s brings a row's largest element so far to [8, 16).  Elements down to 2^-7 of that keep all their bits,
+// smaller ones 2^-28 of it.  One beyond 65504 / s (a row that grows 4096-fold along k) moves s, and the row's results so far with it.
 //
-// bf16 has fp32's exponents: no scaling.  An operand that no bf16 number holds (infinity, NaN, the last 2^-9 below
-// fp32's largest) leaves NaN or infinity in the sums: a tile with an element that is not finite is formed again on the fp32
-// matrix instructions, which takes another one to one and a half times its time.  Parts of an operand below the
-// smallest normal number count as zero: it is exact to 2^-24 of itself or to 2^-126, whichever is more.
+// Bf16x3 (smaller K, and the loss's gradient): x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest: 3 x 8 significant bits and
+// their signs hold all 24), six products, h h', h m', m h', m m', h l', l h'; the three left out are below 2^-26 |x x'|.  bf16
+// has fp32's exponents: no scaling.  Parts of an operand below the smallest normal number count as zero: it is exact to
+// 2^-24 of itself or to 2^-126, whichever is more.
 //
-// v_mfma_f32_16x16x32_bf16 makes 2.1 PFLOP/s with random operands (2.45 with zeros: the chip's power is the limit;
-// the 32x32x16 form 1.8), i.e. 350 TFLOP/s of such fp32 products, where the fp32 matrix instructions make 155.
-// The operands are split on their way from global memory to LDS, in the registers of the thread that loads
-// them: 11 vector instructions per two numbers, 45 % of the matrix instructions' time in a 128 x 128 tile, and
-// issued beside them by the other workgroups of the CU.  LDS holds 16-byte units of 8 consecutive k of one row,
-// [plane][k / 8][row], so that a fragment is one ds_read_b128; an operand that is contiguous along its rows
-// instead of along k is transposed in registers on the way.
+// An operand that the 16-bit numbers cannot hold (infinity, NaN, for bf16 the last 2^-9 below fp32's largest) leaves NaN or infinity in
+// the sums: a tile with an element that is not finite is formed again on the fp32 matrix instructions, in two to four times its time.
 //
-// What bounds it: 32768 x 256, K = 1024 takes 89-93 us, 1.1 PFLOP/s of bf16 products.  Matrix instructions, fragment reads and
-// barriers alone take 67 us (1.56 PFLOP/s), the LDS writes 15 us more, the split 5-10 us, loads that miss the cache 5 us; the
-// clock falls to 1.8-1.9 GHz, so that cycles saved come back as time only in part.  Tried without gain: 256 x 128 tiles
-// (256 registers, spills: 113 us), fragments fetched a dozen matrix instructions ahead (97 us), remainders by
-// v_dot2_f32_bf16 (fewer instructions, 101 us, and it drops denormals).
+// v_mfma_f32_16x16x32_bf16 makes 1.7-2.1 PFLOP/s with random operands and the f16 form 1.5 (2.45 with zeros: the chip's power is
+// the limit), i.e. 490 TFLOP/s of Half2's products and 280-350 of Bf16x3's, where the fp32 matrix instructions make 155.
+//
+// Every wave loads and splits its own rows of A, in the lanes that multiply them; B's rows are split by one wave
+// and handed to the others through LDS, in 16-byte units of 8 k of one row, [plane][k-chunk][row], so that a fragment is one
+// ds_read_b128.  An operand that is contiguous along its rows instead of along k is transposed in registers on the way: a lane's load of T
+// neighbouring rows is a row of each of T tiles.  Splitting takes 7 vector instructions per two numbers (Half2; 21 cycles, 32
+// with v_fma_mixlo_f16, which take 8 each) or 11 (Bf16x3), between the matrix instructions of the step before (the order
+// is pinned: left to itself the compiler sinks the loads behind the products, and every step waits for memory).
 #include "fwp_common.hpp"
 #include "fwp_mfma.hpp"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace fwp {
 
@@ -36,7 +39,6 @@ __device__ v2f llvm_raw_buffer_load_v2f32(v4i rsrc, int voffset, int soffset, in
 
 namespace {
 
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
@@ -56,13 +58,9 @@ __device__ __forceinline__ v4i buffer_of(const float *base, int64_t floats) {
     return v4i{(int)(uint32_t)a, (int)(uint32_t)((a >> 32) & 0xffff), (int)(uint32_t)(floats * 4), 0x00020000};
 }
 
-__device__ __forceinline__ float lane_of(float x, int lane) {
-    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lane));
-}
-
-template <int ROWS>
+template <int P, int ROWS>
 struct Planes {
-    v4u u[3][kBK / 8][ROWS];
+    v4u u[P][kBK / 8][ROWS];
 };
 
 // The place of a row's unit in its k-chunk, such that no access meets a bank twice: a read takes lanes 0-3, 12-15, 20-23
@@ -70,17 +68,19 @@ struct Planes {
 // four chunks (operands contiguous along k) or every other of sixteen rows (the others).  With rows in order and the
 // chunks 32 bytes apart 420 of 1280 LDS cycles per tile step (x W^T), 770 of 1560 (g^T x) were conflicts; 32768 x 256,
 // K = 1024: 4.7e7 -> 4.3e7 cycles of busy CUs, 95.0 -> 92.9 us.
-__device__ __forceinline__ constexpr int unit_of(int row, int chunk) { return row ^ (2 * chunk) ^ ((row >> 3) & 1); }
+__device__ __forceinline__ constexpr int unit_of(int row, int chunk) { return row ^ (2 * chunk) ^ ((row >> 3) & 3); }
 
 // exp(x): 2^(x log2 e) by the hardware, x log2 e rounded to its nearest float and the rest of it as a factor: probabilities
 // are off by at most 4 roundings, down to e^-70 (with x log2 e alone by 60 there; PyTorch's, through the logarithm, by 69).  Arguments below -150 give
 // 0 as that one does (the rest of an infinity would be NaN); a NaN stays.
-__device__ __forceinline__ float exp_of(float x) {
+// exp_of_sum: 0 for a NaN, for logits whose sum of exponentials shows it.
+__device__ __forceinline__ float exp_above(float x) {
     constexpr float kLog2e = 1.44269504f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
-    x = x < -150.f ? -150.f : x;
     const float y = x * kLog2e, rest = fmaf(x, kLog2e, -y), e = __builtin_amdgcn_exp2f(y);
     return fmaf(e, fmaf(rest, kLn2, x * (kLog2eRest * kLn2)), e);
 }
+__device__ __forceinline__ float exp_of(float x) { return exp_above(x < -150.f ? -150.f : x); }
+__device__ __forceinline__ float exp_of_sum(float x) { return exp_above(__builtin_fmaxf(x, -150.f)); }
 
 // What turns stored logits into the gradient of the loss as an operand is loaded:
 // (exp(logit - shift) * scale - [vocabulary entry == target]) * gloss of the token, 0 for an ignored target, NaN for one that
@@ -107,132 +107,285 @@ __device__ __forceinline__ NllToken nll_token(const NllArgs &a, int token) {
     t.g = want == kIgnored ? 0.f : want >= 0 && want < a.vocab ? a.gloss[token] : NAN;
     const float2 s = a.stats ? reinterpret_cast<const float2 *>(a.stats)[token] : make_float2(a.lse[token], 1.f);
     t.shift = s.x;
-    t.scaled = s.y * t.g;
+    t.scaled = s.x > -INFINITY ? s.y * t.g : NAN;
     return t;
 }
 
-__device__ __forceinline__ float nll_grad(float logit, float shift, float scaled, float g, bool hit) {
-    return fmaf(exp_of(logit - shift), scaled, hit ? -g : 0.f);
+
+// The k of element e of the 8 that a lane (A) or a unit in LDS (B) holds of k-chunk c of a step: two runs of four, so that
+// the four chunks' loads of one run are 64 bytes of a row.
+__device__ __forceinline__ constexpr int k_of(int c, int e) { return e < 4 ? 4 * c + e : 16 + 4 * c + (e - 4); }
+
+// x = h + m (+ l) for eight values.  Half2: two fp16 numbers of x * scale; Bf16x3: three bf16 numbers of x.
+struct Half2 {
+    typedef _Float16 frag __attribute__((ext_vector_type(8)));
+    static constexpr int kPlanes = 2;
+    static constexpr bool kScaled = true;
+    static __device__ __forceinline__ unsigned pack(float a, float b) {
+        unsigned r;
+        asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+    }
+    static __device__ __forceinline__ void split2(float a, float b, float scale, unsigned *d) {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        d[0] = pack(a * scale, b * scale);
+        const h2 h = __builtin_bit_cast(h2, d[0]);
+        d[1] = pack(fmaf(a, scale, -(float)h[0]), fmaf(b, scale, -(float)h[1]));
+    }
+    static __device__ __forceinline__ v4f mma(frag x, frag y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, c, 0, 0, 0); }
+    // the planes (of A, of B) that are multiplied, in this order
+    static constexpr int kProducts = 3;
+    static constexpr int kOrder[3][2] = {{1, 0}, {0, 1}, {0, 0}};
+};
+
+struct Bf16x3 {
+    typedef __bf16 frag __attribute__((ext_vector_type(8)));
+    static constexpr int kPlanes = 3;
+    static constexpr bool kScaled = false;
+    static __device__ __forceinline__ void split2(float a, float b, float, unsigned *d) {
+        d[0] = pack2(a, b);
+        const float ra = a - low_f(d[0]), rb = b - high_f(d[0]);
+        d[1] = pack2(ra, rb);
+        d[2] = pack2(ra - low_f(d[1]), rb - high_f(d[1]));
+    }
+    static __device__ __forceinline__ v4f mma(frag x, frag y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0); }
+    static constexpr int kProducts = 6;
+    static constexpr int kOrder[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};
+};
+
+// Elements 2 j and 2 j + 1 of eight values, split, into their place in a fragment of each plane.
+template <class S>
+__device__ __forceinline__ void split_pair(const float *x, int j, float scale, v4u *d) {
+    unsigned y[S::kPlanes];
+    S::split2(x[2 * j], x[2 * j + 1], scale, y);
+#pragma unroll
+    for (int p = 0; p < S::kPlanes; p++) d[p][j] = y[p];
 }
 
-// One operand's share of the loads and LDS writes of a thread.  KC: rows are contiguous along k; a task is 8
-// consecutive k of one row (two 16-byte loads, one unit per plane).  Otherwise contiguous along the rows; a
-// task is VEC consecutive rows x 8 k (8 loads, VEC units per plane).
-// NLL: the operand is the loss gradient, formed from the logits; tokens are the rows (KC) or k.
-template <bool KC, int ROWS, bool NLL>
-struct Operand {
-    static constexpr int kChunks = kBK / 8;
-    static constexpr int VEC = KC ? 1 : ROWS * kChunks / kThreads;          // 2 at 128 rows, 1 at 64
-    static constexpr int kTasks = KC ? ROWS * kChunks / kThreads : 1;
-    static_assert(KC ? kTasks >= 1 : (VEC == 1 || VEC == 2), "a whole number of tasks per thread");
-    float x[kTasks][8 * VEC];
-    unsigned off[kTasks];
-    // the tokens' values for the loss gradient: of this task's row (KC), or of the wave's k-chunk, token j in
-    // the lanes with lane % 8 == j
-    NllToken token[NLL ? kTasks : 1];
+// A row's scale: the power of two that takes `largest` into [2^3, 2^4) (0 for 0: nothing seen yet), and how large an element
+// may be under it.
+struct Scale {
+    float s, limit;
+    __device__ __forceinline__ void none() { s = 0.f, limit = 0.f; }
+    __device__ __forceinline__ void one() { s = 1.f; }
+    __device__ __forceinline__ float inverse() const { return s == 0.f ? 0.f : __uint_as_float((254u << 23) - __float_as_uint(s)); }
+    __device__ __forceinline__ int exponent() const { return s == 0.f ? 0 : 127 - (int)(__float_as_uint(s) >> 23); }      // of the inverse
+    __device__ __forceinline__ void set(float largest) {
+        const int b = 257 - (int)(__float_as_uint(largest) >> 23);
+        s = largest == 0.f ? 0.f : __uint_as_float((unsigned)min(max(b, 4), 250) << 23);
+        limit = 65504.f * inverse();
+    }
+    // for a row with an element of size `largest`: what its results so far are multiplied with
+    __device__ __forceinline__ float fit(float largest) {
+        if (!(largest > limit)) return 1.f;
+        const float was = inverse();
+        set(largest);
+        return was == 0.f ? 1.f : s * was;
+    }
+};
 
-    static __device__ __forceinline__ int row_of(int t) { return KC ? t / kChunks : (t % (ROWS / VEC)) * VEC; }
-    static __device__ __forceinline__ int chunk_of(int t) { return KC ? t % kChunks : t / (ROWS / VEC); }
-
-    __device__ __forceinline__ void init(int tid, int64_t ld, int row0, int rows, const NllArgs &nll) {
+__device__ __forceinline__ float abs_max8(const float *x, float m) {
 #pragma unroll
-        for (int i = 0; i < kTasks; i++) {
-            const int r = row_of(tid + i * kThreads), c = chunk_of(tid + i * kThreads);
-            off[i] = (unsigned)(KC ? r * ld + 8 * c : 8 * c * ld + r) * 4;
-            if constexpr (NLL && KC) token[i] = nll_token(nll, min(row0 + r, rows - 1));
+    for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(x[e]));
+    return m;
+}
+
+// LDS accesses of one wave execute in order; this keeps the compiler from moving them across.
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+// A: a wave's 16 T rows, straight from global memory to the lanes that multiply them.  Lane 16 c + r holds k-chunk c of
+// row r of each of the T matrix-instruction tiles; a tile's rows are 16 consecutive ones (KC: rows are contiguous along
+// k) or every T-th of 16 T (contiguous along the rows: a lane's load is T neighbouring rows).
+// NLL: the operand is the loss gradient, formed from the logits; tokens are the rows (KC) or k.
+template <bool KC, int T, bool NLL>
+struct Direct {
+    // a step's elements as they are loaded, and (NLL, !KC) one of its 32 tokens
+    struct Raw {
+        float x[T][8];
+        NllToken next;
+    };
+    NllToken token[NLL && KC ? T : 1];
+    NllToken *tok;      // LDS, this wave's: a step's tokens
+    Scale s[T];
+    int c, r;
+    unsigned at[2];
+
+    static __device__ __forceinline__ int row_of(int i, int r) { return KC ? 16 * i + r : T * r + i; }
+
+    __device__ __forceinline__ void init(int lane, int row0, int rows, const NllArgs &nll) {
+        c = lane / 16, r = lane % 16;
+        if constexpr (NLL && KC)
+#pragma unroll
+            for (int i = 0; i < T; i++) token[i] = nll_token(nll, min(row0 + row_of(i, r), rows - 1));
+    }
+    // the lanes' offsets for a load of k0 ...: they change where a row ends within the step only
+    __device__ __forceinline__ void aim(int64_t ld, int k0, int K) {
+        if constexpr (KC) {
+            const unsigned o = (unsigned)(r * ld + 4 * c) * 4;
+            at[0] = k0 + 4 * c < K ? o : kOut, at[1] = k0 + 16 + 4 * c < K ? o + 64 : kOut;
+        } else {
+            at[0] = (unsigned)(4 * c * ld + T * r) * 4;
         }
     }
-    // P: the tile's first row at k = 0, `left` rows from there, k0 .. min(k0 + kBK, K)
-    __device__ __forceinline__ void load(const float *P, int64_t ld, int left, int tid, int k0, int K, const NllArgs &nll) {
+    // P: the wave's first row at k = 0, `left` rows from there, k0 .. min(k0 + kBK, K); zeros beyond K
+    __device__ __forceinline__ void load(Raw &w, const float *P, int64_t ld, int left, int k0, int K, const NllArgs &nll, int tokens,
+                                         int lane) const {
         if constexpr (KC) {
-            const v4i rs = buffer_of(P + k0, (int64_t)(min(left, ROWS) - 1) * ld + (K - k0));
+            const v4i rs = buffer_of(P + k0, k0 < K && left > 0 ? (int64_t)(min(left, 16 * T) - 1) * ld + (K - k0) : 0);
 #pragma unroll
-            for (int i = 0; i < kTasks; i++) {
-                const int k = k0 + 8 * chunk_of(tid + i * kThreads);
-                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)(k < K ? off[i] : kOut), 0, 0),
-                          b = llvm_raw_buffer_load_v4f32(rs, (int)(k + 4 < K ? off[i] + 16 : kOut), 0, 0);
+            for (int i = 0; i < T; i++) {
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], (int)(i * ld * 64), 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)at[1], (int)(i * ld * 64), 0);
 #pragma unroll
-                for (int j = 0; j < 4; j++) x[i][j] = a[j], x[i][4 + j] = b[j];
+                for (int j = 0; j < 4; j++) w.x[i][j] = a[j], w.x[i][4 + j] = b[j];
             }
         } else {
-            if constexpr (NLL) token[0] = nll_token(nll, min(k0 + 8 * chunk_of(tid) + tid % 8, K - 1));
-            const v4i rs = buffer_of(P + (int64_t)k0 * ld, (int64_t)(min(K - k0, kBK) - 1) * ld + left);
+            const int64_t size = (int64_t)(min(K - k0, kBK) - 1) * ld + left;
+            const v4i rs = buffer_of(P + (int64_t)k0 * ld, k0 < K && size > 0 ? size : 0);
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                if constexpr (VEC == 1) {
-                    x[0][j] = llvm_raw_buffer_load_f32(rs, (int)off[0], (int)(j * ld * 4), 0);
+            for (int e = 0; e < 8; e++) {
+                const int so = (int)(k_of(0, e) * ld * 4);
+                if constexpr (T == 4) {
+                    const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], so, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) w.x[i][e] = a[i];
+                } else if constexpr (T == 2) {
+                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)at[0], so, 0);
+                    w.x[0][e] = a[0], w.x[1][e] = a[1];
                 } else {
-                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)off[0], (int)(j * ld * 4), 0);
-                    x[0][j] = a[0], x[0][8 + j] = a[1];
+                    static_assert(T == 1, "one, two or four rows per load");
+                    w.x[0][e] = llvm_raw_buffer_load_f32(rs, (int)at[0], so, 0);
                 }
             }
+            if constexpr (NLL) w.next = nll_token(nll, min(k0 + lane % kBK, tokens - 1));
         }
     }
-    // What load() brought: zeros beyond K (a row contiguous along k runs on into the next row there), and the
-    // loss gradient in place of the logits
-    __device__ __forceinline__ void finish(int tid, int row0, int k0, int K, const NllArgs &nll) {
+    // zeros beyond K (a row contiguous along k runs on into the next row there)
+    __device__ __forceinline__ void cut(Raw &w, int k0, int K) const {
+        if constexpr (KC)
+#pragma unroll
+            for (int i = 0; i < T; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) w.x[i][e] = k0 + k_of(c, e) < K ? w.x[i][e] : 0.f;
+    }
+    // the step's tokens to where element() reads them
+    __device__ __forceinline__ void hand_over(const Raw &w, int lane) const {
+        if constexpr (NLL && !KC) {
+            wave_lds_order();
+            if (lane < kBK) tok[lane] = w.next;
+            wave_lds_order();
+        }
+    }
+    // the operand's element: itself, or the loss gradient in place of the logit; `whole`: also where a target or K's end is
+    // within the step (rare())
+    __device__ __forceinline__ float element(const Raw &w, int i, int e, bool whole, int row0, int k0, int K) const {
+        if constexpr (!NLL) return w.x[i][e];
+        else {
+            const NllToken t = KC ? token[i] : tok[k_of(c, e)];
+            if (!whole) return exp_of_sum(w.x[i][e] - t.shift) * t.scaled;
+            const int k = k0 + k_of(c, e);
+            // a token beyond K has the last one's values beside a logit of 0: its exponential may be infinite
+            const float d = fmaf(exp_of(w.x[i][e] - t.shift), t.scaled, t.hit == (KC ? k : row0 + row_of(i, r)) ? -t.g : 0.f);
+            return k < K ? d : 0.f;
+        }
+    }
+    __device__ __forceinline__ bool rare(const Raw &w, int row0, int k0, int K) const {
+        if constexpr (!NLL) return false;
+        bool any = k0 + kBK > K;
+        if constexpr (!KC) any |= (unsigned)(w.next.hit - row0) < 16 * T;
+        else
+#pragma unroll
+            for (int i = 0; i < T; i++) any |= (unsigned)(token[i].hit - k0) < kBK;
+        return __any(any);
+    }
+    // the largest magnitude of a row in this step from its lanes' own
+    static __device__ __forceinline__ float of_row(float m) {
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        return fmaxf(m, __shfl_xor(m, 32, 64));
+    }
+};
+
+// B: a thread's share of the loads of a workgroup's ROWS rows and of their split parts' LDS writes.  KC: a task is one
+// k-chunk of one row; otherwise of VEC neighbouring rows.  A row's four k-chunks are in one wave.
+template <bool KC, int ROWS>
+struct Staged {
+    static constexpr int VEC = KC ? 1 : ROWS / 64;
+    static constexpr int kUnits = ROWS / 64;
+    struct Raw {
+        float x[kUnits][8];
+    };
+    Scale s[kUnits];
+    int c, r, unit;
+    unsigned at[2];
+
+    __device__ __forceinline__ void init(int tid) {
+        c = KC ? tid % 4 : tid % 64 / 16;
+        r = KC ? tid / 4 : (tid / 64 * 16 + tid % 16) * VEC;
+        unit = c * ROWS + unit_of(r, c);
+    }
+    __device__ __forceinline__ int row_of(int t) const { return KC ? r + 64 * t : r + t; }
+    __device__ __forceinline__ void aim(int64_t ld, int k0, int K) {
         if constexpr (KC) {
-            const bool tail = k0 + kBK > K;
+            const unsigned o = (unsigned)(r * ld + 4 * c) * 4;
+            at[0] = k0 + 4 * c < K ? o : kOut, at[1] = k0 + 16 + 4 * c < K ? o + 64 : kOut;
+        } else {
+            at[0] = (unsigned)(4 * c * ld + r) * 4;
+        }
+    }
+    __device__ __forceinline__ void load(Raw &w, const float *P, int64_t ld, int left, int k0, int K) const {
+        if constexpr (KC) {
+            const v4i rs = buffer_of(P + k0, k0 < K ? (int64_t)(min(left, ROWS) - 1) * ld + (K - k0) : 0);
 #pragma unroll
-            for (int i = 0; i < kTasks; i++) {
-                const int k = k0 + 8 * chunk_of(tid + i * kThreads);
-                if constexpr (NLL)
+            for (int t = 0; t < kUnits; t++) {
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], (int)(t * ld * 256), 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)at[1], (int)(t * ld * 256), 0);
 #pragma unroll
-                    for (int j = 0; j < 8; j++)
-                        x[i][j] = nll_grad(x[i][j], token[i].shift, token[i].scaled, token[i].g, token[i].hit == k + j);
-                if (tail)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) x[i][j] = k + j < K ? x[i][j] : 0.f;
+                for (int j = 0; j < 4; j++) w.x[t][j] = a[j], w.x[t][4 + j] = b[j];
             }
-        } else if constexpr (NLL) {
-            static_assert(ROWS / VEC == 64, "a k-chunk per wave");
-            const int k = k0 + 8 * chunk_of(tid), r = row0 + row_of(tid);
+        } else {
+            const v4i rs = buffer_of(P + (int64_t)k0 * ld, k0 < K ? (int64_t)(min(K - k0, kBK) - 1) * ld + left : 0);
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float shift = lane_of(token[0].shift, j), scaled = lane_of(token[0].scaled, j), g = lane_of(token[0].g, j);
-                const int h = __builtin_amdgcn_readlane(token[0].hit, j);
+            for (int e = 0; e < 8; e++) {
+                const int so = (int)(k_of(0, e) * ld * 4);
+                if constexpr (VEC == 4) {
+                    const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], so, 0);
 #pragma unroll
-                for (int c = 0; c < VEC; c++) {
-                    // a token beyond K has the last one's values beside a logit of 0: its exponential may be infinite
-                    const float d = nll_grad(x[0][8 * c + j], shift, scaled, g, h == r + c);
-                    x[0][8 * c + j] = k + j < K ? d : 0.f;
+                    for (int t = 0; t < 4; t++) w.x[t][e] = a[t];
+                } else if constexpr (VEC == 2) {
+                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)at[0], so, 0);
+                    w.x[0][e] = a[0], w.x[1][e] = a[1];
+                } else {
+                    w.x[0][e] = llvm_raw_buffer_load_f32(rs, (int)at[0], so, 0);
                 }
             }
         }
     }
-    __device__ __forceinline__ void store(Planes<ROWS> &L, int tid) const {
+    __device__ __forceinline__ void cut(Raw &w, int k0, int K) const {
+        if constexpr (KC)
 #pragma unroll
-        for (int i = 0; i < kTasks; i++)
+            for (int t = 0; t < kUnits; t++)
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                v4u h, m, l;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float a = x[i][8 * c + 2 * j], b = x[i][8 * c + 2 * j + 1];
-                    h[j] = pack2(a, b);
-                    const float ra = a - low_f(h[j]), rb = b - high_f(h[j]);
-                    m[j] = pack2(ra, rb);
-                    l[j] = pack2(ra - low_f(m[j]), rb - high_f(m[j]));
-                }
-                const int r = row_of(tid + i * kThreads) + c, ch = chunk_of(tid + i * kThreads);
-                const int at = unit_of(r, ch);
-                L.u[0][ch][at] = h;
-                L.u[1][ch][at] = m;
-                L.u[2][ch][at] = l;
-            }
+                for (int e = 0; e < 8; e++) w.x[t][e] = k0 + k_of(c, e) < K ? w.x[t][e] : 0.f;
     }
-    // fp32 as it is: 16-byte units of 4 consecutive k of one row, [k / 4][row], in the same memory
-    static __device__ __forceinline__ v4f *plain(Planes<ROWS> &L) { return reinterpret_cast<v4f *>(&L); }
-    __device__ __forceinline__ void store_plain(Planes<ROWS> &L, int tid) const {
+    static __device__ __forceinline__ float of_row(float m) {
+        m = fmaxf(m, __shfl_xor(m, KC ? 1 : 16, 64));
+        return fmaxf(m, __shfl_xor(m, KC ? 2 : 32, 64));
+    }
+    // the wave that splits the rows of matrix-instruction tile j
+    static constexpr int owner(int j) { return KC ? j % 4 : j / VEC; }
+    // a unit's split parts to LDS
+    template <int P>
+    __device__ __forceinline__ void store(Planes<P, ROWS> &L, int t, const v4u *d) const {
 #pragma unroll
-        for (int i = 0; i < kTasks; i++)
+        for (int p = 0; p < P; p++) L.u[p][0][KC ? unit + 64 * t : unit ^ t] = d[p];
+    }
+    // fp32 as it is: 16-byte units of a chunk's four k, [chunk][half][row]
+    __device__ __forceinline__ void store_plain(v4f *L, const Raw &w) const {
 #pragma unroll
-            for (int c = 0; c < VEC; c++)
+        for (int t = 0; t < kUnits; t++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const float *const y = x[i] + 8 * c + 4 * j;
-                    plain(L)[(2 * chunk_of(tid + i * kThreads) + j) * ROWS + row_of(tid + i * kThreads) + c] = v4f{y[0], y[1], y[2], y[3]};
-                }
+            for (int h = 0; h < 2; h++)
+                L[(2 * c + h) * ROWS + row_of(t)] = v4f{w.x[t][4 * h], w.x[t][4 * h + 1], w.x[t][4 * h + 2], w.x[t][4 * h + 3]};
     }
 };
 
@@ -261,128 +414,320 @@ __device__ __forceinline__ float apply(const fwp_mm_epilogue &e, float x, int64_
     return x;
 }
 
-template <int X>
-__device__ __forceinline__ float rotated(float x) {      // within the 16 lanes of a DPP row
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + X, 0xf, 0xf, true));
-}
-
-// LDS accesses of one wave execute in order; this keeps the compiler from moving them across.
-__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
-
 // What a sum of exp(logit - m) is multiplied with to become one of exp(logit - big).  A part of the vocabulary with no
 // logit but -infinity (masked words; columns beyond the last) has m = -infinity and the sum 0, or NaN if there
 // was one: it stays as it is (exp(-infinity + infinity) would make it NaN).
 __device__ __forceinline__ float to_max(float m, float big) { return m == -INFINITY ? 1.f : exp_of(m - big); }
 
-// The largest of a row's logits and the sum of exp(logit - largest): four logits per lane, LANES (8 or 16) lanes per row.
-template <int LANES>
-__device__ __forceinline__ void lse_of_row(float4 v, int n, int N, int lane, float *out, int at, int pitch) {
-    if (n + 3 >= N) {
-        v.x = n < N ? v.x : -INFINITY, v.y = n + 1 < N ? v.y : -INFINITY;
-        v.z = n + 2 < N ? v.z : -INFINITY, v.w = -INFINITY;
+// What becomes of a column of results on its way out (LDS): 2^exponent, the bias.
+struct Columns {
+    const int *exponent;
+    const float *bias;
+};
+
+// acc[i][j][r] is row m0 + row[i], column n0 + 16 j + 4 lc + r, scaled: B's rows are the rows of the matrix instructions'
+// results, so that a lane has four neighbouring columns of a row, 16 bytes.  `rows`: those of the wave.  The two scales are taken
+// back in one step: one alone can leave fp32's range where both together do not.
+template <bool SCALED, int MT, int NT, int MODE>
+__device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], const int (&row)[MT], int m0, int rows, int n0, int lc,
+                                       const int (&ea)[MT], const Columns &col, int column_tile) {
+    const bool one = gridDim.y == 1;
+    const int left = min(g.M - m0, rows), nl = g.N - n0;
+    if (left <= 0) return;
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const v4f b = *reinterpret_cast<const v4f *>(col.bias + 16 * j + 4 * lc);
+        v4i eb = {0, 0, 0, 0};
+        if constexpr (SCALED) eb = *reinterpret_cast<const v4i *>(col.exponent + 16 * j + 4 * lc);
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][j][e] = (SCALED ? ldexpf(acc[i][j][e], ea[i] + eb[e]) : acc[i][j][e]) + b[e];
     }
-    float m = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w));
-    if constexpr (LANES == 16) {
-        m = fmaxf(m, rotated<8>(m));
-        m = fmaxf(m, rotated<4>(m)), m = fmaxf(m, rotated<2>(m)), m = fmaxf(m, rotated<1>(m));
+    const int64_t first = (int64_t)m0 * g.ldc + n0, size = (int64_t)(left - 1) * g.ldc + nl;
+    float *const C = g.C + blockIdx.y * g.part + first;
+    if (MODE == kLse && !g.C) {
+    } else if (g.vec && nl >= 16 * NT) {
+        // rows beyond M lie behind the resource
+        unsigned at[MT];
+#pragma unroll
+        for (int i = 0; i < MT; i++) at[i] = (unsigned)(row[i] * g.ldc + 4 * lc) * 4;
+        if (one && g.epi.relu)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] = relu(acc[i][j][e]);
+        // a tile's loads all at once: one by one, each waited for, they bound the product
+        const auto with = [&](const float *P, auto f) {
+            const v4i rs = buffer_of(P + first, size);
+#pragma unroll
+            for (int i = 0; i < MT; i++) {
+                v4f y[NT];
+#pragma unroll
+                for (int j = 0; j < NT; j++) y[j] = llvm_raw_buffer_load_v4f32(rs, (int)(at[i] + 64 * j), 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] = f(acc[i][j][e], y[j][e]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        if (one && g.epi.residual) with(g.epi.residual, [](float x, float y) { return x + y; });
+        if (one && g.epi.gate) with(g.epi.gate, [](float x, float y) { return gated(y, x); });
+        const v4i rs = buffer_of(C, size);
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int i = 0; i < MT; i++) llvm_raw_buffer_store_v4f32(acc[i][j], rs, (int)(at[i] + 64 * j), 0, 0);
     } else {
 #pragma unroll
-        for (int o = 4; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    }
-    const float z = m == -INFINITY ? 0.f : m;
-    float s = (exp_of(v.x - z) + exp_of(v.y - z)) + (exp_of(v.z - z) + exp_of(v.w - z));
-    if constexpr (LANES == 16) {
-        s += rotated<8>(s);
-        s += rotated<4>(s), s += rotated<2>(s), s += rotated<1>(s);
-    } else {
+        for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int o = 4; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+            for (int j = 0; j < NT; j++) {
+                const int n = 16 * j + 4 * lc;
+                const int64_t at = row[i] * g.ldc + n;
+                if (row[i] >= left || n >= nl) continue;
+                v4f v = acc[i][j];
+                if (g.vec) {
+                    if (one) {
+                        if (g.epi.relu) v = v4f{relu(v[0]), relu(v[1]), relu(v[2]), relu(v[3])};
+                        if (g.epi.residual) v += *reinterpret_cast<const v4f *>(g.epi.residual + first + at);
+                        if (g.epi.gate) {
+                            const v4f y = *reinterpret_cast<const v4f *>(g.epi.gate + first + at);
+                            v = v4f{gated(y[0], v[0]), gated(y[1], v[1]), gated(y[2], v[2]), gated(y[3], v[3])};
+                        }
+                    }
+                    *reinterpret_cast<v4f *>(C + at) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < nl) C[at + e] = one ? apply(g.epi, v[e], first + at + e) : v[e];
+                }
+            }
     }
-    if (lane % LANES == 0) out[at] = m, out[at + pitch] = s;
+    if constexpr (MODE == kLse) {
+        // the largest of a row's logits here and the sum of exp(logit - largest); four lanes share a row
+        if (nl < 16 * NT)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (16 * j + 4 * lc + e >= nl)
+#pragma unroll
+                        for (int i = 0; i < MT; i++) acc[i][j][e] = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < MT; i++) {
+            const int m = m0 + row[i];
+            if (g.hit) {
+                const int at = row[i] < left ? (int)g.nll.target[m] - n0 - 4 * lc : -1;
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (at == 16 * j + e && at + 4 * lc < nl) g.hit[m] = acc[i][j][e];
+            }
+            float big = -INFINITY, s = 0.f;
+#pragma unroll
+            for (int j = 0; j < NT; j++) big = fmaxf(fmaxf(big, fmaxf(acc[i][j][0], acc[i][j][1])), fmaxf(acc[i][j][2], acc[i][j][3]));
+            big = fmaxf(big, __shfl_xor(big, 16, 64));
+            big = fmaxf(big, __shfl_xor(big, 32, 64));
+            const float z = big == -INFINITY ? 0.f : big;
+#pragma unroll
+            for (int j = 0; j < NT; j++) s += (exp_of(acc[i][j][0] - z) + exp_of(acc[i][j][1] - z)) + (exp_of(acc[i][j][2] - z) + exp_of(acc[i][j][3] - z));
+            s += __shfl_xor(s, 16, 64);
+            s += __shfl_xor(s, 32, 64);
+            if (lc == 0 && row[i] < left) {
+                const int64_t at = (int64_t)column_tile * g.M + m;
+                g.part_max[at] = big, g.part_sum[at] = s;
+            }
+        }
+    }
 }
 
-// Three waves per SIMD, three workgroups on a CU: the products with the loss's gradient are held to 168 registers for it
-// (174 without the bound; one is spilled, outside the loop).
-//
-// BM x BN tile of four waves (two by two), each wave (BM/2) x (BN/2) in 16 x 16 MFMA tiles.
-template <bool AKC, bool BKC, int BM, int BN, int MODE>
-__global__ __launch_bounds__(kThreads, 3) void k_gemm(GemmArgs g) {
-    constexpr int WM = BM / 2, WN = BN / 2, MT = WM / 16, NT = WN / 16;
-    __shared__ Planes<BM> La;
-    __shared__ Planes<BN> Lb;
+// A workgroup: 64 MT rows x 16 NT columns, a wave 16 MT rows of them and all columns; B's rows are staged step by step, in two
+// alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 60 us (one 128 x 128 tile with both
+// operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6.
+template <class S, bool AKC, bool BKC, int MT, int NT, int MODE>
+__global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
+    constexpr int BM = 64 * MT, WM = 16 * MT, BN = 16 * NT;
+    typedef Planes<S::kPlanes, BN> Stage;
+    typedef Direct<AKC, MT, MODE == kGrad> OpA;
+    typedef Staged<BKC, BN> OpB;
+    typedef typename S::frag frag;
+    constexpr size_t kShared = 2 * sizeof(Stage);
+    static_assert(sizeof(v4f) * 8 * BN <= kShared, "fp32 of a step fits");
+    __shared__ __align__(16) char shared[kShared];
+    __shared__ __align__(16) int exponents[BN];
+    __shared__ __align__(16) float biases[BN];
+    // a wave that changed scales of B's rows for step k0 leaves k0 and what those rows' results so far are multiplied with
+    __shared__ __align__(16) int changed[2][4];
+    __shared__ __align__(16) float change_b[S::kScaled ? 2 : 1][S::kScaled ? BN : 4];
+    __shared__ float change_a[S::kScaled ? 4 : 1][WM];
     __shared__ int odd_waves[4];
+    __shared__ NllToken toks[MODE == kGrad && !AKC ? 4 : 1][MODE == kGrad && !AKC ? kBK : 1];
+    Stage *const L = reinterpret_cast<Stage *>(shared);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    const int wm = (wave % 2) * WM, wn = (wave / 2) * WN;
     // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
     // rows of A, through that XCD's L2)
     const int total = g.tm * g.tn, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
     const int id = xcd * each + min(xcd, rest) + blockIdx.x / 8;
-    const int m0 = (id / g.tn) * BM, n0 = (id % g.tn) * BN;
+    const int m0 = (id / g.tn) * BM + wave * WM, n0 = (id % g.tn) * BN;
     const int kb = blockIdx.y * g.ks, ke = min(g.K, kb + g.ks);
-    Operand<AKC, BM, MODE == kGrad> a;
-    Operand<BKC, BN, false> b;
-    a.init(tid, g.lda, m0, g.M, g.nll);
-    b.init(tid, g.ldb, n0, g.N, g.nll);
     const float *Ap = AKC ? g.A + (int64_t)m0 * g.lda : g.A + m0;
     const float *Bp = BKC ? g.B + (int64_t)n0 * g.ldb : g.B + n0;
     const int ml = g.M - m0, nl = g.N - n0;
-    constexpr int CV = AKC ? 1 : Operand<AKC, BM, MODE == kGrad>::VEC;
-    float csum[CV];
-#pragma unroll
-    for (int c = 0; c < CV; c++) csum[c] = 0.f;
+    const int lr = lane % 16, lc = lane / 16;
+    // unit_of(16 j + lr, lc) of even and odd j
+    const int unit[2] = {lc * BN + unit_of(lr, lc), lc * BN + unit_of(16 + lr, lc) - 16};
+    OpA a;
+    OpB b;
+    a.init(lane, m0, g.M, g.nll);
+    b.init(tid);
+    a.tok = toks[MODE == kGrad && !AKC ? wave : 0];
+    const auto load = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0) {
+        a.load(x, Ap, g.lda, ml, k0, ke, g.nll, g.K, lane);
+        b.load(y, Bp, g.ldb, nl, k0, ke);
+    };
+    const auto aim = [&](int k0) { a.aim(g.lda, k0, ke), b.aim(g.ldb, k0, ke); };
+    float csum[MT];
     const bool sums = !AKC && g.colsum && n0 == 0;
     v4f acc[MT][NT];
 #pragma unroll
-    for (int i = 0; i < MT; i++)
+    for (int i = 0; i < MT; i++) {
+        a.s[i].none();
+        csum[i] = 0.f;
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int lr = lane % 16, lc = lane / 16, lu = unit_of(lr, lc);
-    a.load(Ap, g.lda, ml, tid, kb, ke, g.nll);
-    b.load(Bp, g.ldb, nl, tid, kb, ke, g.nll);
-    for (int k0 = kb; k0 < ke; k0 += kBK) {
-        a.finish(tid, m0, k0, ke, g.nll);
-        b.finish(tid, n0, k0, ke, g.nll);
-        if constexpr (!AKC) {
-            if (sums)
+    }
 #pragma unroll
-                for (int c = 0; c < CV; c++)
-#pragma unroll
-                    for (int j = 0; j < 8; j++) csum[c] += a.x[0][8 * c + j];
+    for (int t = 0; t < OpB::kUnits; t++) b.s[t].none();
+    if (tid < 8) changed[tid / 4][tid % 4] = -1;
+
+    typename OpA::Raw ra[2];
+    typename OpB::Raw rb[2];
+    bool change = false;      // of scales of A's rows
+    v4u fa[2][MT][S::kPlanes];
+    float part_sum[MT];       // of a step's elements of A's rows
+    const auto split_a = [&](int i, int j, const typename OpA::Raw &x, v4u (*f)[S::kPlanes], bool whole, int k0) {
+        float v[8];
+        v[2 * j] = a.element(x, i, 2 * j, whole, m0, k0, ke), v[2 * j + 1] = a.element(x, i, 2 * j + 1, whole, m0, k0, ke);
+        if constexpr (!AKC) part_sum[i] = (j ? part_sum[i] : 0.f) + (v[2 * j] + v[2 * j + 1]);
+        else part_sum[i] = 0.f;
+        split_pair<S>(v, j, a.s[i].s, f[i]);
+    };
+    // Pair q of the 4 (units + MT) pairs of a step's split: B's units first, each to LDS when it is whole, then A's tiles
+    v4u part[S::kPlanes];
+    constexpr int kPairs = 4 * (OpB::kUnits + MT);
+    const auto split = [&](int q, const typename OpA::Raw &x, const typename OpB::Raw &y, v4u (*f)[S::kPlanes], Stage &to, int k0) {
+        if (q < 4 * OpB::kUnits) {
+            split_pair<S>(y.x[q / 4], q % 4, b.s[q / 4].s, part);
+            if (q % 4 == 3) b.store(to, q / 4, part);
+            return;
         }
-        a.store(La, tid);
-        b.store(Lb, tid);
-        lds_barrier();
-        if (k0 + kBK < ke) {
-            a.load(Ap, g.lda, ml, tid, k0 + kBK, ke, g.nll);
-            b.load(Bp, g.ldb, nl, tid, k0 + kBK, ke, g.nll);
+        const int j = (q - 4 * OpB::kUnits) / MT, i = q % MT;
+        split_a(i, j, x, f, false, k0);
+    };
+    // once more where split() left something out
+    const auto complete = [&](const typename OpA::Raw &x, v4u (*f)[S::kPlanes], int k0) {
+        if constexpr (MODE == kGrad)
+            if (a.rare(x, m0, k0, ke))
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) split_a(i, j, x, f, true, k0);
+#pragma unroll
+        for (int i = 0; i < MT; i++) csum[i] += part_sum[i];
+    };
+    // What a step's split needs: zeros beyond K, and (parity: the step's) scales that its elements fit
+    const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) {
+        a.hand_over(x, lane);
+        if (ke % 4 && k0 + kBK > ke) a.cut(x, k0, ke), b.cut(y, k0, ke);
+        if constexpr (S::kScaled) {
+            float ma[MT], mb[OpB::kUnits];
+            bool beyond_a = false, beyond_b = false;
+#pragma unroll
+            for (int i = 0; i < MT; i++) ma[i] = abs_max8(x.x[i], 0.f), beyond_a |= ma[i] > a.s[i].limit;
+#pragma unroll
+            for (int t = 0; t < OpB::kUnits; t++) mb[t] = abs_max8(y.x[t], 0.f), beyond_b |= mb[t] > b.s[t].limit;
+            if (__any(beyond_a | beyond_b)) {
+                change = true;
+#pragma unroll
+                for (int i = 0; i < MT; i++) change_a[wave][OpA::row_of(i, lr)] = a.s[i].fit(OpA::of_row(ma[i]));
+#pragma unroll
+                for (int t = 0; t < OpB::kUnits; t++) change_b[parity][b.row_of(t)] = b.s[t].fit(OpB::of_row(mb[t]));
+                if (lane == 0) changed[parity][wave] = k0;
+            }
         }
-        // the products in an order in which three fragment sets are live at a time (six in the order of their size:
-        // 178 registers instead of 162, two workgroups on a CU instead of three)
-        bf8 a1[MT], a2[MT], b1[NT], b2[NT];
-        const auto read_a = [&](bf8 *d, int p) {
+    };
+    // results so far to the scales of step k0
+    const auto follow = [&](int k0, int parity) {
+        if constexpr (S::kScaled) {
+            const int4 w = *reinterpret_cast<const int4 *>(changed[parity]);
+            if (__builtin_amdgcn_readfirstlane(w.x == k0 | w.y == k0 | w.z == k0 | w.w == k0)) {
+                const bool of[4] = {w.x == k0, w.y == k0, w.z == k0, w.w == k0};
 #pragma unroll
-            for (int i = 0; i < MT; i++) d[i] = __builtin_bit_cast(bf8, La.u[p][lc][wm + 16 * i + lu]);
+                for (int j = 0; j < NT; j++)
+                    if (of[OpB::owner(j)])
+#pragma unroll
+                        for (int i = 0; i < MT; i++) acc[i][j] *= *reinterpret_cast<const v4f *>(change_b[parity] + 16 * j + 4 * lc);
+            }
+            if (change) {
+                change = false;
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] *= change_a[wave][OpA::row_of(i, lr)];
+            }
+        }
+    };
+    aim(kb);
+    load(ra[0], rb[0], kb);
+    aim(kb + kBK);
+    load(ra[1], rb[1], kb + kBK);
+    if constexpr (S::kScaled) lds_barrier();      // `changed` is cleared
+    prepare(ra[0], rb[0], kb, 0);
+#pragma unroll
+    for (int q = 0; q < kPairs; q++) split(q, ra[0], rb[0], fa[0], L[0], kb);
+    complete(ra[0], fa[0], kb);
+    lds_barrier();
+    // One step: the products of k0's parts, beside the split of k0 + kBK's elements and the loads of k0 + 2 kBK's.
+    const auto step = [&](auto parity, int k0) {
+        constexpr int p = decltype(parity)::value;
+        if (k0 + 3 * kBK > ke) aim(k0 + 2 * kBK);
+        load(ra[p], rb[p], k0 + 2 * kBK);
+        follow(k0, p);
+        prepare(ra[p ^ 1], rb[p ^ 1], k0 + kBK, p ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        frag fb[2][S::kPlanes];
+        const auto read = [&](int j) {
+#pragma unroll
+            for (int q = 0; q < S::kPlanes; q++) fb[j % 2][q] = __builtin_bit_cast(frag, L[p].u[q][0][unit[j % 2] + 16 * j]);
         };
-        const auto read_b = [&](bf8 *d, int p) {
+        read(0);
 #pragma unroll
-            for (int j = 0; j < NT; j++) d[j] = __builtin_bit_cast(bf8, Lb.u[p][lc][wn + 16 * j + lu]);
-        };
-        const auto products = [&](const bf8 *x, const bf8 *y) {
+        for (int j = 0; j < NT; j++) {
+            if (j + 1 < NT) read(j + 1);
 #pragma unroll
-            for (int i = 0; i < MT; i++)
+            for (int q = j * kPairs / NT; q < (j + 1) * kPairs / NT; q++) split(q, ra[p ^ 1], rb[p ^ 1], fa[p ^ 1], L[p ^ 1], k0 + kBK);
 #pragma unroll
-                for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
-        };
-        read_a(a1, 2), read_b(b1, 0), products(a1, b1);      // l h'
-        read_a(a2, 1), products(a2, b1);                     // m h'
-        read_b(b2, 1), products(a2, b2);                     // m m'
-        read_a(a1, 0), products(a1, b2);                     // h m'
-        products(a1, b1);                                    // h h'
-        read_b(b2, 2), products(a1, b2);                     // h l'
+            for (int q = 0; q < S::kProducts; q++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[i][j] = S::mma(fb[j % 2][S::kOrder[q][1]], __builtin_bit_cast(frag, fa[p][i][S::kOrder[q][0]]), acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        complete(ra[p ^ 1], fa[p ^ 1], k0 + kBK);
         lds_barrier();
+    };
+    for (int k0 = kb; k0 < ke; k0 += 2 * kBK) {      // an odd number of steps: the last one's elements are zeros
+        step(std::integral_constant<int, 0>(), k0);
+        step(std::integral_constant<int, 1>(), k0 + kBK);
     }
 
-    // An element that is not finite (0 times it is NaN): the tile once more from the fp32 operands
+    // An element that is not finite (0 times it is NaN)
     float odd = 0.f;
 #pragma unroll
     for (int i = 0; i < MT; i++)
@@ -394,117 +739,266 @@ __global__ __launch_bounds__(kThreads, 3) void k_gemm(GemmArgs g) {
     if (lane == 0) odd_waves[wave] = wave_odd;
     __syncthreads();
     if (odd_waves[0] | odd_waves[1] | odd_waves[2] | odd_waves[3]) {
+        // the tile once more from the fp32 operands
 #pragma unroll
-        for (int i = 0; i < MT; i++)
+        for (int i = 0; i < MT; i++) {
+            a.s[i].one();
 #pragma unroll
             for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        for (int k0 = kb; k0 < ke; k0 += kBK) {
-            a.load(Ap, g.lda, ml, tid, k0, ke, g.nll);
-            b.load(Bp, g.ldb, nl, tid, k0, ke, g.nll);
-            a.finish(tid, m0, k0, ke, g.nll);
-            b.finish(tid, n0, k0, ke, g.nll);
-            a.store_plain(La, tid);
-            b.store_plain(Lb, tid);
-            __syncthreads();
-            // lane (lc, lr) holds four consecutive k of row lr; register r of both operands is an instruction's four k
+        }
+#pragma unroll
+        for (int t = 0; t < OpB::kUnits; t++) b.s[t].one();
+        v4f *const plain = reinterpret_cast<v4f *>(shared);
 #pragma unroll 1
-            for (int s = 0; s < kBK / 4; s += 4) {
-                v4f y[NT];
+        for (int k0 = kb; k0 < ke; k0 += kBK) {
+            aim(k0);
+            load(ra[0], rb[0], k0);
+            a.hand_over(ra[0], lane);
+            if (ke % 4 && k0 + kBK > ke) a.cut(ra[0], k0, ke), b.cut(rb[0], k0, ke);
 #pragma unroll
-                for (int j = 0; j < NT; j++) y[j] = b.plain(Lb)[(s + lc) * BN + wn + 16 * j + lr];
+            for (int i = 0; i < MT; i++)
 #pragma unroll
-                for (int i = 0; i < MT; i++) {
-                    const v4f x = a.plain(La)[(s + lc) * BM + wm + 16 * i + lr];
+                for (int e = 0; e < 8; e++) ra[0].x[i][e] = a.element(ra[0], i, e, true, m0, k0, ke);
+            b.store_plain(plain, rb[0]);
+            __syncthreads();
 #pragma unroll
-                    for (int r = 0; r < 4; r++)
+            for (int h = 0; h < 2; h++)
 #pragma unroll
-                        for (int j = 0; j < NT; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[r], y[j][r], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NT; j++) {
+                    const v4f y = plain[(2 * lc + h) * BN + 16 * j + lr];
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+#pragma unroll
+                        for (int i = 0; i < MT; i++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[e], ra[0].x[i][4 * h + e], acc[i][j], 0, 0, 0);
                 }
-            }
             __syncthreads();
         }
     }
 
-    // acc[i][j][r] = C[m0 + wm + 16 i + 4 lc + r][n0 + wn + 16 j + lr]
     if constexpr (!AKC) {
-        if (sums) {      // the threads of a row pair's four k-chunks
-            float *s = reinterpret_cast<float *>(&La);
-            using Op = Operand<AKC, BM, MODE == kGrad>;
+        if (sums)      // the four k-chunks of a row
 #pragma unroll
-            for (int c = 0; c < CV; c++) s[Op::chunk_of(tid) * BM + Op::row_of(tid) + c] = csum[c];
-            __syncthreads();
-            for (int r = tid; r < min(BM, ml); r += kThreads)
-                g.colsum[(int64_t)blockIdx.y * g.M + m0 + r] = (s[r] + s[BM + r]) + (s[2 * BM + r] + s[3 * BM + r]);
-        }
-    }
-    // A wave turns its rows round through LDS (its own: no barrier), 16 at a time, so that they leave, and the
-    // residual and the gate arrive, 16 bytes per lane: 4-byte accesses in the MFMA layout, 64-byte pieces of rows, cost
-    // 112 us where this costs 90 at 32768 x 1024, K = 256.
-    constexpr int kPitch = WN + 4;
-    static_assert(4 * 16 * kPitch <= (int)(sizeof(La) / 4), "four waves' strips fit the first operand's planes");
-    float *const strip = reinterpret_cast<float *>(&La) + wave * 16 * kPitch;
-    constexpr int kLanes = WN / 4, kRows = 64 / kLanes;      // lanes per row, rows per access
-    const int c4 = (lane % kLanes) * 4, n = n0 + wn + c4;
-    const bool vec = g.vec && n + 3 < g.N;
-    if constexpr (!AKC) __syncthreads();      // the column sums' reads of the same memory
-    float bias[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) bias[e] = g.epi.bias && n + e < g.N && (gridDim.y == 1) ? g.epi.bias[n + e] : 0.f;
-    float *const C = g.C + blockIdx.y * g.part;
-    const bool one = gridDim.y == 1;
-    float *const sums_of = reinterpret_cast<float *>(&Lb);       // kLse: [2][column half][row]
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-#pragma unroll
-        for (int j = 0; j < NT; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) strip[(4 * lc + r) * kPitch + 16 * j + lr] = acc[i][j][r];
-        wave_lds_order();
-#pragma unroll
-        for (int q = 0; q < 16 / kRows; q++) {
-            const int row = kRows * q + lane / kLanes, m = m0 + wm + 16 * i + row;
-            float4 v = *reinterpret_cast<const float4 *>(strip + row * kPitch + c4);
-            v.x += bias[0], v.y += bias[1], v.z += bias[2], v.w += bias[3];
-            if constexpr (MODE == kLse) {
-                lse_of_row<kLanes>(v, n, g.N, lane, sums_of, (wave / 2) * BM + wm + 16 * i + row, 2 * BM);
-                if (g.hit && m < g.M) {
-                    const int at = (int)g.nll.target[m] - n;
-                    if (at >= 0 && at < 4 && n + at < g.N) g.hit[m] = at == 0 ? v.x : at == 1 ? v.y : at == 2 ? v.z : v.w;
-                }
-                if (!g.C) continue;
+            for (int i = 0; i < MT; i++) {
+                csum[i] += __shfl_xor(csum[i], 16, 64);
+                csum[i] += __shfl_xor(csum[i], 32, 64);
+                const int row = OpA::row_of(i, lr);
+                if (lc == 0 && row < ml) g.colsum[(int64_t)blockIdx.y * g.M + m0 + row] = csum[i];
             }
-            if (m >= g.M) continue;
-            const int64_t at = (int64_t)m * g.ldc + n;
-            if (vec) {
-                if (one) {
-                    if (g.epi.relu) v = make_float4(relu(v.x), relu(v.y), relu(v.z), relu(v.w));
-                    if (g.epi.residual) {
-                        const float4 y = *reinterpret_cast<const float4 *>(g.epi.residual + at);
-                        v.x += y.x, v.y += y.y, v.z += y.z, v.w += y.w;
-                    }
-                    if (g.epi.gate) {
-                        const float4 y = *reinterpret_cast<const float4 *>(g.epi.gate + at);
-                        v = make_float4(gated(y.x, v.x), gated(y.y, v.y), gated(y.z, v.z), gated(y.w, v.w));
-                    }
-                }
-                *reinterpret_cast<float4 *>(C + at) = v;
+    }
+    if (b.c == 0)
+#pragma unroll
+        for (int t = 0; t < OpB::kUnits; t++) exponents[b.row_of(t)] = b.s[t].exponent();
+    if (tid < BN) biases[tid] = g.epi.bias && gridDim.y == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
+    __syncthreads();
+    int row[MT];
+    int ea[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) row[i] = OpA::row_of(i, lr), ea[i] = a.s[i].exponent();
+    finish<S::kScaled, MT, NT, MODE>(g, acc, row, m0, WM, n0, lc, ea, Columns{exponents, biases}, id % g.tn);
+}
+
+// Products with K up to 32 KS: a workgroup keeps 16 NT of B's rows, split, in LDS and its eight waves go over blocks of 32
+// rows of A, each by itself, without barriers: one wave's results leave while others multiply.  32768 x 1024, K = 256 with bias and
+// ReLU 64 us (staged 87; memory alone 35), 24576 x 2048, K = 128 with a gate 100 us (127; 87).
+template <bool BKC, int KS, int NT, int MODE>
+__global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, int per) {
+    typedef Half2 S;
+    typedef S::frag frag;
+    constexpr int BN = 16 * NT, MT = 2, kBlock = 16 * MT, kWaves = 8;
+    typedef Direct<true, MT, false> OpA;
+    __shared__ Planes<S::kPlanes, BN> L[KS];
+    __shared__ unsigned top[BN];                       // the largest magnitude of each of B's rows
+    __shared__ __align__(16) int exponents[2][BN];     // of the scales, zeros
+    __shared__ __align__(16) float biases[BN];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
+    const int id = xcd * each + min(xcd, rest) + blockIdx.x / 8;
+    const int n0 = (id % g.tn) * BN, nl = g.N - n0, K = g.K;
+    const float *const Bp = BKC ? g.B + (int64_t)n0 * g.ldb : g.B + n0;
+    if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
+    __syncthreads();
+    {
+        constexpr int VEC = BKC ? 1 : 2, kTasks = KS * 4 * BN / VEC / (2 * kThreads);
+        static_assert(kTasks >= 1, "a task per thread");
+        float x[kTasks][VEC][8];
+        int row[kTasks], step[kTasks], c[kTasks];
+        const v4i rs = buffer_of(Bp, BKC ? (int64_t)(min(nl, BN) - 1) * g.ldb + K : (int64_t)(K - 1) * g.ldb + nl);
+#pragma unroll
+        for (int t = 0; t < kTasks; t++) {
+            const int task = tid + t * 2 * kThreads;
+            if constexpr (BKC) {
+                c[t] = task % 4, row[t] = task / 4 % BN, step[t] = task / (4 * BN);
+                const int k = 32 * step[t] + 4 * c[t];
+                const unsigned at = (unsigned)(row[t] * g.ldb + k) * 4;
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)(k < K ? at : kOut), 0, 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)(k + 16 < K ? at + 64 : kOut), 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[t][0][j] = a[j], x[t][0][4 + j] = b[j];
             } else {
-                const float w[4] = {v.x, v.y, v.z, v.w};
+                row[t] = task % (BN / 2) * 2, c[t] = task / (BN / 2) % 4, step[t] = task / (2 * BN);
+                const unsigned at = (unsigned)((32 * step[t] + 4 * c[t]) * g.ldb + row[t]) * 4;
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (n + e < g.N) C[at + e] = one ? apply(g.epi, w[e], at + e) : w[e];
+                for (int e = 0; e < 8; e++) {
+                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)(row[t] < nl ? at + (unsigned)(k_of(0, e) * g.ldb) * 4 : kOut), 0, 0);
+                    x[t][0][e] = a[0], x[t][1][e] = row[t] + 1 < nl ? a[1] : 0.f;
+                }
             }
         }
-        wave_lds_order();
-    }
-    if constexpr (MODE == kLse) {
+#pragma unroll
+        for (int t = 0; t < kTasks; t++)
+#pragma unroll
+            for (int v = 0; v < VEC; v++) {
+                if constexpr (BKC)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) x[t][v][e] = 32 * step[t] + k_of(c[t], e) < K ? x[t][v][e] : 0.f;
+                float m = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) m = x[t][v][e] != x[t][v][e] ? INFINITY : fmaxf(m, fabsf(x[t][v][e]));
+                atomicMax(&top[row[t] + v], __float_as_uint(m));
+            }
         __syncthreads();
-        for (int row = tid; row < min(BM, ml); row += kThreads) {
-            const float m1 = sums_of[row], m2 = sums_of[BM + row], mx = fmaxf(m1, m2);
-            const int64_t at = (int64_t)(id % g.tn) * g.M + m0 + row;
-            g.part_max[at] = mx;
-            g.part_sum[at] = sums_of[2 * BM + row] * to_max(m1, mx) + sums_of[3 * BM + row] * to_max(m2, mx);
+#pragma unroll
+        for (int t = 0; t < kTasks; t++)
+#pragma unroll
+            for (int v = 0; v < VEC; v++) {
+                const unsigned m = top[row[t] + v];
+                Scale s;
+                s.set(__uint_as_float(m));
+                v4u d[S::kPlanes];
+#pragma unroll
+                for (int j = 0; j < 4; j++) split_pair<S>(x[t][v], j, s.s, d);
+#pragma unroll
+                for (int p = 0; p < S::kPlanes; p++) L[step[t]].u[p][c[t]][unit_of(row[t] + v, c[t])] = d[p];
+                if (step[t] == 0 && c[t] == 0) exponents[0][row[t] + v] = s.exponent();
+            }
+    }
+    __syncthreads();
+
+    const int lr = lane % 16, lc = lane / 16;
+    const int unit[2] = {lc * BN + unit_of(lr, lc), lc * BN + unit_of(16 + lr, lc) - 16};
+    const int end = min((id / g.tn + 1) * per, (g.M + kBlock - 1) / kBlock);
+    int block = id / g.tn * per + wave;
+    if (block >= end) return;
+    OpA a;
+    a.init(lane, 0, 0, g.nll);
+    const bool ragged = K < 32 * KS;
+    const auto load = [&](OpA::Raw &x, int blk, int k0) {
+        if (ragged) a.aim(g.lda, k0, K);
+        a.load(x, g.A + (int64_t)blk * kBlock * g.lda, g.lda, blk < end ? g.M - blk * kBlock : 0, k0, K, g.nll, 0, lane);
+    };
+    OpA::Raw ra[2];
+    v4u fa[2][MT][S::kPlanes];
+    v4f acc[MT][NT];
+    float change[MT];
+    bool changed = false;
+    // zeros beyond K, and scales that the step's elements fit
+    const auto prepare = [&](OpA::Raw &x, int k0) {
+        if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
+        float m[MT];
+        bool beyond = false;
+#pragma unroll
+        for (int i = 0; i < MT; i++) m[i] = abs_max8(x.x[i], 0.f), beyond |= m[i] > a.s[i].limit;
+        if (__any(beyond)) {
+            changed = true;
+#pragma unroll
+            for (int i = 0; i < MT; i++) change[i] = a.s[i].fit(OpA::of_row(m[i]));
         }
+    };
+    const auto split = [&](int q, const OpA::Raw &x, v4u (*f)[S::kPlanes]) { split_pair<S>(x.x[q % MT], q / MT, a.s[q % MT].s, f[q % MT]); };
+    const auto clear = [&] {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+    a.aim(g.lda, 0, 32 * KS);
+    a.s[0].none(), a.s[1].none();
+    load(ra[0], block, 0);
+    load(ra[1], block, kBK);
+    prepare(ra[0], 0);
+#pragma unroll
+    for (int q = 0; q < 4 * MT; q++) split(q, ra[0], fa[0]);
+    for (; block < end; block += kWaves) {
+        clear();
+        int ea[MT];
+        // the products of step s, beside the split of step s + 1 and the loads of step s + 2, which may be the next block's
+        const auto step = [&](auto parity, int s) {
+            constexpr int p = decltype(parity)::value;
+            load(ra[p], s + 2 < KS ? block : block + kWaves, (s + 2) % KS * kBK);
+            if (changed && s > 0) {      // results so far to the scales of step s
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) acc[i][j] *= change[i];
+            }
+            changed = false;
+            if (s + 1 == KS) {
+#pragma unroll
+                for (int i = 0; i < MT; i++) ea[i] = a.s[i].exponent(), a.s[i].none();
+            }
+            prepare(ra[p ^ 1], (s + 1) % KS * kBK);
+            __builtin_amdgcn_sched_barrier(0);
+            frag fb[2][S::kPlanes];
+            const auto read = [&](int j) {
+#pragma unroll
+                for (int q = 0; q < S::kPlanes; q++) fb[j % 2][q] = __builtin_bit_cast(frag, L[s].u[q][0][unit[j % 2] + 16 * j]);
+            };
+            read(0);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                if (j + 1 < NT) read(j + 1);
+#pragma unroll
+                for (int q = j * 4 * MT / NT; q < (j + 1) * 4 * MT / NT; q++) split(q, ra[p ^ 1], fa[p ^ 1]);
+#pragma unroll
+                for (int q = 0; q < S::kProducts; q++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[i][j] = S::mma(fb[j % 2][S::kOrder[q][1]], __builtin_bit_cast(frag, fa[p][i][S::kOrder[q][0]]), acc[i][j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+#pragma unroll 1
+        for (int s = 0; s < KS; s += 2) {
+            step(std::integral_constant<int, 0>(), s);
+            step(std::integral_constant<int, 1>(), s + 1);
+        }
+        const auto odd = [&] {
+            float x = 0.f;
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) x = fmaf(acc[i][j][r], 0.f, x);
+            return (bool)__any(x != 0.f);
+        };
+        const int *eb = exponents[0];
+        if (odd()) {
+            // an element that is not finite (0 times it is NaN): the block once more from the fp32 operands
+            OpA::Raw x;
+            clear();
+            eb = exponents[1];
+            ea[0] = ea[1] = 0;
+#pragma unroll 1
+            for (int k0 = 0; k0 < K; k0 += kBK) {
+                load(x, block, k0);
+                if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++) {
+                        const int n = 16 * j + lr, k = k0 + k_of(lc, e);
+                        const float y = n < nl && k < K ? Bp[BKC ? n * g.ldb + k : k * g.ldb + n] : 0.f;
+#pragma unroll
+                        for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, x.x[i][e], acc[i][j], 0, 0, 0);
+                    }
+            }
+        }
+        int row[MT];
+#pragma unroll
+        for (int i = 0; i < MT; i++) row[i] = OpA::row_of(i, lr);
+        finish<true, MT, NT, MODE>(g, acc, row, block * kBlock, kBlock, n0, lc, ea, Columns{eb, biases}, id % g.tn);
     }
 }
 
@@ -559,39 +1053,84 @@ __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restric
         for (int i = 0; at + i < total; i++) C[at + i] = v[i];
 }
 
+// Which kernel: the one with B's rows kept in LDS (`steps` of k, 4 or 8; `per` blocks of 32 rows to a workgroup, `groups` of
+// them), or the staged one with tiles of bm x bn and k in `ranges` of ks.
 struct Plan {
-    bool wide;           // 128 x 128 tiles, else 64 x 64
-    int tm, tn, ranges, ks;
+    int steps, per, groups;
+    int bm, bn, tm, tn, ranges, ks;
 };
 
-// 128 x 128 tiles where they fill the chip (two workgroups on each of 256 CUs) or where k can be cut into ranges
-// until they do; the partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k.
-// Without ranges to cut, fewer tiles than CUs: 64 x 64.
+// Kept rows of B, from 128 to 256 k and where workgroups of 256 rows x 128 columns are enough for most CUs: 32768 x 1024,
+// K = 256 64 us (staged 87, both with bias and ReLU), 24576 x 2048, K = 128 with a gate 100 us (staged 127), 8192 x 776, K = 256
+// (224 workgroups) 19 us (22); 16384 x 256, K = 256 (128 workgroups) 19 us (16), 8192 x 392, K = 128 (128) 13 us (11).
+constexpr int kResidentTiles = 200;
+// Half2's error is the smaller one from here on; below, Bf16x3's (K = 64: 1.08e-7 and 1.06e-7, K = 32: 8.8e-8 and 6.3e-8).
+constexpr int kHalfK = 128;
+
+// Staged: 128 x 128 tiles where, with k cut into ranges, they are three for two CUs; else 128 x 64 if those are; else 64 x 64.
+// 32768 x 256, K = 1024 (512 tiles) 60 us, 77, 80; 16384 x 256, K = 1024 (256 tiles) 47, 41, 48 us; 2381 x 1024, K = 256
+// (152, 304, 608 tiles) 16.2, 15.9, 14.3 us; 300 x 256, K = 256 13.9, 10.3, 8.6 us.
+// The partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k.
 Plan plan_of(int M, int N, int K, bool may_cut) {
-    Plan p;
-    const auto tiles = [&](int b) { return (int64_t)((M + b - 1) / b) * ((N + b - 1) / b); };
-    p.wide = tiles(128) >= 256 || (may_cut && tiles(128) * (K / 256) >= 256);
-    const int b = p.wide ? 128 : 64;
-    p.tm = (M + b - 1) / b;
-    p.tn = (N + b - 1) / b;
-    int64_t ranges = 1;
-    if (may_cut) {
-        ranges = 512 / (tiles(b));
-        if (ranges > K / 256) ranges = K / 256;
-        if (ranges < 1) ranges = 1;
+    Plan p{};
+    const auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    const auto ranges = [&](int64_t tiles) { return may_cut ? std::max<int64_t>(1, std::min<int64_t>(512 / tiles, K / 256)) : 1; };
+    const int blocks = (M + 31) / 32;
+    if (K >= kHalfK && K <= 256 && tiles(256, 128) >= kResidentTiles) {
+        p.steps = K <= 128 ? 4 : 8;
+        // the most even division of the blocks over 256 CUs, a workgroup's start (its rows of B) as long as a wave's block
+        double best = 1e30;
+        const int tn = (N + 127) / 128, most = std::min((blocks + 7) / 8, std::max(1, 1024 / tn));
+        for (int n = 1; n <= most; n++) {
+            const int per = (blocks + n - 1) / n;
+            const double cost = (double)(((int64_t)tn * n + 255) / 256) * ((per + 7) / 8 + 1);
+            if (cost < best) best = cost, p.per = per, p.groups = (blocks + per - 1) / per;
+        }
     }
-    p.ks = (int)((K + ranges - 1) / ranges + kBK - 1) / kBK * kBK;
+    p.bm = p.bn = 128;
+    const int64_t wide = tiles(128, 128);
+    if (wide * ranges(wide) < 384) {
+        p.bn = 64;
+        if (tiles(128, 64) < 384) p.bm = 64;
+    }
+    p.tm = (M + p.bm - 1) / p.bm;
+    p.tn = (N + p.bn - 1) / p.bn;
+    const int64_t n = ranges(tiles(p.bm, p.bn));
+    p.ks = (int)((K + n - 1) / n + 2 * kBK - 1) / (2 * kBK) * (2 * kBK);
     p.ranges = (K + p.ks - 1) / p.ks;
     return p;
 }
 
-template <bool AKC, bool BKC, int MODE>
-void launch(const GemmArgs &g, const Plan &p, hipStream_t s) {
+template <class S, bool AKC, bool BKC, int MODE>
+void launch_staged(const GemmArgs &g, const Plan &p, hipStream_t s) {
     const dim3 grid((unsigned)(p.tm * p.tn), (unsigned)p.ranges);
-    if (p.wide) hipLaunchKernelGGL((k_gemm<AKC, BKC, 128, 128, MODE>), grid, dim3(kThreads), 0, s, g);
-    else hipLaunchKernelGGL((k_gemm<AKC, BKC, 64, 64, MODE>), grid, dim3(kThreads), 0, s, g);
+    if (p.bm == 64) hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 1, 4, MODE>), grid, dim3(kThreads), 0, s, g);
+    else if (p.bn == 64) hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 2, 4, MODE>), grid, dim3(kThreads), 0, s, g);
+    else hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 2, 8, MODE>), grid, dim3(kThreads), 0, s, g);
 }
 
+// The loss gradient's products stay with Bf16x3: a word's probabilities over the tokens, or a token's over the words, are
+// held to their own size, however far below the largest.
+template <bool AKC, bool BKC, int MODE>
+void launch(GemmArgs g, const Plan &p, hipStream_t s) {
+    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
+    if constexpr (MODE == kGrad) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
+    else if (g.K < kHalfK) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
+    else {
+        if constexpr (AKC) {
+            if (p.steps) {
+                g.tn = (g.N + 127) / 128;
+                const dim3 grid((unsigned)(g.tn * p.groups)), block(2 * kThreads);
+                if (p.steps == 4) hipLaunchKernelGGL((k_gemm_resident<BKC, 4, 8, MODE>), grid, block, 0, s, g, p.per);
+                else hipLaunchKernelGGL((k_gemm_resident<BKC, 8, 8, MODE>), grid, block, 0, s, g, p.per);
+                return;
+            }
+        }
+        launch_staged<Half2, AKC, BKC, MODE>(g, p, s);
+    }
+}
+
+constexpr int kMaxPitch = 1 << 22;      // of 64 rows that 32-bit offsets reach
 bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // a partial result, in whole 16-byte groups
@@ -610,12 +1149,11 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
     if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target, nll->vocab};
     const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace));
-    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
     const bool cut = p.ranges > 1;
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
     g.part = part_of(M, N);
-    g.vec = g.ldc % 4 == 0 && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
+    g.vec = g.ldc % 4 == 0 && N % 4 == 0 && g.ldc <= kMaxPitch && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
     float *const col = cut ? workspace + p.ranges * g.part : epi.colsum;
     g.colsum = layout == FWP_MM_TN && epi.colsum ? col : nullptr;
     if (layout == FWP_MM_NT) launch<true, true, kPlain>(g, p, s);
@@ -676,14 +1214,14 @@ int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *ta
     g.epi.bias = bias;
     g.nll.target = target;
     const Plan p = plan_of(rows, vocab, dim, false);
-    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
+    const int tn = p.steps ? (vocab + 127) / 128 : p.tn;
     g.part_max = workspace;
-    g.part_sum = workspace + (int64_t)p.tn * rows;
-    g.hit = logits ? nullptr : g.part_sum + (int64_t)p.tn * rows;
-    g.vec = vocab % 4 == 0 && aligned(logits);
+    g.part_sum = workspace + (int64_t)tn * rows;
+    g.hit = logits ? nullptr : g.part_sum + (int64_t)tn * rows;
+    g.vec = vocab % 4 == 0 && vocab <= kMaxPitch && aligned(logits);
     launch<true, true, kLse>(g, p, s);
     hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, logits, target, loss,
-                       lse, stats, rows, vocab, p.tn);
+                       lse, stats, rows, vocab, tn);
     return (int)hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
 """The language model's matrix products, negative log-likelihood and LayerNorm kernels through the C ABI, against
-float64.  Tolerance of a product: every one of the six roundings per 32 terms, and the split of an operand into
+float64.  Tolerance of a product: every one of the up to six roundings per 32 terms, and the split of an operand into
 three bf16 numbers, is at most 2^-24 of the sum of the terms' magnitudes."""
 import ctypes
 
@@ -278,6 +278,55 @@ def test_loss_gradients_of_an_infinite_upstream_gradient(fwp):
         odd = ~w.isfinite()      # at the target PyTorch forms infinity - p infinity, NaN, and (p - 1) infinity is also right
         assert torch.equal(~g.isfinite(), odd) and bool((g == w)[w.isinf()].all()), name
         assert float((g.double() - w)[~odd].abs().max() if bool((~odd).any()) else 0.0) <= 2e-5 * 10, name
+
+
+# 64 x 64, 128 x 64 and 128 x 128 tiles, k in ranges; B's rows kept in LDS (4 and 8 steps of k, whole and not)
+HALF_SHAPES = [(70, 130, 128), (8190, 509, 300), (2100, 3001, 260), (131, 776, 3001), (6433, 1030, 131), (6433, 1030, 200),
+               (3201, 2048, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", HALF_SHAPES)
+@pytest.mark.parametrize("layout", [NT, NN, TN])
+@pytest.mark.parametrize("case", ["even", "growing", "sparse"])
+def test_products_of_two_fp16_parts(fwp, M, N, K, layout, case):
+    """Rows of the same size throughout, rows that grow along k far beyond fp16's range (up and down again), rows of zeros
+    with a few elements; with every epilogue, operands apart and unaligned."""
+    a, b = randn(M, K, seed=1), randn(N, K, seed=2)
+    if case == "growing":
+        step = torch.arange(K, device="cuda") / K
+        a = a * torch.exp2(60 * step - 40) * torch.exp2(20 * randn(M, 1, seed=6))
+        b = b * torch.exp2(40 * (0.5 - (step - 0.5).abs()))
+    elif case == "sparse":
+        a, b = a * (randn(M, K, seed=6) > 2), b * (randn(N, K, seed=7) > 2) * 1e-20
+        a[5], b[3] = 0, 0
+    bias, residual, gate = randn(N, seed=3), randn(M, N, seed=4), randn(M, N, seed=5)
+    x, y = a.double(), b.double()
+    raw, mag = x @ y.t(), x.abs() @ y.abs().t()
+    # an operand's parts: 2^-22 of an element, or 2^-28 of its row's largest where the element is below 2^-7 of that
+    err = 2.0 ** -28 * (x.abs().amax(1)[:, None] * y.abs().sum(1) + x.abs().sum(1)[:, None] * y.abs().amax(1))
+    err = bound(K, mag) + 3 * 2.0 ** -22 * mag + err
+    A, B = a.t().contiguous() if layout == TN else a, b if layout == NT else b.t().contiguous()
+    for by, first in ((0, 0), (3, 1)):
+        p, q = spread(A, by, first), spread(B, by, first)
+        assert bool(((matmul(fwp._lib, layout, p, q).double() - raw).abs() <= err).all())
+        got = matmul(fwp._lib, layout, p, q, bias=bias, relu=1, residual=residual, gate=gate)
+        want = torch.where(gate > 0, torch.relu(raw + bias.double()) + residual.double(), 0.0)
+        assert bool(((got.double() - want).abs() <= err + 2 * EPS * (raw.abs() + bias.abs() + residual.abs())).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(8190, 509, 300), (6433, 1030, 200), (3201, 2048, 128)])
+@pytest.mark.parametrize("layout", [NT, NN, TN])
+def test_infinities_in_larger_products(fwp, M, N, K, layout):
+    a, b = randn(M, K, seed=1), randn(N, K, seed=2)
+    a[7, 3], a[M - 1, K - 1], a[900, 0], b[N - 1, 5] = float("inf"), float("nan"), 2e37, float("inf")
+    want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+    A, B = a.t().contiguous() if layout == TN else a, b if layout == NT else b.t().contiguous()
+    got = matmul(fwp._lib, layout, A, B).double()
+    assert torch.equal(got.isnan(), want.isnan()) and bool((got == want)[want.isinf()].all())
+    ok = want.isfinite()
+    amax, bmax = (t.double().abs().nan_to_num(0.0, 0.0, 0.0) for t in (a, b))
+    err = 2.0 ** -28 * (amax.amax(1)[:, None] * bmax.sum(1) + amax.sum(1)[:, None] * bmax.amax(1))
+    assert bool(((got - want).abs() <= bound(K, mag) + K * EPS * mag + err)[ok].all())
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 36), (3000, 128), (2500, 256), (9, 260), (70, 1024)])
