@@ -169,6 +169,20 @@ int fwp_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff,
                   int chunk, void *stream);
 
 /*
+ * fwp_delta_fwd_strided and fwp_delta_bwd for few long sequences: given `work` (16-byte aligned,
+ * fwp_delta_segment_floats floats, which may be 0) a sequence is cut into segments that run at the same time.
+ * `work` is scratch of the call; NULL: as the two above.  A sum's terms are grouped differently then.
+ */
+long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk);
+int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W,
+                           fwp_out_view out, float *vdiff, float *ckpt, float *work, int N, int H, int L,
+                           int E, int M, int chunk, void *stream);
+int fwp_delta_bwd_segments(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff,
+                           fwp_view grad_out, const float *ckpt, float *gq, float *gk,
+                           float *gv, float *gbeta, float *work, int N, int H, int L, int E, int M,
+                           int chunk, void *stream);
+
+/*
  * Sum update rule (causal linear attention) forward.  Replaces causal_dot_product
  * (algorithmic/fast_transformers/causal_product_cuda.cu:99-141, kernel :15-96).
  *   W += k (x) v ; out = W^T q per step.  q,k [N,H,L,E]  v [N,H,L,M]

@@ -50,6 +50,8 @@ _SIGNATURES = {
     "fwp_deltanet_prep_fwd": [_P] * 5 + [_I] * 4 + [ctypes.c_float, _P],
     "fwp_deltanet_prep_bwd": [_P] * 6 + [_I] * 4 + [ctypes.c_float, _P],
     "fwp_delta_fwd_strided": [_V] * 4 + [_P, OutView] + [_P] * 2 + [_I] * 6 + [_P],
+    "fwp_delta_fwd_segments": [_V] * 4 + [_P, OutView] + [_P] * 3 + [_I] * 6 + [_P],
+    "fwp_delta_bwd_segments": [_V] * 3 + [_P, _V, _P] + [_P] * 5 + [_I] * 6 + [_P],
     "fwp_rec_fwd": [_V] * 4 + [_P] * 12 + [_I] * 5 + [_P],
     "fwp_rec_bwd": [_P] * 6 + [_V] + [_P] * 14 + [_I] * 5 + [_P],
     "fwp_rec_bwd_static": [_P] * 6 + [_V] + [_P] * 13 + [_I] * 5 + [_P],
@@ -70,7 +72,7 @@ _MODEL_SIGNATURES = {
 }
 _WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
 EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",
-                                       "fwp_delta_ckpt_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
+                                       "fwp_delta_ckpt_floats", "fwp_delta_segment_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
 KIND_LDS, KIND_SCAN, KIND_CHUNKED, KIND_SPLIT, KIND_PHASE, KIND_STEP = 0, 1, 2, 3, 4, 5
 CFG_DELTA_KERNELS, DELTA_AUTO, DELTA_SCAN, DELTA_CHUNKED, DELTA_SPLIT, DELTA_PHASE = 0, 0, 1, 2, 3, 4
 CFG_STEP_KERNELS = 1
@@ -99,6 +101,8 @@ def lib():
         handle.fwp_check_device.restype = ctypes.c_int
         handle.fwp_delta_ckpt_floats.argtypes = [ctypes.c_int] * 6
         handle.fwp_delta_ckpt_floats.restype = ctypes.c_longlong
+        handle.fwp_delta_segment_floats.argtypes = [ctypes.c_int] * 6
+        handle.fwp_delta_segment_floats.restype = ctypes.c_longlong
         for name, argtypes in _MODEL_SIGNATURES.items():
             if hasattr(handle, name):
                 getattr(handle, name).argtypes = argtypes
@@ -149,6 +153,12 @@ def delta_ckpt_floats(N, H, L, E, M, chunk):
             _ckpt_floats_cache.clear()
         _ckpt_floats_cache[key] = n
     return n
+
+
+def segment_work(N, H, L, E, M, chunk, device):
+    """Scratch for a delta-rule call whose sequences run as several segments at once, or ``None``: they do not."""
+    n = int(lib().fwp_delta_segment_floats(N, H, L, E, M, chunk))
+    return torch.empty(n, device=device, dtype=torch.float32) if n > 0 else None
 
 
 def config(key, value):

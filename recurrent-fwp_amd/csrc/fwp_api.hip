@@ -184,11 +184,17 @@ int fwp_check_device(void) {
     return static_scratch_init();        // per-device set-up of the entry point that allocates nothing
 }
 
-int fwp_delta_fwd_strided(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,
-                          float *vdiff, float *ckpt, int N, int H, int L, int E, int M, int chunk,
-                          void *stream) {
+long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
+    if (check_dims(N, H, L, E, M, chunk)) return -1;
+    return delta_segment_floats(N, H, L, E, M, chunk);
+}
+
+int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,
+                           float *vdiff, float *ckpt, float *work, int N, int H, int L, int E, int M, int chunk,
+                           void *stream) {
     if (bad_view(q) || bad_view(k) || bad_view(v) || bad_view(beta) || !W || !out.ptr)
         return FWP_E_NULL;
+    if (!aligned16(work)) return FWP_E_SHAPE;
     if ((vdiff == nullptr) != (ckpt == nullptr)) return FWP_E_NULL;
     if (int rc = check_dims(N, H, L, E, M, chunk)) return rc;
     const int dk = g_delta_kernels;          // the one read of the switch in this call
@@ -201,7 +207,7 @@ int fwp_delta_fwd_strided(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, flo
         case FWP_KIND_PHASE:
             return phase_delta_fwd(q, k, v, beta, W, out, vdiff, ckpt, N, H, L, chunk, (hipStream_t)stream);
         case FWP_KIND_SPLIT:
-            return split_delta_fwd(q, k, v, beta, W, out, vdiff, ckpt, N, H, L, E, M, chunk, (hipStream_t)stream);
+            return split_delta_fwd(q, k, v, beta, W, out, vdiff, ckpt, work, N, H, L, E, M, chunk, (hipStream_t)stream);
         case FWP_KIND_CHUNKED:
             return mfma_delta_fwd(q, k, v, beta, W, out, vdiff, ckpt, N, H, L, E, chunk, (hipStream_t)stream);
         case FWP_KIND_SCAN:
@@ -211,6 +217,12 @@ int fwp_delta_fwd_strided(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, flo
     if (int rc = delta_aux_invalidate(ckpt, N, H, L, E, M, chunk, (hipStream_t)stream)) return rc;
     return generic_delta_fwd(q, k, v, beta, W, out, vdiff, ckpt, N, H, L, E, M, chunk,
                              (hipStream_t)stream);
+}
+
+int fwp_delta_fwd_strided(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,
+                          float *vdiff, float *ckpt, int N, int H, int L, int E, int M, int chunk,
+                          void *stream) {
+    return fwp_delta_fwd_segments(q, k, v, beta, W, out, vdiff, ckpt, nullptr, N, H, L, E, M, chunk, stream);
 }
 
 int fwp_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, float *out,
@@ -224,14 +236,21 @@ int fwp_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, f
 int fwp_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp_view grad_out,
                   const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, int N, int H,
                   int L, int E, int M, int chunk, void *stream) {
+    return fwp_delta_bwd_segments(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, nullptr, N, H, L, E, M, chunk, stream);
+}
+
+int fwp_delta_bwd_segments(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp_view grad_out,
+                           const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, float *work, int N, int H,
+                           int L, int E, int M, int chunk, void *stream) {
     if (bad_view(q) || bad_view(k) || bad_view(beta) || bad_view(grad_out) || !vdiff || !ckpt ||
         !gq || !gk || !gv || !gbeta)
         return FWP_E_NULL;
+    if (!aligned16(work)) return FWP_E_SHAPE;
     if (int rc = check_dims(N, H, L, E, M, chunk)) return rc;
     const bool aligned = aligned16(vdiff) && aligned16(ckpt) && aligned16(gq) && aligned16(gk) && aligned16(gv);
     switch (delta_kind(g_delta_kernels, true, aligned, q, k, grad_out, beta, nullptr, N, H, L, E, M)) {
         case FWP_KIND_SPLIT:
-            return split_delta_bwd(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, N, H, L, E, M, chunk,
+            return split_delta_bwd(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, work, N, H, L, E, M, chunk,
                                    (hipStream_t)stream);
         case FWP_KIND_CHUNKED:
             return mfma_delta_bwd(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, N, H, L, E, chunk,

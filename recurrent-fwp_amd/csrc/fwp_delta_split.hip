@@ -20,12 +20,83 @@
 // needs no code of its own: every tensor is read and written through a buffer resource of exactly
 // the sequence's size, so its missing rows read as zeros (beta = 0: nothing is written to the
 // state; zero upstream gradient) and stores to them are dropped; the loops stay straight-line.
+//
+// Few long sequences leave most CUs without work (a block of the chain takes 0.65 us, forward, D = 32, however few there
+// are).  What a run of blocks does to the state is the map S -> S + D S + R, and to its gradient dS -> dS + D^T dS + G: a
+// sequence is cut into segments, a first launch forms the maps of all segments at once (for D by the same chain from
+// zero, with -K for the values), and in a second one every segment's workgroup goes through the maps of those before it
+// (behind it, backward) and then does its blocks as above.  Twice the chain's products, over a chain as much shorter as
+// there are segments.  32 x 32 states, 8 sequences of 2381 steps: forward 93 -> 30 us, with backward 264 -> 77 us; 32 of 2048
+// steps: 83 -> 35, 232 -> 82 us; 64 x 64, 32 of 1024 steps: 118 -> 64, 345 -> 145 us.
 #include "fwp_common.hpp"
 #include "fwp_wave.hpp"
 #include "fwp_mfma.hpp"
 
+#include <algorithm>
+
 namespace fwp {
 namespace {
+
+// A sequence's segments: `count` of `blocks` blocks each (whole checkpoint intervals; the last may be shorter).  work, per
+// sequence: the state it starts from [E,M] (forward), then per segment but the last (forward) or the first (backward) R or G
+// [E,M] and D or D^T [E,E], row-major.
+struct Segments {
+    float *work;
+    int count, blocks;
+};
+template <int E, int M>
+__device__ __forceinline__ int64_t map_at(const Segments &s, int64_t seq, int j) {
+    return seq * (E * M + (int64_t)(s.count - 1) * (E * M + E * E)) + E * M + (int64_t)j * (E * M + E * E);
+}
+
+// Tiles eb of D and R of the map at `at`, for a wave's 16 columns
+template <int NE, int M>
+struct MapRow {
+    v4f D[NE], R;
+    __device__ __forceinline__ void load(const float *at, int eb, int mb, int g, int c) {
+        constexpr int E = 16 * NE;
+#pragma unroll
+        for (int r = 0; r < 4; r++) R[r] = at[(16 * eb + 4 * g + r) * M + 16 * mb + c];
+#pragma unroll
+        for (int b = 0; b < NE; b++) D[b] = from_float4(*reinterpret_cast<const float4 *>(at + E * M + (16 * eb + c) * E + 16 * b + 4 * g));
+    }
+};
+
+// X <- X + D X + R for n maps in turn, at(i) the i-th; X: a wave's 16 columns, tiles as in the accumulator layout.  With keys of
+// up to 32 features the next map is in flight meanwhile.
+template <int NE, int M, class At>
+__device__ __forceinline__ void apply_maps(v4f (&X)[NE], int n, int mb, int g, int c, At at) {
+    constexpr int kAhead = NE <= 2 ? 2 : 1;
+    MapRow<NE, M> m[kAhead][NE];
+    const auto load = [&](int to, int i) {
+#pragma unroll
+        for (int eb = 0; eb < NE; eb++) m[to][eb].load(at(i), eb, mb, g, c);
+    };
+    const auto apply = [&](int from) {
+        v4f Y[NE];
+#pragma unroll
+        for (int eb = 0; eb < NE; eb++) {
+            Y[eb] = m[from][eb].R;      // the small terms first
+#pragma unroll
+            for (int b = 0; b < NE; b++) Y[eb] = tn(m[from][eb].D[b], X[b], Y[eb]);
+        }
+#pragma unroll
+        for (int eb = 0; eb < NE; eb++) X[eb] += Y[eb];
+    };
+    if (n <= 0) return;
+    if constexpr (kAhead == 1) {
+        for (int i = 0; i < n; i++) load(0, i), apply(0);
+    } else {
+        load(0, 0);
+        for (int i = 0; i < n; i += 2) {
+            load(1, min(i + 1, n - 1));
+            apply(0);
+            if (i + 1 >= n) break;
+            load(0, min(i + 2, n - 1));
+            apply(1);
+        }
+    }
+}
 
 // ------------------------------------------------------------------ forward
 
@@ -59,18 +130,19 @@ struct OutRaw {
 // block behind the state waves, which hand it their columns of the state and of U.
 // With one state wave and the output wave a fourth wave only keeps the barriers: the four waves of a
 // 256-thread workgroup take one SIMD each, three-wave workgroups are placed unevenly.
-template <int NE, int NM, int PF, bool OUT>   // E = 16 NE, M = 16 NM, PF = blocks in flight
-__global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void k_delta_fwd_split(fwp_view q, fwp_view k, fwp_view v,
+// MAP: the map of a segment instead; state waves mb >= NM hold the columns of D.
+template <int NE, int NM, int PF, bool OUT, bool MAP = false>   // E = 16 NE, M = 16 NM, PF = blocks in flight
+__global__ __launch_bounds__(64 * (MAP ? NM + NE + 1 : OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void k_delta_fwd_split(fwp_view q, fwp_view k, fwp_view v,
                                                                   fwp_view beta, float *__restrict__ W,
                                                                   fwp_out_view out,
                                                                   float *__restrict__ vdiff,
                                                                   float *__restrict__ ckpt,
                                                                   float *__restrict__ aux, int H, int L,
-                                                                  int chunk, int nchunk) {
-    constexpr int E = 16 * NE, M = 16 * NM;
+                                                                  int chunk, int nchunk, Segments segs) {
+    constexpr int E = 16 * NE, M = 16 * NM, NS = MAP ? NM + NE : NM;
     // lower(Q K^T)^T: with one state wave that wave forms it itself, with several the preparing
     // wave does it once for all
-    constexpr bool kPrepQK = NM > 1;
+    constexpr bool kPrepQK = NM > 1 && !MAP;
     // What the preparing wave hands over, per block of a group of four, two groups alternately:
     // (I + A)^-T and (with several state waves) lower(Q K^T)^T
     __shared__ LdsMat tmat[2][kGrp], rmat[kPrepQK ? 2 : 1][kPrepQK ? kGrp : 1];
@@ -83,13 +155,17 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
     const int lane = threadIdx.x % 64;
     const Geo16 p(lane);
     const int g = p.g, c = p.c;
-    const int64_t seq = blockIdx.x;
+    const int parts = MAP ? segs.count - 1 : segs.count, part = parts > 1 ? (int)(blockIdx.x % parts) : 0;
+    const int64_t seq = parts > 1 ? blockIdx.x / parts : blockIdx.x;
     const int n = (int)(seq / H), h = (int)(seq % H);
-    // rows of this sequence; lane offsets and block steps in bytes
-    const RowBuf qb(row(q, n, h, 0), (uint32_t)(((L - 1) * q.sL + E) * 4)),
-        kb(row(k, n, h, 0), (uint32_t)(((L - 1) * k.sL + E) * 4)),
-        vb(row(v, n, h, 0), (uint32_t)(((L - 1) * v.sL + M) * 4)),
-        bb(row(beta, n, h, 0), (uint32_t)(((L - 1) * beta.sL + 1) * 4));
+    // this segment: its first step and block, its length
+    const int t0 = part * segs.blocks * kBlk, b0 = part * segs.blocks, L_all = L, nblk_all = (L + kBlk - 1) / kBlk;
+    if (segs.count > 1) L = min(L - t0, segs.blocks * kBlk);
+    // its rows; lane offsets and block steps in bytes
+    const RowBuf qb(row(q, n, h, t0), (uint32_t)(((L - 1) * q.sL + E) * 4)),
+        kb(row(k, n, h, t0), (uint32_t)(((L - 1) * k.sL + E) * 4)),
+        vb(row(v, n, h, t0), (uint32_t)(((L - 1) * v.sL + M) * 4)),
+        bb(row(beta, n, h, t0), (uint32_t)(((L - 1) * beta.sL + 1) * 4));
     const unsigned q_step = (unsigned)(kBlk * q.sL * 4), k_step = (unsigned)(kBlk * k.sL * 4),
                    v_step = (unsigned)(kBlk * v.sL * 4), b_step = (unsigned)(kBlk * beta.sL * 4);
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
@@ -99,7 +175,7 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
 #pragma unroll
     for (int r = 0; r < 4; r++) o_br[r] = (unsigned)((4 * g + r) * beta.sL) * 4;
 
-    if (wave == NM) {
+    if (wave == NS) {
         // ------------------------------------------------ preparing wave
         // While the state waves do the four blocks of group m (one block per round, a barrier
         // after each), it prepares group m + 1 in four steps, one per round: K K^T of two blocks,
@@ -195,7 +271,7 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
     }
 
     const unsigned m_step = (unsigned)(kBlk * M * 4), out_step = (unsigned)(kBlk * out.sL * 4);
-    float *const out_rows = out.ptr + n * out.sN + h * out.sH;
+    float *const out_rows = MAP ? nullptr : out.ptr + n * out.sN + h * out.sH + t0 * out.sL;
     const uint32_t out_bytes = (uint32_t)(((L - 1) * out.sL + M) * 4);
     // With one state wave a fourth wave fills the workgroup up to four (one SIMD each); it forms
     // lower(Q K^T)^T for the output wave, in the round in which the state wave does the block
@@ -271,24 +347,27 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
     // ---------------------------------------------------- state wave of columns [16 mb, 16 mb + 16)
     __builtin_amdgcn_s_setprio(3);      // the wave on the chain goes first where waves share a SIMD
     const int mb = wave;
+    const bool values = !MAP || mb < NM;      // else -K's columns for values
+    const RowBuf xb = values ? vb : kb;
+    const unsigned x_step = values ? v_step : k_step;
     unsigned o_kr[4], o_vr[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         o_kr[r] = (unsigned)((4 * g + r) * k.sL + c) * 4;
-        o_vr[r] = (unsigned)((4 * g + r) * v.sL + 16 * mb + c) * 4;
+        o_vr[r] = (unsigned)((4 * g + r) * (values ? v.sL : k.sL) + 16 * (values ? mb : mb - NM) + c) * 4;
     }
-    using StateRaw = MainRaw<NE, !OUT>;
+    using StateRaw = MainRaw<NE, !OUT && !MAP>;
     auto load = [&](StateRaw &w, int ib) {
-        const unsigned ks = ib * k_step, qs = ib * q_step, vs = ib * v_step, bs = ib * b_step;
+        const unsigned ks = ib * k_step, qs = ib * q_step, vs = ib * x_step, bs = ib * b_step;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             w.brow[r] = bb.f(o_br[r], bs);
-            w.Vc[r] = vb.f(o_vr[r], vs);
+            w.Vc[r] = xb.f(o_vr[r], vs);
         }
 #pragma unroll
         for (int b = 0; b < NE; b++) {
             w.Kt[b] = kb.f4(o_kt + 64 * b, ks);
-            if constexpr (!OUT) w.Qt[b] = qb.f4(o_qt + 64 * b, qs);
+            if constexpr (!OUT && !MAP) w.Qt[b] = qb.f4(o_qt + 64 * b, qs);
 #pragma unroll
             for (int r = 0; r < 4; r++) w.Kc[b][r] = kb.f(o_kr[r] + 64 * b, ks);
         }
@@ -296,14 +375,27 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
 
     // S[eb]: register r holds S[16 eb + 4g + r][16 mb + c]
     v4f S[NE];
+    // the state in front of the sequence; the last segment overwrites W while others may not have read it: they
+    // read the copy that the maps' launch made
+    const float *const start = !MAP && segs.count > 1 ? segs.work + map_at<E, M>(segs, seq, 0) - E * M : W + seq * E * M;
 #pragma unroll
     for (int eb = 0; eb < NE; eb++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) S[eb][r] = W[(seq * E + 16 * eb + 4 * g + r) * M + 16 * mb + c];
+        for (int r = 0; r < 4; r++) {
+            const int at = (16 * eb + 4 * g + r) * M + 16 * mb + c;
+            if constexpr (MAP) {
+                if (part == 0 && values) segs.work[map_at<E, M>(segs, seq, 0) - E * M + at] = start[at];
+                S[eb][r] = 0.f;
+            } else {
+                S[eb][r] = start[at];
+            }
+        }
+    if constexpr (!MAP)
+        if (segs.count > 1) apply_maps<NE, M>(S, part, mb, g, c, [&](int j) { return segs.work + map_at<E, M>(segs, seq, j); });
     const ChunkOf chunk_of(chunk);
-    const RowBuf ob(out_rows, out_bytes), db(vdiff ? vdiff + seq * L * M : nullptr, vdiff ? (uint32_t)(L * M * 4) : 0);
+    const RowBuf ob(out_rows, out_bytes), db(vdiff ? vdiff + (seq * L_all + t0) * M : nullptr, vdiff ? (uint32_t)(L * M * 4) : 0);
     const unsigned o_out = (unsigned)(c * out.sL + 16 * mb + 4 * g) * 4, o_vd = (unsigned)(4 * g * M + 16 * mb + c) * 4;
-    const RowBuf tb(aux && mb == 0 ? aux + kAuxHeader + seq * nblk * 256 : nullptr,
+    const RowBuf tb(aux && mb == 0 ? aux + kAuxHeader + (seq * nblk_all + b0) * 256 : nullptr,
                     aux && mb == 0 ? (uint32_t)(nblk * 1024) : 0);
     auto block = [&](int ib, const StateRaw &cur) {
         const int grp = (ib / kGrp) & 1, j = ib % kGrp;
@@ -313,22 +405,23 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
         if constexpr (OUT) {
 #pragma unroll
             for (int eb = 0; eb < NE; eb++) hx[ib & 1][mb][eb].put(lane, S[eb]);
-        } else {
+        } else if constexpr (!MAP) {
 #pragma unroll
             for (int eb = 0; eb < NE; eb++) Ot = tn(S[eb], cur.Qt[eb], Ot);      // O^T, state part (old state)
         }
         const v4f Tt = tmat[grp][j].get(lane);
-        tb.st4(Tt, (unsigned)(c * 16 + 4 * g) * 4, (unsigned)ib * 1024);      // register r = T[c][4g + r]
-        const v4f X = cur.Vc - KS;
+        if constexpr (!MAP) tb.st4(Tt, (unsigned)(c * 16 + 4 * g) * 4, (unsigned)ib * 1024);      // register r = T[c][4g + r]
+        const v4f X = values ? cur.Vc - KS : -cur.Vc - KS;
         v4f Y;
 #pragma unroll
         for (int r = 0; r < 4; r++) Y[r] = cur.brow[r] * X[r];
         const v4f U = tn(Tt, Y, zero);
 #pragma unroll
         for (int eb = 0; eb < NE; eb++) S[eb] = tn(cur.Kc[eb], U, S[eb]);
+        if constexpr (MAP) return;
         if constexpr (OUT) {
             hx[ib & 1][mb][NE].put(lane, U);
-        } else {
+        } else if constexpr (!MAP) {
             v4f Rm;
             if constexpr (kPrepQK) {
                 Rm = rmat[grp][j].get(lane);
@@ -361,7 +454,7 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
             for (int r = 0; r < 4; r++) db.st(Dd[r], o_vd + r * M * 4, ib * m_step);
         }
         if (ckpt && (chunk_of.closes(ib) || ib + 1 == nblk)) {
-            float *dst = ckpt + (seq * nchunk + chunk_of(ib)) * E * M;
+            float *dst = ckpt + (seq * nchunk + chunk_of(b0 + ib)) * E * M;
 #pragma unroll
             for (int eb = 0; eb < NE; eb++)
 #pragma unroll
@@ -372,10 +465,22 @@ __global__ __launch_bounds__(64 * (OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void 
     lds_barrier();      // the preparing wave's block 0
     ring_loop<PF, StateRaw>(nblk, load, block);
     if constexpr (OUT) lds_barrier();      // the output wave's last block
+    if constexpr (MAP) {
+        float *const to = segs.work + map_at<E, M>(segs, seq, part);
 #pragma unroll
-    for (int eb = 0; eb < NE; eb++)
+        for (int eb = 0; eb < NE; eb++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) W[(seq * E + 16 * eb + 4 * g + r) * M + 16 * mb + c] = S[eb][r];
+            for (int r = 0; r < 4; r++) {
+                const int e = 16 * eb + 4 * g + r;
+                if (mb < NM) to[e * M + 16 * mb + c] = S[eb][r];
+                else to[E * M + e * E + 16 * (mb - NM) + c] = S[eb][r];
+            }
+    } else if (part == parts - 1) {
+#pragma unroll
+        for (int eb = 0; eb < NE; eb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) W[(seq * E + 16 * eb + 4 * g + r) * M + 16 * mb + c] = S[eb][r];
+    }
 }
 
 // ----------------------------------------------------------------- backward
@@ -410,7 +515,7 @@ struct QuadP {
 };
 template <int NE>
 struct QuadC {
-    v4f Kt[NE], Kc[NE], T;
+    v4f Kt[NE], Kc[NE], Kx, T;      // Kx: a map's own columns of K
     float bcol, brow[4];
 };
 template <int NEW, int NM>
@@ -429,13 +534,14 @@ constexpr int quad_lds_mats() {
 }
 
 // PW = 2: P on two waves, one with the products of Pm, one with the others.
-template <int NE, int NM, int WR, int PW, int PF>
-__global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
+// MAP: the map of a segment instead, by P and C alone; C's waves mb >= NM hold the columns of D^T.
+template <int NE, int NM, int WR, int PW, int PF, bool MAP = false>
+__global__ __launch_bounds__(64 * (MAP ? PW + NM + NE : PW + NM + 2 * WR)) void k_delta_bwd_quad(
     fwp_view q, fwp_view k, fwp_view beta, const float *__restrict__ vdiff, fwp_view go,
     const float *__restrict__ ckpt, const float *__restrict__ aux, float *__restrict__ gq,
     float *__restrict__ gk, float *__restrict__ gv, float *__restrict__ gbeta, int H, int L, int chunk,
-    int nchunk) {
-    constexpr int E = 16 * NE, M = 16 * NM, NEW = NE / WR;
+    int nchunk, Segments segs) {
+    constexpr int E = 16 * NE, M = 16 * NM, NEW = NE / WR, NC = MAP ? NM + NE : NM;
     static_assert(NE % WR == 0, "key tiles divide evenly over the waves of a role");
     __shared__ LdsMat pc[2][NM + NE * NM];     // P -> C: Pm^T dO per mb, then Q^T dO per (eb, mb)
     // With narrow keys P reads the block's rows for everybody: it hands K (transposed on the way) to C,
@@ -450,20 +556,25 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
     __shared__ __align__(16) float pb[3][16];  // P -> C, G, R: beta[t0 + c]
     __shared__ LdsMat cg[2][NE * NM + NM];     // C -> G, R: dS^T per (eb, mb) before the block's update, dY^T per mb
     __shared__ LdsMat rg[2][NE];               // R -> G: -dX S0^T per eb, transposed like g_k
-    __shared__ LdsMat inv[NM][2];              // the inverse inside C where forward left none
+    __shared__ LdsMat inv[NC][2];              // the inverse inside C where forward left none
     __shared__ LdsMat own[WR];                 // the transpose inside G
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int lane = threadIdx.x % 64;
     const Geo16 p(lane);
     const int g = p.g, c = p.c;
-    const int64_t seq = blockIdx.x;
+    const int parts = MAP ? segs.count - 1 : segs.count, part = (parts > 1 ? (int)(blockIdx.x % parts) : 0) + MAP;
+    const int64_t seq = parts > 1 ? blockIdx.x / parts : blockIdx.x;
     const int n = (int)(seq / H), h = (int)(seq % H);
-    const int nblk = (L + kBlk - 1) / kBlk;
-    const RowBuf qb(row(q, n, h, 0), (uint32_t)(((L - 1) * q.sL + E) * 4)),
-        kb(row(k, n, h, 0), (uint32_t)(((L - 1) * k.sL + E) * 4)),
-        gob(row(go, n, h, 0), (uint32_t)(((L - 1) * go.sL + M) * 4)),
-        bb(row(beta, n, h, 0), (uint32_t)(((L - 1) * beta.sL + 1) * 4)),
-        db(vdiff + seq * L * M, (uint32_t)(L * M * 4));
+    // this segment: its first block, its rows in contiguous tensors, its length
+    const int b0 = part * segs.blocks, nblk_all = (L + kBlk - 1) / kBlk;
+    const int64_t row0 = seq * L + b0 * kBlk;
+    if (segs.count > 1) L = min(L - b0 * kBlk, segs.blocks * kBlk);
+    const int nblk = (L + kBlk - 1) / kBlk, t0 = b0 * kBlk;
+    const RowBuf qb(row(q, n, h, t0), (uint32_t)(((L - 1) * q.sL + E) * 4)),
+        kb(row(k, n, h, t0), (uint32_t)(((L - 1) * k.sL + E) * 4)),
+        gob(row(go, n, h, t0), (uint32_t)(((L - 1) * go.sL + M) * 4)),
+        bb(row(beta, n, h, t0), (uint32_t)(((L - 1) * beta.sL + 1) * 4)),
+        db(vdiff + row0 * M, (uint32_t)(L * M * 4));
     const unsigned q_step = (unsigned)(kBlk * q.sL * 4), k_step = (unsigned)(kBlk * k.sL * 4),
                    o_step = (unsigned)(kBlk * go.sL * 4), b_step = (unsigned)(kBlk * beta.sL * 4),
                    d_step = (unsigned)(kBlk * M * 4), e_step = (unsigned)(kBlk * E * 4);
@@ -505,7 +616,7 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
             }
 #pragma unroll
             for (int b = 0; b < NM; b++) {
-                if (with_rest) {
+                if (with_rest && !MAP) {
                     w.Ot[b] = gob.f4(o_ot + 64 * b, os);
                     w.Dt[b] = db.f4(o_dt + 64 * b, ds);
                 }
@@ -534,10 +645,11 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
                 LdsMat *to = pg[s3];
 #pragma unroll
                 for (int mb = 0; mb < NM; mb++) {
-                    Z = tn(w.Ot[mb], w.bcol * w.Dt[mb], Z);         // dO U^T
 #pragma unroll
                     for (int eb = 0; eb < NE; eb++)
                         pc[e & 1][NM + eb * NM + mb].put(lane, tn(w.Qc[eb], w.Oc[mb], zero));
+                    if constexpr (MAP) continue;
+                    Z = tn(w.Ot[mb], w.bcol * w.Dt[mb], Z);         // dO U^T
                     to[2 + mb].put(lane, w.Dt[mb]);
                     to[2 + NM + mb].put(lane, w.Ot[mb]);
                     if constexpr (kShareG) to[kGD + mb].put_t(p, w.Dt[mb]);      // read back as d[4g + r][c]
@@ -545,9 +657,11 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
                 v4f dPm;
 #pragma unroll
                 for (int r = 0; r < 4; r++) dPm[r] = (p.lo[r] || p.di[r]) ? Z[r] : 0.f;
-                to[0].put(lane, dPm);
-                to[1].put_t(p, dPm);
-                if constexpr (kShareG) {
+                if constexpr (!MAP) {
+                    to[0].put(lane, dPm);
+                    to[1].put_t(p, dPm);
+                }
+                if constexpr (kShareG && !MAP) {
 #pragma unroll
                     for (int b = 0; b < NE; b++) to[kGQ + b].put(lane, w.Qc[b]);
                 }
@@ -560,14 +674,14 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
         lds_barrier();
         return;
     }
-    if (wave < PW + NM) {
+    if (wave < PW + NC) {
         // ------------------------------------------------ C of value columns [16 mb, 16 mb + 16)
         __builtin_amdgcn_s_setprio(3);      // the chain goes first where waves share a SIMD
         const int mb = wave - PW;
         using Raw = QuadC<NE>;
         // T = (I + A)^-1 per block as left by the blocked forward (row-major), if it ran
         const bool have_T = aux && aux[0] == 1.f;
-        const RowBuf tb(have_T ? aux + kAuxHeader + seq * nblk * 256 : nullptr, have_T ? nblk * 1024 : 0);
+        const RowBuf tb(have_T ? aux + kAuxHeader + (seq * nblk_all + b0) * 256 : nullptr, have_T ? nblk * 1024 : 0);
         const unsigned o_t = (unsigned)(4 * g * 16 + c) * 4, o_tt = (unsigned)(c * 16 + 4 * g) * 4;
         v4f ident;
 #pragma unroll
@@ -597,10 +711,16 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
                     for (int r = 0; r < 4; r++) w.Kc[b][r] = kb.f(o_kr[r] + 64 * b, ks);
                 }
             }
+            if constexpr (MAP && !kShareG)
+#pragma unroll
+                for (int r = 0; r < 4; r++) w.Kx[r] = kb.f(o_kr[r] + 64 * max(mb - NM, 0), ks);
         };
         v4f dS[NE];           // register r = dS[16 eb + 4g + r][16 mb + c]
 #pragma unroll
         for (int eb = 0; eb < NE; eb++) dS[eb] = zero;
+        if constexpr (!MAP)
+            if (segs.count > 1)
+                apply_maps<NE, M>(dS, segs.count - 1 - part, mb, g, c, [&](int j) { return segs.work + map_at<E, M>(segs, seq, segs.count - 2 - j); });
         auto block = [&](int e, const Raw &w) {
             // beta[t0 + 4g + r] and K[t0 + 4g + r][.]: loaded, or from what P left a round ago
             float brow[4];
@@ -638,34 +758,47 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
             }
             const LdsMat *from = pc[e & 1];
             LdsMat *to = cg[e & 1];
-            v4f dU = from[mb].get(lane);
+            const bool values = !MAP || mb < NM;      // else those of K times the unit matrix
+            v4f dU = values ? from[mb].get(lane) : kShareG ? pg[third(e)][kGK + max(mb - NM, 0)].get(lane) : w.Kx;
 #pragma unroll
             for (int eb = 0; eb < NE; eb++) {
-                to[eb * NM + mb].put_t(p, dS[eb]);
+                if constexpr (!MAP) to[eb * NM + mb].put_t(p, dS[eb]);
                 dU = tn(w.Kt[eb], dS[eb], dU);
             }
             const v4f dY = tn(T, dU, zero);
-            to[NE * NM + mb].put_t(p, dY);
+            if constexpr (!MAP) to[NE * NM + mb].put_t(p, dY);
             v4f ndX;
 #pragma unroll
             for (int r = 0; r < 4; r++) ndX[r] = -(brow[r] * dY[r]);
 #pragma unroll
-            for (int eb = 0; eb < NE; eb++) dS[eb] = tn(Kc[eb], ndX, dS[eb] + from[NM + eb * NM + mb].get(lane));
+            for (int eb = 0; eb < NE; eb++) dS[eb] = tn(Kc[eb], ndX, values ? dS[eb] + from[NM + eb * NM + mb].get(lane) : dS[eb]);
         };
         lds_barrier();
         ring_loop<PF, Raw>(nblk, load, block);
         lds_barrier();
         lds_barrier();
+        if constexpr (MAP) {
+            float *const to = segs.work + map_at<E, M>(segs, seq, part - 1);
+#pragma unroll
+            for (int eb = 0; eb < NE; eb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int e = 16 * eb + 4 * g + r;
+                    if (mb < NM) to[e * M + 16 * mb + c] = dS[eb][r];
+                    else to[E * M + e * E + 16 * (mb - NM) + c] = dS[eb][r];
+                }
+        }
         return;
     }
+    if constexpr (MAP) return;
     if (wave < PW + NM + WR) {
         // ------------------------------------------------ R of key tiles [eb0, eb0 + NEW)
         const int j = wave - PW - NM, eb0 = j * NEW;
         using Raw = QuadR<NEW, NM>;
-        const RowBuf cb(ckpt + seq * nchunk * E * M, (uint32_t)(nchunk * E * M * 4)),
-            gqb(gq + seq * L * E, (uint32_t)(L * E * 4)),
-            gvb(j == 0 ? gv + seq * L * M : nullptr, j == 0 ? (uint32_t)(L * M * 4) : 0);
         const ChunkOf chunk_of(chunk);
+        const RowBuf cb(ckpt + (seq * nchunk + chunk_of(b0)) * E * M, (uint32_t)((nchunk - chunk_of(b0)) * E * M * 4)),
+            gqb(gq + row0 * E, (uint32_t)(L * E * 4)),
+            gvb(j == 0 ? gv + row0 * M : nullptr, j == 0 ? (uint32_t)(L * M * 4) : 0);
         auto load = [&](Raw &w, int e) {
             const int ib = nblk - 1 - e;
             const unsigned cs = chunk_of(ib) * (E * M * 4), ks = ib * k_step, bs = ib * b_step, ds = ib * d_step;
@@ -746,8 +879,8 @@ __global__ __launch_bounds__(64 * (PW + NM + 2 * WR)) void k_delta_bwd_quad(
     // ---------------------------------------------------- G of key tiles [eb0, eb0 + NEW)
     const int j = wave - PW - NM - WR, eb0 = j * NEW;
     using Raw = QuadG<NEW>;
-    const RowBuf gkb(gk + seq * L * E, (uint32_t)(L * E * 4)),
-        gbb(j == 0 ? gbeta + seq * L : nullptr, j == 0 ? (uint32_t)(L * 4) : 0);
+    const RowBuf gkb(gk + row0 * E, (uint32_t)(L * E * 4)),
+        gbb(j == 0 ? gbeta + row0 : nullptr, j == 0 ? (uint32_t)(L * 4) : 0);
     auto load = [&](Raw &w, int e) {
         if constexpr (!kShareG) {
             const int ib = nblk - 1 - e;
@@ -840,6 +973,7 @@ bool split_delta_supported(int L) { return L >= 1; }
 namespace {
 constexpr int fwd_ring(int ne) { return ne <= 2 ? 4 : ne <= 4 ? 3 : ne <= 8 ? 2 : 1; }     // (NE = 8: 56 us with two, 67 with one)
 constexpr int bwd_ring(int ne) { return ne <= 2 ? 3 : ne <= 4 ? 2 : 1; }
+constexpr bool segment_dims(int ne, int nm) { return ne <= 6 && nm <= 4; }
 
 // The output wave is built for one or two state waves; with one (a workgroup of four waves, one per
 // SIMD) it is always used, with two up to one and a half waves per SIMD (D = 16, forward at 256 / 512 /
@@ -847,33 +981,65 @@ constexpr int bwd_ring(int ne) { return ne <= 2 ? 3 : ne <= 4 ? 2 : 1; }
 // without; D = 32, 256 sequences of 1024 steps: 54 against 62 us).
 template <int NE, int NM>
 void launch_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out, float *vdiff,
-                float *ckpt, float *aux, int nseq, int H, int L, int chunk, int nchunk, hipStream_t s) {
+                float *ckpt, float *aux, int nseq, int H, int L, int chunk, int nchunk, const Segments &segs, hipStream_t s) {
+    if constexpr (segment_dims(NE, NM))
+        if (segs.count > 1)
+            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false, true>), dim3(nseq * (segs.count - 1)),
+                               dim3(64 * (NM + NE + 1)), 0, s, q, k, v, beta, W, out, nullptr, nullptr, nullptr, H, L, chunk, nchunk, segs);
+    const int wgs = nseq * segs.count;
     if constexpr (NM <= 2) {
-        if (NM == 1 || (int64_t)nseq * (NM + 2) <= 1536) {
-            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), true>), dim3(nseq),
+        if (NM == 1 || (int64_t)wgs * (NM + 2) <= 1536) {
+            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), true>), dim3(wgs),
                                dim3(64 * (NM == 1 ? 4 : NM + 2)),
                                0,
-                               s, q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk);
+                               s, q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk, segs);
             return;
         }
     }
     if constexpr (NM > 1)
-        hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false>), dim3(nseq), dim3(64 * (NM + 1)),
+        hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false>), dim3(wgs), dim3(64 * (NM + 1)),
                            0, s,
-                           q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk);
+                           q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk, segs);
+}
+
+// How sequences are cut: one workgroup to a CU (two of 16 x 16 states), segments of four blocks or more, of more with wide keys,
+// whose maps take longer to go through (E = 96: 3 us each); not into fewer than four, since the maps cost a pass, and
+// not where a sequence is so short that the additional launches, 7 us of the host's, are what a step waits for.
+// Forward / with backward, us: 64 sequences of 2048 steps, 32 x 32, 4 segments 54 / 127, one 88 / 235, 8 60 / 144; 128 of 1024
+// steps 2 53 / 124, 1 48 / 127; 128 of 2048 steps, 16 x 16 4 40 / 94, 1 50 / 138, 2 54 / 132; 8 of 2048 steps, E = 96, M = 16 16
+// 97 / 200, 32 148 / 294, 1 136 / 386; 8 of 512 steps, 32 x 32 8 18 / 79, 1 24 / 64.
+Segments segments_of(int nseq, int L, int E, int M, int chunk) {
+    Segments s{nullptr, 1, 0};
+    const int ne = E / 16, nm = M / 16, nblk = (L + kBlk - 1) / kBlk, per = chunk / kBlk;
+    if (!split_delta_dims(E, M) || !segment_dims(ne, nm)) return s;
+    const bool small = ne == 1 && nm == 1;
+    const int most = (small ? 512 : 256) / nseq;
+    if (most < 4 || nblk < (small ? 80 : 40)) return s;
+    int blocks = std::max((nblk + most - 1) / most, 2 * std::max(ne, 2));
+    blocks = (blocks + per - 1) / per * per;
+    const int count = (nblk + blocks - 1) / blocks;
+    if (count >= 4) s.count = count, s.blocks = blocks;
+    return s;
 }
 }  // namespace
+
+int64_t delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
+    const Segments s = segments_of(N * H, L, E, M, chunk);
+    return s.count > 1 ? (int64_t)N * H * (E * M + (int64_t)(s.count - 1) * (E * M + E * E)) : 0;
+}
 
 // the (NE, NM) pairs of split_delta_dims
 #define FWP_SPLIT_SHAPES(X) X(1, 1) X(1, 2) X(1, 4) X(2, 1) X(2, 2) X(2, 4) X(4, 1) X(4, 2) X(4, 4) X(6, 1) X(6, 2) X(8, 1) X(8, 2) X(12, 1)
 
 int split_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,
-                    float *vdiff, float *ckpt, int N, int H, int L, int E, int M, int chunk, hipStream_t s) {
+                    float *vdiff, float *ckpt, float *work, int N, int H, int L, int E, int M, int chunk, hipStream_t s) {
     const int nchunk = (L + chunk - 1) / chunk;
+    Segments segs = work ? segments_of(N * H, L, E, M, chunk) : Segments{nullptr, 1, 0};
+    segs.work = work;
     float *aux = delta_aux_of(ckpt, N, H, L, E, M, chunk);
 #define X(ne, nm)                                                                                        \
     if (E == 16 * ne && M == 16 * nm) {                                                                  \
-        launch_fwd<ne, nm>(q, k, v, beta, W, out, vdiff, ckpt, aux, N * H, H, L, chunk, nchunk, s);      \
+        launch_fwd<ne, nm>(q, k, v, beta, W, out, vdiff, ckpt, aux, N * H, H, L, chunk, nchunk, segs, s); \
         return (int)hipGetLastError();                                                                   \
     }
     FWP_SPLIT_SHAPES(X)
@@ -882,22 +1048,27 @@ int split_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W,
 }
 
 int split_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp_view go,
-                    const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, int N, int H,
+                    const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, float *work, int N, int H,
                     int L, int E, int M, int chunk, hipStream_t s) {
     const int nchunk = (L + chunk - 1) / chunk;
+    Segments segs = work ? segments_of(N * H, L, E, M, chunk) : Segments{nullptr, 1, 0};
+    segs.work = work;
     const float *aux = delta_aux_of(ckpt, N, H, L, E, M, chunk);
     // four roles; the hand-over of the last five shapes takes 77 to 99 KB of LDS, one or two workgroups to a CU
 #define Q(ne, nm, wr, pw, pf)                                                                               \
     if (E == 16 * ne && M == 16 * nm) {                                                                     \
         static_assert(quad_lds_mats<ne, nm, wr>() * sizeof(LdsMat) + 192 <= 160 * 1024, "LDS of the hand-over"); \
-        hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf>), dim3(N * H), dim3(64 * (pw + nm + 2 * wr)), \
-                           0,                        \
-                           s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk);    \
+        if constexpr (segment_dims(ne, nm))                                                                 \
+            if (segs.count > 1)                                                                             \
+                hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf, true>), dim3(N * H * (segs.count - 1)), dim3(64 * (pw + nm + ne)), \
+                                   0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
+        hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf>), dim3(N * H * segs.count), dim3(64 * (pw + nm + 2 * wr)), \
+                           0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
         return (int)hipGetLastError();                                                                      \
     }
     // blocks in flight per wave: short sequences start sooner with two (all sequences ask for their first rows
     // at once, and a deeper ring puts more requests in front of them), long ones stream better with three
-    if (L <= 512) { Q(1, 1, 1, 1, 2) }
+    if (L <= 512 || segs.count > 1) { Q(1, 1, 1, 1, 2) }
     Q(1, 1, 1, 1, 3) Q(2, 1, 1, 1, 3) Q(1, 2, 1, 1, 3) Q(2, 2, 2, 2, 3) Q(4, 1, 2, 1, 2) Q(6, 1, 3, 1, 2)
     Q(4, 2, 2, 1, 2) Q(1, 4, 1, 1, 2) Q(2, 4, 1, 1, 2) Q(6, 2, 3, 1, 1)
     // 64 x 64: ten waves (two for P, four on the chain, two each for R and G with two key tiles apiece), one block

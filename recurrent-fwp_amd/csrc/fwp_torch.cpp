@@ -139,10 +139,11 @@ struct DeltaBackward : torch::autograd::Node {
                 if (!tq.defined()) tq = at::empty_like(res[0]), tk = at::empty_like(res[1]), tb = at::empty_like(res[3]);
                 gq = tq, gk = tk, gb = tb;
             }
-            check(fwp_delta_bwd(qv, kv, bv, vdiff, gv_, ckpt, gq.data_ptr<float>(), gk.data_ptr<float>(),
-                                gv_s.data_ptr<float>(), gb.data_ptr<float>(), (int)N, (int)H, (int)L, (int)E,
-                                (int)sl.width, chunk_, stream_of(Q)),
-                  "fwp_delta_bwd");
+            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk_, Q.options());
+            check(fwp_delta_bwd_segments(qv, kv, bv, vdiff, gv_, ckpt, gq.data_ptr<float>(), gk.data_ptr<float>(),
+                                         gv_s.data_ptr<float>(), gb.data_ptr<float>(), work.defined() ? work.data_ptr<float>() : nullptr,
+                                         (int)N, (int)H, (int)L, (int)E, (int)sl.width, chunk_, stream_of(Q)),
+                  "fwp_delta_bwd_segments");
             if (!whole) res[2].slice(3, sl.first, sl.last).copy_(pad ? gv_s.slice(3, 0, cols) : gv_s);
             if (i > 0) {
                 res[0].add_(tq);
@@ -235,9 +236,11 @@ at::Tensor delta_forward(const at::Tensor &Q_in, const at::Tensor &K_in, const a
                 ckpt = vdiff + n_vdiff;
                 bufs.push_back(saved);
             }
-            check(fwp_delta_fwd_strided(qv, kv, vv, bv, W_s.data_ptr<float>(), ov, vdiff, ckpt, (int)N, (int)H,
-                                        (int)L, (int)E, (int)sl.width, chunk, stream_of(Q)),
-                  "fwp_delta_fwd_strided");
+            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk, opts);
+            check(fwp_delta_fwd_segments(qv, kv, vv, bv, W_s.data_ptr<float>(), ov, vdiff, ckpt,
+                                         work.defined() ? work.data_ptr<float>() : nullptr, (int)N, (int)H, (int)L, (int)E,
+                                         (int)sl.width, chunk, stream_of(Q)),
+                  "fwp_delta_fwd_segments");
             if (!whole && (pad || M % 4)) out.slice(3, sl.first, sl.last).copy_(out_s.slice(3, 0, cols));
         }
         // the state after the last step, in place, once every slice has run: a rejected slice leaves W as it was

@@ -108,6 +108,12 @@ inline fwp_view view_of(const at::Tensor &t) {
     return {static_cast<const float *>(t.const_data_ptr()), t.stride(0), t.stride(1), t.stride(2)};
 }
 
+// Scratch for a delta-rule call whose sequences run as several segments at once; undefined: they do not.
+inline at::Tensor segment_work(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M, int chunk, const at::TensorOptions &opts) {
+    const int64_t n = fwp_delta_segment_floats((int)N, (int)H, (int)L, (int)E, (int)M, chunk);
+    return n > 0 ? at::empty({n}, opts) : at::Tensor();
+}
+
 // Several contiguous fp32 results of one call in one allocation: `sizes[i]` floats each, every part
 // starting at a multiple of 4 floats (16 bytes, which the kernels that store 16 bytes at a time need).
 struct Parts {

@@ -200,9 +200,11 @@ at::Tensor projection_grad(const at::Tensor &go, const at::Tensor &qkvb, const a
     const at::Tensor gq = parts.take(B, H, T, D), gk = parts.take(B, H, T, D), gv = parts.take(B, H, T, D), gb = parts.take(B, H, T, 1);
     const float *vdiff = ptr(buf), *ckpt = vdiff + rows * H * D;
     const fwp_view gov = {ptr(go), H * D, D, B * H * D};
-    check(fwp_delta_bwd(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), (int)B, (int)H, (int)T,
-                        (int)D, (int)D, fwp_query(FWP_Q_DEFAULT_CHUNK), s),
-          "fwp_delta_bwd");
+    const int chunk = fwp_query(FWP_Q_DEFAULT_CHUNK);
+    const at::Tensor work = segment_work(B, H, T, D, D, chunk, go.options());
+    check(fwp_delta_bwd_segments(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(work), (int)B,
+                                 (int)H, (int)T, (int)D, (int)D, chunk, s),
+          "fwp_delta_bwd_segments");
     const at::Tensor gp = at::empty_like(qkvb);
     check(fwp_deltanet_prep_bwd(ptr(qkvb), ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(gp), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
           "fwp_deltanet_prep_bwd");
@@ -263,9 +265,10 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
             vdiff = ptr(saved);
             ckpt = vdiff + n_vdiff;
         }
-        check(fwp_delta_fwd_strided(view_of(q), view_of(k), view_of(v), view_of(beta), ptr(state), ov, vdiff, ckpt, (int)B,
-                                    (int)H, (int)T, (int)D, (int)D, chunk, s),
-              "fwp_delta_fwd_strided");
+        const at::Tensor work = segment_work(B, H, T, D, D, chunk, opts);
+        check(fwp_delta_fwd_segments(view_of(q), view_of(k), view_of(v), view_of(beta), ptr(state), ov, vdiff, ckpt, ptr(work), (int)B,
+                                     (int)H, (int)T, (int)D, (int)D, chunk, s),
+              "fwp_delta_fwd_segments");
         fwp_mm_epilogue e{};
         e.residual = residual ? ptr(x) : nullptr;
         const at::Tensor y = matmul(FWP_MM_NT, out, Wo, rows, d, H * D, x_in.sizes(), e);

@@ -68,10 +68,12 @@ class DeltaFastWeight(torch.autograd.Function):
             vdiff = saved.data_ptr()
             ckpt = vdiff + 4 * n_vdiff
         with _lib.on_device(Q):
-            rc = _lib.lib().fwp_delta_fwd_strided(qv, kv, vv, bv, _lib.ptr(W), ov, vdiff, ckpt,
-                                                  N, H, L, E, M, chunk, _lib.stream_of(Q))
+            work = _lib.segment_work(N, H, L, E, M, chunk, Q.device)
+            rc = _lib.lib().fwp_delta_fwd_segments(qv, kv, vv, bv, _lib.ptr(W), ov, vdiff, ckpt,
+                                                   work if work is None else _lib.ptr(work),
+                                                   N, H, L, E, M, chunk, _lib.stream_of(Q))
         if rc:
-            _lib.check(rc, "fwp_delta_fwd_strided")
+            _lib.check(rc, "fwp_delta_fwd_segments")
         if need_grad:
             ctx.save_for_backward(Q, K, beta, saved)
             ctx.dims = (N, H, L, E, M, chunk)
@@ -95,12 +97,13 @@ class DeltaFastWeight(torch.autograd.Function):
         grad_V = torch.empty((N, H, L, M), device=Q.device, dtype=torch.float32)
         grad_beta = torch.empty((N, H, L, 1), device=Q.device, dtype=torch.float32)
         with _lib.on_device(Q):
-            rc = _lib.lib().fwp_delta_bwd(
+            work = _lib.segment_work(N, H, L, E, M, chunk, Q.device)
+            rc = _lib.lib().fwp_delta_bwd_segments(
                 qv, kv, bv, vdiff, gv_, ckpt, _lib.ptr(grad_Q),
-                _lib.ptr(grad_K), _lib.ptr(grad_V), _lib.ptr(grad_beta), N, H, L, E, M, chunk,
-                _lib.stream_of(Q))
+                _lib.ptr(grad_K), _lib.ptr(grad_V), _lib.ptr(grad_beta), work if work is None else _lib.ptr(work),
+                N, H, L, E, M, chunk, _lib.stream_of(Q))
         if rc:
-            _lib.check(rc, "fwp_delta_bwd")
+            _lib.check(rc, "fwp_delta_bwd_segments")
         return grad_Q, grad_K, grad_V, grad_beta, None, None
 
 

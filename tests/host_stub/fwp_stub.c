@@ -84,6 +84,16 @@ int fwp_delta_fwd_strided(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, flo
     if (ckpt) fill(ckpt, fwp_delta_ckpt_floats(N, H, L, E, M, chunk), s);
     return 0;
 }
+/* a sequence of 256 steps or more is "cut": the call's scratch is overwritten to its end */
+long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
+    (void)chunk;
+    return L < 256 ? 0 : (long long)N * H * (L / 64) * (E * M + E * E);
+}
+int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out, float *vdiff,
+                           float *ckpt, float *work, int N, int H, int L, int E, int M, int chunk, void *stream) {
+    if (work) fill(work, fwp_delta_segment_floats(N, H, L, E, M, chunk), 1);
+    return fwp_delta_fwd_strided(q, k, v, beta, W, out, vdiff, ckpt, N, H, L, E, M, chunk, stream);
+}
 int fwp_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, float *out, float *vdiff,
                   float *ckpt, int N, int H, int L, int E, int M, int chunk, void *stream) {
     fwp_out_view ov = {out, (int64_t)H * L * M, (int64_t)L * M, M};
@@ -103,6 +113,12 @@ int fwp_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp
     fill(gv, T * M, s + 2);
     fill(gbeta, T, s + 3);
     return 0;
+}
+int fwp_delta_bwd_segments(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp_view grad_out,
+                           const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, float *work, int N, int H, int L,
+                           int E, int M, int chunk, void *stream) {
+    if (work) fill(work, fwp_delta_segment_floats(N, H, L, E, M, chunk), 1);
+    return fwp_delta_bwd(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, N, H, L, E, M, chunk, stream);
 }
 
 int fwp_sum_fwd(fwp_view q, fwp_view k, fwp_view v, float *W, float *out, float *ckpt, int N, int H, int L,
