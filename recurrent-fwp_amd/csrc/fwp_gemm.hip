@@ -396,7 +396,7 @@ struct GemmArgs {
     int M, N, K;
     int ks;                      // k per range (a multiple of kBK)
     int vec;                     // C, residual and gate can be accessed 16 bytes at a time
-    int tm, tn;                  // tiles
+    int tm, tn, ranges;          // tiles, of k
     float *colsum;               // sums over k of A's rows, per range [M] (A contiguous along its rows), or NULL
     fwp_mm_epilogue epi;         // applied here when there is one range
     NllArgs nll;
@@ -430,8 +430,8 @@ struct Columns {
 // back in one step: one alone can leave fp32's range where both together do not.
 template <bool SCALED, int MT, int NT, int MODE>
 __device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], const int (&row)[MT], int m0, int rows, int n0, int lc,
-                                       const int (&ea)[MT], const Columns &col, int column_tile) {
-    const bool one = gridDim.y == 1;
+                                       const int (&ea)[MT], const Columns &col, int range, int column_tile) {
+    const bool one = g.ranges == 1;
     const int left = min(g.M - m0, rows), nl = g.N - n0;
     if (left <= 0) return;
 #pragma unroll
@@ -445,7 +445,7 @@ __device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], co
             for (int e = 0; e < 4; e++) acc[i][j][e] = (SCALED ? ldexpf(acc[i][j][e], ea[i] + eb[e]) : acc[i][j][e]) + b[e];
     }
     const int64_t first = (int64_t)m0 * g.ldc + n0, size = (int64_t)(left - 1) * g.ldc + nl;
-    float *const C = g.C + blockIdx.y * g.part + first;
+    float *const C = g.C + range * g.part + first;
     if (MODE == kLse && !g.C) {
     } else if (g.vec && nl >= 16 * NT) {
         // rows beyond M lie behind the resource
@@ -571,11 +571,12 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     Stage *const L = reinterpret_cast<Stage *>(shared);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
-    // rows of A, through that XCD's L2)
-    const int total = g.tm * g.tn, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
-    const int id = xcd * each + min(xcd, rest) + blockIdx.x / 8;
+    // rows of A, through that XCD's L2), of whole ranges of k where there are several: the tiles of a range read the
+    // same k of A and B (2048 x 128, K = 24576 in 32 ranges: 65 us, with each XCD a tile of all ranges 74)
+    const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
+    const int tile = xcd * each + min(xcd, rest) + blockIdx.x / 8, range = tile / (g.tm * g.tn), id = tile % (g.tm * g.tn);
     const int m0 = (id / g.tn) * BM + wave * WM, n0 = (id % g.tn) * BN;
-    const int kb = blockIdx.y * g.ks, ke = min(g.K, kb + g.ks);
+    const int kb = range * g.ks, ke = min(g.K, kb + g.ks);
     const float *Ap = AKC ? g.A + (int64_t)m0 * g.lda : g.A + m0;
     const float *Bp = BKC ? g.B + (int64_t)n0 * g.ldb : g.B + n0;
     const int ml = g.M - m0, nl = g.N - n0;
@@ -783,19 +784,111 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
                 csum[i] += __shfl_xor(csum[i], 16, 64);
                 csum[i] += __shfl_xor(csum[i], 32, 64);
                 const int row = OpA::row_of(i, lr);
-                if (lc == 0 && row < ml) g.colsum[(int64_t)blockIdx.y * g.M + m0 + row] = csum[i];
+                if (lc == 0 && row < ml) g.colsum[(int64_t)range * g.M + m0 + row] = csum[i];
             }
     }
     if (b.c == 0)
 #pragma unroll
         for (int t = 0; t < OpB::kUnits; t++) exponents[b.row_of(t)] = b.s[t].exponent();
-    if (tid < BN) biases[tid] = g.epi.bias && gridDim.y == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
+    if (tid < BN) biases[tid] = g.epi.bias && g.ranges == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
     __syncthreads();
     int row[MT];
     int ea[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) row[i] = OpA::row_of(i, lr), ea[i] = a.s[i].exponent();
-    finish<S::kScaled, MT, NT, MODE>(g, acc, row, m0, WM, n0, lc, ea, Columns{exponents, biases}, id % g.tn);
+    finish<S::kScaled, MT, NT, MODE>(g, acc, row, m0, WM, n0, lc, ea, Columns{exponents, biases}, range, id % g.tn);
+}
+
+// B's rows split for a whole product at once: a thread's share of THREADS threads' of BN rows x 32 KS k.  A task is a k-chunk of
+// one row (KC) or of two neighbouring ones.
+template <bool KC, int KS, int BN, int THREADS>
+struct Kept {
+    static constexpr int VEC = KC ? 1 : 2, kTasks = KS * 4 * BN / VEC / THREADS;
+    static_assert(kTasks >= 1, "a task per thread");
+    float x[kTasks][VEC][8];
+
+    static __device__ __forceinline__ int chunk(int task) { return KC ? task % 4 : task / (BN / 2) % 4; }
+    static __device__ __forceinline__ int row(int task) { return KC ? task / 4 % BN : task % (BN / 2) * 2; }
+    static __device__ __forceinline__ int step(int task) { return KC ? task / (4 * BN) : task / (2 * BN); }
+
+    // P: the first row at the first k, `left` rows from there, K of k
+    __device__ __forceinline__ void load(const float *P, int64_t ld, int left, int K, int tid) {
+        const v4i rs = buffer_of(P, KC ? (int64_t)(min(left, BN) - 1) * ld + K : (int64_t)(K - 1) * ld + left);
+#pragma unroll
+        for (int t = 0; t < kTasks; t++) {
+            const int task = tid + t * THREADS, r = row(task), k = 32 * step(task) + 4 * chunk(task);
+            if constexpr (KC) {
+                const unsigned at = (unsigned)(r * ld + k) * 4;
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)(k < K ? at : kOut), 0, 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)(k + 16 < K ? at + 64 : kOut), 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[t][0][j] = a[j], x[t][0][4 + j] = b[j];
+            } else {
+                const unsigned at = (unsigned)(k * ld + r) * 4;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)(r < left ? at + (unsigned)(k_of(0, e) * ld) * 4 : kOut), 0, 0);
+                    x[t][0][e] = a[0], x[t][1][e] = r + 1 < left ? a[1] : 0.f;
+                }
+            }
+        }
+    }
+    // the largest magnitude of each row to `top` (LDS, zeros)
+    __device__ __forceinline__ void largest(unsigned *top, int K, int tid) {
+#pragma unroll
+        for (int t = 0; t < kTasks; t++)
+#pragma unroll
+            for (int v = 0; v < VEC; v++) {
+                const int task = tid + t * THREADS;
+                if constexpr (KC)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) x[t][v][e] = 32 * step(task) + k_of(chunk(task), e) < K ? x[t][v][e] : 0.f;
+                atomicMax(&top[row(task) + v], __float_as_uint(abs_max8(x[t][v], 0.f)));
+            }
+    }
+    __device__ __forceinline__ void store(Planes<Half2::kPlanes, BN> *L, int *exponents, const unsigned *top, int tid) const {
+#pragma unroll
+        for (int t = 0; t < kTasks; t++)
+#pragma unroll
+            for (int v = 0; v < VEC; v++) {
+                const int task = tid + t * THREADS, r = row(task) + v, c = chunk(task);
+                Scale s;
+                s.set(__uint_as_float(top[r]));
+                v4u d[Half2::kPlanes];
+#pragma unroll
+                for (int j = 0; j < 4; j++) split_pair<Half2>(x[t][v], j, s.s, d);
+#pragma unroll
+                for (int p = 0; p < Half2::kPlanes; p++) L[step(task)].u[p][c][unit_of(r, c)] = d[p];
+                if (step(task) == 0 && c == 0) exponents[r] = s.exponent();
+            }
+    }
+};
+
+// acc += the fp32 products of a wave's rows (x: a step's elements of A) with B's rows from memory
+template <bool BKC, int MT, int NT>
+__device__ __forceinline__ void plain_step(v4f (&acc)[MT][NT], const float (&x)[MT][8], const float *Bp, int64_t ldb, int nl, int k0, int K,
+                                           int lr, int lc) {
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) {
+            const int n = 16 * j + lr, k = k0 + k_of(lc, e);
+            const float y = n < nl && k < K ? Bp[BKC ? n * ldb + k : k * ldb + n] : 0.f;
+#pragma unroll
+            for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, x[i][e], acc[i][j], 0, 0, 0);
+        }
+}
+
+template <int MT, int NT>
+__device__ __forceinline__ bool any_odd(const v4f (&acc)[MT][NT]) {      // 0 times what is not finite is NaN
+    float x = 0.f;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) x = fmaf(acc[i][j][r], 0.f, x);
+    return __any(x != 0.f);
 }
 
 // Products with K up to 32 KS: a workgroup keeps 16 NT of B's rows, split, in LDS and its eight waves go over blocks of 32
@@ -819,59 +912,11 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
     __syncthreads();
     {
-        constexpr int VEC = BKC ? 1 : 2, kTasks = KS * 4 * BN / VEC / (2 * kThreads);
-        static_assert(kTasks >= 1, "a task per thread");
-        float x[kTasks][VEC][8];
-        int row[kTasks], step[kTasks], c[kTasks];
-        const v4i rs = buffer_of(Bp, BKC ? (int64_t)(min(nl, BN) - 1) * g.ldb + K : (int64_t)(K - 1) * g.ldb + nl);
-#pragma unroll
-        for (int t = 0; t < kTasks; t++) {
-            const int task = tid + t * 2 * kThreads;
-            if constexpr (BKC) {
-                c[t] = task % 4, row[t] = task / 4 % BN, step[t] = task / (4 * BN);
-                const int k = 32 * step[t] + 4 * c[t];
-                const unsigned at = (unsigned)(row[t] * g.ldb + k) * 4;
-                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)(k < K ? at : kOut), 0, 0),
-                          b = llvm_raw_buffer_load_v4f32(rs, (int)(k + 16 < K ? at + 64 : kOut), 0, 0);
-#pragma unroll
-                for (int j = 0; j < 4; j++) x[t][0][j] = a[j], x[t][0][4 + j] = b[j];
-            } else {
-                row[t] = task % (BN / 2) * 2, c[t] = task / (BN / 2) % 4, step[t] = task / (2 * BN);
-                const unsigned at = (unsigned)((32 * step[t] + 4 * c[t]) * g.ldb + row[t]) * 4;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)(row[t] < nl ? at + (unsigned)(k_of(0, e) * g.ldb) * 4 : kOut), 0, 0);
-                    x[t][0][e] = a[0], x[t][1][e] = row[t] + 1 < nl ? a[1] : 0.f;
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < kTasks; t++)
-#pragma unroll
-            for (int v = 0; v < VEC; v++) {
-                if constexpr (BKC)
-#pragma unroll
-                    for (int e = 0; e < 8; e++) x[t][v][e] = 32 * step[t] + k_of(c[t], e) < K ? x[t][v][e] : 0.f;
-                float m = 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; e++) m = x[t][v][e] != x[t][v][e] ? INFINITY : fmaxf(m, fabsf(x[t][v][e]));
-                atomicMax(&top[row[t] + v], __float_as_uint(m));
-            }
+        Kept<BKC, KS, BN, 2 * kThreads> kept;
+        kept.load(Bp, g.ldb, nl, K, tid);
+        kept.largest(top, K, tid);
         __syncthreads();
-#pragma unroll
-        for (int t = 0; t < kTasks; t++)
-#pragma unroll
-            for (int v = 0; v < VEC; v++) {
-                const unsigned m = top[row[t] + v];
-                Scale s;
-                s.set(__uint_as_float(m));
-                v4u d[S::kPlanes];
-#pragma unroll
-                for (int j = 0; j < 4; j++) split_pair<S>(x[t][v], j, s.s, d);
-#pragma unroll
-                for (int p = 0; p < S::kPlanes; p++) L[step[t]].u[p][c[t]][unit_of(row[t] + v, c[t])] = d[p];
-                if (step[t] == 0 && c[t] == 0) exponents[0][row[t] + v] = s.exponent();
-            }
+        kept.store(L, exponents[0], top, tid);
     }
     __syncthreads();
 
@@ -963,18 +1008,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             step(std::integral_constant<int, 0>(), s);
             step(std::integral_constant<int, 1>(), s + 1);
         }
-        const auto odd = [&] {
-            float x = 0.f;
-#pragma unroll
-            for (int i = 0; i < MT; i++)
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) x = fmaf(acc[i][j][r], 0.f, x);
-            return (bool)__any(x != 0.f);
-        };
         const int *eb = exponents[0];
-        if (odd()) {
+        if (any_odd(acc)) {
             // an element that is not finite (0 times it is NaN): the block once more from the fp32 operands
             OpA::Raw x;
             clear();
@@ -984,22 +1019,102 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             for (int k0 = 0; k0 < K; k0 += kBK) {
                 load(x, block, k0);
                 if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++) {
-                        const int n = 16 * j + lr, k = k0 + k_of(lc, e);
-                        const float y = n < nl && k < K ? Bp[BKC ? n * g.ldb + k : k * g.ldb + n] : 0.f;
-#pragma unroll
-                        for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, x.x[i][e], acc[i][j], 0, 0, 0);
-                    }
+                plain_step<BKC>(acc, x.x, Bp, g.ldb, nl, k0, K, lr, lc);
             }
         }
         int row[MT];
 #pragma unroll
         for (int i = 0; i < MT; i++) row[i] = OpA::row_of(i, lr);
-        finish<true, MT, NT, MODE>(g, acc, row, block * kBlock, kBlock, n0, lc, ea, Columns{eb, biases}, id % g.tn);
+        finish<true, MT, NT, MODE>(g, acc, row, block * kBlock, kBlock, n0, lc, ea, Columns{eb, biases}, 0, id % g.tn);
     }
+}
+
+// Small products, 64 x 64 tiles with up to 32 KS k each: everything is asked for at once and split as it arrives, three barriers in
+// all.  Bound by latency, one trip to memory and a chain of 12 KS matrix instructions: 300 x 256, K = 256 7.0 us (step by step
+// 8.5; 2 are an empty kernel's), 300 x 128, K = 128 4.6 (6.3), x^T y of 1000 rows, 1024 x 256 11.6 with the ranges' sum (15.8).
+template <bool AKC, bool BKC, int KS, int MODE>
+__global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
+    typedef Half2 S;
+    constexpr int NT = 4, BN = 16 * NT;
+    typedef Direct<AKC, 1, false> OpA;
+    __shared__ Planes<S::kPlanes, BN> L[KS];
+    __shared__ unsigned top[BN];
+    __shared__ __align__(16) int exponents[2][BN];
+    __shared__ __align__(16) float biases[BN];
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), lr = lane % 16, lc = lane / 16;
+    const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
+    const int tile = xcd * each + min(xcd, rest) + blockIdx.x / 8, range = tile / (g.tm * g.tn), id = tile % (g.tm * g.tn);
+    const int m0 = id / g.tn * 64 + wave * 16, n0 = id % g.tn * BN, ml = g.M - m0, nl = g.N - n0;
+    const int kb = range * g.ks, K = min(g.K - kb, g.ks);
+    const float *const Ap = AKC ? g.A + (int64_t)m0 * g.lda + kb : g.A + m0 + kb * g.lda;
+    const float *const Bp = BKC ? g.B + (int64_t)n0 * g.ldb + kb : g.B + n0 + kb * g.ldb;
+    if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && g.ranges == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
+    Kept<BKC, KS, BN, kThreads> kept;
+    OpA a;
+    typename OpA::Raw x[KS];
+    kept.load(Bp, g.ldb, nl, K, tid);
+    a.init(lane, m0, g.M, g.nll);
+    const auto load = [&](typename OpA::Raw &y, int k0) {
+        a.aim(g.lda, k0, K);
+        a.load(y, Ap, g.lda, ml, k0, K, g.nll, 0, lane);
+    };
+#pragma unroll
+    for (int s = 0; s < KS; s++) load(x[s], 32 * s);
+    lds_barrier();
+    kept.largest(top, K, tid);
+    lds_barrier();
+    kept.store(L, exponents[0], top, tid);
+    float m = 0.f, csum = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        if (K % 4 && 32 * s + 32 > K) a.cut(x[s], 32 * s, K);
+        m = abs_max8(x[s].x[0], m);
+    }
+    a.s[0].set(OpA::of_row(m));
+    if constexpr (!AKC) {
+        if (g.colsum && n0 == 0)
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) csum += x[s].x[0][e];
+    }
+    lds_barrier();
+    v4f acc[1][NT];
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[0][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    const int unit[2] = {lc * BN + unit_of(lr, lc), lc * BN + unit_of(16 + lr, lc) - 16};
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        v4u f[S::kPlanes];
+#pragma unroll
+        for (int q = 0; q < 4; q++) split_pair<S>(x[s].x[0], q, a.s[0].s, f);
+#pragma unroll
+        for (int q = 0; q < S::kProducts; q++)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                acc[0][j] = S::mma(__builtin_bit_cast(S::frag, L[s].u[S::kOrder[q][1]][0][unit[j % 2] + 16 * j]),
+                                   __builtin_bit_cast(S::frag, f[S::kOrder[q][0]]), acc[0][j]);
+    }
+    const int *eb = exponents[0];
+    int ea[1] = {a.s[0].exponent()}, row[1] = {OpA::row_of(0, lr)};
+    if (any_odd(acc)) {      // the wave's rows once more from the fp32 operands
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[0][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        eb = exponents[1], ea[0] = 0;
+#pragma unroll 1
+        for (int k0 = 0; k0 < K; k0 += kBK) {
+            load(x[0], k0);
+            if (K % 4 && k0 + kBK > K) a.cut(x[0], k0, K);
+            plain_step<BKC>(acc, x[0].x, Bp, g.ldb, nl, k0, K, lr, lc);
+        }
+    }
+    if constexpr (!AKC)
+        if (g.colsum && n0 == 0) {
+            csum = csum + __shfl_xor(csum, 16, 64);
+            csum += __shfl_xor(csum, 32, 64);
+            if (lc == 0 && lr < ml) g.colsum[(int64_t)range * g.M + m0 + lr] = csum;
+        }
+    finish<true, 1, NT, MODE>(g, acc, row, m0, 16, n0, lc, ea, Columns{eb, biases}, range, id % g.tn);
 }
 
 // C[M,N] = the sum of `ranges` partial results `stride` floats apart (whole 16-byte groups: the last may reach beyond M N),
@@ -1054,11 +1169,13 @@ __global__ __launch_bounds__(kThreads) void k_gemm_reduce(const float *__restric
 }
 
 // Which kernel: the one with B's rows kept in LDS (`steps` of k, 4 or 8; `per` blocks of 32 rows to a workgroup, `groups` of
-// them), or the staged one with tiles of bm x bn and k in `ranges` of ks.
+// them), the one that asks for everything at once (`once`, tiles of 64 x 64), or the staged one with tiles of bm x bn; k in `ranges` of ks.
 struct Plan {
     int steps, per, groups;
+    bool once;
     int bm, bn, tm, tn, ranges, ks;
 };
+
 
 // Kept rows of B, from 128 to 256 k and where workgroups of 256 rows x 128 columns are enough for most CUs: 32768 x 1024,
 // K = 256 64 us (staged 87, both with bias and ReLU), 24576 x 2048, K = 128 with a gate 100 us (staged 127), 8192 x 776, K = 256
@@ -1069,7 +1186,9 @@ constexpr int kHalfK = 128;
 
 // Staged: 128 x 128 tiles where, with k cut into ranges, they are three for two CUs; else 128 x 64 if those are; else 64 x 64.
 // 32768 x 256, K = 1024 (512 tiles) 60 us, 77, 80; 16384 x 256, K = 1024 (256 tiles) 47, 41, 48 us; 2381 x 1024, K = 256
-// (152, 304, 608 tiles) 16.2, 15.9, 14.3 us; 300 x 256, K = 256 13.9, 10.3, 8.6 us.
+// (152, 304, 608 tiles) 16.2, 15.9, 14.3 us; 300 x 256, K = 256 13.9, 10.3, 8.6 us.  Those of 64 x 64 all at once where a tile's k
+// is at most 256 or can be cut into ranges that are, and that makes no more than two workgroups for a CU: 300 x 256, K = 256
+// 7.0 us, 1000 x 256, K = 1024 (256 workgroups) 11.9 us staged 13.2, 2381 x 256, K = 1024 (608) 20.8 us, staged 19.1.
 // The partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k.
 Plan plan_of(int M, int N, int K, bool may_cut) {
     Plan p{};
@@ -1095,15 +1214,20 @@ Plan plan_of(int M, int N, int K, bool may_cut) {
     }
     p.tm = (M + p.bm - 1) / p.bm;
     p.tn = (N + p.bn - 1) / p.bn;
-    const int64_t n = ranges(tiles(p.bm, p.bn));
-    p.ks = (int)((K + n - 1) / n + 2 * kBK - 1) / (2 * kBK) * (2 * kBK);
+    int64_t n = ranges(tiles(p.bm, p.bn));
+    if (p.bm == 64 && K >= kHalfK) {
+        const int64_t parts = (K + 255) / 256;
+        if (parts == 1 || (may_cut && parts * tiles(64, 64) <= 512)) p.once = true, n = parts;
+    }
+    const int whole = p.once ? kBK : 2 * kBK;
+    p.ks = (int)((K + n - 1) / n + whole - 1) / whole * whole;
     p.ranges = (K + p.ks - 1) / p.ks;
     return p;
 }
 
 template <class S, bool AKC, bool BKC, int MODE>
 void launch_staged(const GemmArgs &g, const Plan &p, hipStream_t s) {
-    const dim3 grid((unsigned)(p.tm * p.tn), (unsigned)p.ranges);
+    const dim3 grid((unsigned)(p.tm * p.tn * p.ranges));
     if (p.bm == 64) hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 1, 4, MODE>), grid, dim3(kThreads), 0, s, g);
     else if (p.bn == 64) hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 2, 4, MODE>), grid, dim3(kThreads), 0, s, g);
     else hipLaunchKernelGGL((k_gemm<S, AKC, BKC, 2, 8, MODE>), grid, dim3(kThreads), 0, s, g);
@@ -1113,7 +1237,7 @@ void launch_staged(const GemmArgs &g, const Plan &p, hipStream_t s) {
 // held to their own size, however far below the largest.
 template <bool AKC, bool BKC, int MODE>
 void launch(GemmArgs g, const Plan &p, hipStream_t s) {
-    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn;
+    g.ks = p.ks, g.tm = p.tm, g.tn = p.tn, g.ranges = p.ranges;
     if constexpr (MODE == kGrad) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
     else if (g.K < kHalfK) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
     else {
@@ -1125,6 +1249,12 @@ void launch(GemmArgs g, const Plan &p, hipStream_t s) {
                 else hipLaunchKernelGGL((k_gemm_resident<BKC, 8, 8, MODE>), grid, block, 0, s, g, p.per);
                 return;
             }
+        }
+        if (p.once) {
+            const dim3 grid((unsigned)(p.tm * p.tn * p.ranges));
+            if (p.ks <= 128) hipLaunchKernelGGL((k_gemm_once<AKC, BKC, 4, MODE>), grid, dim3(kThreads), 0, s, g);
+            else hipLaunchKernelGGL((k_gemm_once<AKC, BKC, 8, MODE>), grid, dim3(kThreads), 0, s, g);
+            return;
         }
         launch_staged<Half2, AKC, BKC, MODE>(g, p, s);
     }

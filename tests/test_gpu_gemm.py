@@ -280,8 +280,8 @@ def test_loss_gradients_of_an_infinite_upstream_gradient(fwp):
         assert float((g.double() - w)[~odd].abs().max() if bool((~odd).any()) else 0.0) <= 2e-5 * 10, name
 
 
-# 64 x 64, 128 x 64 and 128 x 128 tiles, k in ranges; B's rows kept in LDS (4 and 8 steps of k, whole and not)
-HALF_SHAPES = [(70, 130, 128), (8190, 509, 300), (2100, 3001, 260), (131, 776, 3001), (6433, 1030, 131), (6433, 1030, 200),
+# 64 x 64 (all at once, cut or not; step by step), 128 x 64 and 128 x 128 tiles, k in ranges; B's rows kept in LDS (4 and 8 steps of k, whole and not)
+HALF_SHAPES = [(70, 130, 128), (3, 5, 131), (65, 66, 256), (200, 70, 257), (64, 64, 2111), (8190, 509, 300), (2100, 3001, 260), (131, 776, 3001), (6433, 1030, 131), (6433, 1030, 200),
                (3201, 2048, 256)]
 
 
@@ -298,7 +298,7 @@ def test_products_of_two_fp16_parts(fwp, M, N, K, layout, case):
         b = b * torch.exp2(40 * (0.5 - (step - 0.5).abs()))
     elif case == "sparse":
         a, b = a * (randn(M, K, seed=6) > 2), b * (randn(N, K, seed=7) > 2) * 1e-20
-        a[5], b[3] = 0, 0
+        a[M // 2], b[N // 2] = 0, 0
     bias, residual, gate = randn(N, seed=3), randn(M, N, seed=4), randn(M, N, seed=5)
     x, y = a.double(), b.double()
     raw, mag = x @ y.t(), x.abs() @ y.abs().t()
@@ -314,7 +314,7 @@ def test_products_of_two_fp16_parts(fwp, M, N, K, layout, case):
         assert bool(((got.double() - want).abs() <= err + 2 * EPS * (raw.abs() + bias.abs() + residual.abs())).all())
 
 
-@pytest.mark.parametrize("M,N,K", [(8190, 509, 300), (6433, 1030, 200), (3201, 2048, 128)])
+@pytest.mark.parametrize("M,N,K", [(8190, 509, 300), (6433, 1030, 200), (3201, 2048, 128), (1000, 70, 200), (1000, 130, 700)])
 @pytest.mark.parametrize("layout", [NT, NN, TN])
 def test_infinities_in_larger_products(fwp, M, N, K, layout):
     a, b = randn(M, K, seed=1), randn(N, K, seed=2)
