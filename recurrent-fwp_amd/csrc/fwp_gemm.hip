@@ -307,10 +307,10 @@ struct Direct {
 
 // B: a thread's share of the loads of a workgroup's ROWS rows and of their split parts' LDS writes.  KC: a task is one
 // k-chunk of one row; otherwise of VEC neighbouring rows.  A row's four k-chunks are in one wave.
-template <bool KC, int ROWS>
+template <bool KC, int ROWS, int WAVES>
 struct Staged {
-    static constexpr int VEC = KC ? 1 : ROWS / 64;
-    static constexpr int kUnits = ROWS / 64;
+    static constexpr int kUnits = ROWS / (16 * WAVES);
+    static constexpr int VEC = KC ? 1 : kUnits;
     struct Raw {
         float x[kUnits][8];
     };
@@ -323,7 +323,7 @@ struct Staged {
         r = KC ? tid / 4 : (tid / 64 * 16 + tid % 16) * VEC;
         unit = c * ROWS + unit_of(r, c);
     }
-    __device__ __forceinline__ int row_of(int t) const { return KC ? r + 64 * t : r + t; }
+    __device__ __forceinline__ int row_of(int t) const { return KC ? r + 16 * WAVES * t : r + t; }
     __device__ __forceinline__ void aim(int64_t ld, int k0, int K) {
         if constexpr (KC) {
             const unsigned o = (unsigned)(r * ld + 4 * c) * 4;
@@ -337,8 +337,8 @@ struct Staged {
             const v4i rs = buffer_of(P + k0, k0 < K ? (int64_t)(min(left, ROWS) - 1) * ld + (K - k0) : 0);
 #pragma unroll
             for (int t = 0; t < kUnits; t++) {
-                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], (int)(t * ld * 256), 0),
-                          b = llvm_raw_buffer_load_v4f32(rs, (int)at[1], (int)(t * ld * 256), 0);
+                const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], (int)(t * ld * 64 * WAVES), 0),
+                          b = llvm_raw_buffer_load_v4f32(rs, (int)at[1], (int)(t * ld * 64 * WAVES), 0);
 #pragma unroll
                 for (int j = 0; j < 4; j++) w.x[t][j] = a[j], w.x[t][4 + j] = b[j];
             }
@@ -372,12 +372,12 @@ struct Staged {
         return fmaxf(m, __shfl_xor(m, KC ? 2 : 32, 64));
     }
     // the wave that splits the rows of matrix-instruction tile j
-    static constexpr int owner(int j) { return KC ? j % 4 : j / VEC; }
+    static constexpr int owner(int j) { return KC ? j % WAVES : j / VEC; }
     // a unit's split parts to LDS
     template <int P>
     __device__ __forceinline__ void store(Planes<P, ROWS> &L, int t, const v4u *d) const {
 #pragma unroll
-        for (int p = 0; p < P; p++) L.u[p][0][KC ? unit + 64 * t : unit ^ t] = d[p];
+        for (int p = 0; p < P; p++) L.u[p][0][KC ? unit + 16 * WAVES * t : unit ^ t] = d[p];
     }
     // fp32 as it is: 16-byte units of a chunk's four k, [chunk][half][row]
     __device__ __forceinline__ void store_plain(v4f *L, const Raw &w) const {
@@ -547,15 +547,16 @@ __device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], co
     }
 }
 
-// A workgroup: 64 MT rows x 16 NT columns, a wave 16 MT rows of them and all columns; B's rows are staged step by step, in two
+// A workgroup of WAVES waves: a wave 16 MT rows and all 16 NT columns; B's rows are staged step by step, in two
 // alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 60 us (one 128 x 128 tile with both
 // operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6.
-template <class S, bool AKC, bool BKC, int MT, int NT, int MODE>
-__global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
-    constexpr int BM = 64 * MT, WM = 16 * MT, BN = 16 * NT;
+template <class S, bool AKC, bool BKC, int MT, int NT, int MODE, int WAVES = 4>
+__global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
+    constexpr int WM = 16 * MT, BM = WAVES * WM, BN = 16 * NT;
+    static_assert(WAVES == 4 || !S::kScaled, "four waves' changes of scales");
     typedef Planes<S::kPlanes, BN> Stage;
     typedef Direct<AKC, MT, MODE == kGrad> OpA;
-    typedef Staged<BKC, BN> OpB;
+    typedef Staged<BKC, BN, WAVES> OpB;
     typedef typename S::frag frag;
     constexpr size_t kShared = 2 * sizeof(Stage);
     static_assert(sizeof(v4f) * 8 * BN <= kShared, "fp32 of a step fits");
@@ -566,8 +567,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     __shared__ __align__(16) int changed[2][4];
     __shared__ __align__(16) float change_b[S::kScaled ? 2 : 1][S::kScaled ? BN : 4];
     __shared__ float change_a[S::kScaled ? 4 : 1][WM];
-    __shared__ int odd_waves[4];
-    __shared__ NllToken toks[MODE == kGrad && !AKC ? 4 : 1][MODE == kGrad && !AKC ? kBK : 1];
+    __shared__ int odd_waves[WAVES];
+    __shared__ NllToken toks[MODE == kGrad && !AKC ? WAVES : 1][MODE == kGrad && !AKC ? kBK : 1];
     Stage *const L = reinterpret_cast<Stage *>(shared);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
@@ -739,7 +740,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm(GemmArgs g) {
     const bool wave_odd = __any(odd != 0.f);
     if (lane == 0) odd_waves[wave] = wave_odd;
     __syncthreads();
-    if (odd_waves[0] | odd_waves[1] | odd_waves[2] | odd_waves[3]) {
+    bool odd_tile = false;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) odd_tile |= odd_waves[w] != 0;
+    if (odd_tile) {
         // the tile once more from the fp32 operands
 #pragma unroll
         for (int i = 0; i < MT; i++) {
@@ -1234,11 +1238,19 @@ void launch_staged(const GemmArgs &g, const Plan &p, hipStream_t s) {
 }
 
 // The loss gradient's products stay with Bf16x3: a word's probabilities over the tokens, or a token's over the words, are
-// held to their own size, however far below the largest.
+// held to their own size, however far below the largest.  Its elements cost an exponential each: 128 x 256 tiles of eight waves,
+// where a 128 x 128 one leaves columns over, form them once (32768 x 256, K = 32768 3.12 ms and, x^T y, 3.33; 128 x 128 3.45, 3.85).
 template <bool AKC, bool BKC, int MODE>
 void launch(GemmArgs g, const Plan &p, hipStream_t s) {
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn, g.ranges = p.ranges;
-    if constexpr (MODE == kGrad) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
+    if constexpr (MODE == kGrad) {
+        if (p.bn == 128 && g.N > 128) {
+            g.tn = (g.N + 255) / 256;
+            hipLaunchKernelGGL((k_gemm<Bf16x3, AKC, BKC, 1, 16, MODE, 8>), dim3((unsigned)(g.tm * g.tn * g.ranges)), dim3(512), 0, s, g);
+        } else {
+            launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
+        }
+    }
     else if (g.K < kHalfK) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
     else {
         if constexpr (AKC) {
