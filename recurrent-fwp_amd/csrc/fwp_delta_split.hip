@@ -44,6 +44,9 @@ struct Segments {
     float *work;
     int count, blocks;
 };
+// What a launch does: whole sequences, segments, or the segments' maps.  Known when compiled: with the choice read from the
+// arguments, uncut sequences took 0.3-0.8 % longer (32 x 32, 256 sequences of 1024 steps: backward 77.3 -> 77.9 us).
+enum { kWhole = 0, kSegments = 1, kMaps = 2 };
 template <int E, int M>
 __device__ __forceinline__ int64_t map_at(const Segments &s, int64_t seq, int j) {
     return seq * (E * M + (int64_t)(s.count - 1) * (E * M + E * E)) + E * M + (int64_t)j * (E * M + E * E);
@@ -130,15 +133,17 @@ struct OutRaw {
 // block behind the state waves, which hand it their columns of the state and of U.
 // With one state wave and the output wave a fourth wave only keeps the barriers: the four waves of a
 // 256-thread workgroup take one SIMD each, three-wave workgroups are placed unevenly.
-// MAP: the map of a segment instead; state waves mb >= NM hold the columns of D.
-template <int NE, int NM, int PF, bool OUT, bool MAP = false>   // E = 16 NE, M = 16 NM, PF = blocks in flight
-__global__ __launch_bounds__(64 * (MAP ? NM + NE + 1 : OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void k_delta_fwd_split(fwp_view q, fwp_view k, fwp_view v,
+// kMaps: the map of a segment instead; state waves mb >= NM hold the columns of D.
+template <int NE, int NM, int PF, bool OUT, int WHAT = kWhole>   // E = 16 NE, M = 16 NM, PF = blocks in flight
+__global__ __launch_bounds__(64 * (WHAT == kMaps ? NM + NE + 1 : OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void k_delta_fwd_split(fwp_view q, fwp_view k, fwp_view v,
                                                                   fwp_view beta, float *__restrict__ W,
                                                                   fwp_out_view out,
                                                                   float *__restrict__ vdiff,
                                                                   float *__restrict__ ckpt,
                                                                   float *__restrict__ aux, int H, int L,
-                                                                  int chunk, int nchunk, Segments segs) {
+                                                                  int chunk, int nchunk, Segments cut) {
+    constexpr bool MAP = WHAT == kMaps;
+    const Segments segs = WHAT == kWhole ? Segments{nullptr, 1, 0} : cut;
     constexpr int E = 16 * NE, M = 16 * NM, NS = MAP ? NM + NE : NM;
     // lower(Q K^T)^T: with one state wave that wave forms it itself, with several the preparing
     // wave does it once for all
@@ -534,13 +539,15 @@ constexpr int quad_lds_mats() {
 }
 
 // PW = 2: P on two waves, one with the products of Pm, one with the others.
-// MAP: the map of a segment instead, by P and C alone; C's waves mb >= NM hold the columns of D^T.
-template <int NE, int NM, int WR, int PW, int PF, bool MAP = false>
-__global__ __launch_bounds__(64 * (MAP ? PW + NM + NE : PW + NM + 2 * WR)) void k_delta_bwd_quad(
+// kMaps: the map of a segment instead, by P and C alone; C's waves mb >= NM hold the columns of D^T.
+template <int NE, int NM, int WR, int PW, int PF, int WHAT = kWhole>
+__global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * WR)) void k_delta_bwd_quad(
     fwp_view q, fwp_view k, fwp_view beta, const float *__restrict__ vdiff, fwp_view go,
     const float *__restrict__ ckpt, const float *__restrict__ aux, float *__restrict__ gq,
     float *__restrict__ gk, float *__restrict__ gv, float *__restrict__ gbeta, int H, int L, int chunk,
-    int nchunk, Segments segs) {
+    int nchunk, Segments cut) {
+    constexpr bool MAP = WHAT == kMaps;
+    const Segments segs = WHAT == kWhole ? Segments{nullptr, 1, 0} : cut;
     constexpr int E = 16 * NE, M = 16 * NM, NEW = NE / WR, NC = MAP ? NM + NE : NM;
     static_assert(NE % WR == 0, "key tiles divide evenly over the waves of a role");
     __shared__ LdsMat pc[2][NM + NE * NM];     // P -> C: Pm^T dO per mb, then Q^T dO per (eb, mb)
@@ -983,13 +990,17 @@ template <int NE, int NM>
 void launch_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out, float *vdiff,
                 float *ckpt, float *aux, int nseq, int H, int L, int chunk, int nchunk, const Segments &segs, hipStream_t s) {
     if constexpr (segment_dims(NE, NM))
-        if (segs.count > 1)
-            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false, true>), dim3(nseq * (segs.count - 1)),
+        if (segs.count > 1) {
+            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false, kMaps>), dim3(nseq * (segs.count - 1)),
                                dim3(64 * (NM + NE + 1)), 0, s, q, k, v, beta, W, out, nullptr, nullptr, nullptr, H, L, chunk, nchunk, segs);
-    const int wgs = nseq * segs.count;
+            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), (NM <= 2), kSegments>), dim3(nseq * segs.count),
+                               dim3(64 * (NM <= 2 ? 4 : NM + 1)), 0, s, q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk,
+                               nchunk, segs);
+            return;
+        }
     if constexpr (NM <= 2) {
-        if (NM == 1 || (int64_t)wgs * (NM + 2) <= 1536) {
-            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), true>), dim3(wgs),
+        if (NM == 1 || (int64_t)nseq * (NM + 2) <= 1536) {
+            hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), true>), dim3(nseq),
                                dim3(64 * (NM == 1 ? 4 : NM + 2)),
                                0,
                                s, q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk, segs);
@@ -997,7 +1008,7 @@ void launch_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp
         }
     }
     if constexpr (NM > 1)
-        hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false>), dim3(wgs), dim3(64 * (NM + 1)),
+        hipLaunchKernelGGL((k_delta_fwd_split<NE, NM, fwd_ring(NE), false>), dim3(nseq), dim3(64 * (NM + 1)),
                            0, s,
                            q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk, segs);
 }
@@ -1059,10 +1070,14 @@ int split_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, f
     if (E == 16 * ne && M == 16 * nm) {                                                                     \
         static_assert(quad_lds_mats<ne, nm, wr>() * sizeof(LdsMat) + 192 <= 160 * 1024, "LDS of the hand-over"); \
         if constexpr (segment_dims(ne, nm))                                                                 \
-            if (segs.count > 1)                                                                             \
-                hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf, true>), dim3(N * H * (segs.count - 1)), dim3(64 * (pw + nm + ne)), \
+            if (segs.count > 1) {                                                                           \
+                hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf, kMaps>), dim3(N * H * (segs.count - 1)), dim3(64 * (pw + nm + ne)), \
                                    0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
-        hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf>), dim3(N * H * segs.count), dim3(64 * (pw + nm + 2 * wr)), \
+                hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf, kSegments>), dim3(N * H * segs.count), dim3(64 * (pw + nm + 2 * wr)), \
+                                   0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
+                return (int)hipGetLastError();                                                              \
+            }                                                                                               \
+        hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf>), dim3(N * H), dim3(64 * (pw + nm + 2 * wr)), \
                            0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
         return (int)hipGetLastError();                                                                      \
     }
