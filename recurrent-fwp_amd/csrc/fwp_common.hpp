@@ -190,7 +190,7 @@ int deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *be
 int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,
                       const float *gbeta, float *gqkvb, int T, int B, int H, int D, float q_scale, hipStream_t s);
 
-// fp32 matrix products on the bf16 matrix cores (fwp_matmul); `nll`: A holds logits and stands for the gradient of
+// fp32 matrix products on the 16-bit matrix cores (fwp_matmul); `nll`: A holds logits and stands for the gradient of
 // the loss that nll_fwd computed from them.
 struct NllView {
     const float *lse, *stats, *gloss;      // lse [rows] or stats [rows,2], whichever nll_fwd wrote

@@ -15,7 +15,7 @@
 // 2^-24 of itself or to 2^-126, whichever is more.
 //
 // An operand that the 16-bit numbers cannot hold (infinity, NaN, for bf16 the last 2^-9 below fp32's largest) leaves NaN or infinity in
-// the sums: a tile with an element that is not finite is formed again on the fp32 matrix instructions, in two to four times its time.
+// the sums: a tile with an element that is not finite is formed again on the fp32 matrix instructions, a third of the rate or less.
 //
 // v_mfma_f32_16x16x32_bf16 makes 1.7-2.1 PFLOP/s with random operands and the f16 form 1.5 (2.45 with zeros: the chip's power is
 // the limit), i.e. 490 TFLOP/s of Half2's products and 280-350 of Bf16x3's, where the fp32 matrix instructions make 155.

@@ -1,6 +1,6 @@
 """The language model's matrix products, negative log-likelihood and LayerNorm kernels through the C ABI, against
 float64.  Tolerance of a product: every one of the up to six roundings per 32 terms, and the split of an operand into
-three bf16 numbers, is at most 2^-24 of the sum of the terms' magnitudes."""
+three bf16 numbers (K < 128), is at most 2^-24 of the sum of the terms' magnitudes; into two fp16 numbers: see the tests."""
 import ctypes
 
 import pytest
