@@ -1069,7 +1069,7 @@ int split_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, f
 #define Q(ne, nm, wr, pw, pf)                                                                               \
     if (E == 16 * ne && M == 16 * nm) {                                                                     \
         static_assert(quad_lds_mats<ne, nm, wr>() * sizeof(LdsMat) + 192 <= 160 * 1024, "LDS of the hand-over"); \
-        if constexpr (segment_dims(ne, nm))                                                                 \
+        if constexpr (segment_dims(ne, nm) && (ne + nm > 2 || pf == 2))                                     \
             if (segs.count > 1) {                                                                           \
                 hipLaunchKernelGGL((k_delta_bwd_quad<ne, nm, wr, pw, pf, kMaps>), dim3(N * H * (segs.count - 1)), dim3(64 * (pw + nm + ne)), \
                                    0, s, q, k, beta, vdiff, go, ckpt, aux, gq, gk, gv, gbeta, H, L, chunk, nchunk, segs); \
