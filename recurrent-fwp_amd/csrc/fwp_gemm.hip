@@ -2,12 +2,14 @@
 // numbers, their products summed in fp32.
 //
 // Half2 (K >= 128): x s = h + m, h = fp16(x s), m = fp16(x s - h), three products m h', h m', h h'.  s is a power of two for each row
-// of an operand (the rows of C, the columns of C).  h and m hold x to the last or the last but one of its 24 bits; m m' is below
+// of an operand (the rows of C, the columns of C).  h and m hold x to 2^-23 of itself; m m' is below
 // 2^-22 |x x'|.  That is 7e-8 of a product, at random, where a sum's roundings, three per 32 terms, make more: relative error
 // against float64 (N(0,1) operands, 2-norm; in brackets Bf16x3, then hipBLASLt's fp32): K = 128 1.39e-7 (1.61e-7), 32768 x 1024, K = 256
 // 1.87e-7 (2.36e-7, 2.9e-7); 32768 x 256, K = 1024 3.6e-7 (4.9e-7, 5.7e-7); 1024 x 256, K = 32768 in ranges 3.9e-7 (5.75e-7, 2.0e-6).
-// fp16 has few exponents: s brings a row's largest element so far to [8, 16).  Elements down to 2^-7 of that keep all their bits,
-// smaller ones 2^-28 of it.  One beyond 65504 / s (a row that grows 4096-fold along k) moves s, and the row's results so far with it.
+// fp16 has few exponents: s brings a row's largest element so far to [2^13, 2^14).  One beyond 65504 / s (a row that grows fourfold
+// or more along k) moves s, and the row's results so far with it.  An element below about 2^-20 of its row's largest would lose bits: the
+// waves look for those, and what two numbers leave of them is multiplied apart, so that an element counts to 2^-19 of itself or better
+// whatever is in its row (a result may be made of small elements alone).  The search costs 4 to 7 us of 65, 32768 x 256, K = 1024.
 //
 // Bf16x3 (smaller K, and the loss's gradient): x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest: 3 x 8 significant bits and
 // their signs hold all 24), six products, h h', h m', m h', m m', h l', l h'; the three left out are below 2^-26 |x x'|.  bf16
@@ -116,6 +118,12 @@ __device__ __forceinline__ NllToken nll_token(const NllArgs &a, int token) {
 // the four chunks' loads of one run are 64 bytes of a row.
 __device__ __forceinline__ constexpr int k_of(int c, int e) { return e < 4 ? 4 * c + e : 16 + 4 * c + (e - 4); }
 
+// Sizes of scaled elements.  Beyond kLargest they do not fit fp16.  From 2^-2 on two fp16 numbers hold them to 2^-23 of themselves, at
+// kSmall to 2^-19: what is left of smaller ones is multiplied apart (add_rests), the whole of those below kTiny, fp16's smallest normal
+// number (products with others cut the sum they are added to at 2^-24 of what that number would give).  With one below kLeast the whole
+// tile is formed on fp32.
+constexpr float kLargest = 65504.f, kSmall = 0x1p-6f, kTiny = 0x1p-14f, kLeast = 0x1p-31f;
+
 // x = h + m (+ l) for eight values.  Half2: two fp16 numbers of x * scale; Bf16x3: three bf16 numbers of x.
 struct Half2 {
     typedef _Float16 frag __attribute__((ext_vector_type(8)));
@@ -132,10 +140,36 @@ struct Half2 {
         const h2 h = __builtin_bit_cast(h2, d[0]);
         d[1] = pack(fmaf(a, scale, -(float)h[0]), fmaf(b, scale, -(float)h[1]));
     }
+    // what is left of an element (scaled)
+    static __device__ __forceinline__ float rest(float x) {
+        const float h = (float)(_Float16)x, r = x - h;
+        return fabsf(h) < kTiny ? x : r - (float)(_Float16)r;
+    }
+    // the two numbers of elements below kTiny become zero
+    static __device__ __forceinline__ void drop_tiny(v4u *d) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const unsigned keep = (d[0][j] & 0x7c00u ? 0xffffu : 0u) | (d[0][j] & 0x7c000000u ? 0xffff0000u : 0u);
+            d[0][j] &= keep, d[1][j] &= keep;
+        }
+    }
     static __device__ __forceinline__ v4f mma(frag x, frag y, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, c, 0, 0, 0); }
     // the planes (of A, of B) that are multiplied, in this order
     static constexpr int kProducts = 3;
     static constexpr int kOrder[3][2] = {{1, 0}, {0, 1}, {0, 0}};
+};
+
+// The same with the second number 2^11 times as large: its products are summed apart, and elements from 2^-16 on (of a row's largest
+// in [2^14, 2^15)) are held to 2^-20 of themselves.
+struct WideHalf2 : Half2 {
+    static constexpr float kRest = 0x1p-11f;      // what those sums are multiplied with
+    static constexpr float kLeast = 0x1p-16f;
+    static __device__ __forceinline__ void split2(float a, float b, float scale, unsigned *d) {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        d[0] = pack(a * scale, b * scale);
+        const h2 h = __builtin_bit_cast(h2, d[0]);
+        d[1] = pack(fmaf(a, scale, -(float)h[0]) / kRest, fmaf(b, scale, -(float)h[1]) / kRest);
+    }
 };
 
 struct Bf16x3 {
@@ -162,31 +196,107 @@ __device__ __forceinline__ void split_pair(const float *x, int j, float scale, v
     for (int p = 0; p < S::kPlanes; p++) d[p][j] = y[p];
 }
 
-// A row's scale: the power of two that takes `largest` into [2^3, 2^4) (0 for 0: nothing seen yet), and how large an element
-// may be under it.
+// The largest and the smallest magnitude of eight elements that are not NaN.  By hand: fmaxf() and fminf() quiet every operand first, 104
+// instead of 40 instructions a step.
+__device__ __forceinline__ float abs_max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float abs_min3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float abs_max8(const float *x) {
+    return abs_max3(abs_max3(x[0], x[1], x[2]), abs_max3(x[3], x[4], x[5]), abs_max3(x[6], x[7], x[7]));
+}
+__device__ __forceinline__ float abs_min8(const float *x) {
+    return abs_min3(abs_min3(x[0], x[1], x[2]), abs_min3(x[3], x[4], x[5]), abs_min3(x[6], x[7], x[7]));
+}
+// the same of those that are not zero, to one unit of the last place (NaN: all are zero)
+__device__ __forceinline__ float nonzero_min8(const float *x) {
+    unsigned m = ~0u;
+#pragma unroll
+    for (int e = 0; e < 8; e++) m = min(m, (__float_as_uint(x[e]) << 1) - 1);
+    return __uint_as_float(m >> 1);
+}
+__device__ __forceinline__ float pick(const float *x, int e) {      // x[e] of a wave-uniform e, in registers
+    typedef float v8f __attribute__((ext_vector_type(8)));
+    const v8f v = {x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
+    return v[e];
+}
+
+// A row's scale: the power of two that takes its largest element so far into [2^13, 2^14).
 struct Scale {
-    float s, limit;
-    __device__ __forceinline__ void none() { s = 0.f, limit = 0.f; }
+    static constexpr unsigned kNone = 254u << 23;      // 2^127: no element but zeros yet, or below 2^-111
+    float s, first;                                    // first: the largest s so far
+    __device__ __forceinline__ void none() { s = __uint_as_float(kNone); }
     __device__ __forceinline__ void one() { s = 1.f; }
-    __device__ __forceinline__ float inverse() const { return s == 0.f ? 0.f : __uint_as_float((254u << 23) - __float_as_uint(s)); }
-    __device__ __forceinline__ int exponent() const { return s == 0.f ? 0 : 127 - (int)(__float_as_uint(s) >> 23); }      // of the inverse
-    __device__ __forceinline__ void set(float largest) {
-        const int b = 257 - (int)(__float_as_uint(largest) >> 23);
-        s = largest == 0.f ? 0.f : __uint_as_float((unsigned)min(max(b, 4), 250) << 23);
-        limit = 65504.f * inverse();
+    __device__ __forceinline__ int exponent() const { return 127 - (int)(__float_as_uint(s) >> 23); }      // of 1 / s
+    // top: 14 where no larger element can come
+    __device__ __forceinline__ void set(float largest, int top = 13) {
+        s = __uint_as_float((unsigned)min(254 + top - (int)(__float_as_uint(largest) >> 23), 254) << 23);
     }
     // for a row with an element of size `largest`: what its results so far are multiplied with
     __device__ __forceinline__ float fit(float largest) {
-        if (!(largest > limit)) return 1.f;
-        const float was = inverse();
+        if (!(largest * s > kLargest)) return 1.f;
+        const unsigned was = __float_as_uint(s);
         set(largest);
-        return was == 0.f ? 1.f : s * was;
+        if (was == kNone) first = s;
+        return ldexpf(1.f, (int)(__float_as_uint(s) >> 23) - (int)(was >> 23));
     }
+    // s was once so much larger that the row's results so far may not be what fp32 holds
+    __device__ __forceinline__ bool shrunk() const { return __float_as_uint(s) != kNone && s < first * 0x1p-25f; }
 };
 
-__device__ __forceinline__ float abs_max8(const float *x, float m) {
+__device__ __forceinline__ void drop_tiny8(float *x, float s) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(x[e]));
+    for (int e = 0; e < 8; e++) x[e] = fabsf((float)(_Float16)(x[e] * s)) < kTiny ? 0.f : x[e];
+}
+
+// A lane's elements of ROWS rows, scaled: the largest magnitude, and each row's before that; the smallest; the smallest that is not zero
+// (a third more instructions, but where there are zeros, ReLU's, no second look).
+template <int ROWS>
+__device__ __forceinline__ float largest_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS], float (&m)[ROWS]) {
+    float all = 0.f;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) m[i] = abs_max8(x[i]), all = abs_max3(all, m[i] * s[i].s, 0.f);
+    return all;
+}
+template <int ROWS>
+__device__ __forceinline__ float smallest_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS]) {
+    float all = INFINITY;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) all = abs_min3(all, abs_min8(x[i]) * s[i].s, INFINITY);
+    return all;
+}
+template <int ROWS>
+__device__ __forceinline__ float smallest_nonzero_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS]) {
+    float all = INFINITY;
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) all = abs_min3(all, nonzero_min8(x[i]) * s[i].s, INFINITY);
+    return all;
+}
+// Which of the wave's lanes' elements are small (bit e: those at e; bit 8: some are tiny); far: one is too small even for its rest.  Short
+// code: it is run so rarely that it is fetched each time.
+constexpr unsigned kSomeTiny = 1u << 8;
+template <int ROWS>
+__device__ __forceinline__ unsigned small_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS], bool &far) {
+    const float least = smallest_nonzero_of(x, s);
+    if (!__any(least < kSmall)) return 0;
+    far |= least < kLeast;
+    unsigned m = __any(least < kTiny) ? kSomeTiny : 0u;
+#pragma unroll 1
+    for (int e = 0; e < 8; e++) {
+        bool small = false;
+#pragma unroll
+        for (int i = 0; i < ROWS; i++) {
+            const float v = pick(x[i], e);
+            small |= v != 0.f && fabsf(v * s[i].s) < kSmall;
+        }
+        m |= __any(small) ? 1u << e : 0u;
+    }
     return m;
 }
 
@@ -547,6 +657,43 @@ __device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], co
     }
 }
 
+// What two fp16 numbers leave of small elements, in fp32: the step's products of the rest of A with B and of A with the rest of B, for
+// the k of bit e of `small_a` (a wave's rows) and of `small_b`.  x, f: the step's elements of A, split.  has, rest: whether column tile j has a
+// rest at e, and this lane's of it.
+template <int MT, int NT, class Has, class Rest>
+__device__ __forceinline__ void add_rests(v4f (&acc)[MT][NT], const float (&x)[MT][8], const Scale (&s)[MT], unsigned small_a, unsigned small_b,
+                                          v4u (&f)[MT][Half2::kPlanes], const Planes<Half2::kPlanes, 16 * NT> &L, const int (&unit)[2], Has has, Rest rest) {
+    if (small_a & kSomeTiny)
+#pragma unroll
+        for (int i = 0; i < MT; i++) Half2::drop_tiny(f[i]);
+#pragma unroll 1
+    for (unsigned left = (small_a | small_b) & 0xff; left; left &= left - 1) {
+        const int e = __builtin_ctz(left);
+        float v[MT];
+#pragma unroll
+        for (int i = 0; i < MT; i++) v[i] = pick(x[i], e) * s[i].s;
+        if (small_b >> e & 1)
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                if (has(j, e)) {
+                    const float y = rest(j, e);
+#pragma unroll
+                    for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, v[i], acc[i][j], 0, 0, 0);
+                }
+        if (small_a >> e & 1) {
+#pragma unroll
+            for (int i = 0; i < MT; i++) v[i] = Half2::rest(v[i]);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const _Float16 *const h = reinterpret_cast<const _Float16 *>(&L.u[0][0][unit[j % 2] + 16 * j]) + e;
+                const float y = (float)h[0] + (float)h[sizeof(L.u[0]) / sizeof(_Float16)];
+#pragma unroll
+                for (int i = 0; i < MT; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y, v[i], acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+}
+
 // A workgroup of WAVES waves: a wave 16 MT rows and all 16 NT columns; B's rows are staged step by step, in two
 // alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 60 us (one 128 x 128 tile with both
 // operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6.
@@ -563,9 +710,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     __shared__ __align__(16) char shared[kShared];
     __shared__ __align__(16) int exponents[BN];
     __shared__ __align__(16) float biases[BN];
-    // a wave that changed scales of B's rows for step k0 leaves k0 and what those rows' results so far are multiplied with
-    __shared__ __align__(16) int changed[2][4];
+    // Of the steps' B, alternately: what each wave did to its rows' scales (kChange: what their results so far are multiplied with is in
+    // change_b) and which of its elements are small (bit e; scaled_b: its rows' elements)
+    constexpr int kChange = 1 << 9;
+    __shared__ __align__(16) int news[2][4];
     __shared__ __align__(16) float change_b[S::kScaled ? 2 : 1][S::kScaled ? BN : 4];
+    __shared__ v4f scaled_b[S::kScaled ? 2 : 1][2][4][S::kScaled ? BN : 1];
     __shared__ float change_a[S::kScaled ? 4 : 1][WM];
     __shared__ int odd_waves[WAVES];
     __shared__ NllToken toks[MODE == kGrad && !AKC ? WAVES : 1][MODE == kGrad && !AKC ? kBK : 1];
@@ -606,11 +756,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     }
 #pragma unroll
     for (int t = 0; t < OpB::kUnits; t++) b.s[t].none();
-    if (tid < 8) changed[tid / 4][tid % 4] = -1;
 
     typename OpA::Raw ra[2];
     typename OpB::Raw rb[2];
     bool change = false;      // of scales of A's rows
+    unsigned small_a = 0;
+    bool far = false;         // an element too small even for that
     v4u fa[2][MT][S::kPlanes];
     float part_sum[MT];       // of a step's elements of A's rows
     const auto split_a = [&](int i, int j, const typename OpA::Raw &x, v4u (*f)[S::kPlanes], bool whole, int k0) {
@@ -644,35 +795,51 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
         for (int i = 0; i < MT; i++) csum[i] += part_sum[i];
     };
     // What a step's split needs: zeros beyond K, and (parity: the step's) scales that its elements fit
-    const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) {
+    const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) __attribute__((always_inline)) {
         a.hand_over(x, lane);
         if (ke % 4 && k0 + kBK > ke) a.cut(x, k0, ke), b.cut(y, k0, ke);
         if constexpr (S::kScaled) {
             float ma[MT], mb[OpB::kUnits];
-            bool beyond_a = false, beyond_b = false;
+            const bool beyond = fmaxf(largest_of(x.x, a.s, ma), largest_of(y.x, b.s, mb)) > kLargest;
+            float la = smallest_nonzero_of(x.x, a.s), lb = smallest_of(y.x, b.s);
+            int word = 0;
+            small_a = 0;
+            if (__any(beyond || fminf(la, lb) < kSmall)) {
+                if (__any(beyond)) {
+                    change = true, word = kChange;
+                    la = lb = 0.f;
 #pragma unroll
-            for (int i = 0; i < MT; i++) ma[i] = abs_max8(x.x[i], 0.f), beyond_a |= ma[i] > a.s[i].limit;
+                    for (int i = 0; i < MT; i++) change_a[wave][OpA::row_of(i, lr)] = a.s[i].fit(OpA::of_row(ma[i])), far |= a.s[i].shrunk();
 #pragma unroll
-            for (int t = 0; t < OpB::kUnits; t++) mb[t] = abs_max8(y.x[t], 0.f), beyond_b |= mb[t] > b.s[t].limit;
-            if (__any(beyond_a | beyond_b)) {
-                change = true;
+                    for (int t = 0; t < OpB::kUnits; t++) change_b[parity][b.row_of(t)] = b.s[t].fit(OpB::of_row(mb[t])), far |= b.s[t].shrunk();
+                }
+                if (__any(la < kSmall)) small_a = small_of(x.x, a.s, far);
+                if (__any(lb < kSmall)) word |= small_of(y.x, b.s, far);
+                if (word & 0xff)
 #pragma unroll
-                for (int i = 0; i < MT; i++) change_a[wave][OpA::row_of(i, lr)] = a.s[i].fit(OpA::of_row(ma[i]));
+                    for (int t = 0; t < OpB::kUnits; t++)
 #pragma unroll
-                for (int t = 0; t < OpB::kUnits; t++) change_b[parity][b.row_of(t)] = b.s[t].fit(OpB::of_row(mb[t]));
-                if (lane == 0) changed[parity][wave] = k0;
+                        for (int h = 0; h < 2; h++)
+                            scaled_b[parity][h][b.c][b.row_of(t)] =
+                                v4f{y.x[t][4 * h], y.x[t][4 * h + 1], y.x[t][4 * h + 2], y.x[t][4 * h + 3]} * b.s[t].s;
+                if (word & kSomeTiny)
+#pragma unroll
+                    for (int t = 0; t < OpB::kUnits; t++) drop_tiny8(y.x[t], b.s[t].s);
             }
+            if (lane == 0) news[parity][wave] = word;
         }
     };
-    // results so far to the scales of step k0
-    const auto follow = [&](int k0, int parity) {
+    // Before step k0's products (x: its elements of A): results so far to its scales, and what is left of its small elements
+    const auto follow = [&](int parity, const typename OpA::Raw &x) __attribute__((always_inline)) {
         if constexpr (S::kScaled) {
-            const int4 w = *reinterpret_cast<const int4 *>(changed[parity]);
-            if (__builtin_amdgcn_readfirstlane(w.x == k0 | w.y == k0 | w.z == k0 | w.w == k0)) {
-                const bool of[4] = {w.x == k0, w.y == k0, w.z == k0, w.w == k0};
+            const int4 w = *reinterpret_cast<const int4 *>(news[parity]);
+            const int of[4] = {__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
+                               __builtin_amdgcn_readfirstlane(w.w)};
+            const int all = of[0] | of[1] | of[2] | of[3];
+            if (all & kChange) {
 #pragma unroll
                 for (int j = 0; j < NT; j++)
-                    if (of[OpB::owner(j)])
+                    if (of[OpB::owner(j)] & kChange)
 #pragma unroll
                         for (int i = 0; i < MT; i++) acc[i][j] *= *reinterpret_cast<const v4f *>(change_b[parity] + 16 * j + 4 * lc);
             }
@@ -683,24 +850,26 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
 #pragma unroll
                     for (int j = 0; j < NT; j++) acc[i][j] *= change_a[wave][OpA::row_of(i, lr)];
             }
+            if (small_a | (all & 0xff))
+                add_rests(acc, x.x, a.s, small_a, all & 0xff, fa[parity], L[parity], unit, [&](int j, int e) { return of[OpB::owner(j)] >> e & 1; },
+                          [&](int j, int e) { return Half2::rest(reinterpret_cast<const float *>(&scaled_b[parity][e / 4][lc][16 * j + lr])[e % 4]); });
         }
     };
     aim(kb);
     load(ra[0], rb[0], kb);
     aim(kb + kBK);
     load(ra[1], rb[1], kb + kBK);
-    if constexpr (S::kScaled) lds_barrier();      // `changed` is cleared
     prepare(ra[0], rb[0], kb, 0);
 #pragma unroll
     for (int q = 0; q < kPairs; q++) split(q, ra[0], rb[0], fa[0], L[0], kb);
     complete(ra[0], fa[0], kb);
     lds_barrier();
     // One step: the products of k0's parts, beside the split of k0 + kBK's elements and the loads of k0 + 2 kBK's.
-    const auto step = [&](auto parity, int k0) {
+    const auto step = [&](auto parity, int k0) __attribute__((always_inline)) {
         constexpr int p = decltype(parity)::value;
+        follow(p, ra[p]);
         if (k0 + 3 * kBK > ke) aim(k0 + 2 * kBK);
         load(ra[p], rb[p], k0 + 2 * kBK);
-        follow(k0, p);
         prepare(ra[p ^ 1], rb[p ^ 1], k0 + kBK, p ^ 1);
         __builtin_amdgcn_sched_barrier(0);
         frag fb[2][S::kPlanes];
@@ -737,7 +906,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
         for (int j = 0; j < NT; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++) odd = fmaf(acc[i][j][r], 0.f, odd);
-    const bool wave_odd = __any(odd != 0.f);
+    const bool wave_odd = __any(odd != 0.f || far);
     if (lane == 0) odd_waves[wave] = wave_odd;
     __syncthreads();
     bool odd_tile = false;
@@ -803,9 +972,26 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     finish<S::kScaled, MT, NT, MODE>(g, acc, row, m0, WM, n0, lc, ea, Columns{exponents, biases}, range, id % g.tn);
 }
 
+// What two fp16 numbers leave of the small elements of rows of B that are split for a whole product: bit 8 s + e of `bits` for those at
+// e of step s, `far` if one is too small even for that, and of the first kKept of those bits the values.
+template <int BN>
+struct Rests {
+    static constexpr int kKept = 896 / BN;
+    unsigned bits[2];
+    int far;
+    float kept[kKept][4][BN];
+    static __device__ __forceinline__ int place(uint64_t all, int bit) { return __popcll(all & ((1ull << bit) - 1)); }
+    __device__ __forceinline__ void clear(int tid) {
+        if (tid == 0) bits[0] = bits[1] = 0, far = 0;
+    }
+    __device__ __forceinline__ uint64_t all() const {
+        return (unsigned)__builtin_amdgcn_readfirstlane(bits[0]) | (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane(bits[1]) << 32;
+    }
+};
+
 // B's rows split for a whole product at once: a thread's share of THREADS threads' of BN rows x 32 KS k.  A task is a k-chunk of
 // one row (KC) or of two neighbouring ones.
-template <bool KC, int KS, int BN, int THREADS>
+template <class S, bool KC, int KS, int BN, int THREADS>
 struct Kept {
     static constexpr int VEC = KC ? 1 : 2, kTasks = KS * 4 * BN / VEC / THREADS;
     static_assert(kTasks >= 1, "a task per thread");
@@ -847,26 +1033,66 @@ struct Kept {
                 if constexpr (KC)
 #pragma unroll
                     for (int e = 0; e < 8; e++) x[t][v][e] = 32 * step(task) + k_of(chunk(task), e) < K ? x[t][v][e] : 0.f;
-                atomicMax(&top[row(task) + v], __float_as_uint(abs_max8(x[t][v], 0.f)));
+                atomicMax(&top[row(task) + v], __float_as_uint(abs_max8(x[t][v])));
             }
     }
-    __device__ __forceinline__ void store(Planes<Half2::kPlanes, BN> *L, int *exponents, const unsigned *top, int tid) const {
+    // look(task, elements, scale, split) besides
+    template <class Look>
+    __device__ __forceinline__ void store(Planes<S::kPlanes, BN> *L, int *exponents, const unsigned *top, int tid, Look look) const {
 #pragma unroll
         for (int t = 0; t < kTasks; t++)
 #pragma unroll
             for (int v = 0; v < VEC; v++) {
                 const int task = tid + t * THREADS, r = row(task) + v, c = chunk(task);
                 Scale s;
-                s.set(__uint_as_float(top[r]));
-                v4u d[Half2::kPlanes];
+                s.set(__uint_as_float(top[r]), 14);
+                v4u d[S::kPlanes];
 #pragma unroll
-                for (int j = 0; j < 4; j++) split_pair<Half2>(x[t][v], j, s.s, d);
+                for (int j = 0; j < 4; j++) split_pair<S>(x[t][v], j, s.s, d);
+                look(task, x[t][v], s.s, d);
 #pragma unroll
-                for (int p = 0; p < Half2::kPlanes; p++) L[step(task)].u[p][c][unit_of(r, c)] = d[p];
+                for (int p = 0; p < S::kPlanes; p++) L[step(task)].u[p][c][unit_of(r, c)] = d[p];
                 if (step(task) == 0 && c == 0) exponents[r] = s.exponent();
             }
     }
+    // a task's small elements to the bits of all
+    static __device__ __forceinline__ void note_small(Rests<BN> &rests, int task, const float *y, float s, v4u *d) {
+        const float least = nonzero_min8(y) * s;
+        if (least < kSmall) {
+            unsigned m = 0;
+#pragma unroll
+            for (int e = 0; e < 8; e++) m |= y[e] != 0.f && fabsf(y[e] * s) < kSmall ? 1u << e : 0u;
+            atomicOr(&rests.bits[step(task) / 4], m << 8 * (step(task) % 4));
+            if (least < kTiny) S::drop_tiny(d);
+            if (least < kLeast) rests.far = 1;
+        }
+    }
+    // `all`: the bits of all threads' small elements
+    __device__ __forceinline__ void store_rests(Rests<BN> &rests, const unsigned *top, uint64_t all, int tid) const {
+#pragma unroll
+        for (int t = 0; t < kTasks; t++) {
+            const int task = tid + t * THREADS, first = 8 * __builtin_amdgcn_readfirstlane(step(task));
+#pragma unroll 1
+            for (unsigned left = (unsigned)(all >> first) & 0xff; left; left &= left - 1) {
+                const int e = __builtin_ctz(left), at = Rests<BN>::place(all, first + e);
+                if (at >= Rests<BN>::kKept) break;
+#pragma unroll
+                for (int v = 0; v < VEC; v++) {
+                    Scale s;
+                    s.set(__uint_as_float(top[row(task) + v]), 14);
+                    rests.kept[at][chunk(task)][row(task) + v] = Half2::rest(pick(x[t][v], e) * s.s);
+                }
+            }
+        }
+    }
 };
+
+// What is left of B's element at e of step s in row n, from memory
+template <bool BKC>
+__device__ __forceinline__ float rest_of(const float *Bp, int64_t ldb, int n, int nl, int k, int K, const int *exponents) {
+    const float y = n < nl && k < K ? Bp[BKC ? n * ldb + k : k * ldb + n] : 0.f;
+    return Half2::rest(ldexpf(y, -exponents[n]));
+}
 
 // acc += the fp32 products of a wave's rows (x: a step's elements of A) with B's rows from memory
 template <bool BKC, int MT, int NT>
@@ -908,21 +1134,30 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     __shared__ unsigned top[BN];                       // the largest magnitude of each of B's rows
     __shared__ __align__(16) int exponents[2][BN];     // of the scales, zeros
     __shared__ __align__(16) float biases[BN];
+    __shared__ Rests<BN> rests;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
     const int id = xcd * each + min(xcd, rest) + blockIdx.x / 8;
     const int n0 = (id % g.tn) * BN, nl = g.N - n0, K = g.K;
     const float *const Bp = BKC ? g.B + (int64_t)n0 * g.ldb : g.B + n0;
     if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
+    rests.clear(tid);
     __syncthreads();
+    uint64_t small_b;
     {
-        Kept<BKC, KS, BN, 2 * kThreads> kept;
+        Kept<S, BKC, KS, BN, 2 * kThreads> kept;
         kept.load(Bp, g.ldb, nl, K, tid);
         kept.largest(top, K, tid);
         __syncthreads();
-        kept.store(L, exponents[0], top, tid);
+        kept.store(L, exponents[0], top, tid, [&](int task, const float *y, float scale, v4u *d) { kept.note_small(rests, task, y, scale, d); });
+        __syncthreads();
+        small_b = rests.all();
+        if (small_b) {
+            kept.store_rests(rests, top, small_b, tid);
+            __syncthreads();
+        }
     }
-    __syncthreads();
+    const bool far_b = __builtin_amdgcn_readfirstlane(rests.far);
 
     const int lr = lane % 16, lc = lane / 16;
     const int unit[2] = {lc * BN + unit_of(lr, lc), lc * BN + unit_of(16 + lr, lc) - 16};
@@ -940,18 +1175,21 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     v4u fa[2][MT][S::kPlanes];
     v4f acc[MT][NT];
     float change[MT];
-    bool changed = false;
-    // zeros beyond K, and scales that the step's elements fit
-    const auto prepare = [&](OpA::Raw &x, int k0) {
+    bool changed = false, far = false;
+    unsigned small_a = 0;
+    // zeros beyond K, scales that the step's elements fit, and which of them are small
+    const auto prepare = [&](OpA::Raw &x, int k0) __attribute__((always_inline)) {
         if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
         float m[MT];
-        bool beyond = false;
+        const bool beyond = largest_of(x.x, a.s, m) > kLargest;
+        small_a = 0;
+        if (__any(beyond || smallest_nonzero_of(x.x, a.s) < kSmall)) {
+            if (__any(beyond)) {
+                changed = true;
 #pragma unroll
-        for (int i = 0; i < MT; i++) m[i] = abs_max8(x.x[i], 0.f), beyond |= m[i] > a.s[i].limit;
-        if (__any(beyond)) {
-            changed = true;
-#pragma unroll
-            for (int i = 0; i < MT; i++) change[i] = a.s[i].fit(OpA::of_row(m[i]));
+                for (int i = 0; i < MT; i++) change[i] = a.s[i].fit(OpA::of_row(m[i])), far |= a.s[i].shrunk();
+            }
+            small_a = small_of(x.x, a.s, far);
         }
     };
     const auto split = [&](int q, const OpA::Raw &x, v4u (*f)[S::kPlanes]) { split_pair<S>(x.x[q % MT], q / MT, a.s[q % MT].s, f[q % MT]); };
@@ -971,10 +1209,10 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     for (; block < end; block += kWaves) {
         clear();
         int ea[MT];
+        bool odd = far_b;
         // the products of step s, beside the split of step s + 1 and the loads of step s + 2, which may be the next block's
-        const auto step = [&](auto parity, int s) {
+        const auto step = [&](auto parity, int s) __attribute__((always_inline)) {
             constexpr int p = decltype(parity)::value;
-            load(ra[p], s + 2 < KS ? block : block + kWaves, (s + 2) % KS * kBK);
             if (changed && s > 0) {      // results so far to the scales of step s
 #pragma unroll
                 for (int i = 0; i < MT; i++)
@@ -982,7 +1220,16 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
                     for (int j = 0; j < NT; j++) acc[i][j] *= change[i];
             }
             changed = false;
+            const unsigned b_here = (unsigned)(small_b >> 8 * s) & 0xff;
+            if (small_a | b_here)
+                add_rests(acc, ra[p].x, a.s, small_a, b_here, fa[p], L[s], unit, [&](int, int e) { return b_here >> e & 1; }, [&](int j, int e) {
+                    const int at = Rests<BN>::place(small_b, 8 * s + e);
+                    return at < Rests<BN>::kKept ? rests.kept[at][lc][16 * j + lr]
+                                                 : rest_of<BKC>(Bp, g.ldb, 16 * j + lr, nl, 32 * s + k_of(lc, e), K, exponents[0]);
+                });
+            load(ra[p], s + 2 < KS ? block : block + kWaves, (s + 2) % KS * kBK);
             if (s + 1 == KS) {
+                odd |= far, far = false;
 #pragma unroll
                 for (int i = 0; i < MT; i++) ea[i] = a.s[i].exponent(), a.s[i].none();
             }
@@ -1013,8 +1260,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             step(std::integral_constant<int, 1>(), s + 1);
         }
         const int *eb = exponents[0];
-        if (any_odd(acc)) {
-            // an element that is not finite (0 times it is NaN): the block once more from the fp32 operands
+        if (any_odd(acc) || __any(odd)) {
+            // an element that is not finite (0 times it is NaN) or too small: the block once more from the fp32 operands
             OpA::Raw x;
             clear();
             eb = exponents[1];
@@ -1038,13 +1285,14 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
 // 8.5; 2 are an empty kernel's), 300 x 128, K = 128 4.6 (6.3), x^T y of 1000 rows, 1024 x 256 11.6 with the ranges' sum (15.8).
 template <bool AKC, bool BKC, int KS, int MODE>
 __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
-    typedef Half2 S;
+    typedef WideHalf2 S;
     constexpr int NT = 4, BN = 16 * NT;
     typedef Direct<AKC, 1, false> OpA;
     __shared__ Planes<S::kPlanes, BN> L[KS];
     __shared__ unsigned top[BN];
     __shared__ __align__(16) int exponents[2][BN];
     __shared__ __align__(16) float biases[BN];
+    __shared__ int far_b;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), lr = lane % 16, lc = lane / 16;
     const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
     const int tile = xcd * each + min(xcd, rest) + blockIdx.x / 8, range = tile / (g.tm * g.tn), id = tile % (g.tm * g.tn);
@@ -1053,7 +1301,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     const float *const Ap = AKC ? g.A + (int64_t)m0 * g.lda + kb : g.A + m0 + kb * g.lda;
     const float *const Bp = BKC ? g.B + (int64_t)n0 * g.ldb + kb : g.B + n0 + kb * g.ldb;
     if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && g.ranges == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
-    Kept<BKC, KS, BN, kThreads> kept;
+    if (tid == 0) far_b = 0;
+    Kept<S, BKC, KS, BN, kThreads> kept;
     OpA a;
     typename OpA::Raw x[KS];
     kept.load(Bp, g.ldb, nl, K, tid);
@@ -1067,14 +1316,16 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     lds_barrier();
     kept.largest(top, K, tid);
     lds_barrier();
-    kept.store(L, exponents[0], top, tid);
+    kept.store(L, exponents[0], top, tid, [&](int, const float *y, float scale, v4u *) {
+        if (nonzero_min8(y) * scale < S::kLeast) far_b = 1;
+    });
     float m = 0.f, csum = 0.f;
 #pragma unroll
     for (int s = 0; s < KS; s++) {
         if (K % 4 && 32 * s + 32 > K) a.cut(x[s], 32 * s, K);
-        m = abs_max8(x[s].x[0], m);
+        m = fmaxf(m, abs_max8(x[s].x[0]));
     }
-    a.s[0].set(OpA::of_row(m));
+    a.s[0].set(OpA::of_row(m), 14);
     if constexpr (!AKC) {
         if (g.colsum && n0 == 0)
 #pragma unroll
@@ -1083,9 +1334,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
                 for (int e = 0; e < 8; e++) csum += x[s].x[0][e];
     }
     lds_barrier();
-    v4f acc[1][NT];
+    v4f acc[1][NT], low[NT];
 #pragma unroll
-    for (int j = 0; j < NT; j++) acc[0][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NT; j++) acc[0][j] = low[j] = v4f{0.f, 0.f, 0.f, 0.f};
     const int unit[2] = {lc * BN + unit_of(lr, lc), lc * BN + unit_of(16 + lr, lc) - 16};
 #pragma unroll
     for (int s = 0; s < KS; s++) {
@@ -1095,13 +1346,20 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
 #pragma unroll
         for (int q = 0; q < S::kProducts; q++)
 #pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[0][j] = S::mma(__builtin_bit_cast(S::frag, L[s].u[S::kOrder[q][1]][0][unit[j % 2] + 16 * j]),
-                                   __builtin_bit_cast(S::frag, f[S::kOrder[q][0]]), acc[0][j]);
+            for (int j = 0; j < NT; j++) {
+                v4f &to = S::kOrder[q][0] + S::kOrder[q][1] ? low[j] : acc[0][j];
+                to = S::mma(__builtin_bit_cast(S::frag, L[s].u[S::kOrder[q][1]][0][unit[j % 2] + 16 * j]),
+                            __builtin_bit_cast(S::frag, f[S::kOrder[q][0]]), to);
+            }
     }
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[0][j] += low[j] * S::kRest;
+    bool far = far_b;
+#pragma unroll
+    for (int s = 0; s < KS; s++) far |= smallest_nonzero_of(x[s].x, a.s) < S::kLeast;
     const int *eb = exponents[0];
     int ea[1] = {a.s[0].exponent()}, row[1] = {OpA::row_of(0, lr)};
-    if (any_odd(acc)) {      // the wave's rows once more from the fp32 operands
+    if (any_odd(acc) || __any(far)) {      // the wave's rows once more from the fp32 operands
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[0][j] = v4f{0.f, 0.f, 0.f, 0.f};
         eb = exponents[1], ea[0] = 0;
