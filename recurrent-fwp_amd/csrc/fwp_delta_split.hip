@@ -22,12 +22,17 @@
 // state; zero upstream gradient) and stores to them are dropped; the loops stay straight-line.
 //
 // Few long sequences leave most CUs without work (a block of the chain takes 0.65 us, forward, D = 32, however few there
-// are).  What a run of blocks does to the state is the map S -> S + D S + R, and to its gradient dS -> dS + D^T dS + G: a
-// sequence is cut into segments, a first launch forms the maps of all segments at once (for D by the same chain from
-// zero, with -K for the values), and in a second one every segment's workgroup goes through the maps of those before it
+// are).  What a run of blocks does to the state is the map S -> P S + R, and to its gradient dS -> P^T dS + G: a
+// sequence is cut into segments, a first launch forms the maps of all segments at once (for P by the same chain),
+// and in a second one every segment's workgroup goes through the maps of those before it
 // (behind it, backward) and then does its blocks as above.  Twice the chain's products, over a chain as much shorter as
-// there are segments.  32 x 32 states, 8 sequences of 2381 steps: forward 93 -> 30 us, with backward 264 -> 77 us; 32 of 2048
-// steps: 83 -> 35, 232 -> 82 us; 64 x 64, 32 of 1024 steps: 118 -> 64, 345 -> 145 us.
+// there are segments.  A column of P starts as D, P less the unit matrix's column: from zero, with -K for the values.  A segment that
+// forgets little leaves D small, and S + D S + R rounds once where the chain rounds in every block.  One that forgets much would leave S and
+// D S nearly opposite, with an error of the forgotten state's size: when a column's diagonal of P falls below 1/2, its chain goes on as
+// P's, with zeros for values, and its errors shrink as the chain's do.  Relative errors of the states after 256 steps (float32 emulation; one
+// chain, D throughout, as it is; unit-norm keys, a carried state 1000 times the values): 16 keys 3.2e-7, 2.9e-5, 3.2e-7; 32 keys
+// 2.4e-7, 2.1e-6, 2.5e-7; softmax keys, 32 1.0e-7, 4.6e-8, 4.6e-8.  32 x 32 states, 8 sequences of 2381 steps:
+// forward 93 -> 26 us, with backward 263 -> 60 us; 32 of 2048 steps: 83 -> 35, 233 -> 82 us; 64 x 64, 32 of 1024 steps: 118 -> 63, 352 -> 142 us.
 #include "fwp_common.hpp"
 #include "fwp_wave.hpp"
 #include "fwp_mfma.hpp"
@@ -39,7 +44,7 @@ namespace {
 
 // A sequence's segments: `count` of `blocks` blocks each (whole checkpoint intervals; the last may be shorter).  work, per
 // sequence: the state it starts from [E,M] (forward), then per segment but the last (forward) or the first (backward) R or G
-// [E,M] and D or D^T [E,E], row-major.
+// [E,M], P or P^T [E,E], row-major, and for each of its columns whether it is without the unit matrix's (1) or whole (0) [E].
 struct Segments {
     float *work;
     int count, blocks;
@@ -49,47 +54,72 @@ struct Segments {
 enum { kWhole = 0, kSegments = 1, kMaps = 2 };
 template <int E, int M>
 __device__ __forceinline__ int64_t map_at(const Segments &s, int64_t seq, int j) {
-    return seq * (E * M + (int64_t)(s.count - 1) * (E * M + E * E)) + E * M + (int64_t)j * (E * M + E * E);
+    constexpr int kMap = E * M + E * E + E;
+    return seq * (E * M + (int64_t)(s.count - 1) * kMap) + E * M + (int64_t)j * kMap;
 }
 
-// Tiles eb of D and R of the map at `at`, for a wave's 16 columns
+// Tiles eb of D and R of the map at `at`, for a wave's 16 columns; unit: for the rows of tile eb, that of the unit matrix
 template <int NE, int M>
 struct MapRow {
-    v4f D[NE], R;
+    v4f D[NE], R, unit;
     __device__ __forceinline__ void load(const float *at, int eb, int mb, int g, int c) {
         constexpr int E = 16 * NE;
 #pragma unroll
         for (int r = 0; r < 4; r++) R[r] = at[(16 * eb + 4 * g + r) * M + 16 * mb + c];
 #pragma unroll
         for (int b = 0; b < NE; b++) D[b] = from_float4(*reinterpret_cast<const float4 *>(at + E * M + (16 * eb + c) * E + 16 * b + 4 * g));
+        unit = from_float4(*reinterpret_cast<const float4 *>(at + E * M + E * E + 16 * eb + 4 * g));
     }
 };
 
-// X <- X + D X + R for n maps in turn, at(i) the i-th; X: a wave's 16 columns, tiles as in the accumulator layout.  With keys of
-// up to 32 features the next map is in flight meanwhile.
+// After a block: the columns of tile b of D (in X, a wave's 16 columns) whose diagonal of P has fallen below 1/2 become P's; unit: 1 or 0 of
+// this lane's column.
+template <int NE>
+__device__ __forceinline__ void make_whole(v4f (&X)[NE], int b, const Geo16 &p, float &unit) {
+    float d = 0.f;
+#pragma unroll
+    for (int eb = 0; eb < NE; eb++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) d = eb == b && p.di[r] ? X[eb][r] : d;
+    const bool now = __ballot(unit != 0.f && d < -0.5f) >> (16 * (p.c / 4) + p.c) & 1;      // the lane on the diagonal says so
+    if (!now) return;
+    unit = 0.f;
+#pragma unroll
+    for (int eb = 0; eb < NE; eb++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) X[eb][r] += eb == b && p.di[r] ? 1.f : 0.f;
+}
+
+// X <- P X + R for n maps in turn, at(i) the i-th; X: a wave's 16 columns, tiles as in the accumulator layout.  With keys of up to 32
+// features the next map is in flight meanwhile, with more the next tile of rows.  Their loads are pinned: left alone the compiler asks late for
+// what is used last, a trip to memory for each map (8 sequences of 2048 steps, 32 x 32, forward 46.7 -> 28.1 us).
 template <int NE, int M, class At>
 __device__ __forceinline__ void apply_maps(v4f (&X)[NE], int n, int mb, int g, int c, At at) {
-    constexpr int kAhead = NE <= 2 ? 2 : 1;
-    MapRow<NE, M> m[kAhead][NE];
-    const auto load = [&](int to, int i) {
-#pragma unroll
-        for (int eb = 0; eb < NE; eb++) m[to][eb].load(at(i), eb, mb, g, c);
-    };
-    const auto apply = [&](int from) {
-        v4f Y[NE];
-#pragma unroll
-        for (int eb = 0; eb < NE; eb++) {
-            Y[eb] = m[from][eb].R;      // the small terms first
-#pragma unroll
-            for (int b = 0; b < NE; b++) Y[eb] = tn(m[from][eb].D[b], X[b], Y[eb]);
-        }
-#pragma unroll
-        for (int eb = 0; eb < NE; eb++) X[eb] += Y[eb];
-    };
     if (n <= 0) return;
-    if constexpr (kAhead == 1) {
-        for (int i = 0; i < n; i++) load(0, i), apply(0);
-    } else {
+    v4f Y[NE], unit[NE];
+    const auto row = [&](const MapRow<NE, M> &m, int eb) {
+        Y[eb] = m.R, unit[eb] = m.unit;      // the small terms first
+#pragma unroll
+        for (int b = 0; b < NE; b++) Y[eb] = tn(m.D[b], X[b], Y[eb]);
+    };
+    const auto finish = [&] {
+#pragma unroll
+        for (int eb = 0; eb < NE; eb++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) X[eb][r] = fmaf(unit[eb][r], X[eb][r], Y[eb][r]);
+    };
+    if constexpr (NE <= 2) {
+        MapRow<NE, M> m[2][NE];
+        const auto load = [&](int to, int i) {
+#pragma unroll
+            for (int eb = 0; eb < NE; eb++) m[to][eb].load(at(i), eb, mb, g, c);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const auto apply = [&](int from) {
+#pragma unroll
+            for (int eb = 0; eb < NE; eb++) row(m[from][eb], eb);
+            finish();
+        };
         load(0, 0);
         for (int i = 0; i < n; i += 2) {
             load(1, min(i + 1, n - 1));
@@ -97,6 +127,19 @@ __device__ __forceinline__ void apply_maps(v4f (&X)[NE], int n, int mb, int g, i
             if (i + 1 >= n) break;
             load(0, min(i + 2, n - 1));
             apply(1);
+        }
+    } else {
+        MapRow<NE, M> m[2];
+        m[0].load(at(0), 0, mb, g, c);
+        for (int i = 0; i < n; i++) {
+#pragma unroll
+            for (int eb = 0; eb < NE; eb++) {
+                const bool last = eb + 1 == NE;
+                m[(eb + 1) % 2].load(at(last ? min(i + 1, n - 1) : i), last ? 0 : eb + 1, mb, g, c);
+                __builtin_amdgcn_sched_barrier(0);
+                row(m[eb % 2], eb);
+            }
+            finish();
         }
     }
 }
@@ -133,7 +176,7 @@ struct OutRaw {
 // block behind the state waves, which hand it their columns of the state and of U.
 // With one state wave and the output wave a fourth wave only keeps the barriers: the four waves of a
 // 256-thread workgroup take one SIMD each, three-wave workgroups are placed unevenly.
-// kMaps: the map of a segment instead; state waves mb >= NM hold the columns of D.
+// kMaps: the map of a segment instead; state waves mb >= NM hold the columns of D or P.
 template <int NE, int NM, int PF, bool OUT, int WHAT = kWhole>   // E = 16 NE, M = 16 NM, PF = blocks in flight
 __global__ __launch_bounds__(64 * (WHAT == kMaps ? NM + NE + 1 : OUT ? (NM == 1 ? 4 : NM + 2) : NM + 1)) void k_delta_fwd_split(fwp_view q, fwp_view k, fwp_view v,
                                                                   fwp_view beta, float *__restrict__ W,
@@ -352,7 +395,8 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? NM + NE + 1 : OUT ? (NM == 1 
     // ---------------------------------------------------- state wave of columns [16 mb, 16 mb + 16)
     __builtin_amdgcn_s_setprio(3);      // the wave on the chain goes first where waves share a SIMD
     const int mb = wave;
-    const bool values = !MAP || mb < NM;      // else -K's columns for values
+    const bool values = !MAP || mb < NM;      // else -K's columns for values, while they are D's
+    float unit = 1.f;
     const RowBuf xb = values ? vb : kb;
     const unsigned x_step = values ? v_step : k_step;
     unsigned o_kr[4], o_vr[4];
@@ -416,14 +460,17 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? NM + NE + 1 : OUT ? (NM == 1 
         }
         const v4f Tt = tmat[grp][j].get(lane);
         if constexpr (!MAP) tb.st4(Tt, (unsigned)(c * 16 + 4 * g) * 4, (unsigned)ib * 1024);      // register r = T[c][4g + r]
-        const v4f X = values ? cur.Vc - KS : -cur.Vc - KS;
+        const v4f X = values ? cur.Vc - KS : -unit * cur.Vc - KS;
         v4f Y;
 #pragma unroll
         for (int r = 0; r < 4; r++) Y[r] = cur.brow[r] * X[r];
         const v4f U = tn(Tt, Y, zero);
 #pragma unroll
         for (int eb = 0; eb < NE; eb++) S[eb] = tn(cur.Kc[eb], U, S[eb]);
-        if constexpr (MAP) return;
+        if constexpr (MAP) {
+            if (!values) make_whole(S, mb - NM, p, unit);
+            return;
+        }
         if constexpr (OUT) {
             hx[ib & 1][mb][NE].put(lane, U);
         } else if constexpr (!MAP) {
@@ -480,6 +527,7 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? NM + NE + 1 : OUT ? (NM == 1 
                 if (mb < NM) to[e * M + 16 * mb + c] = S[eb][r];
                 else to[E * M + e * E + 16 * (mb - NM) + c] = S[eb][r];
             }
+        if (!values && g == 0) to[E * M + E * E + 16 * (mb - NM) + c] = unit;
     } else if (part == parts - 1) {
 #pragma unroll
         for (int eb = 0; eb < NE; eb++)
@@ -539,7 +587,7 @@ constexpr int quad_lds_mats() {
 }
 
 // PW = 2: P on two waves, one with the products of Pm, one with the others.
-// kMaps: the map of a segment instead, by P and C alone; C's waves mb >= NM hold the columns of D^T.
+// kMaps: the map of a segment instead, by P and C alone; C's waves mb >= NM hold the columns of D^T or P^T.
 template <int NE, int NM, int WR, int PW, int PF, int WHAT = kWhole>
 __global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * WR)) void k_delta_bwd_quad(
     fwp_view q, fwp_view k, fwp_view beta, const float *__restrict__ vdiff, fwp_view go,
@@ -728,6 +776,8 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * 
         if constexpr (!MAP)
             if (segs.count > 1)
                 apply_maps<NE, M>(dS, segs.count - 1 - part, mb, g, c, [&](int j) { return segs.work + map_at<E, M>(segs, seq, segs.count - 2 - j); });
+        const bool values = !MAP || mb < NM;      // else those of K times the unit matrix, while they are D^T's
+        float unit = 1.f;
         auto block = [&](int e, const Raw &w) {
             // beta[t0 + 4g + r] and K[t0 + 4g + r][.]: loaded, or from what P left a round ago
             float brow[4];
@@ -765,8 +815,7 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * 
             }
             const LdsMat *from = pc[e & 1];
             LdsMat *to = cg[e & 1];
-            const bool values = !MAP || mb < NM;      // else those of K times the unit matrix
-            v4f dU = values ? from[mb].get(lane) : kShareG ? pg[third(e)][kGK + max(mb - NM, 0)].get(lane) : w.Kx;
+            v4f dU = values ? from[mb].get(lane) : unit * (kShareG ? pg[third(e)][kGK + max(mb - NM, 0)].get(lane) : w.Kx);
 #pragma unroll
             for (int eb = 0; eb < NE; eb++) {
                 if constexpr (!MAP) to[eb * NM + mb].put_t(p, dS[eb]);
@@ -779,6 +828,8 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * 
             for (int r = 0; r < 4; r++) ndX[r] = -(brow[r] * dY[r]);
 #pragma unroll
             for (int eb = 0; eb < NE; eb++) dS[eb] = tn(Kc[eb], ndX, values ? dS[eb] + from[NM + eb * NM + mb].get(lane) : dS[eb]);
+            if constexpr (MAP)
+                if (!values) make_whole(dS, mb - NM, p, unit);
         };
         lds_barrier();
         ring_loop<PF, Raw>(nblk, load, block);
@@ -794,6 +845,7 @@ __global__ __launch_bounds__(64 * (WHAT == kMaps ? PW + NM + NE : PW + NM + 2 * 
                     if (mb < NM) to[e * M + 16 * mb + c] = dS[eb][r];
                     else to[E * M + e * E + 16 * (mb - NM) + c] = dS[eb][r];
                 }
+            if (!values && g == 0) to[E * M + E * E + 16 * (mb - NM) + c] = unit;
         }
         return;
     }
@@ -1036,7 +1088,7 @@ Segments segments_of(int nseq, int L, int E, int M, int chunk) {
 
 int64_t delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
     const Segments s = segments_of(N * H, L, E, M, chunk);
-    return s.count > 1 ? (int64_t)N * H * (E * M + (int64_t)(s.count - 1) * (E * M + E * E)) : 0;
+    return s.count > 1 ? (int64_t)N * H * (E * M + (int64_t)(s.count - 1) * (E * M + E * E + E)) : 0;
 }
 
 // the (NE, NM) pairs of split_delta_dims

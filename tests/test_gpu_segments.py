@@ -37,6 +37,70 @@ def test_segments_against_the_oracle(fwp, N, H, L, E, M, steps_first):
     assert within(torch.cat(pieces, 2).cpu().numpy(), want[0], 1e-4, 1e-5) and within(W2.cpu().numpy(), want[1], 1e-4, 1e-5)
 
 
+def run(fwp, arrays, cut, chunk=64, kind=None):
+    """Forward and backward through the C ABI, cut or whole; `kind`: of the forward kernels (the backward ones are chosen)."""
+    L_ = fwp._lib
+    lib = L_.lib()
+    q, k, v, beta, W0, go = (torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda() for a in arrays)
+    N, H, L, E = q.shape
+    M = v.shape[-1]
+    view = lambda t: L_.View(t.data_ptr(), t.stride(0), t.stride(1), t.stride(2))
+    W, out, vdiff, gv = W0.clone(), torch.empty_like(v), torch.empty_like(v), torch.empty_like(v)
+    ckpt = torch.ones(L_.delta_ckpt_floats(N, H, L, E, M, chunk), device="cuda")
+    gq, gk, gb = torch.empty_like(q), torch.empty_like(k), torch.empty_like(beta)
+    n = lib.fwp_delta_segment_floats(N, H, L, E, M, chunk)
+    assert n > 0
+    work = torch.full((n,), float("nan"), device="cuda") if cut else None
+    w, dims, stream = (L_.ptr(work) if cut else None), (N, H, L, E, M, chunk), L_.stream_of(q)
+    try:
+        L_.config(L_.CFG_DELTA_KERNELS, L_.DELTA_AUTO if kind is None else kind)
+        L_.check(lib.fwp_delta_fwd_segments(view(q), view(k), view(v), view(beta), L_.ptr(W),
+                                            L_.OutView(out.data_ptr(), *out.stride()[:3]), L_.ptr(vdiff), L_.ptr(ckpt), w, *dims, stream), "fwd")
+        if cut:
+            work.fill_(float("nan"))
+    finally:
+        L_.config(L_.CFG_DELTA_KERNELS, L_.DELTA_AUTO)
+    L_.check(lib.fwp_delta_bwd_segments(view(q), view(k), view(beta), L_.ptr(vdiff), view(go), L_.ptr(ckpt), L_.ptr(gq), L_.ptr(gk),
+                                        L_.ptr(gv), L_.ptr(gb), w, *dims, stream), "bwd")
+    return dict(zip(("out", "W", "q", "k", "v", "beta"), (t.cpu().numpy() for t in (out, W, gq, gk, gv, gb))))
+
+
+def oracle_of(arrays):
+    x = [np.asarray(a, np.float32).astype(np.float64) for a in arrays]
+    return dict(zip(("out", "W", "q", "k", "v", "beta"), [*oracle.delta_fwd(*x[:5])[:2], *oracle.delta_bwd(*x)]))
+
+
+@pytest.mark.parametrize("N,H,L,E,M", [(1, 8, 2048, 16, 16), (1, 4, 2048, 32, 32), (1, 2, 1500, 64, 32), (1, 2, 1400, 96, 16)])
+@pytest.mark.parametrize("keys", ["unit", "half", "weak"])
+def test_segments_that_forget(fwp, N, H, L, E, M, keys):
+    """Keys of unit norm forget the state before: a large one carried in, and the gradient that comes in at the end.  Every stretch of 64 steps
+    to its own size, as precise as whole sequences are: twice their error (they round once a block, segments in their own
+    blocks and in the maps of those before) and a rounding's worth.  half: only half of the directions are ever written;
+    weak: nothing is forgotten."""
+    g = np.random.default_rng(5)
+    k, q = (g.standard_normal((N, H, L, E)) for _ in range(2))
+    if keys == "half":
+        k[..., E // 2:] = 0
+    k /= np.linalg.norm(k, axis=-1, keepdims=True)
+    beta = 1 / (1 + np.exp(-g.standard_normal((N, H, L, 1)) + (6 if keys == "weak" else 0)))
+    go = g.standard_normal((N, H, L, M))
+    go[:, :, :-70] = 0
+    arrays = (q / np.sqrt(E), k, g.standard_normal((N, H, L, M)), beta, 1e3 * g.standard_normal((N, H, E, M)), go)
+    arrays = [a.astype(np.float32) for a in arrays]
+    want = oracle_of(arrays)
+    cut, whole = run(fwp, arrays, True), run(fwp, arrays, False)
+    for name, w in want.items():
+        steps = range(0, L, 64) if name != "W" else (0,)
+        top = np.linalg.norm(w)
+        for t in steps:
+            part = (lambda a: a) if name == "W" else (lambda a: a[:, :, t:t + 64])
+            size = np.linalg.norm(part(w))
+            if size <= 1e-12 * top:
+                continue
+            err = lambda got: np.linalg.norm(part(got[name]) - part(w)) / size
+            assert err(cut) <= 2 * err(whole) + 3e-7, (name, t, err(cut), err(whole))
+
+
 def test_segments_in_a_graph(fwp):
     """Captured and replayed several times, eager calls between."""
     *x, W0, go = delta_inputs(4, 1, 8, 1000, 32, 32, np.float32, w0=True)
