@@ -10,6 +10,9 @@
 // or more along k) moves s, and the row's results so far with it.  An element below about 2^-20 of its row's largest would lose bits: the
 // waves look for those, and what two numbers leave of them is multiplied apart, so that an element counts to 2^-19 of itself or better
 // whatever is in its row (a result may be made of small elements alone).  The search costs 4 to 7 us of 65, 32768 x 256, K = 1024.
+// Where small elements are many (tokens' gradients, features of very different sizes) that is left: step by step kernels go on with Bf16x3,
+// those with B's rows kept make the products of the small elements once more, small products are formed again on fp32.  x^T y, 1024 x 256, K = 32768,
+// the size of k exp(a N(0,1)), a = 0 / 1.5 / 3 / 5: 86 / 103 / 100 / 98 us (Bf16x3 alone 96; element by element 84 / 122 / 301 / 460).
 //
 // Bf16x3 (smaller K, and the loss's gradient): x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest: 3 x 8 significant bits and
 // their signs hold all 24), six products, h h', h m', m h', m m', h l', l h'; the three left out are below 2^-26 |x x'|.  bf16
@@ -120,9 +123,12 @@ __device__ __forceinline__ constexpr int k_of(int c, int e) { return e < 4 ? 4 *
 
 // Sizes of scaled elements.  Beyond kLargest they do not fit fp16.  From 2^-2 on two fp16 numbers hold them to 2^-23 of themselves, at
 // kSmall to 2^-19: what is left of smaller ones is multiplied apart (add_rests), the whole of those below kTiny, fp16's smallest normal
-// number (products with others cut the sum they are added to at 2^-24 of what that number would give).  With one below kLeast the whole
-// tile is formed on fp32.
+// number (products with others cut the sum they are added to at 2^-24 of what that number would give).  With one below kLeast that is
+// not enough either.
 constexpr float kLargest = 65504.f, kSmall = 0x1p-6f, kTiny = 0x1p-14f, kLeast = 0x1p-31f;
+// One wave's small elements at one place of a step's k cost a workgroup of the step by step kernels about as much as four steps gain over Bf16x3
+// (a = 1.5 as above: 103 us, 120 when counted as one): the steps owed, beyond kGrace of them the rest of k is Bf16x3's.
+constexpr int kPatience = 4, kGrace = 16;
 
 // x = h + m (+ l) for eight values.  Half2: two fp16 numbers of x * scale; Bf16x3: three bf16 numbers of x.
 struct Half2 {
@@ -694,6 +700,58 @@ __device__ __forceinline__ void add_rests(v4f (&acc)[MT][NT], const float (&x)[M
     }
 }
 
+// The same for A alone with whole steps of 16-bit products: small elements leave f and come back 2^20 times as large, those that are small then 2^40
+// times, to results as much larger meanwhile (below 2^(28 + 8) before, K <= 256).  Each is the step's products once more, however many elements:
+// 32768 x 1024, K = 256, features of sizes exp(a N(0,1)), a = 0 / 1.5 / 3 / 5 66 / 74 / 128 / 140 us (Bf16x3 97; element by element 68 / 76 / 183 / 581).
+constexpr float kLevel = 0x1p20f, kFarthest = 0x1p-50f;
+template <int MT, int NT>
+__device__ __forceinline__ void add_small(v4f (&acc)[MT][NT], const float (&x)[MT][8], const Scale (&s)[MT], v4u (&f)[MT][Half2::kPlanes],
+                                          const Planes<Half2::kPlanes, 16 * NT> &L, const int (&unit)[2]) {
+    typedef Half2 S;
+    const float least = smallest_nonzero_of(x, s);
+    // elements of row tile i of sizes (scaled) from `from` below `to` (also infinities: infinity), times up
+    const auto part = [&](int i, float from, float to, float up, v4u *d) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float y[2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const float v = x[i][2 * j + e] * s[i].s;
+                y[e] = fabsf(v) < from || (to < INFINITY && fabsf(v) >= to) ? 0.f : v;
+            }
+            unsigned w[S::kPlanes];
+            S::split2(y[0], y[1], up, w);
+#pragma unroll
+            for (int p = 0; p < S::kPlanes; p++) d[p][j] = w[p];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+        part(i, kSmall, INFINITY, 1.f, f[i]);
+        float to = kSmall, up = 1.f;
+#pragma unroll 1
+        do {
+            const float from = to / kLevel;
+            v4u d[S::kPlanes];
+            up *= kLevel;
+            part(i, from, to, up, d);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                acc[i][j] *= kLevel;
+#pragma unroll
+                for (int q = 0; q < S::kProducts; q++)
+                    acc[i][j] = S::mma(__builtin_bit_cast(S::frag, L.u[S::kOrder[q][1]][0][unit[j % 2] + 16 * j]),
+                                       __builtin_bit_cast(S::frag, d[S::kOrder[q][0]]), acc[i][j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            to = from;
+        } while (__any(least < to));
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] *= 1.f / up;
+    }
+}
+
 // A workgroup of WAVES waves: a wave 16 MT rows and all 16 NT columns; B's rows are staged step by step, in two
 // alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 60 us (one 128 x 128 tile with both
 // operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6.
@@ -701,25 +759,25 @@ template <class S, bool AKC, bool BKC, int MT, int NT, int MODE, int WAVES = 4>
 __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     constexpr int WM = 16 * MT, BM = WAVES * WM, BN = 16 * NT;
     static_assert(WAVES == 4 || !S::kScaled, "four waves' changes of scales");
-    typedef Planes<S::kPlanes, BN> Stage;
     typedef Direct<AKC, MT, MODE == kGrad> OpA;
     typedef Staged<BKC, BN, WAVES> OpB;
-    typedef typename S::frag frag;
-    constexpr size_t kShared = 2 * sizeof(Stage);
+    // the two places of a step's B, and (scaled) behind them its elements in fp32 where some are small; later Bf16x3's places
+    typedef v4f Elements[2][4][BN];
+    constexpr size_t kStages = 2 * sizeof(Planes<S::kPlanes, BN>), kShared = kStages + (S::kScaled ? 2 * sizeof(Elements) : 0);
+    static_assert(2 * sizeof(Planes<Bf16x3::kPlanes, BN>) <= kShared, "Bf16x3's places fit");
     static_assert(sizeof(v4f) * 8 * BN <= kShared, "fp32 of a step fits");
     __shared__ __align__(16) char shared[kShared];
     __shared__ __align__(16) int exponents[BN];
     __shared__ __align__(16) float biases[BN];
     // Of the steps' B, alternately: what each wave did to its rows' scales (kChange: what their results so far are multiplied with is in
-    // change_b) and which of its elements are small (bit e; scaled_b: its rows' elements)
-    constexpr int kChange = 1 << 9;
+    // change_b) and which of its elements are small (bit e); of how many e there are small elements of A; whether an element is too small for that
+    constexpr int kChange = 1 << 9, kStop = 1 << 10, kCountA = 1 << 12;
     __shared__ __align__(16) int news[2][4];
     __shared__ __align__(16) float change_b[S::kScaled ? 2 : 1][S::kScaled ? BN : 4];
-    __shared__ v4f scaled_b[S::kScaled ? 2 : 1][2][4][S::kScaled ? BN : 1];
     __shared__ float change_a[S::kScaled ? 4 : 1][WM];
     __shared__ int odd_waves[WAVES];
     __shared__ NllToken toks[MODE == kGrad && !AKC ? WAVES : 1][MODE == kGrad && !AKC ? kBK : 1];
-    Stage *const L = reinterpret_cast<Stage *>(shared);
+    Elements *const scaled_b = reinterpret_cast<Elements *>(shared + kStages);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     // workgroups go round the 8 XCDs: each XCD gets a run of neighbouring tiles (a row of tiles reads the same
     // rows of A, through that XCD's L2), of whole ranges of k where there are several: the tiles of a range read the
@@ -759,144 +817,184 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
 
     typename OpA::Raw ra[2];
     typename OpB::Raw rb[2];
-    bool change = false;      // of scales of A's rows
-    unsigned small_a = 0;
-    bool far = false;         // an element too small even for that
-    v4u fa[2][MT][S::kPlanes];
-    float part_sum[MT];       // of a step's elements of A's rows
-    const auto split_a = [&](int i, int j, const typename OpA::Raw &x, v4u (*f)[S::kPlanes], bool whole, int k0) {
-        float v[8];
-        v[2 * j] = a.element(x, i, 2 * j, whole, m0, k0, ke), v[2 * j + 1] = a.element(x, i, 2 * j + 1, whole, m0, k0, ke);
-        if constexpr (!AKC) part_sum[i] = (j ? part_sum[i] : 0.f) + (v[2 * j] + v[2 * j + 1]);
-        else part_sum[i] = 0.f;
-        split_pair<S>(v, j, a.s[i].s, f[i]);
-    };
-    // Pair q of the 4 (units + MT) pairs of a step's split: B's units first, each to LDS when it is whole, then A's tiles
-    v4u part[S::kPlanes];
-    constexpr int kPairs = 4 * (OpB::kUnits + MT);
-    const auto split = [&](int q, const typename OpA::Raw &x, const typename OpB::Raw &y, v4u (*f)[S::kPlanes], Stage &to, int k0) {
-        if (q < 4 * OpB::kUnits) {
-            split_pair<S>(y.x[q / 4], q % 4, b.s[q / 4].s, part);
-            if (q % 4 == 3) b.store(to, q / 4, part);
-            return;
-        }
-        const int j = (q - 4 * OpB::kUnits) / MT, i = q % MT;
-        split_a(i, j, x, f, false, k0);
-    };
-    // once more where split() left something out
-    const auto complete = [&](const typename OpA::Raw &x, v4u (*f)[S::kPlanes], int k0) {
-        if constexpr (MODE == kGrad)
-            if (a.rare(x, m0, k0, ke))
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) split_a(i, j, x, f, true, k0);
-#pragma unroll
-        for (int i = 0; i < MT; i++) csum[i] += part_sum[i];
-    };
-    // What a step's split needs: zeros beyond K, and (parity: the step's) scales that its elements fit
-    const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) __attribute__((always_inline)) {
-        a.hand_over(x, lane);
-        if (ke % 4 && k0 + kBK > ke) a.cut(x, k0, ke), b.cut(y, k0, ke);
-        if constexpr (S::kScaled) {
-            float ma[MT], mb[OpB::kUnits];
-            const bool beyond = fmaxf(largest_of(x.x, a.s, ma), largest_of(y.x, b.s, mb)) > kLargest;
-            float la = smallest_nonzero_of(x.x, a.s), lb = smallest_of(y.x, b.s);
-            int word = 0;
-            small_a = 0;
-            if (__any(beyond || fminf(la, lb) < kSmall)) {
-                if (__any(beyond)) {
-                    change = true, word = kChange;
-                    la = lb = 0.f;
-#pragma unroll
-                    for (int i = 0; i < MT; i++) change_a[wave][OpA::row_of(i, lr)] = a.s[i].fit(OpA::of_row(ma[i])), far |= a.s[i].shrunk();
-#pragma unroll
-                    for (int t = 0; t < OpB::kUnits; t++) change_b[parity][b.row_of(t)] = b.s[t].fit(OpB::of_row(mb[t])), far |= b.s[t].shrunk();
-                }
-                if (__any(la < kSmall)) small_a = small_of(x.x, a.s, far);
-                if (__any(lb < kSmall)) word |= small_of(y.x, b.s, far);
-                if (word & 0xff)
-#pragma unroll
-                    for (int t = 0; t < OpB::kUnits; t++)
-#pragma unroll
-                        for (int h = 0; h < 2; h++)
-                            scaled_b[parity][h][b.c][b.row_of(t)] =
-                                v4f{y.x[t][4 * h], y.x[t][4 * h + 1], y.x[t][4 * h + 2], y.x[t][4 * h + 3]} * b.s[t].s;
-                if (word & kSomeTiny)
-#pragma unroll
-                    for (int t = 0; t < OpB::kUnits; t++) drop_tiny8(y.x[t], b.s[t].s);
-            }
-            if (lane == 0) news[parity][wave] = word;
-        }
-    };
-    // Before step k0's products (x: its elements of A): results so far to its scales, and what is left of its small elements
-    const auto follow = [&](int parity, const typename OpA::Raw &x) __attribute__((always_inline)) {
-        if constexpr (S::kScaled) {
-            const int4 w = *reinterpret_cast<const int4 *>(news[parity]);
-            const int of[4] = {__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
-                               __builtin_amdgcn_readfirstlane(w.w)};
-            const int all = of[0] | of[1] | of[2] | of[3];
-            if (all & kChange) {
-#pragma unroll
-                for (int j = 0; j < NT; j++)
-                    if (of[OpB::owner(j)] & kChange)
-#pragma unroll
-                        for (int i = 0; i < MT; i++) acc[i][j] *= *reinterpret_cast<const v4f *>(change_b[parity] + 16 * j + 4 * lc);
-            }
-            if (change) {
-                change = false;
-#pragma unroll
-                for (int i = 0; i < MT; i++)
-#pragma unroll
-                    for (int j = 0; j < NT; j++) acc[i][j] *= change_a[wave][OpA::row_of(i, lr)];
-            }
-            if (small_a | (all & 0xff))
-                add_rests(acc, x.x, a.s, small_a, all & 0xff, fa[parity], L[parity], unit, [&](int j, int e) { return of[OpB::owner(j)] >> e & 1; },
-                          [&](int j, int e) { return Half2::rest(reinterpret_cast<const float *>(&scaled_b[parity][e / 4][lc][16 * j + lr])[e % 4]); });
-        }
-    };
-    aim(kb);
-    load(ra[0], rb[0], kb);
-    aim(kb + kBK);
-    load(ra[1], rb[1], kb + kBK);
-    prepare(ra[0], rb[0], kb, 0);
-#pragma unroll
-    for (int q = 0; q < kPairs; q++) split(q, ra[0], rb[0], fa[0], L[0], kb);
-    complete(ra[0], fa[0], kb);
-    lds_barrier();
-    // One step: the products of k0's parts, beside the split of k0 + kBK's elements and the loads of k0 + 2 kBK's.
-    const auto step = [&](auto parity, int k0) __attribute__((always_inline)) {
-        constexpr int p = decltype(parity)::value;
-        follow(p, ra[p]);
-        if (k0 + 3 * kBK > ke) aim(k0 + 2 * kBK);
-        load(ra[p], rb[p], k0 + 2 * kBK);
-        prepare(ra[p ^ 1], rb[p ^ 1], k0 + kBK, p ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-        frag fb[2][S::kPlanes];
-        const auto read = [&](int j) {
-#pragma unroll
-            for (int q = 0; q < S::kPlanes; q++) fb[j % 2][q] = __builtin_bit_cast(frag, L[p].u[q][0][unit[j % 2] + 16 * j]);
+    bool far = false;         // results that may not be what fp32 holds
+    // The steps from k = first on with operands split as T; returns the k it stopped at (scaled).
+    const auto steps = [&](auto split_as, int first) __attribute__((always_inline)) -> int {
+        typedef decltype(split_as) T;
+        typedef typename T::frag frag;
+        typedef Planes<T::kPlanes, BN> Stage;
+        Stage *const L = reinterpret_cast<Stage *>(shared);
+        bool change = false;      // of scales of A's rows
+        unsigned small_a = 0;
+        int spent = 0;
+        v4u fa[2][MT][T::kPlanes];
+        float part_sum[MT];       // of a step's elements of A's rows
+        const auto split_a = [&](int i, int j, const typename OpA::Raw &x, v4u (*f)[T::kPlanes], bool whole, int k0) {
+            float v[8];
+            v[2 * j] = a.element(x, i, 2 * j, whole, m0, k0, ke), v[2 * j + 1] = a.element(x, i, 2 * j + 1, whole, m0, k0, ke);
+            if constexpr (!AKC) part_sum[i] = (j ? part_sum[i] : 0.f) + (v[2 * j] + v[2 * j + 1]);
+            else part_sum[i] = 0.f;
+            split_pair<T>(v, j, a.s[i].s, f[i]);
         };
-        read(0);
+        // Pair q of the 4 (units + MT) pairs of a step's split: B's units first, each to LDS when it is whole, then A's tiles
+        v4u part[T::kPlanes];
+        constexpr int kPairs = 4 * (OpB::kUnits + MT);
+        const auto split = [&](int q, const typename OpA::Raw &x, const typename OpB::Raw &y, v4u (*f)[T::kPlanes], Stage &to, int k0) {
+            if (q < 4 * OpB::kUnits) {
+                split_pair<T>(y.x[q / 4], q % 4, b.s[q / 4].s, part);
+                if (q % 4 == 3) b.store(to, q / 4, part);
+                return;
+            }
+            const int j = (q - 4 * OpB::kUnits) / MT, i = q % MT;
+            split_a(i, j, x, f, false, k0);
+        };
+        // once more where split() left something out
+        const auto complete = [&](const typename OpA::Raw &x, v4u (*f)[T::kPlanes], int k0) {
+            if constexpr (MODE == kGrad)
+                if (a.rare(x, m0, k0, ke))
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
-            if (j + 1 < NT) read(j + 1);
+                    for (int i = 0; i < MT; i++)
 #pragma unroll
-            for (int q = j * kPairs / NT; q < (j + 1) * kPairs / NT; q++) split(q, ra[p ^ 1], rb[p ^ 1], fa[p ^ 1], L[p ^ 1], k0 + kBK);
+                        for (int j = 0; j < 4; j++) split_a(i, j, x, f, true, k0);
+        };
+        // What a step's split needs: zeros beyond K, and (parity: the step's) scales that its elements fit
+        const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) __attribute__((always_inline)) {
+            a.hand_over(x, lane);
+            if (ke % 4 && k0 + kBK > ke) a.cut(x, k0, ke), b.cut(y, k0, ke);
+            if constexpr (T::kScaled) {
+                float ma[MT], mb[OpB::kUnits];
+                const bool beyond = fmaxf(largest_of(x.x, a.s, ma), largest_of(y.x, b.s, mb)) > kLargest;
+                float la = smallest_nonzero_of(x.x, a.s), lb = smallest_of(y.x, b.s);
+                int word = 0;
+                small_a = 0;
+                if (__any(beyond || fminf(la, lb) < kSmall)) {
+                    if (__any(beyond)) {
+                        change = true, word = kChange;
+                        la = lb = 0.f;
 #pragma unroll
-            for (int q = 0; q < S::kProducts; q++)
+                        for (int i = 0; i < MT; i++) change_a[wave][OpA::row_of(i, lr)] = a.s[i].fit(OpA::of_row(ma[i])), far |= a.s[i].shrunk();
 #pragma unroll
-                for (int i = 0; i < MT; i++)
-                    acc[i][j] = S::mma(fb[j % 2][S::kOrder[q][1]], __builtin_bit_cast(frag, fa[p][i][S::kOrder[q][0]]), acc[i][j]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        complete(ra[p ^ 1], fa[p ^ 1], k0 + kBK);
+                        for (int t = 0; t < OpB::kUnits; t++) change_b[parity][b.row_of(t)] = b.s[t].fit(OpB::of_row(mb[t])), far |= b.s[t].shrunk();
+                    }
+                    bool stop = false;
+                    if (__any(la < kSmall)) small_a = small_of(x.x, a.s, stop), word |= __popc(small_a) * kCountA;
+                    if (__any(lb < kSmall)) word |= small_of(y.x, b.s, stop);
+                    if (__any(stop)) word |= kStop;
+                    if (word & 0xff)
+#pragma unroll
+                        for (int t = 0; t < OpB::kUnits; t++)
+#pragma unroll
+                            for (int h = 0; h < 2; h++)
+                                scaled_b[parity][h][b.c][b.row_of(t)] =
+                                    v4f{y.x[t][4 * h], y.x[t][4 * h + 1], y.x[t][4 * h + 2], y.x[t][4 * h + 3]} * b.s[t].s;
+                    if (word & kSomeTiny)
+#pragma unroll
+                        for (int t = 0; t < OpB::kUnits; t++) drop_tiny8(y.x[t], b.s[t].s);
+                }
+                if (lane == 0) news[parity][wave] = word;
+            }
+        };
+        // Before step k0's products (x: its elements of A): results so far to its scales, and what is left of its small elements
+        // True (in all waves): the step is not for fp16.
+        const auto follow = [&](int parity, const typename OpA::Raw &x) __attribute__((always_inline)) -> bool {
+            if constexpr (T::kScaled) {
+                const int4 w = *reinterpret_cast<const int4 *>(news[parity]);
+                const int of[4] = {__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
+                                   __builtin_amdgcn_readfirstlane(w.w)};
+                const int all = of[0] | of[1] | of[2] | of[3];
+                if (all & kChange) {
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        if (of[OpB::owner(j)] & kChange)
+#pragma unroll
+                            for (int i = 0; i < MT; i++) acc[i][j] *= *reinterpret_cast<const v4f *>(change_b[parity] + 16 * j + 4 * lc);
+                }
+                if (change) {
+                    change = false;
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+#pragma unroll
+                        for (int j = 0; j < NT; j++) acc[i][j] *= change_a[wave][OpA::row_of(i, lr)];
+                }
+                if (all & (0xff | kStop | 0xf * kCountA)) {
+                    spent += kPatience * (of[0] / kCountA + of[1] / kCountA + of[2] / kCountA + of[3] / kCountA + __popc(all & 0xff));
+                    if (all & kStop || spent > kGrace) return true;
+                    add_rests(acc, x.x, a.s, small_a, all & 0xff, fa[parity], L[parity], unit, [&](int j, int e) { return of[OpB::owner(j)] >> e & 1; },
+                              [&](int j, int e) { return Half2::rest(reinterpret_cast<const float *>(&scaled_b[parity][e / 4][lc][16 * j + lr])[e % 4]); });
+                }
+                spent = max(spent - 1, 0);
+            }
+            return false;
+        };
+        aim(first);
+        load(ra[0], rb[0], first);
+        aim(first + kBK);
+        load(ra[1], rb[1], first + kBK);
+        prepare(ra[0], rb[0], first, 0);
+#pragma unroll
+        for (int q = 0; q < kPairs; q++) split(q, ra[0], rb[0], fa[0], L[0], first);
+        complete(ra[0], fa[0], first);
         lds_barrier();
+        // One step: the products of k0's parts, beside the split of k0 + kBK's elements and the loads of k0 + 2 kBK's.
+        const auto step = [&](auto parity, int k0) __attribute__((always_inline)) -> bool {
+            constexpr int p = decltype(parity)::value;
+            if (follow(p, ra[p])) return false;
+#pragma unroll
+            for (int i = 0; i < MT; i++) csum[i] += part_sum[i];
+            if (k0 + 3 * kBK > ke) aim(k0 + 2 * kBK);
+            load(ra[p], rb[p], k0 + 2 * kBK);
+            prepare(ra[p ^ 1], rb[p ^ 1], k0 + kBK, p ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            frag fb[2][T::kPlanes];
+            const auto read = [&](int j) {
+#pragma unroll
+                for (int q = 0; q < T::kPlanes; q++) fb[j % 2][q] = __builtin_bit_cast(frag, L[p].u[q][0][unit[j % 2] + 16 * j]);
+            };
+            read(0);
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                if (j + 1 < NT) read(j + 1);
+#pragma unroll
+                for (int q = j * kPairs / NT; q < (j + 1) * kPairs / NT; q++) split(q, ra[p ^ 1], rb[p ^ 1], fa[p ^ 1], L[p ^ 1], k0 + kBK);
+#pragma unroll
+                for (int q = 0; q < T::kProducts; q++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[i][j] = T::mma(fb[j % 2][T::kOrder[q][1]], __builtin_bit_cast(frag, fa[p][i][T::kOrder[q][0]]), acc[i][j]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            complete(ra[p ^ 1], fa[p ^ 1], k0 + kBK);
+            lds_barrier();
+            return true;
+        };
+        for (int k0 = first; k0 < ke; k0 += 2 * kBK) {      // an odd number of steps: the last one's elements are zeros
+            if (!step(std::integral_constant<int, 0>(), k0)) return k0;
+            if (!step(std::integral_constant<int, 1>(), k0 + kBK)) return k0 + kBK;
+        }
+        return ke;
     };
-    for (int k0 = kb; k0 < ke; k0 += 2 * kBK) {      // an odd number of steps: the last one's elements are zeros
-        step(std::integral_constant<int, 0>(), k0);
-        step(std::integral_constant<int, 1>(), k0 + kBK);
-    }
+    const int stopped = steps(S(), kb);
+    if constexpr (S::kScaled)
+        if (stopped < ke) {
+            // the rest of k as Bf16x3, to results of the size they have
+            if (b.c == 0)
+#pragma unroll
+                for (int t = 0; t < OpB::kUnits; t++) exponents[b.row_of(t)] = b.s[t].exponent();
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const v4i eb = *reinterpret_cast<const v4i *>(exponents + 16 * j + 4 * lc);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[i][j][e] = ldexpf(acc[i][j][e], a.s[i].exponent() + eb[e]);
+                }
+#pragma unroll
+            for (int i = 0; i < MT; i++) a.s[i].one();
+#pragma unroll
+            for (int t = 0; t < OpB::kUnits; t++) b.s[t].one();
+            steps(Bf16x3(), stopped);
+        }
 
     // An element that is not finite (0 times it is NaN)
     float odd = 0.f;
@@ -1064,8 +1162,21 @@ struct Kept {
             for (int e = 0; e < 8; e++) m |= y[e] != 0.f && fabsf(y[e] * s) < kSmall ? 1u << e : 0u;
             atomicOr(&rests.bits[step(task) / 4], m << 8 * (step(task) % 4));
             if (least < kTiny) S::drop_tiny(d);
-            if (least < kLeast) rests.far = 1;
+            if (least < kFarthest) rests.far = 1;
         }
+    }
+    // fp32 as it is, [step][half][chunk][row]
+    __device__ __forceinline__ void store_plain(v4f (*L)[2][4][BN], int tid) const {
+#pragma unroll
+        for (int t = 0; t < kTasks; t++)
+#pragma unroll
+            for (int v = 0; v < VEC; v++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int task = tid + t * THREADS;
+                    const float *const y = x[t][v] + 4 * h;
+                    L[step(task)][h][chunk(task)][row(task) + v] = v4f{y[0], y[1], y[2], y[3]};
+                }
     }
     // `all`: the bits of all threads' small elements
     __device__ __forceinline__ void store_rests(Rests<BN> &rests, const unsigned *top, uint64_t all, int tid) const {
@@ -1086,6 +1197,12 @@ struct Kept {
         }
     }
 };
+
+// Keeps what is computed from it in rare code from being held in registers outside
+__device__ __forceinline__ int afresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 // What is left of B's element at e of step s in row n, from memory
 template <bool BKC>
@@ -1176,20 +1293,22 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     v4f acc[MT][NT];
     float change[MT];
     bool changed = false, far = false;
-    unsigned small_a = 0;
-    // zeros beyond K, scales that the step's elements fit, and which of them are small
+    bool small_a = false;
+    // zeros beyond K, scales that the step's elements fit, and whether some are small
     const auto prepare = [&](OpA::Raw &x, int k0) __attribute__((always_inline)) {
         if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
         float m[MT];
         const bool beyond = largest_of(x.x, a.s, m) > kLargest;
-        small_a = 0;
+        small_a = false;
         if (__any(beyond || smallest_nonzero_of(x.x, a.s) < kSmall)) {
             if (__any(beyond)) {
                 changed = true;
 #pragma unroll
                 for (int i = 0; i < MT; i++) change[i] = a.s[i].fit(OpA::of_row(m[i])), far |= a.s[i].shrunk();
             }
-            small_a = small_of(x.x, a.s, far);
+            const float least = smallest_nonzero_of(x.x, a.s);
+            small_a = __any(least < kSmall);
+            far |= least < kFarthest;
         }
     };
     const auto split = [&](int q, const OpA::Raw &x, v4u (*f)[S::kPlanes]) { split_pair<S>(x.x[q % MT], q / MT, a.s[q % MT].s, f[q % MT]); };
@@ -1221,11 +1340,12 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             }
             changed = false;
             const unsigned b_here = (unsigned)(small_b >> 8 * s) & 0xff;
-            if (small_a | b_here)
-                add_rests(acc, ra[p].x, a.s, small_a, b_here, fa[p], L[s], unit, [&](int, int e) { return b_here >> e & 1; }, [&](int j, int e) {
+            if (small_a) add_small(acc, ra[p].x, a.s, fa[p], L[s], unit);
+            if (b_here)
+                add_rests(acc, ra[p].x, a.s, 0, b_here, fa[p], L[s], unit, [&](int, int e) { return b_here >> e & 1; }, [&](int j, int e) {
                     const int at = Rests<BN>::place(small_b, 8 * s + e);
                     return at < Rests<BN>::kKept ? rests.kept[at][lc][16 * j + lr]
-                                                 : rest_of<BKC>(Bp, g.ldb, 16 * j + lr, nl, 32 * s + k_of(lc, e), K, exponents[0]);
+                                                 : rest_of<BKC>(Bp, g.ldb, 16 * j + afresh(lr), nl, 32 * s + k_of(lc, e), K, exponents[0]);
                 });
             load(ra[p], s + 2 < KS ? block : block + kWaves, (s + 2) % KS * kBK);
             if (s + 1 == KS) {
@@ -1264,13 +1384,14 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             // an element that is not finite (0 times it is NaN) or too small: the block once more from the fp32 operands
             OpA::Raw x;
             clear();
+            const int r = afresh(lr);
             eb = exponents[1];
             ea[0] = ea[1] = 0;
 #pragma unroll 1
             for (int k0 = 0; k0 < K; k0 += kBK) {
                 load(x, block, k0);
                 if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
-                plain_step<BKC>(acc, x.x, Bp, g.ldb, nl, k0, K, lr, lc);
+                plain_step<BKC>(acc, x.x, Bp, g.ldb, nl, k0, K, r, lc);
             }
         }
         int row[MT];
@@ -1292,7 +1413,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     __shared__ unsigned top[BN];
     __shared__ __align__(16) int exponents[2][BN];
     __shared__ __align__(16) float biases[BN];
-    __shared__ int far_b;
+    __shared__ int odd;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), lr = lane % 16, lc = lane / 16;
     const int total = gridDim.x, xcd = blockIdx.x % 8, each = total / 8, rest = total % 8;
     const int tile = xcd * each + min(xcd, rest) + blockIdx.x / 8, range = tile / (g.tm * g.tn), id = tile % (g.tm * g.tn);
@@ -1301,7 +1422,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     const float *const Ap = AKC ? g.A + (int64_t)m0 * g.lda + kb : g.A + m0 + kb * g.lda;
     const float *const Bp = BKC ? g.B + (int64_t)n0 * g.ldb + kb : g.B + n0 + kb * g.ldb;
     if (tid < BN) top[tid] = 0, exponents[1][tid] = 0, biases[tid] = g.epi.bias && g.ranges == 1 && tid < nl ? g.epi.bias[n0 + tid] : 0.f;
-    if (tid == 0) far_b = 0;
+    if (tid == 0) odd = 0;
     Kept<S, BKC, KS, BN, kThreads> kept;
     OpA a;
     typename OpA::Raw x[KS];
@@ -1317,7 +1438,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     kept.largest(top, K, tid);
     lds_barrier();
     kept.store(L, exponents[0], top, tid, [&](int, const float *y, float scale, v4u *) {
-        if (nonzero_min8(y) * scale < S::kLeast) far_b = 1;
+        if (nonzero_min8(y) * scale < S::kLeast) odd = 1;
     });
     float m = 0.f, csum = 0.f;
 #pragma unroll
@@ -1354,21 +1475,31 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_once(GemmArgs g) {
     }
 #pragma unroll
     for (int j = 0; j < NT; j++) acc[0][j] += low[j] * S::kRest;
-    bool far = far_b;
+    bool far = any_odd(acc);
 #pragma unroll
     for (int s = 0; s < KS; s++) far |= smallest_nonzero_of(x[s].x, a.s) < S::kLeast;
+    if (far) odd = 1;
     const int *eb = exponents[0];
     int ea[1] = {a.s[0].exponent()}, row[1] = {OpA::row_of(0, lr)};
-    if (any_odd(acc) || __any(far)) {      // the wave's rows once more from the fp32 operands
+    __syncthreads();
+    if (odd) {
+        // the tile once more in fp32, B through LDS: 15.5 us for 2000 rows of very different sizes, x^T y, 256 x 128 (11.3 without; B from memory 37.6)
+        eb = exponents[1], ea[0] = 0;
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[0][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        eb = exponents[1], ea[0] = 0;
-#pragma unroll 1
-        for (int k0 = 0; k0 < K; k0 += kBK) {
-            load(x[0], k0);
-            if (K % 4 && k0 + kBK > K) a.cut(x[0], k0, K);
-            plain_step<BKC>(acc, x[0].x, Bp, g.ldb, nl, k0, K, lr, lc);
-        }
+        v4f(*const plain)[2][4][BN] = reinterpret_cast<v4f(*)[2][4][BN]>(L);
+        kept.store_plain(plain, tid);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KS; s++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const v4f y = plain[s][h][lc][16 * j + lr];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) acc[0][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[e], x[s].x[0][4 * h + e], acc[0][j], 0, 0, 0);
+                }
     }
     if constexpr (!AKC)
         if (g.colsum && n0 == 0) {

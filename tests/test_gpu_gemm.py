@@ -318,6 +318,8 @@ def test_products_of_two_fp16_parts(fwp, M, N, K, layout, case):
 def test_infinities_in_larger_products(fwp, M, N, K, layout):
     a, b = randn(M, K, seed=1), randn(N, K, seed=2)
     a[7, 3], a[M - 1, K - 1], a[900, 0], b[N - 1, 5] = float("inf"), float("nan"), 2e37, float("inf")
+    a[39], a[40] = 0, a[40] * 2.0 ** (-24 * (torch.arange(K, device="cuda") % 5 == 0))      # an infinity alone beside small elements
+    a[39, 3] = float("inf")
     want, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
     A, B = a.t().contiguous() if layout == TN else a, b if layout == NT else b.t().contiguous()
     got = matmul(fwp._lib, layout, A, B).double()
@@ -348,12 +350,18 @@ def wide_operands(case, M, N, K):
         r = lambda i, *s: torch.rand(*s, generator=torch.Generator().manual_seed(i)).cuda()
         a = a * torch.exp2(-40 * r(3, M, K)) * (r(4, M, K) < 0.5)
         b = b * torch.exp2(-40 * r(5, N, K)) * (r(6, N, K) < 0.5)
+    elif case in ("spread", "weights"):        # every k of one operand has a size of its own, over 2^56 (beyond the second time of small elements)
+        x = a if case == "spread" else b
+        x *= torch.exp2(-56 * torch.rand(K, generator=torch.Generator().manual_seed(3)).cuda())
+    elif case == "few":                        # small elements now and then: too few to give up on fp16
+        a[:, ::41] *= 2.0 ** -24
+        b[:, 7::97] *= 2.0 ** -30
     return a, b
 
 
 @pytest.mark.parametrize("M,N,K", HALF_SHAPES)
 @pytest.mark.parametrize("layout", [NT, NN, TN])
-@pytest.mark.parametrize("case", ["outlier", "weight", "late", "groups", "picked", "even"])
+@pytest.mark.parametrize("case", ["outlier", "weight", "late", "groups", "picked", "even", "spread", "weights", "few"])
 def test_rows_of_elements_of_very_different_sizes(fwp, M, N, K, layout, case):
     """An element counts to its own size, whatever else is in its row."""
     a, b = wide_operands(case, M, N, K)
@@ -363,6 +371,30 @@ def test_rows_of_elements_of_very_different_sizes(fwp, M, N, K, layout, case):
     for cut in (True, False):
         got = matmul(fwp._lib, layout, A, B, cut).double()
         assert bool(((got - want).abs() <= bound(K, mag)).all())
+
+
+@pytest.mark.parametrize("M,N,K,layout", [(256, 1024, 32768, TN), (32768, 256, 1024, NT), (32768, 1024, 256, NT), (256, 128, 2000, TN)])
+def test_sizes_that_are_spread_cost_no_multiple(fwp, M, N, K, layout):
+    """Where every k has a size of its own (tokens' gradients; features) three bf16 numbers' six products take over from three, or
+    three more are made: twice the time, and something for the change.  (Element by element: 6 to 9 times.)"""
+    def microseconds(A, B):
+        matmul(fwp._lib, layout, A, B)
+        times = []
+        for _ in range(9):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                matmul(fwp._lib, layout, A, B)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return sorted(times)[4]
+
+    a, b = randn(M, K, seed=1), randn(N, K, seed=2)
+    sizes = torch.exp(5 * randn(K, seed=3))
+    A, S = (a.t().contiguous(), (a * sizes).t().contiguous()) if layout == TN else (a, a * sizes)
+    B = b if layout == NT else b.t().contiguous()
+    assert microseconds(S, B) <= 3.5 * microseconds(A, B)
 
 
 @pytest.mark.parametrize("rows,vocab", [(70, 300), (6500, 6600)])
