@@ -1582,13 +1582,17 @@ constexpr int kHalfK = 128;
 // (152, 304, 608 tiles) 16.2, 15.9, 14.3 us; 300 x 256, K = 256 13.9, 10.3, 8.6 us.  Those of 64 x 64 all at once where a tile's k
 // is at most 256 or can be cut into ranges that are, and that makes no more than two workgroups for a CU: 300 x 256, K = 256
 // 7.0 us, 1000 x 256, K = 1024 (256 workgroups) 11.9 us staged 13.2, 2381 x 256, K = 1024 (608) 20.8 us, staged 19.1.
-// The partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k.
-Plan plan_of(int M, int N, int K, bool may_cut) {
+// The partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k; all at once, 129.
+// The loss's gradients (`grad`): 128 x 256 tiles of eight waves, which form an element once for twice the columns, where those divide over the
+// chip as well as 128 x 128 ones, one of them to a CU or two of the others, the latter 1.12 times as long.  dX and dW, tokens = words = 32768: 256 columns
+// 3.09 and 3.36 ms (128-column tiles 3.45, 3.85), 288 (512 tiles, two turns) 5.85 and 6.61 (768 tiles, one and a half: 5.10, 5.94); 8192, in two
+// ranges: 288 columns 0.37 and 0.43 ms (0.38, 0.46); 640 (192 tiles) 0.69 and 0.83 (128 x 64 tiles 0.81, 1.05).
+Plan plan_of(int M, int N, int K, bool may_cut, bool grad) {
     Plan p{};
     const auto tiles = [&](int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const auto ranges = [&](int64_t tiles) { return may_cut ? std::max<int64_t>(1, std::min<int64_t>(512 / tiles, K / 256)) : 1; };
     const int blocks = (M + 31) / 32;
-    if (K >= kHalfK && K <= 256 && tiles(256, 128) >= kResidentTiles) {
+    if (!grad && K >= kHalfK && K <= 256 && tiles(256, 128) >= kResidentTiles) {
         p.steps = K <= 128 ? 4 : 8;
         // the most even division of the blocks over 256 CUs, a workgroup's start (its rows of B) as long as a wave's block
         double best = 1e30;
@@ -1600,15 +1604,16 @@ Plan plan_of(int M, int N, int K, bool may_cut) {
         }
     }
     p.bm = p.bn = 128;
-    const int64_t wide = tiles(128, 128);
-    if (wide * ranges(wide) < 384) {
+    const int64_t wide = tiles(128, 128), turns = tiles(128, 256) * ranges(wide);
+    if (wide * ranges(wide) < 384 && !(grad && N > 128 && turns >= 160)) {
         p.bn = 64;
         if (tiles(128, 64) < 384) p.bm = 64;
     }
+    if (grad && N > 128 && p.bn == 128 && (turns + 255) / 256 <= 1.12 * std::max(1.0, wide * ranges(wide) / 512.0)) p.bn = 256;
     p.tm = (M + p.bm - 1) / p.bm;
     p.tn = (N + p.bn - 1) / p.bn;
-    int64_t n = ranges(tiles(p.bm, p.bn));
-    if (p.bm == 64 && K >= kHalfK) {
+    int64_t n = ranges(p.bn == 256 ? wide : tiles(p.bm, p.bn));
+    if (!grad && p.bm == 64 && K >= kHalfK) {
         const int64_t parts = (K + 255) / 256;
         if (parts == 1 || (may_cut && parts * tiles(64, 64) <= 512)) p.once = true, n = parts;
     }
@@ -1627,18 +1632,15 @@ void launch_staged(const GemmArgs &g, const Plan &p, hipStream_t s) {
 }
 
 // The loss gradient's products stay with Bf16x3: a word's probabilities over the tokens, or a token's over the words, are
-// held to their own size, however far below the largest.  Its elements cost an exponential each: 128 x 256 tiles of eight waves,
-// where a 128 x 128 one leaves columns over, form them once (32768 x 256, K = 32768 3.12 ms and, x^T y, 3.33; 128 x 128 3.45, 3.85).
+// held to their own size, however far below the largest.
 template <bool AKC, bool BKC, int MODE>
 void launch(GemmArgs g, const Plan &p, hipStream_t s) {
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn, g.ranges = p.ranges;
     if constexpr (MODE == kGrad) {
-        if (p.bn == 128 && g.N > 128) {
-            g.tn = (g.N + 255) / 256;
+        if (p.bn == 256)
             hipLaunchKernelGGL((k_gemm<Bf16x3, AKC, BKC, 1, 16, MODE, 8>), dim3((unsigned)(g.tm * g.tn * g.ranges)), dim3(512), 0, s, g);
-        } else {
+        else
             launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
-        }
     }
     else if (g.K < kHalfK) launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
     else {
@@ -1670,8 +1672,8 @@ int64_t part_of(int M, int N) { return ((int64_t)M * N + 3) / 4 * 4; }
 }  // namespace
 
 int64_t matmul_workspace(int M, int N, int K) {
-    const Plan p = plan_of(M, N, K, true);
-    return p.ranges > 1 ? p.ranges * (part_of(M, N) + M) : 0;
+    const int ranges = std::max(plan_of(M, N, K, true, false).ranges, plan_of(M, N, K, true, true).ranges);      // of a product and of a loss's gradient
+    return ranges > 1 ? ranges * (part_of(M, N) + M) : 0;
 }
 
 int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
@@ -1679,7 +1681,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     GemmArgs g{};
     g.A = A, g.B = B, g.lda = lda, g.ldb = ldb, g.M = M, g.N = N, g.K = K, g.epi = epi;
     if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target, nll->vocab};
-    const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace));
+    const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace), nll != nullptr);
     const bool cut = p.ranges > 1;
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
@@ -1744,7 +1746,7 @@ int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *ta
     g.A = x, g.B = W, g.lda = dim, g.ldb = dim, g.M = rows, g.N = vocab, g.K = dim, g.C = logits, g.ldc = vocab;
     g.epi.bias = bias;
     g.nll.target = target;
-    const Plan p = plan_of(rows, vocab, dim, false);
+    const Plan p = plan_of(rows, vocab, dim, false, false);
     const int tn = p.steps ? (vocab + 127) / 128 : p.tn;
     g.part_max = workspace;
     g.part_sum = workspace + (int64_t)tn * rows;

@@ -71,7 +71,8 @@ def test_epilogues_and_column_sums(fwp, M, N, K):
     assert bool(((colsum.double() - G.double().sum(0)).abs() <= K * EPS * G.double().abs().sum(0)).all())
 
 
-@pytest.mark.parametrize("rows,vocab,dim", [(1, 5, 4), (70, 211, 64), (64, 64, 36), (300, 4099, 128), (520, 33000, 256), (6500, 6600, 132)])
+@pytest.mark.parametrize("rows,vocab,dim", [(1, 5, 4), (70, 211, 64), (64, 64, 36), (300, 4099, 128), (520, 33000, 256), (6500, 6600, 132),
+                                            (70, 33000, 288), (600, 8200, 640)])
 def test_negative_log_likelihood(fwp, rows, vocab, dim):
     L = fwp._lib
     x, W, b = randn(rows, dim, seed=1), randn(vocab, dim, seed=2) * 0.3, randn(vocab, seed=3)
