@@ -411,7 +411,7 @@ long long fwp_matmul_workspace(int M, int N, int K) {
 }
 
 // rows further apart than this could leave the 32-bit offsets within a tile
-static bool pitch_ok(long long ld, long long least) { return ld >= least && ld <= (1 << 21); }
+static bool pitch_ok(long long ld, long long least) { return ld >= least && ld <= kMatmulMaxLd; }
 
 int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C, long long ldc,
                int M, int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream) {

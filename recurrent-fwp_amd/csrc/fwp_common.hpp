@@ -190,6 +190,7 @@ int deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *be
 int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,
                       const float *gbeta, float *gqkvb, int T, int B, int H, int D, float q_scale, hipStream_t s);
 
+constexpr int kMatmulMaxLd = 1 << 21;      // floats between an operand's rows
 // fp32 matrix products on the 16-bit matrix cores (fwp_matmul); `nll`: A holds logits and stands for the gradient of
 // the loss that nll_fwd computed from them.
 struct NllView {

@@ -50,6 +50,10 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 constexpr int kBK = 32;          // k per LDS tile
 constexpr int kThreads = 256;
 constexpr unsigned kOut = 0x80000000u;      // an offset beyond every buffer: reads as zero
+// Offsets within a buffer are 32 bits: floats between operands' rows (Kept: up to 128 rows of B or 256 of k; kOut stays beyond), and between those of
+// results (at most 64 to a wave)
+constexpr int64_t kMaxLd = kMatmulMaxLd, kMaxPitch = 1 << 22;
+static_assert((255 * kMaxLd + 256) * 4 <= kOut && 64 * kMaxPitch * 4 < (int64_t)1 << 32, "offsets within a tile fit 32 bits");
 
 __device__ __forceinline__ unsigned pack2(float a, float b) {
     const bf2 r = {(__bf16)a, (__bf16)b};
@@ -361,15 +365,11 @@ struct Direct {
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int so = (int)(k_of(0, e) * ld * 4);
-                if constexpr (T == 4) {
-                    const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], so, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) w.x[i][e] = a[i];
-                } else if constexpr (T == 2) {
+                if constexpr (T == 2) {
                     const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)at[0], so, 0);
                     w.x[0][e] = a[0], w.x[1][e] = a[1];
                 } else {
-                    static_assert(T == 1, "one, two or four rows per load");
+                    static_assert(T == 1, "one or two rows per load");
                     w.x[0][e] = llvm_raw_buffer_load_f32(rs, (int)at[0], so, 0);
                 }
             }
@@ -463,14 +463,11 @@ struct Staged {
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int so = (int)(k_of(0, e) * ld * 4);
-                if constexpr (VEC == 4) {
-                    const v4f a = llvm_raw_buffer_load_v4f32(rs, (int)at[0], so, 0);
-#pragma unroll
-                    for (int t = 0; t < 4; t++) w.x[t][e] = a[t];
-                } else if constexpr (VEC == 2) {
+                if constexpr (VEC == 2) {
                     const v2f a = llvm_raw_buffer_load_v2f32(rs, (int)at[0], so, 0);
                     w.x[0][e] = a[0], w.x[1][e] = a[1];
                 } else {
+                    static_assert(VEC == 1, "one or two rows per load");
                     w.x[0][e] = llvm_raw_buffer_load_f32(rs, (int)at[0], so, 0);
                 }
             }
@@ -1594,13 +1591,15 @@ Plan plan_of(int M, int N, int K, bool may_cut, bool grad) {
     const int blocks = (M + 31) / 32;
     if (!grad && K >= kHalfK && K <= 256 && tiles(256, 128) >= kResidentTiles) {
         p.steps = K <= 128 ? 4 : 8;
-        // the most even division of the blocks over 256 CUs, a workgroup's start (its rows of B) as long as a wave's block
-        double best = 1e30;
+        // the most even division of the blocks over 256 CUs, a workgroup's start (its rows of B) as long as a wave's block: of those that
+        // take as many turns of 256 workgroups the one with most, and of those whose waves have as many blocks that with fewest
+        int64_t best = INT64_MAX;
         const int tn = (N + 127) / 128, most = std::min((blocks + 7) / 8, std::max(1, 1024 / tn));
-        for (int n = 1; n <= most; n++) {
-            const int per = (blocks + n - 1) / n;
-            const double cost = (double)(((int64_t)tn * n + 255) / 256) * ((per + 7) / 8 + 1);
-            if (cost < best) best = cost, p.per = per, p.groups = (blocks + per - 1) / per;
+        for (int turns = (tn + 255) / 256, n = 0; n < most; turns++) {
+            n = std::min(most, 256 * turns / tn);
+            const int each = ((blocks + n - 1) / n + 7) / 8, least = (blocks + 8 * each - 1) / (8 * each);
+            const int64_t cost = (int64_t)turns * (each + 1);
+            if (cost < best) best = cost, p.per = (blocks + least - 1) / least, p.groups = (blocks + p.per - 1) / p.per;
         }
     }
     p.bm = p.bn = 128;
@@ -1663,7 +1662,6 @@ void launch(GemmArgs g, const Plan &p, hipStream_t s) {
     }
 }
 
-constexpr int kMaxPitch = 1 << 22;      // of 64 rows that 32-bit offsets reach
 bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // a partial result, in whole 16-byte groups
