@@ -508,7 +508,7 @@ struct GemmArgs {
     int64_t lda, ldb, ldc, part;
     int M, N, K;
     int ks;                      // k per range (a multiple of kBK)
-    int vec;                     // C, residual and gate can be accessed 16 bytes at a time
+    int vec;                     // C, residual and gate lie 16-byte aligned, in rows of whole 16-byte groups
     int tm, tn, ranges;          // tiles, of k
     float *colsum;               // sums over k of A's rows, per range [M] (A contiguous along its rows), or NULL
     fwp_mm_epilogue epi;         // applied here when there is one range
@@ -560,8 +560,9 @@ __device__ __forceinline__ void finish(const GemmArgs &g, v4f (&acc)[MT][NT], co
     const int64_t first = (int64_t)m0 * g.ldc + n0, size = (int64_t)(left - 1) * g.ldc + nl;
     float *const C = g.C + range * g.part + first;
     if (MODE == kLse && !g.C) {
-    } else if (g.vec && nl >= 16 * NT) {
-        // rows beyond M lie behind the resource
+    } else if (nl >= 16 * NT && g.ldc <= kMaxPitch) {
+        // Rows beyond M lie behind the resource.  Buffer accesses need 4-byte alignment only, whatever N is (32768 x 1029, K = 256 74 us, element by
+        // element 116).
         unsigned at[MT];
 #pragma unroll
         for (int i = 0; i < MT; i++) at[i] = (unsigned)(row[i] * g.ldc + 4 * lc) * 4;
@@ -1684,7 +1685,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
     g.part = part_of(M, N);
-    g.vec = g.ldc % 4 == 0 && N % 4 == 0 && g.ldc <= kMaxPitch && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
+    g.vec = g.ldc % 4 == 0 && N % 4 == 0 && aligned(g.C) && aligned(epi.residual) && aligned(epi.gate);
     float *const col = cut ? workspace + p.ranges * g.part : epi.colsum;
     g.colsum = layout == FWP_MM_TN && epi.colsum ? col : nullptr;
     if (layout == FWP_MM_NT) launch<true, true, kPlain>(g, p, s);
@@ -1749,7 +1750,7 @@ int nll_fwd(const float *x, const float *W, const float *bias, const int64_t *ta
     g.part_max = workspace;
     g.part_sum = workspace + (int64_t)tn * rows;
     g.hit = logits ? nullptr : g.part_sum + (int64_t)tn * rows;
-    g.vec = vocab % 4 == 0 && vocab <= kMaxPitch && aligned(logits);
+    g.vec = vocab % 4 == 0 && aligned(logits);
     launch<true, true, kLse>(g, p, s);
     hipLaunchKernelGGL(k_nll, dim3((rows + 63) / 64), dim3(kThreads), 0, s, g.part_max, g.part_sum, g.hit, logits, target, loss,
                        lse, stats, rows, vocab, tn);
