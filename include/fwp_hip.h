@@ -170,10 +170,12 @@ int fwp_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff,
 
 /*
  * fwp_delta_fwd_strided and fwp_delta_bwd for few long sequences: given `work` (16-byte aligned,
- * fwp_delta_segment_floats floats, which may be 0) a sequence is cut into segments that run at the same time.
+ * fwp_delta_segment_floats floats, for backward fwp_delta_bwd_segment_floats, no more than those; each may be 0) a sequence is cut
+ * into segments that run at the same time.
  * `work` is scratch of the call; NULL: as the two above.  A sum's terms are grouped differently then.
  */
 long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk);
+long long fwp_delta_bwd_segment_floats(int N, int H, int L, int E, int M, int chunk);
 int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W,
                            fwp_out_view out, float *vdiff, float *ckpt, float *work, int N, int H, int L,
                            int E, int M, int chunk, void *stream);

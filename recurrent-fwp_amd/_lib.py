@@ -72,7 +72,7 @@ _MODEL_SIGNATURES = {
 }
 _WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
 EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",
-                                       "fwp_delta_ckpt_floats", "fwp_delta_segment_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
+                                       "fwp_delta_ckpt_floats", "fwp_delta_segment_floats", "fwp_delta_bwd_segment_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
 KIND_LDS, KIND_SCAN, KIND_CHUNKED, KIND_SPLIT, KIND_PHASE, KIND_STEP = 0, 1, 2, 3, 4, 5
 CFG_DELTA_KERNELS, DELTA_AUTO, DELTA_SCAN, DELTA_CHUNKED, DELTA_SPLIT, DELTA_PHASE = 0, 0, 1, 2, 3, 4
 CFG_STEP_KERNELS = 1
@@ -101,8 +101,9 @@ def lib():
         handle.fwp_check_device.restype = ctypes.c_int
         handle.fwp_delta_ckpt_floats.argtypes = [ctypes.c_int] * 6
         handle.fwp_delta_ckpt_floats.restype = ctypes.c_longlong
-        handle.fwp_delta_segment_floats.argtypes = [ctypes.c_int] * 6
-        handle.fwp_delta_segment_floats.restype = ctypes.c_longlong
+        for name in ("fwp_delta_segment_floats", "fwp_delta_bwd_segment_floats"):
+            getattr(handle, name).argtypes = [ctypes.c_int] * 6
+            getattr(handle, name).restype = ctypes.c_longlong
         for name, argtypes in _MODEL_SIGNATURES.items():
             if hasattr(handle, name):
                 getattr(handle, name).argtypes = argtypes
@@ -155,9 +156,10 @@ def delta_ckpt_floats(N, H, L, E, M, chunk):
     return n
 
 
-def segment_work(N, H, L, E, M, chunk, device):
+def segment_work(N, H, L, E, M, chunk, device, backward=False):
     """Scratch for a delta-rule call whose sequences run as several segments at once, or ``None``: they do not."""
-    n = int(lib().fwp_delta_segment_floats(N, H, L, E, M, chunk))
+    floats = lib().fwp_delta_bwd_segment_floats if backward else lib().fwp_delta_segment_floats
+    n = int(floats(N, H, L, E, M, chunk))
     return torch.empty(n, device=device, dtype=torch.float32) if n > 0 else None
 
 

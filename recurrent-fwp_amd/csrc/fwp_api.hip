@@ -186,7 +186,12 @@ int fwp_check_device(void) {
 
 long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
     if (check_dims(N, H, L, E, M, chunk)) return -1;
-    return delta_segment_floats(N, H, L, E, M, chunk);
+    return delta_segment_floats(N, H, L, E, M, chunk, false);
+}
+
+long long fwp_delta_bwd_segment_floats(int N, int H, int L, int E, int M, int chunk) {
+    if (check_dims(N, H, L, E, M, chunk)) return -1;
+    return delta_segment_floats(N, H, L, E, M, chunk, true);
 }
 
 int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,

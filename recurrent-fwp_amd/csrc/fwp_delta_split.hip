@@ -1065,19 +1065,33 @@ void launch_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp
                            q, k, v, beta, W, out, vdiff, ckpt, aux, H, L, chunk, nchunk, segs);
 }
 
-// How sequences are cut: one workgroup to a CU (two of 16 x 16 states), segments of four blocks or more, of more with wide keys,
-// whose maps take longer to go through (E = 96: 3 us each); not into fewer than four, since the maps cost a pass, and
-// not where a sequence is so short that the additional launches, 7 us of the host's, are what a step waits for.
+// From how many blocks on sequences are cut into `most` segments or fewer.  Forward alone / a training step with forward cut, with both cut, in us, 8 and
+// 64 sequences; a launch more is 3 to 5 us of the host's, which are what a short step of narrow states waits for (77 to 87 here):
+//   32 x 32:  640 steps  forward 20, 29 (uncut 30, 31), step 81, 82 / 87, 98 (80, 84); 832 steps 82, 98 / 87, 85 (100, 104)
+//   32 x 16:  640 steps  forward 18, 24 (23, 24), step 83, 83 / 86, 86 (77, 77); 1152 steps 84, 95 / 87, 87 (103, 105)
+//   16 x 32:  640 steps  forward 15, 22 (23, 23), step 80, 80 / 86, 86 (72, 77); 896 steps 80, 92 / 87, 63 (96, 98)
+//   64 x 16:  640 steps  forward 34, 43 (36, 37), step 96, 105 / 86, 96 (102, 103); 896 steps forward 38, 50 (48, 50)
+//   96 x 16:  640 steps  forward 59, 61 (49, 50), both cut 136, 142, backward alone 130, 136 (130, 136); 1024 steps forward 65, 77 (73, 74), 148, 176, 148, 183 (200, 208)
+// Backward goes from 49 to 19 us at 640 steps, 32 x 32, and gains with wider states at once; with keys of 96 features forward's maps take 3 us each to
+// go through.
+int least_blocks(int ne, int nm, int most, bool backward) {
+    if (ne == 1 && nm == 1) return 80;
+    if (backward) return ne == 2 && nm == 1 ? 72 : ne == 1 && nm == 2 ? 60 : ne == 2 && nm == 2 ? 52 : 40;
+    return ne == 6 ? most < 8 ? 60 : 52 : ne == 4 && nm == 1 && most < 8 ? 56 : 40;
+}
+
+// How sequences are cut: one workgroup to a CU (two of 16 x 16 states), segments of four blocks or more, of more with wide keys;
+// not into fewer than four, since the maps cost a pass.
 // Forward / with backward, us: 64 sequences of 2048 steps, 32 x 32, 4 segments 54 / 127, one 88 / 235, 8 60 / 144; 128 of 1024
 // steps 2 53 / 124, 1 48 / 127; 128 of 2048 steps, 16 x 16 4 40 / 94, 1 50 / 138, 2 54 / 132; 8 of 2048 steps, E = 96, M = 16 16
-// 97 / 200, 32 148 / 294, 1 136 / 386; 8 of 512 steps, 32 x 32 8 18 / 79, 1 24 / 64.
-Segments segments_of(int nseq, int L, int E, int M, int chunk) {
+// 97 / 200, 32 148 / 294, 1 136 / 386.
+Segments segments_of(int nseq, int L, int E, int M, int chunk, bool backward) {
     Segments s{nullptr, 1, 0};
     const int ne = E / 16, nm = M / 16, nblk = (L + kBlk - 1) / kBlk, per = chunk / kBlk;
     if (!split_delta_dims(E, M) || !segment_dims(ne, nm)) return s;
     const bool small = ne == 1 && nm == 1;
     const int most = (small ? 512 : 256) / nseq;
-    if (most < 4 || nblk < (small ? 80 : 40)) return s;
+    if (most < 4 || nblk < least_blocks(ne, nm, most, backward)) return s;
     int blocks = std::max((nblk + most - 1) / most, 2 * std::max(ne, 2));
     blocks = (blocks + per - 1) / per * per;
     const int count = (nblk + blocks - 1) / blocks;
@@ -1086,8 +1100,9 @@ Segments segments_of(int nseq, int L, int E, int M, int chunk) {
 }
 }  // namespace
 
-int64_t delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
-    const Segments s = segments_of(N * H, L, E, M, chunk);
+int64_t delta_segment_floats(int N, int H, int L, int E, int M, int chunk, bool backward) {
+    Segments s = segments_of(N * H, L, E, M, chunk, true);
+    if (!backward && s.count == 1) s = segments_of(N * H, L, E, M, chunk, false);      // forward's is enough for backward
     return s.count > 1 ? (int64_t)N * H * (E * M + (int64_t)(s.count - 1) * (E * M + E * E + E)) : 0;
 }
 
@@ -1097,7 +1112,7 @@ int64_t delta_segment_floats(int N, int H, int L, int E, int M, int chunk) {
 int split_delta_fwd(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out,
                     float *vdiff, float *ckpt, float *work, int N, int H, int L, int E, int M, int chunk, hipStream_t s) {
     const int nchunk = (L + chunk - 1) / chunk;
-    Segments segs = work ? segments_of(N * H, L, E, M, chunk) : Segments{nullptr, 1, 0};
+    Segments segs = work ? segments_of(N * H, L, E, M, chunk, false) : Segments{nullptr, 1, 0};
     segs.work = work;
     float *aux = delta_aux_of(ckpt, N, H, L, E, M, chunk);
 #define X(ne, nm)                                                                                        \
@@ -1114,7 +1129,7 @@ int split_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, f
                     const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, float *work, int N, int H,
                     int L, int E, int M, int chunk, hipStream_t s) {
     const int nchunk = (L + chunk - 1) / chunk;
-    Segments segs = work ? segments_of(N * H, L, E, M, chunk) : Segments{nullptr, 1, 0};
+    Segments segs = work ? segments_of(N * H, L, E, M, chunk, true) : Segments{nullptr, 1, 0};
     segs.work = work;
     const float *aux = delta_aux_of(ckpt, N, H, L, E, M, chunk);
     // four roles; the hand-over of the last five shapes takes 77 to 99 KB of LDS, one or two workgroups to a CU

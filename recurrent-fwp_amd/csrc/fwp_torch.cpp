@@ -139,7 +139,7 @@ struct DeltaBackward : torch::autograd::Node {
                 if (!tq.defined()) tq = at::empty_like(res[0]), tk = at::empty_like(res[1]), tb = at::empty_like(res[3]);
                 gq = tq, gk = tk, gb = tb;
             }
-            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk_, Q.options());
+            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk_, Q.options(), true);
             check(fwp_delta_bwd_segments(qv, kv, bv, vdiff, gv_, ckpt, gq.data_ptr<float>(), gk.data_ptr<float>(),
                                          gv_s.data_ptr<float>(), gb.data_ptr<float>(), work.defined() ? work.data_ptr<float>() : nullptr,
                                          (int)N, (int)H, (int)L, (int)E, (int)sl.width, chunk_, stream_of(Q)),
@@ -236,7 +236,7 @@ at::Tensor delta_forward(const at::Tensor &Q_in, const at::Tensor &K_in, const a
                 ckpt = vdiff + n_vdiff;
                 bufs.push_back(saved);
             }
-            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk, opts);
+            const at::Tensor work = segment_work(N, H, L, E, sl.width, chunk, opts, false);
             check(fwp_delta_fwd_segments(qv, kv, vv, bv, W_s.data_ptr<float>(), ov, vdiff, ckpt,
                                          work.defined() ? work.data_ptr<float>() : nullptr, (int)N, (int)H, (int)L, (int)E,
                                          (int)sl.width, chunk, stream_of(Q)),

@@ -109,8 +109,9 @@ inline fwp_view view_of(const at::Tensor &t) {
 }
 
 // Scratch for a delta-rule call whose sequences run as several segments at once; undefined: they do not.
-inline at::Tensor segment_work(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M, int chunk, const at::TensorOptions &opts) {
-    const int64_t n = fwp_delta_segment_floats((int)N, (int)H, (int)L, (int)E, (int)M, chunk);
+inline at::Tensor segment_work(int64_t N, int64_t H, int64_t L, int64_t E, int64_t M, int chunk, const at::TensorOptions &opts,
+                               bool backward) {
+    const int64_t n = (backward ? fwp_delta_bwd_segment_floats : fwp_delta_segment_floats)((int)N, (int)H, (int)L, (int)E, (int)M, chunk);
     return n > 0 ? at::empty({n}, opts) : at::Tensor();
 }
 

@@ -201,7 +201,7 @@ at::Tensor projection_grad(const at::Tensor &go, const at::Tensor &qkvb, const a
     const float *vdiff = ptr(buf), *ckpt = vdiff + rows * H * D;
     const fwp_view gov = {ptr(go), H * D, D, B * H * D};
     const int chunk = fwp_query(FWP_Q_DEFAULT_CHUNK);
-    const at::Tensor work = segment_work(B, H, T, D, D, chunk, go.options());
+    const at::Tensor work = segment_work(B, H, T, D, D, chunk, go.options(), true);
     check(fwp_delta_bwd_segments(view_of(q), view_of(k), view_of(beta), vdiff, gov, ckpt, ptr(gq), ptr(gk), ptr(gv), ptr(gb), ptr(work), (int)B,
                                  (int)H, (int)T, (int)D, (int)D, chunk, s),
           "fwp_delta_bwd_segments");
@@ -265,7 +265,7 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
             vdiff = ptr(saved);
             ckpt = vdiff + n_vdiff;
         }
-        const at::Tensor work = segment_work(B, H, T, D, D, chunk, opts);
+        const at::Tensor work = segment_work(B, H, T, D, D, chunk, opts, false);
         check(fwp_delta_fwd_segments(view_of(q), view_of(k), view_of(v), view_of(beta), ptr(state), ov, vdiff, ckpt, ptr(work), (int)B,
                                      (int)H, (int)T, (int)D, (int)D, chunk, s),
               "fwp_delta_fwd_segments");

@@ -97,7 +97,7 @@ class DeltaFastWeight(torch.autograd.Function):
         grad_V = torch.empty((N, H, L, M), device=Q.device, dtype=torch.float32)
         grad_beta = torch.empty((N, H, L, 1), device=Q.device, dtype=torch.float32)
         with _lib.on_device(Q):
-            work = _lib.segment_work(N, H, L, E, M, chunk, Q.device)
+            work = _lib.segment_work(N, H, L, E, M, chunk, Q.device, True)
             rc = _lib.lib().fwp_delta_bwd_segments(
                 qv, kv, bv, vdiff, gv_, ckpt, _lib.ptr(grad_Q),
                 _lib.ptr(grad_K), _lib.ptr(grad_V), _lib.ptr(grad_beta), work if work is None else _lib.ptr(work),

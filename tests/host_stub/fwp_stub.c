@@ -89,6 +89,9 @@ long long fwp_delta_segment_floats(int N, int H, int L, int E, int M, int chunk)
     (void)chunk;
     return L < 256 ? 0 : (long long)N * H * (L / 64) * (E * M + E * E);
 }
+long long fwp_delta_bwd_segment_floats(int N, int H, int L, int E, int M, int chunk) {
+    return L < 320 ? 0 : fwp_delta_segment_floats(N, H, L, E, M, chunk) - 1;
+}
 int fwp_delta_fwd_segments(fwp_view q, fwp_view k, fwp_view v, fwp_view beta, float *W, fwp_out_view out, float *vdiff,
                            float *ckpt, float *work, int N, int H, int L, int E, int M, int chunk, void *stream) {
     if (work) fill(work, fwp_delta_segment_floats(N, H, L, E, M, chunk), 1);
@@ -117,7 +120,7 @@ int fwp_delta_bwd(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp
 int fwp_delta_bwd_segments(fwp_view q, fwp_view k, fwp_view beta, const float *vdiff, fwp_view grad_out,
                            const float *ckpt, float *gq, float *gk, float *gv, float *gbeta, float *work, int N, int H, int L,
                            int E, int M, int chunk, void *stream) {
-    if (work) fill(work, fwp_delta_segment_floats(N, H, L, E, M, chunk), 1);
+    if (work) fill(work, fwp_delta_bwd_segment_floats(N, H, L, E, M, chunk), 1);
     return fwp_delta_bwd(q, k, beta, vdiff, grad_out, ckpt, gq, gk, gv, gbeta, N, H, L, E, M, chunk, stream);
 }
 

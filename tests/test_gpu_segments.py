@@ -8,15 +8,16 @@ from helpers import delta_inputs, within
 
 pytestmark = pytest.mark.gpu
 
-# N, H, L, E, M: the shortest that is cut, a last segment of one step, of whole blocks, key widths of each kernel
+# N, H, L, E, M: the shortest that is cut, a last segment of one step, of whole blocks, key widths of each kernel; values in slices of columns
 SHAPES = [(1, 8, 640, 32, 32), (1, 1, 641, 32, 16), (2, 3, 1281, 16, 16), (1, 5, 1408, 16, 32), (2, 2, 700, 16, 64), (1, 2, 1000, 64, 16),
-          (1, 2, 777, 64, 64), (1, 3, 900, 96, 16), (2, 1, 830, 96, 32), (1, 2, 650, 32, 64), (8, 8, 1000, 32, 32)]
+          (1, 2, 777, 64, 64), (1, 3, 900, 96, 16), (2, 1, 830, 96, 32), (1, 2, 650, 32, 64), (8, 8, 1000, 32, 32),
+          (1, 2, 900, 64, 32), (1, 1, 1200, 32, 16), (1, 2, 1200, 96, 97)]
 
 
 @pytest.mark.parametrize("N,H,L,E,M", SHAPES)
 @pytest.mark.parametrize("steps_first", [False, True])
 def test_segments_against_the_oracle(fwp, N, H, L, E, M, steps_first):
-    assert fwp._lib.lib().fwp_delta_segment_floats(N, H, L, E, M, 64) > 0
+    assert fwp._lib.lib().fwp_delta_segment_floats(N, H, L, E, M if M % 16 == 0 else 16, 64) > 0
     *x, W0, go = delta_inputs(3, N, H, L, E, M, np.float32, w0=True)
     dev = lambda a: (torch.from_numpy(a).permute(2, 0, 1, 3).contiguous().cuda().permute(1, 2, 0, 3) if steps_first
                      else torch.from_numpy(a).cuda())
@@ -130,3 +131,26 @@ def test_what_is_cut(fwp):
     assert floats(1, 8, 639 - 15, 32, 32) == 0 and floats(8, 8, 2048, 32, 32) > 0 and floats(9, 8, 2048, 32, 32) == 0
     assert floats(1, 8, 1264, 16, 16) == 0 and floats(16, 8, 2048, 16, 16) > 0 and floats(17, 8, 2048, 16, 16) == 0
     assert floats(1, 8, 4096, 128, 16) == 0 and floats(1, 8, 4096, 24, 24) == 0 and floats(0, 8, 4096, 16, 16) == -1
+
+
+def test_backward_is_cut_on_its_own(fwp):
+    """Forward and backward are cut from other lengths on; what forward's scratch holds is enough for backward."""
+    lib = fwp._lib.lib()
+    fwd, bwd = lib.fwp_delta_segment_floats, lib.fwp_delta_bwd_segment_floats
+    for E in (16, 32, 64, 96):
+        for M in (16, 32, 64):
+            for seqs in (1, 8, 32, 64, 100):
+                for L in range(600, 1400, 16):
+                    assert 0 <= bwd(1, seqs, L, E, M, 64) <= fwd(1, seqs, L, E, M, 64)
+    assert fwd(1, 8, 768, 32, 32, 64) > 0 and bwd(1, 8, 768, 32, 32, 64) == 0 and bwd(1, 8, 832, 32, 32, 64) > 0
+    assert bwd(1, 64, 640, 96, 16, 64) > 0
+
+
+@pytest.mark.parametrize("N,H,L,E,M", [(1, 2, 800, 64, 32), (1, 8, 1000, 32, 32), (1, 2, 1300, 16, 16), (1, 2, 1300, 96, 16)])
+@pytest.mark.parametrize("chunk,kind", [(64, "DELTA_SCAN"), (128, "DELTA_AUTO"), (256, "DELTA_AUTO")])
+def test_segments_of_other_chunks_and_forward_kernels(fwp, N, H, L, E, M, chunk, kind):
+    """Backward in segments behind a forward whose kernels leave no inverses; checkpoints further apart."""
+    arrays = delta_inputs(6, N, H, L, E, M, np.float32, w0=True)
+    got, want = run(fwp, arrays, True, chunk, getattr(fwp._lib, kind)), oracle_of(arrays)
+    for name, w in want.items():
+        assert within(got[name], w, 1e-4, 1e-5), name
