@@ -48,6 +48,8 @@ typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kBK = 32;          // k per LDS tile
+// Registers are spilled in rare code first
+__device__ __forceinline__ bool rarely(bool x) { return __builtin_expect(x, false); }
 constexpr int kThreads = 256;
 constexpr unsigned kOut = 0x80000000u;      // an offset beyond every buffer: reads as zero
 // Offsets within a buffer are 32 bits: floats between operands' rows (Kept: up to 128 rows of B or 256 of k; kOut stays beyond), and between those of
@@ -265,8 +267,9 @@ __device__ __forceinline__ void drop_tiny8(float *x, float s) {
     for (int e = 0; e < 8; e++) x[e] = fabsf((float)(_Float16)(x[e] * s)) < kTiny ? 0.f : x[e];
 }
 
-// A lane's elements of ROWS rows, scaled: the largest magnitude, and each row's before that; the smallest; the smallest that is not zero
-// (a third more instructions, but where there are zeros, ReLU's, no second look).
+// A lane's elements of ROWS rows, scaled: the largest magnitude, and each row's before that; the smallest; the smallest that is not zero, which takes
+// three times the instructions: looked for from the first zero on (32768 x 256, K = 1024 always 72.4 us, so 71.1; where a zero of B's rows, beyond the last
+// of 776, led to a second look at every step, 8192 x 776, K = 1024 70.1 -> 62.9).
 template <int ROWS>
 __device__ __forceinline__ float largest_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS], float (&m)[ROWS]) {
     float all = 0.f;
@@ -824,6 +827,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
         Stage *const L = reinterpret_cast<Stage *>(shared);
         bool change = false;      // of scales of A's rows
         unsigned small_a = 0;
+        bool zeros_a = false, zeros_b = false;      // there are zeros: ReLU's, rows beyond the last
         int spent = 0;
         v4u fa[2][MT][T::kPlanes];
         float part_sum[MT];       // of a step's elements of A's rows
@@ -862,10 +866,12 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
             if constexpr (T::kScaled) {
                 float ma[MT], mb[OpB::kUnits];
                 const bool beyond = fmaxf(largest_of(x.x, a.s, ma), largest_of(y.x, b.s, mb)) > kLargest;
-                float la = smallest_nonzero_of(x.x, a.s), lb = smallest_of(y.x, b.s);
+                float la = zeros_a ? smallest_nonzero_of(x.x, a.s) : smallest_of(x.x, a.s);
+            float lb = zeros_b ? smallest_nonzero_of(y.x, b.s) : smallest_of(y.x, b.s);
                 int word = 0;
                 small_a = 0;
-                if (__any(beyond || fminf(la, lb) < kSmall)) {
+                if (rarely(__any(beyond || fminf(la, lb) < kSmall))) {
+                zeros_a |= __any(la == 0.f) != 0, zeros_b |= __any(lb == 0.f) != 0;
                     if (__any(beyond)) {
                         change = true, word = kChange;
                         la = lb = 0.f;
@@ -900,21 +906,21 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
                 const int of[4] = {__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y), __builtin_amdgcn_readfirstlane(w.z),
                                    __builtin_amdgcn_readfirstlane(w.w)};
                 const int all = of[0] | of[1] | of[2] | of[3];
-                if (all & kChange) {
+                if (rarely(all & kChange)) {
 #pragma unroll
                     for (int j = 0; j < NT; j++)
                         if (of[OpB::owner(j)] & kChange)
 #pragma unroll
                             for (int i = 0; i < MT; i++) acc[i][j] *= *reinterpret_cast<const v4f *>(change_b[parity] + 16 * j + 4 * lc);
                 }
-                if (change) {
+                if (rarely(change)) {
                     change = false;
 #pragma unroll
                     for (int i = 0; i < MT; i++)
 #pragma unroll
                         for (int j = 0; j < NT; j++) acc[i][j] *= change_a[wave][OpA::row_of(i, lr)];
                 }
-                if (all & (0xff | kStop | 0xf * kCountA)) {
+                if (rarely(all & (0xff | kStop | 0xf * kCountA))) {
                     spent += kPatience * (of[0] / kCountA + of[1] / kCountA + of[2] / kCountA + of[3] / kCountA + __popc(all & 0xff));
                     if (all & kStop || spent > kGrace) return true;
                     add_rests(acc, x.x, a.s, small_a, all & 0xff, fa[parity], L[parity], unit, [&](int j, int e) { return of[OpB::owner(j)] >> e & 1; },
@@ -1008,7 +1014,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     bool odd_tile = false;
 #pragma unroll
     for (int w = 0; w < WAVES; w++) odd_tile |= odd_waves[w] != 0;
-    if (odd_tile) {
+    if (rarely(odd_tile)) {
         // the tile once more from the fp32 operands
 #pragma unroll
         for (int i = 0; i < MT; i++) {
@@ -1291,14 +1297,16 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
     v4f acc[MT][NT];
     float change[MT];
     bool changed = false, far = false;
-    bool small_a = false;
+    bool small_a = false, zeros = false;      // zeros: A has elements that are zero, ReLU's
     // zeros beyond K, scales that the step's elements fit, and whether some are small
     const auto prepare = [&](OpA::Raw &x, int k0) __attribute__((always_inline)) {
         if (K % 4 && k0 + kBK > K) a.cut(x, k0, K);
         float m[MT];
         const bool beyond = largest_of(x.x, a.s, m) > kLargest;
         small_a = false;
-        if (__any(beyond || smallest_nonzero_of(x.x, a.s) < kSmall)) {
+        const float smallest = zeros ? smallest_nonzero_of(x.x, a.s) : smallest_of(x.x, a.s);
+        if (rarely(__any(beyond || smallest < kSmall))) {
+            zeros |= __any(smallest == 0.f) != 0;
             if (__any(beyond)) {
                 changed = true;
 #pragma unroll
@@ -1330,7 +1338,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
         // the products of step s, beside the split of step s + 1 and the loads of step s + 2, which may be the next block's
         const auto step = [&](auto parity, int s) __attribute__((always_inline)) {
             constexpr int p = decltype(parity)::value;
-            if (changed && s > 0) {      // results so far to the scales of step s
+            if (rarely(changed && s > 0)) {      // results so far to the scales of step s
 #pragma unroll
                 for (int i = 0; i < MT; i++)
 #pragma unroll
@@ -1338,8 +1346,8 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             }
             changed = false;
             const unsigned b_here = (unsigned)(small_b >> 8 * s) & 0xff;
-            if (small_a) add_small(acc, ra[p].x, a.s, fa[p], L[s], unit);
-            if (b_here)
+            if (rarely(small_a)) add_small(acc, ra[p].x, a.s, fa[p], L[s], unit);
+            if (rarely(b_here != 0))
                 add_rests(acc, ra[p].x, a.s, 0, b_here, fa[p], L[s], unit, [&](int, int e) { return b_here >> e & 1; }, [&](int j, int e) {
                     const int at = Rests<BN>::place(small_b, 8 * s + e);
                     return at < Rests<BN>::kKept ? rests.kept[at][lc][16 * j + lr]
@@ -1378,7 +1386,7 @@ __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, i
             step(std::integral_constant<int, 1>(), s + 1);
         }
         const int *eb = exponents[0];
-        if (any_odd(acc) || __any(odd)) {
+        if (rarely(any_odd(acc) || __any(odd))) {
             // an element that is not finite (0 times it is NaN) or too small: the block once more from the fp32 operands
             OpA::Raw x;
             clear();
