@@ -289,9 +289,9 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
 /*
  * fp32 matrix product C[M,N] on the 16-bit matrix cores, fp32 sums: each operand as the sum of three bf16 numbers (K < 128),
  * or, scaled by a power of two for each row of A and column of B, of two fp16 numbers.  These hold an element to 2^-23 of itself; one so
- * small beside its row's or column's largest that they would lose more than 2^-19 of it is multiplied apart, on fp32.  For the projections and feed-forward layers around the operators
- * (language_modeling/src/utils/cuda_fast_weight_layer.py:108,163, utils/model_utils.py:45-50), which the
- * reference leaves to its BLAS.
+ * small beside its row's or column's largest that they would lose more than 2^-19 of it is multiplied apart.
+ * For the projections and feed-forward layers around the operators (language_modeling/src/utils/cuda_fast_weight_layer.py:108,163,
+ * utils/model_utils.py:45-50), which the reference leaves to its BLAS.
  *   FWP_MM_NT: C = A B^T, A [M,K], B [N,K]      FWP_MM_NN: C = A B, A [M,K], B [K,N]
  *   FWP_MM_TN: C = A^T B, A [K,M], B [K,N]      row-major, rows lda, ldb, ldc floats apart
  * epi (NULL: none): C = relu(C + bias) + residual, 0 where gate <= 0, each part optional (a NaN passes relu and gate, as in

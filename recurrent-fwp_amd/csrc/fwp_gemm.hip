@@ -9,10 +9,10 @@
 // fp16 has few exponents: s brings a row's largest element so far to [2^13, 2^14).  One beyond 65504 / s (a row that grows fourfold
 // or more along k) moves s, and the row's results so far with it.  An element below about 2^-20 of its row's largest would lose bits: the
 // waves look for those, and what two numbers leave of them is multiplied apart, so that an element counts to 2^-19 of itself or better
-// whatever is in its row (a result may be made of small elements alone).  The search costs 4 to 7 us of 65, 32768 x 256, K = 1024.
+// whatever is in its row (a result may be made of small elements alone).  The search costs 7 us of 71, 32768 x 256, K = 1024.
 // Where small elements are many (tokens' gradients, features of very different sizes) that is left: step by step kernels go on with Bf16x3,
 // those with B's rows kept make the products of the small elements once more, small products are formed again on fp32.  x^T y, 1024 x 256, K = 32768,
-// the size of k exp(a N(0,1)), a = 0 / 1.5 / 3 / 5: 86 / 103 / 100 / 98 us (Bf16x3 alone 96; element by element 84 / 122 / 301 / 460).
+// the size of k exp(a N(0,1)), a = 0 / 1.5 / 3 / 5: 82 / 103 / 100 / 98 us (Bf16x3 alone 96; element by element 84 / 122 / 301 / 460).
 //
 // Bf16x3 (smaller K, and the loss's gradient): x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest: 3 x 8 significant bits and
 // their signs hold all 24), six products, h h', h m', m h', m m', h l', l h'; the three left out are below 2^-26 |x x'|.  bf16
@@ -754,8 +754,8 @@ __device__ __forceinline__ void add_small(v4f (&acc)[MT][NT], const float (&x)[M
 }
 
 // A workgroup of WAVES waves: a wave 16 MT rows and all 16 NT columns; B's rows are staged step by step, in two
-// alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 60 us (one 128 x 128 tile with both
-// operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6.
+// alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 71 us (one 128 x 128 tile with both
+// operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6, the look for small elements 7.
 template <class S, bool AKC, bool BKC, int MT, int NT, int MODE, int WAVES = 4>
 __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     constexpr int WM = 16 * MT, BM = WAVES * WM, BN = 16 * NT;
@@ -1244,7 +1244,7 @@ __device__ __forceinline__ bool any_odd(const v4f (&acc)[MT][NT]) {      // 0 ti
 
 // Products with K up to 32 KS: a workgroup keeps 16 NT of B's rows, split, in LDS and its eight waves go over blocks of 32
 // rows of A, each by itself, without barriers: one wave's results leave while others multiply.  32768 x 1024, K = 256 with bias and
-// ReLU 64 us (staged 87; memory alone 35), 24576 x 2048, K = 128 with a gate 100 us (127; 87).
+// ReLU 64 us (staged 87; memory alone 35), 24576 x 2048, K = 128 with a gate 100 us (127; 87), all before the look for small elements (4 to 8 us).
 template <bool BKC, int KS, int NT, int MODE>
 __global__ __launch_bounds__(2 * kThreads, 2) void k_gemm_resident(GemmArgs g, int per) {
     typedef Half2 S;
@@ -1583,6 +1583,7 @@ constexpr int kResidentTiles = 200;
 // Half2's error is the smaller one from here on; below, Bf16x3's (K = 64: 1.08e-7 and 1.06e-7, K = 32: 8.8e-8 and 6.3e-8).
 constexpr int kHalfK = 128;
 
+// (These times and those below are without the look for small elements, which takes a tenth on either side.)
 // Staged: 128 x 128 tiles where, with k cut into ranges, they are three for two CUs; else 128 x 64 if those are; else 64 x 64.
 // 32768 x 256, K = 1024 (512 tiles) 60 us, 77, 80; 16384 x 256, K = 1024 (256 tiles) 47, 41, 48 us; 2381 x 1024, K = 256
 // (152, 304, 608 tiles) 16.2, 15.9, 14.3 us; 300 x 256, K = 256 13.9, 10.3, 8.6 us.  Those of 64 x 64 all at once where a tile's k
