@@ -12,7 +12,7 @@
 // whatever is in its row (a result may be made of small elements alone).  The search costs 7 us of 71, 32768 x 256, K = 1024.
 // Where small elements are many (tokens' gradients, features of very different sizes) that is left: step by step kernels go on with Bf16x3,
 // those with B's rows kept make the products of the small elements once more, small products are formed again on fp32.  x^T y, 1024 x 256, K = 32768,
-// the size of k exp(a N(0,1)), a = 0 / 1.5 / 3 / 5: 82 / 103 / 100 / 98 us (Bf16x3 alone 96; element by element 84 / 122 / 301 / 460).
+// the size of k exp(a N(0,1)), a = 0 / 1.5 / 3 / 5: 80 / 102 / 103 / 98 us (Bf16x3 alone 96; element by element 84 / 122 / 301 / 460).
 //
 // Bf16x3 (smaller K, and the loss's gradient): x = h + m + l (h = bf16(x), m = bf16(x - h), l = the rest: 3 x 8 significant bits and
 // their signs hold all 24), six products, h h', h m', m h', m m', h l', l h'; the three left out are below 2^-26 |x x'|.  bf16
@@ -291,23 +291,23 @@ __device__ __forceinline__ float smallest_nonzero_of(const float (&x)[ROWS][8], 
     for (int i = 0; i < ROWS; i++) all = abs_min3(all, nonzero_min8(x[i]) * s[i].s, INFINITY);
     return all;
 }
-// Which of the wave's lanes' elements are small (bit e: those at e; bit 8: some are tiny); far: one is too small even for its rest.  Short
-// code: it is run so rarely that it is fetched each time.
+// Which of the wave's lanes' elements are small (bit e: those at e; bit 8: some are tiny); far: one is too small even for its rest.  Two
+// instructions an element: with gradients as operands it is run every few steps (a loop over e that picks the elements: 10 an element, a training step of the
+// benchmark's model 0.3 ms more).
 constexpr unsigned kSomeTiny = 1u << 8;
 template <int ROWS>
 __device__ __forceinline__ unsigned small_of(const float (&x)[ROWS][8], const Scale (&s)[ROWS], bool &far) {
     const float least = smallest_nonzero_of(x, s);
     if (!__any(least < kSmall)) return 0;
     far |= least < kLeast;
-    unsigned m = __any(least < kTiny) ? kSomeTiny : 0u;
-#pragma unroll 1
+    unsigned m = __any(least < kTiny) ? kSomeTiny : 0u, below[ROWS];      // below: twice the bits of kSmall / s, as a zero's are largest
+#pragma unroll
+    for (int i = 0; i < ROWS; i++) below[i] = (__float_as_uint(ldexpf(kSmall, s[i].exponent())) << 1) - 1;
+#pragma unroll
     for (int e = 0; e < 8; e++) {
         bool small = false;
 #pragma unroll
-        for (int i = 0; i < ROWS; i++) {
-            const float v = pick(x[i], e);
-            small |= v != 0.f && fabsf(v * s[i].s) < kSmall;
-        }
+        for (int i = 0; i < ROWS; i++) small |= (__float_as_uint(x[i][e]) << 1) - 1 < below[i];
         m |= __any(small) ? 1u << e : 0u;
     }
     return m;
