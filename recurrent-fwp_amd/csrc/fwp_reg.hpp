@@ -259,6 +259,101 @@ __device__ __forceinline__ float row_reduce(float x, Op op) {
     return x;
 }
 
+// 32 x 32 matrices and vectors of 32 without conversions.  A vector is held in one of two forms, by rows of 16 lanes (x0: its
+// entries 0 .. 15, x1: 16 .. 31): half form x0 x1 x0 x1 (lane l: entry l % 32) or pair form x0 x0 x1 x1.  Either is what the row
+// rotations of a product take whose results come out in the other one: a lane has 16 entries of a matrix, those of one result
+// and of the half of the terms that its row holds; the two lanes of a result are added by one exchange of rows.  So a chain of
+// products alternates between the forms, and between matrices held for either, where lanes l = 2 col + s need a
+// ds_bpermute per 16 entries (60 cycles before its result can be used) between any two.
+namespace forms {
+__device__ __forceinline__ int half(int lane) { return lane % 32; }
+__device__ __forceinline__ int pair(int lane) { return lane / 32 * 16 + lane % 16; }
+// the terms that register j of a matrix belongs to: with results in half form (terms in pair form), and the other way round
+__device__ __forceinline__ int terms_of_half(int lane, int j) { return lane / 32 * 16 + ((lane - j) & 15); }
+__device__ __forceinline__ int terms_of_pair(int lane, int j) { return lane / 16 % 2 * 16 + ((lane - j) & 15); }
+
+// x is about to be rotated by an asm statement below: the wait states between a vector instruction that wrote it and a DPP
+// read of it, which the compiler cannot see there.
+__device__ __forceinline__ float ready(float x) {
+    asm volatile("s_nop 1" : "+v"(x));
+    return x;
+}
+
+__device__ __forceinline__ void ready(float &x, float &y) { asm volatile("s_nop 1" : "+v"(x), "+v"(y)); }
+
+// Products J of N dots that share x, NA accumulators each.  N NA is four or more: between two asm statements of which the second adds to
+// the first's result the compiler wants three others, or puts wait states there.
+template <int N, int NA, int J>
+__device__ __forceinline__ void dots1(const float (*const (&w)[N])[16], float x, float (&acc)[N][NA]) {
+#pragma unroll
+    for (int n = 0; n < N; n++) acc[n][J % NA] = J < NA ? mul_ror<J>(x, (*w[n])[J]) : fmac_ror<J>(acc[n][J % NA], x, (*w[n])[J]);
+}
+template <int N, int NA, int FROM = 0, int... J>
+__device__ __forceinline__ void dots(const float (*const (&w)[N])[16], float x, float (&acc)[N][NA], std::integer_sequence<int, J...>) {
+    (dots1<N, NA, FROM + J>(w, x, acc), ...);
+}
+// products FROM .. FROM + 3 of a dot with four accumulators
+template <int FROM>
+__device__ __forceinline__ void dot_part(const float (&w)[16], float x, float (&acc)[1][4]) {
+    dots<1, 4, FROM>({&w}, x, acc, std::make_integer_sequence<int, 4>{});
+}
+template <bool NEG, int... J>
+__device__ __forceinline__ void rank1_1(float *w, float x, float y, std::integer_sequence<int, J...>) {
+    ((w[J] = fmac_ror<J, NEG>(w[J], x, y)), ...);
+}
+// a lane's share of a product: sum_j w[j] x[terms(j)]; of three products with the same vector
+__device__ __forceinline__ float dot(const float (&w)[16], float x) {
+    float a[1][4];
+    dots({&w}, x, a, std::make_integer_sequence<int, 16>{});
+    return (a[0][0] + a[0][1]) + (a[0][2] + a[0][3]);
+}
+__device__ __forceinline__ void dot3(const float (&w0)[16], const float (&w1)[16], const float (&w2)[16], float x, float &r0, float &r1, float &r2) {
+    float a[3][2];
+    dots({&w0, &w1, &w2}, x, a, std::make_integer_sequence<int, 16>{});
+    r0 = a[0][0] + a[0][1], r1 = a[1][0] + a[1][1], r2 = a[2][0] + a[2][1];
+}
+__device__ __forceinline__ void dot2(const float (&w0)[16], const float (&w1)[16], float x, float &r0, float &r1) {
+    float a[2][2];
+    dots({&w0, &w1}, x, a, std::make_integer_sequence<int, 16>{});
+    r0 = a[0][0] + a[0][1], r1 = a[1][0] + a[1][1];
+}
+// w[j] += x[terms(j)] * y  (NEG: -=)
+template <bool NEG = false>
+__device__ __forceinline__ void rank1(float (&w)[16], float x, float y) {
+    rank1_1<NEG>(w, x, y, std::make_integer_sequence<int, 16>{});
+}
+
+// Shares to results: in half form (the shares lie 32 lanes apart), in pair form (16 lanes apart), or the former's shares in
+// pair form, which takes one more exchange.
+__device__ __forceinline__ float sum_to_half(float x) {
+    float y = x;
+    swap32(x, y);
+    return x + y;
+}
+__device__ __forceinline__ float sum_to_pair(float x) {
+    float y = x;
+    swap16(x, y);
+    return x + y;
+}
+__device__ __forceinline__ float half_shares_to_pair(float x) {
+    float y = x;
+    swap16(x, y);
+    swap32(x, y);
+    return x + y;
+}
+// The sum over a row's 16 lanes, added in the same order (to the last bit) for all of them: pairs, quads, mirrored halves.
+__device__ __forceinline__ float row_sum(float x) {
+    x += dpp<kQuadXor1>(x);
+    x += dpp<kQuadXor2>(x);
+    x += dpp<0x141>(x);      // row_half_mirror
+    x += dpp<0x140>(x);      // row_mirror
+    return x;
+}
+// the sum over a vector's entries: of one in pair form; of two in half form, one in each half of the wave
+__device__ __forceinline__ float sum_of_pair(float x) { return sum_to_half(row_sum(x)); }
+__device__ __forceinline__ float sums_of_halves(float x) { return sum_to_pair(row_sum(x)); }
+}  // namespace forms
+
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace fwp

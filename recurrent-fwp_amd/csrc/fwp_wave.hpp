@@ -33,15 +33,17 @@ __device__ __forceinline__ float group_sum(float x) {
     return x;
 }
 
-// Exchange between the four 16-lane rows of the wave.  The compiler's builtins
-// for these two gfx950 instructions drop the second result, hence the asm.
-// After swap16: a = {r0,r0,r2,r2}, b = {r1,r1,r3,r3} for a = b = {r0,r1,r2,r3};
-// after swap32: a = {lo,lo}, b = {hi,hi}.
+// Exchange between the four 16-lane rows of the wave.
+// After swap16: a = {a0,b0,a2,b2}, b = {a1,b1,a3,b3} for a = {a0,a1,a2,a3}, b = {b0,b1,b2,b3};
+// after swap32: a = {a0,a1,b0,b1}, b = {a2,a3,b2,b3}.
+// (The builtins' two results have to go through variables: __builtin_bit_cast of the second element gives the first.)
 __device__ __forceinline__ void swap16(float &a, float &b) {
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
 }
 __device__ __forceinline__ void swap32(float &a, float &b) {
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
 }
 
 // Forces x to be computed by every lane at this point.  Values that come out of cross-lane
