@@ -6,8 +6,9 @@
 // operand with one ds_bpermute per 16 entries.  In backward the softmax of the delayed output does
 // not sit on the sequential path: it is recomputed for a whole tile when the tile is committed.
 // Up to 1024 sequences the forward step is divided between two waves of a sequence, the backward step
-// between three (up to 512 sequences) or two, which hand tiles over through LDS.
+// between four (up to 512 sequences; 16 x 16: three) or two, which hand tiles over through LDS.
 #include "fwp_reg.hpp"
+#include "fwp_mfma.hpp"
 
 namespace fwp {
 namespace {
@@ -1014,17 +1015,282 @@ __global__ __launch_bounds__(kWave * 6) void k_rnn_bwd_tri(
     else rnn_bwd_tri_a<D>(M, gv, gbeta, L, seq, lane);
 }
 
+// ------------------------------------------- 32 x 32 states, backward: four waves per sequence
+//
+// The division of the three waves with grad_k's two parts on a wave each, and vectors in half and pair form (fwp_reg.hpp), so that
+// no wave converts an operand: wave X carries the gradient of h through W and the softmax; one tile behind, wave A keeps G by columns and
+// forms r = G^T k, grad_v, a and grad_beta's terms; two tiles behind, wave D keeps G by rows and forms G u, and wave E forms W a, loads and
+// stores.  256 steps, 8 / 256 / 512 sequences: 54 / 57 / 71 us where three waves take 72 / 76 / 79.  Bound by X's chain while a sequence has a CU
+// to itself, beyond by issue: 70 to 80 instructions a step of each wave, two waves to a SIMD.
+typedef float rnn_v4f __attribute__((ext_vector_type(4)));
+constexpr int kRnnTile = 16;                // steps to a tile (8: 59 / 73 us)
+constexpr int kRnnRows = kRnnTile / 8;      // of eight rows each: a wave's 16-byte accesses to a tile
+struct RnnBwdLds {
+    static constexpr int T = kRnnTile * 32;
+    float k[4][T], u[4][T], s[4][T], d[4][T], b[4][kRnnTile];      // u = beta (v - v_old), s = softmax(h_{t-1})
+    float go[2][T], g[3][T], a[2][T], pd[2][T], gu[2][T], wa[2][T];
+};
+
+struct RnnBwdArgs {
+    fwp_view k, beta, go;
+    const float *vdiff, *out, *h_init, *ckpt;
+    float *gz, *gk, *gv, *gbeta;
+    int H, L, chunk, nchunk, nseq;
+};
+
+// Every wave runs the same rounds: the one that is LAG tiles behind works on tile ntile - 1 - (j - LAG) in round j, if there is one.
+template <int LAG, class Work>
+__device__ __forceinline__ void rnn_rounds(int ntile, Work work) {
+#pragma unroll 1
+    for (int j = 0; j < ntile + 2; j++) {
+        const int t = ntile - 1 - (j - LAG);
+        if (t >= 0 && t < ntile) work(t);
+        lds_barrier();
+    }
+}
+
+// The steps of a tile, last first, the operands of the next one asked for ahead
+template <class Ops, class Load, class Step>
+__device__ __forceinline__ void rnn_steps_back(int nst, Load load, Step step) {
+    if (nst == kRnnTile) {
+        Ops ring[2];
+        load(ring[(kRnnTile - 1) & 1], kRnnTile - 1);
+#pragma unroll
+        for (int tt = kRnnTile - 1; tt >= 0; tt--) {
+            if (tt) load(ring[(tt - 1) & 1], tt - 1);
+            step(ring[tt & 1], tt);
+        }
+    } else {
+#pragma unroll 1
+        for (int tt = nst - 1; tt >= 0; tt--) {
+            Ops o;
+            load(o, tt);
+            step(o, tt);
+        }
+    }
+}
+
+// The state after the last step of chunk c, by rows (results of products over its values in half form)
+__device__ __forceinline__ void rnn_state_rows(float (&W)[16], const RnnBwdArgs &g, int64_t seq, int c, int lane) {
+    const float *src = g.ckpt + ((seq * g.nchunk + c) * 32 + forms::half(lane)) * 32;
+#pragma unroll
+    for (int j = 0; j < 16; j++) W[j] = src[forms::terms_of_half(lane, j)];
+}
+
+__device__ __forceinline__ void rnn_bwd_x(RnnBwdLds &M, const RnnBwdArgs &g, int64_t seq, int lane) {
+    using namespace forms;
+    constexpr int D = 32, TL = kRnnTile;
+    const int half = forms::half(lane), pair = forms::pair(lane), L = g.L, ntile = (L + TL - 1) / TL;
+    float W[16], Wnext[16], dh = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; j++) W[j] = 0.f;
+    rnn_state_rows(Wnext, g, seq, g.nchunk - 1, lane);
+    struct Ops {
+        float u, k, s, go;
+    };
+    lds_barrier();
+    rnn_rounds<0>(ntile, [&](int it) {
+        const int t0 = it * TL, nst = min(TL, L - t0), slot = it & 3;
+        if ((t0 + nst) % g.chunk == 0 || it == ntile - 1)
+#pragma unroll
+            for (int j = 0; j < 16; j++) W[j] = pinned(Wnext[j]);
+        if (it && t0 % g.chunk == 0) rnn_state_rows(Wnext, g, seq, t0 / g.chunk - 1, lane);
+        const float *const u_at = M.u[slot] + pair, *const k_at = M.k[slot] + half, *const s_at = M.s[slot] + pair, *const go_at = M.go[it & 1] + pair;
+        float *const hand = M.g[it % 3] + pair;
+        rnn_steps_back<Ops>(
+            nst, [&](Ops &o, int tt) { o.u = u_at[tt * D], o.k = k_at[tt * D], o.s = s_at[tt * D], o.go = go_at[tt * D]; },
+            [&](const Ops &o, int tt) __attribute__((always_inline)) {
+                const float h = dh + o.go;                    // the gradient of h_t = grad_z
+                hand[tt * D] = h;
+                // the gradient of s_t = W_t g, through the softmax to h_{t-1}
+                const float ds = half_shares_to_pair(dot(W, ready(h)));
+                rank1<true>(W, o.u, o.k);                     // W_{t-1}
+                dh = o.s * (ds - sum_of_pair(ds * o.s));
+            });
+    });
+}
+
+__device__ __forceinline__ void rnn_bwd_a(RnnBwdLds &M, const RnnBwdArgs &g, int64_t seq, int lane) {
+    using namespace forms;
+    constexpr int D = 32, TL = kRnnTile;
+    const int half = forms::half(lane), pair = forms::pair(lane), L = g.L, ntile = (L + TL - 1) / TL;
+    float G[16];      // by columns
+#pragma unroll
+    for (int j = 0; j < 16; j++) G[j] = 0.f;
+    struct Ops {
+        float s, k, g, d, b;
+    };
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    lds_barrier();
+    rnn_rounds<1>(ntile, [&](int it) {
+        const int slot = it & 3;
+        const float *const s_at = M.s[slot] + pair, *const k_at = M.k[slot] + pair, *const g_at = M.g[it % 3] + half, *const d_at = M.d[slot] + half,
+                    *const b_at = M.b[slot] + zero;
+        float *const hand = (lane < 32 ? M.a[it & 1] : M.pd[it & 1]) + half;
+        rnn_steps_back<Ops>(
+            min(TL, L - it * TL),
+            [&](Ops &o, int tt) { o.s = s_at[tt * D], o.k = k_at[tt * D], o.g = g_at[tt * D], o.d = d_at[tt * D], o.b = b_at[tt]; },
+            [&](const Ops &o, int tt) __attribute__((always_inline)) {
+                rank1(G, o.s, o.g);                           // G' = G + s (x) g
+                const float r = sum_to_half(dot(G, o.k));     // G'^T k
+                const float a = -(o.b * r);                   // the gradient of v_old; grad_v = -a
+                rank1(G, o.k, a);
+                const float o_a = pinned(a), o_p = pinned(r * o.d);
+                hand[tt * D] = lane < 32 ? o_a : o_p;
+            });
+    });
+}
+
+__device__ __forceinline__ void rnn_bwd_d(RnnBwdLds &M, const RnnBwdArgs &g, int64_t seq, int lane) {
+    using namespace forms;
+    constexpr int D = 32, TL = kRnnTile;
+    const int half = forms::half(lane), pair = forms::pair(lane), L = g.L, ntile = (L + TL - 1) / TL;
+    float G[16];      // by rows
+#pragma unroll
+    for (int j = 0; j < 16; j++) G[j] = 0.f;
+    struct Ops {
+        float g, a, u, s, k;
+    };
+    lds_barrier();
+    rnn_rounds<2>(ntile, [&](int it) {
+        const int slot = it & 3;
+        const float *const g_at = M.g[it % 3] + pair, *const a_at = M.a[it & 1] + pair, *const u_at = M.u[slot] + pair, *const s_at = M.s[slot] + half,
+                    *const k_at = M.k[slot] + half;
+        float *const hand = M.gu[it & 1] + half;
+        rnn_steps_back<Ops>(
+            min(TL, L - it * TL),
+            [&](Ops &o, int tt) { o.g = g_at[tt * D], o.a = a_at[tt * D], o.u = u_at[tt * D], o.s = s_at[tt * D], o.k = k_at[tt * D]; },
+            [&](const Ops &o, int tt) __attribute__((always_inline)) {
+                rank1(G, o.g, o.s);
+                hand[tt * D] = sum_to_half(dot(G, o.u));
+                rank1(G, o.a, o.k);
+            });
+    });
+}
+
+__device__ __forceinline__ void rnn_bwd_e(RnnBwdLds &M, const RnnBwdArgs &g, int64_t seq, int lane) {
+    using namespace forms;
+    constexpr int D = 32, TL = kRnnTile;
+    const int half = forms::half(lane), pair = forms::pair(lane), L = g.L, ntile = (L + TL - 1) / TL;
+    const int n = (int)(seq / g.H), hd = (int)(seq % g.H), row8 = lane / 8, c4 = lane % 8 * 4;
+    const float *k = row(g.k, n, hd, 0), *go = row(g.go, n, hd, 0), *b = row(g.beta, n, hd, 0);
+    const int64_t first = seq * L * D;
+    rnn_v4f pk[kRnnRows], pg[kRnnRows], pd[kRnnRows], ph[kRnnRows];
+    float pb[kRnnRows];
+    const auto fetch = [&](int it) {
+#pragma unroll
+        for (int i = 0; i < kRnnRows; i++) {
+            const int64_t t = min(it * TL + row8 + 8 * i, L - 1);      // rows beyond L are no step's
+            pk[i] = *reinterpret_cast<const rnn_v4f *>(k + t * g.k.sL + c4);
+            pg[i] = *reinterpret_cast<const rnn_v4f *>(go + t * g.go.sL + c4);
+            pd[i] = *reinterpret_cast<const rnn_v4f *>(g.vdiff + first + t * D + c4);
+            // row t of the delayed output is out[t-1], or the initial state for t = 0
+            ph[i] = *reinterpret_cast<const rnn_v4f *>(t ? g.out + first + (t - 1) * D + c4 : g.h_init + seq * D + c4);
+            pb[i] = b[t * g.beta.sL];
+        }
+    };
+    const auto commit = [&](int it) {
+        const int slot = it & 3;
+#pragma unroll
+        for (int i = 0; i < kRnnRows; i++) {
+            const rnn_v4f h = ph[i];
+            const float m = row_reduce<D>(OpMax()(OpMax()(h[0], h[1]), OpMax()(h[2], h[3])), OpMax());
+            rnn_v4f e = {__expf(h[0] - m), __expf(h[1] - m), __expf(h[2] - m), __expf(h[3] - m)};
+            e *= fast_div(1.f, row_reduce<D>((e[0] + e[1]) + (e[2] + e[3]), OpSum()));
+            const int at = 256 * i + 4 * lane;
+            *reinterpret_cast<rnn_v4f *>(M.k[slot] + at) = pk[i];
+            *reinterpret_cast<rnn_v4f *>(M.go[it & 1] + at) = pg[i];
+            *reinterpret_cast<rnn_v4f *>(M.d[slot] + at) = pd[i];
+            *reinterpret_cast<rnn_v4f *>(M.u[slot] + at) = pb[i] * pd[i];
+            *reinterpret_cast<rnn_v4f *>(M.s[slot] + at) = e;
+            if (c4 == 0) M.b[slot][row8 + 8 * i] = pb[i];
+        }
+    };
+    const auto stored = [&](const float *from, int i) { return *reinterpret_cast<const rnn_v4f *>(from + 256 * i + 4 * lane); };
+    // what the others left of their last tiles: X of tile it, A of it + 1, D and E of it + 2
+    const auto store = [&](int it) {
+#pragma unroll
+        for (int i = 0; i < kRnnRows; i++) {
+            const int r = row8 + 8 * i;
+            const auto put = [&](int t, float *to, const rnn_v4f &x) {
+                if (t * TL + r < L) *reinterpret_cast<rnn_v4f *>(to + first + (int64_t)(t * TL + r) * D + c4) = x;
+            };
+            if (it >= 0 && it < ntile) put(it, g.gz, stored(M.g[it % 3], i));
+            if (it + 1 >= 0 && it + 1 < ntile) {
+                const int t = it + 1;
+                put(t, g.gv, -stored(M.a[t & 1], i));
+                const rnn_v4f x = stored(M.pd[t & 1], i);
+                const float sum = row_reduce<D>((x[0] + x[1]) + (x[2] + x[3]), OpSum());
+                if (c4 == 0 && t * TL + r < L) g.gbeta[seq * L + t * TL + r] = sum;
+            }
+            if (it + 2 >= 0 && it + 2 < ntile) put(it + 2, g.gk, stored(M.gu[it & 1], i) + stored(M.wa[it & 1], i));
+        }
+    };
+    float W[16], Wnext[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) W[j] = 0.f;
+    rnn_state_rows(Wnext, g, seq, g.nchunk - 1, lane);
+    fetch(ntile - 1);
+    commit(ntile - 1);
+    if (ntile > 1) fetch(ntile - 2);
+    lds_barrier();
+    struct Ops {
+        float u, k, a;
+    };
+#pragma unroll 1
+    for (int j = 0; j < ntile + 2; j++) {
+        const int x = ntile - 1 - j, it = x + 2;      // X's tile, this wave's
+        if (x > 0) commit(x - 1);
+        if (x > 1) fetch(x - 2);
+        store(x + 1);
+        if (it < ntile) {
+            const int t0 = it * TL, nst = min(TL, L - t0), slot = it & 3;
+            if ((t0 + nst) % g.chunk == 0 || it == ntile - 1)
+#pragma unroll
+                for (int i = 0; i < 16; i++) W[i] = pinned(Wnext[i]);
+            if (it && t0 % g.chunk == 0) rnn_state_rows(Wnext, g, seq, t0 / g.chunk - 1, lane);
+            const float *const u_at = M.u[slot] + pair, *const k_at = M.k[slot] + half, *const a_at = M.a[it & 1] + pair;
+            float *const hand = M.wa[it & 1] + half;
+            rnn_steps_back<Ops>(
+                nst, [&](Ops &o, int tt) { o.u = u_at[tt * D], o.k = k_at[tt * D], o.a = a_at[tt * D]; },
+                [&](const Ops &o, int tt) __attribute__((always_inline)) {
+                    rank1<true>(W, o.u, o.k);                 // W_{t-1}
+                    hand[tt * D] = sum_to_half(dot(W, o.a));
+                });
+        }
+        lds_barrier();
+    }
+    store(-2);
+}
+
+template <int NS>
+__global__ __launch_bounds__(kWave * 4 * NS) void k_rnn_bwd_quad(RnnBwdArgs g) {
+    extern __shared__ __align__(16) unsigned char quad_lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave, role = wave / NS;
+    const int64_t seq = (int64_t)blockIdx.x * NS + wave % NS;
+    RnnBwdLds &M = reinterpret_cast<RnnBwdLds *>(quad_lds)[wave % NS];
+    if (seq >= g.nseq) {      // spare waves only keep the barriers' count
+        for (int j = (g.L + kRnnTile - 1) / kRnnTile + 3; j; j--) lds_barrier();
+        return;
+    }
+    if (role == 0) rnn_bwd_x(M, g, seq, lane);
+    else if (role == 1) rnn_bwd_a(M, g, seq, lane);
+    else if (role == 2) rnn_bwd_d(M, g, seq, lane);
+    else rnn_bwd_e(M, g, seq, lane);
+}
+
 }  // namespace
 
 // up to this many sequences the forward pass puts two waves on each (D = 32 over 256 steps, two waves
 // against one: 512 sequences 67 against 74 us, 768: 91 against 105 us, 1024: 93 against 107 us)
 constexpr int kFwdPairMaxSeq = 1024;
 
-// Up to this many sequences (one workgroup of two sequences on each CU) the backward pass puts three
-// waves on each, beyond it two, four sequences to a workgroup (D = 32 over 256 steps, 512 sequences:
-// one wave 131 us, two 98 us, three 79 us; 768: one 130, two 115 us; 1024: one 143, two 123 us;
-// 2048: one 270, two 239 us).
-constexpr int kTriMaxSeq = 512;
+// Up to this many sequences the backward pass puts four waves on each (16 x 16: three), one sequence to a workgroup while that is
+// one for each CU, then two, and beyond it two waves, four sequences to a workgroup (32 x 32 over 256 steps, 512 sequences:
+// one wave 131 us, two 98, three 79, four 71; 768: one 130, two 113, four 117; 1024: one 143, two 117, four 132;
+// 2048: one 270, two 240, four 264).
+constexpr int kQuadMaxSeq = 512;
 bool reg_rnn_supported(int D) { return D == 16 || D == 32; }
 
 int reg_rnn_fwd(fwp_view z, fwp_view k, fwp_view v, fwp_view beta, float *W, float *h, float *out,
@@ -1059,6 +1325,18 @@ int reg_rnn_bwd(fwp_view k, fwp_view beta, const float *vdiff, const float *out,
                 const float *h_init, fwp_view go, const float *ckpt, float *gz, float *gk,
                 float *gv, float *gbeta, int N, int H, int L, int D, int chunk, hipStream_t s) {
     const int nchunk = (L + chunk - 1) / chunk, nseq = N * H;
+    if (D == 32 && nseq <= kQuadMaxSeq) {
+        const RnnBwdArgs g{k, beta, go, vdiff, out, h_init, ckpt, gz, gk, gv, gbeta, H, L, chunk, nchunk, nseq};
+        const auto run = [&](auto ns) {
+            constexpr int NS = decltype(ns)::value;
+            if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_rnn_bwd_quad<NS>),
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NS * sizeof(RnnBwdLds))))
+                return (int)e;
+            hipLaunchKernelGGL(k_rnn_bwd_quad<NS>, dim3((nseq + NS - 1) / NS), dim3(4 * NS * kWave), NS * sizeof(RnnBwdLds), s, g);
+            return (int)hipGetLastError();
+        };
+        return nseq <= 256 ? run(std::integral_constant<int, 1>()) : run(std::integral_constant<int, 2>());
+    }
     auto launch_on = [&](auto kernel, int waves, size_t lds, int ns = 2) {
         if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
@@ -1067,9 +1345,7 @@ int reg_rnn_bwd(fwp_view k, fwp_view beta, const float *vdiff, const float *out,
                            go, ckpt, gz, gk, gv, gbeta, H, L, chunk, nchunk, nseq);
         return (int)hipGetLastError();
     };
-    if (nseq <= kTriMaxSeq)
-        return D == 16 ? launch_on(k_rnn_bwd_tri<16>, 6, 2 * sizeof(RnnTriLds<16>))
-                       : launch_on(k_rnn_bwd_tri<32>, 6, 2 * sizeof(RnnTriLds<32>));
+    if (nseq <= kQuadMaxSeq) return launch_on(k_rnn_bwd_tri<16>, 6, 2 * sizeof(RnnTriLds<16>));
     return D == 16 ? launch_on(k_rnn_bwd_pair<16, 4>, 8, 4 * sizeof(RnnPairLds<16>), 4)
                    : launch_on(k_rnn_bwd_pair<32, 4>, 8, 4 * sizeof(RnnPairLds<32>), 4);
 }

@@ -8,7 +8,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 import oracle
-from helpers import rec_inputs
+from helpers import rec_inputs, rnn_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -53,6 +53,21 @@ def test_rec_tiles_and_workgroups(fwp, N, H, L):
         check(name, a, b, L)
     grads = oracle.rec_bwd(*x64, np.asarray(go, np.float32).astype(np.float64))
     for name, t, g in zip("qx kx vx bx R_q R_k R_v r_b".split(), ts, grads):
+        check("grad " + name, t.grad, g, L)
+
+
+@pytest.mark.parametrize("N,H,L", [(1, 3, L) for L in LENGTHS] + [(64, 4, 18), (85, 3, 33), (257, 1, 20), (171, 3, 17)])
+def test_rnn_tiles_and_workgroups(fwp, N, H, L):
+    """256, 255, 257 and 513 sequences: one and two sequences to a workgroup, a spare place in the last one, fewer waves to a sequence."""
+    z, k, v, W0, beta, h0, go = (np.asarray(a, np.float32) for a in rnn_inputs(L + N, N, H, L, 32, w0=True))
+    ts = [dev(a, True) for a in (z, k, v, beta)]
+    W, h = dev(W0), dev(h0)
+    out = fwp.fast_rnn_v2(ts[0], ts[1], ts[2], W, ts[3], h)
+    out.backward(dev(go))
+    x64 = [a.astype(np.float64) for a in (z, k, v, W0, beta, h0)]
+    for name, a, b in zip(("out", "W", "h"), (out, W, h), oracle.rnn_fwd(*x64)):
+        check(name, a, b, L)
+    for name, t, g in zip("z k v beta".split(), ts, oracle.rnn_bwd(*x64, go.astype(np.float64))):
         check("grad " + name, t.grad, g, L)
 
 
