@@ -1,55 +1,76 @@
 // LayerNorm of the language model's layers and its adjoint (reference: language_modeling/src/utils/
 // model_utils.py:52-66, cuda_fast_weight_layer.py:168-176).
 //
-// One wave per row, a float4 of the row per lane and 256 columns (up to four of them): a row is read once, its mean
-// and its variance (of the differences from the mean, as exact as two passes over memory) are butterflies
-// inside the wave.  The adjoint forms the gradient of x in the same one pass and keeps the column sums for gamma and
-// beta in registers over the rows a wave takes; the workgroups' sums are added up by a second, small kernel in
-// a fixed order.  Bound by HBM: 2 (forward) and 3 (adjoint) passes over rows x cols floats.
+// A lane holds four columns of every 64 (rows of up to 256 columns: 16 lanes to a row, four rows to a wave) or of every 256 (up to
+// 1024 columns: the wave's 64 lanes): a row is read once, its mean and its variance (of the differences from the mean, as exact as
+// two passes over memory) are DPP moves and, over a whole wave, row exchanges.  The adjoint forms the gradient of x in the same
+// one pass and keeps the column sums for gamma and beta in registers over the rows a lane takes; the workgroups' sums are added
+// up by a second, small kernel in a fixed order.
+//
+// Bound by HBM: 2 (forward) and 3 (adjoint) passes over rows x cols floats, 5.9 and 5.5 TB/s at 32768 x 256.  Four rows to a wave have
+// four times the bytes in flight, and a sum is four moves instead of six shuffles one after the other through the LDS's crossbar; one
+// wave per row took 13.3 us forward and 26.0 us backward there against 11.3 and 21.9 now, 8.9 and 19.2 against 6.0 and 11.9 at 24576 x
+// 128, as much up to 2400 rows, where a pass is as long as its launches.  For the adjoint, 1024 workgroups instead of 512 took 2 us more, 256 of eight waves
+// 0.2 us less there and 1.4 us more at 2384 rows; loads a turn ahead nothing.
 #include "fwp_common.hpp"
+#include "fwp_wave.hpp"
 
 namespace fwp {
 namespace {
 
 constexpr int kWaves = 4, kBlocks = 512;
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
-    return x;
+// The sum over the four 16-lane rows of the wave, in all of them
+__device__ __forceinline__ float rows_sum(float x) {
+    float y = x;
+    swap16(x, y);
+    x += y, y = x;
+    swap32(x, y);
+    return x + y;
+}
+
+// The sum over the L lanes of a row, in all of them
+template <int L>
+__device__ __forceinline__ float row_sum(float x) {
+    x += dpp<kQuadXor1>(x);
+    x += dpp<kQuadXor2>(x);
+    x += dpp<0x141>(x);             // row_half_mirror
+    x += dpp<0x140>(x);             // row_mirror
+    return L == 64 ? rows_sum(x) : x;
 }
 
 __device__ __forceinline__ float4 load4(const float *p, bool ok) {
     return ok ? *reinterpret_cast<const float4 *>(p) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-template <int V>
+template <int L, int V>
 __global__ __launch_bounds__(64 * kWaves) void k_norm_fwd(const float *__restrict__ x, const float *__restrict__ gamma,
                                                           const float *__restrict__ beta, float *__restrict__ y,
                                                           float *__restrict__ stats, int rows, int cols, float eps) {
-    const int lane = threadIdx.x % 64, row = blockIdx.x * kWaves + threadIdx.x / 64;
-    if (row >= rows) return;
+    const int lane = threadIdx.x % L, row = blockIdx.x * (64 * kWaves / L) + threadIdx.x / L;
+    if (row >= rows) return;        // all lanes of a row together
     const float *src = x + (int64_t)row * cols;
     float4 v[V];
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const int c = 4 * (lane + 64 * i);
+        const int c = 4 * (lane + L * i);
         v[i] = load4(src + c, c < cols);
-        s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
-    const float mean = wave_sum(s) / cols;
+#pragma unroll
+    for (int i = 0; i < V; i++) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    const float mean = row_sum<L>(s) / cols;
     s = 0.f;
 #pragma unroll
     for (int i = 0; i < V; i++)
-        if (4 * (lane + 64 * i) < cols) {
+        if (4 * (lane + L * i) < cols) {
             const float a = v[i].x - mean, b = v[i].y - mean, c = v[i].z - mean, d = v[i].w - mean;
             s += (a * a + b * b) + (c * c + d * d);
         }
-    const float rstd = 1.f / sqrtf(wave_sum(s) / cols + eps);
+    const float rstd = 1.f / sqrtf(row_sum<L>(s) / cols + eps);
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const int c = 4 * (lane + 64 * i);
+        const int c = 4 * (lane + L * i);
         if (c >= cols) continue;
         const float4 g = load4(gamma + c, true), b = load4(beta + c, true);
         float4 o;
@@ -61,28 +82,33 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_fwd(const float *__restric
 }
 
 // gx = rstd (g - mean(g) - xh mean(g xh)),  g = gy gamma, xh = (x - mean) rstd
-template <int V>
+template <int L, int V>
 __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restrict__ gy, const float *__restrict__ x,
                                                           const float *__restrict__ stats, const float *__restrict__ gamma,
                                                           float *__restrict__ gx,
                                                           float *__restrict__ part, int rows, int cols) {
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    constexpr int R = 64 * kWaves / L;      // rows of a workgroup at once
+    const int lane = threadIdx.x % L, wave = threadIdx.x / 64;
     float4 gam[V], sg[V], sb[V];
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const int c = 4 * (lane + 64 * i);
+        const int c = 4 * (lane + L * i);
         gam[i] = load4(gamma + c, c < cols);
         sg[i] = sb[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    for (int row = blockIdx.x * kWaves + wave; row < rows; row += gridDim.x * kWaves) {
-        const int64_t at = (int64_t)row * cols;
-        const float2 st = *reinterpret_cast<const float2 *>(stats + 2 * (int64_t)row);
+    for (int64_t row = (int64_t)blockIdx.x * R + threadIdx.x / L; row < rows; row += (int64_t)gridDim.x * R) {
+        const int64_t at = row * cols;
+        const float2 st = *reinterpret_cast<const float2 *>(stats + 2 * row);
         float4 g[V], xh[V];
         float s = 0.f, t = 0.f;
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const int c = 4 * (lane + 64 * i);
-            const float4 d = load4(gy + at + c, c < cols), w = load4(x + at + c, c < cols);
+            const int c = 4 * (lane + L * i);
+            g[i] = load4(gy + at + c, c < cols), xh[i] = load4(x + at + c, c < cols);
+        }
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const float4 d = g[i], w = xh[i];
             xh[i] = make_float4((w.x - st.x) * st.y, (w.y - st.x) * st.y, (w.z - st.x) * st.y, (w.w - st.x) * st.y);
             sb[i].x += d.x, sb[i].y += d.y, sb[i].z += d.z, sb[i].w += d.w;
             sg[i].x += d.x * xh[i].x, sg[i].y += d.y * xh[i].y, sg[i].z += d.z * xh[i].z, sg[i].w += d.w * xh[i].w;
@@ -90,11 +116,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restric
             s += (g[i].x + g[i].y) + (g[i].z + g[i].w);
             t += (g[i].x * xh[i].x + g[i].y * xh[i].y) + (g[i].z * xh[i].z + g[i].w * xh[i].w);
         }
-        s = wave_sum(s) / cols;
-        t = wave_sum(t) / cols;
+        s = row_sum<L>(s) / cols;
+        t = row_sum<L>(t) / cols;
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const int c = 4 * (lane + 64 * i);
+            const int c = 4 * (lane + L * i);
             if (c >= cols) continue;
             float4 o = make_float4(st.y * (g[i].x - s - xh[i].x * t), st.y * (g[i].y - s - xh[i].y * t),
                                    st.y * (g[i].z - s - xh[i].z * t), st.y * (g[i].w - s - xh[i].w * t));
@@ -102,65 +128,85 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restric
         }
     }
     // this workgroup's column sums: [gamma | beta][cols]
-    __shared__ float4 sh[kWaves][64];
+    __shared__ float4 sh[kWaves][L];
 #pragma unroll
     for (int i = 0; i < V; i++)
+#pragma unroll
         for (int w = 0; w < 2; w++) {
+            float4 o = w ? sb[i] : sg[i];
+            if constexpr (L == 16) o = make_float4(rows_sum(o.x), rows_sum(o.y), rows_sum(o.z), rows_sum(o.w));
             __syncthreads();
-            sh[wave][lane] = w ? sb[i] : sg[i];
+            if (threadIdx.x % 64 < L) sh[wave][lane] = o;
             __syncthreads();
-            const int c = 4 * (lane + 64 * i);
-            if (wave || c >= cols) continue;
-            float4 o = sh[0][lane];
+            const int c = 4 * (lane + L * i);
+            if (threadIdx.x >= L || c >= cols) continue;
+            o = sh[0][lane];
 #pragma unroll
             for (int k = 1; k < kWaves; k++) o.x += sh[k][lane].x, o.y += sh[k][lane].y, o.z += sh[k][lane].z, o.w += sh[k][lane].w;
             *reinterpret_cast<float4 *>(part + ((int64_t)blockIdx.x * 2 + w) * cols + c) = o;
         }
 }
 
-// ggamma, gbeta = the workgroups' sums added up: 16 columns x 16 slices of the workgroups per workgroup
-__global__ __launch_bounds__(256) void k_norm_params(const float *__restrict__ part, float *__restrict__ ggamma,
-                                                     float *__restrict__ gbeta, int blocks, int cols) {
-    __shared__ float sh[16][17];
+// ggamma, gbeta = the workgroups' sums added up: 16 columns x 64 slices of the workgroups per workgroup (16 slices: 0.8 us more at 512)
+__global__ __launch_bounds__(1024) void k_norm_params(const float *__restrict__ part, float *__restrict__ ggamma,
+                                                      float *__restrict__ gbeta, int blocks, int cols) {
+    __shared__ float sh[16][16];
     const int c = threadIdx.x % 16, q = threadIdx.x / 16, col = blockIdx.x * 16 + c;
     float s = 0.f;
     if (col < 2 * cols) {
 #pragma unroll 8
-        for (int b = q; b < blocks; b += 16) s += part[(int64_t)b * 2 * cols + col];
+        for (int b = q; b < blocks; b += 64) s += part[(int64_t)b * 2 * cols + col];
     }
-    sh[q][c] = s;
+    s = rows_sum(s);
+    if (q % 4 == 0) sh[q / 4][c] = s;
     __syncthreads();
     if (q || col >= 2 * cols) return;
+    s = sh[0][c];
+#pragma unroll
     for (int k = 1; k < 16; k++) s += sh[k][c];
     (col < cols ? ggamma : gbeta)[col < cols ? col : col - cols] = s;
 }
 
-int blocks_of(int rows) { return rows < kBlocks * kWaves ? (rows + kWaves - 1) / kWaves : kBlocks; }
+// Lanes to a row
+int lanes_of(int cols) { return cols <= 256 ? 16 : 64; }
+
+int blocks_of(int rows, int cols) {
+    const int at_once = 64 * kWaves / lanes_of(cols);
+    return (int)std::min<int64_t>(((int64_t)rows + at_once - 1) / at_once, kBlocks);
+}
 
 }  // namespace
 
 bool layer_norm_supported(int cols) { return cols >= 4 && cols <= 1024 && cols % 4 == 0; }
-int64_t layer_norm_workspace(int rows, int cols) { return (int64_t)blocks_of(rows) * 2 * cols; }
+int64_t layer_norm_workspace(int rows, int cols) { return (int64_t)blocks_of(rows, cols) * 2 * cols; }
+
+#define FWP_BY_COLS(LAUNCH)                                                                                                  \
+    if (cols <= 64) LAUNCH(16, 1);                                                                                           \
+    else if (cols <= 128) LAUNCH(16, 2);                                                                                     \
+    else if (cols <= 256) LAUNCH(16, 4);                                                                                     \
+    else if (cols <= 512) LAUNCH(64, 2);                                                                                     \
+    else LAUNCH(64, 4)
 
 int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows, int cols,
                    float eps, hipStream_t s) {
-    const dim3 grid((rows + kWaves - 1) / kWaves), block(64 * kWaves);
-    const int v = (cols + 255) / 256;
-    if (v == 1) hipLaunchKernelGGL(k_norm_fwd<1>, grid, block, 0, s, x, gamma, beta, y, stats, rows, cols, eps);
-    else if (v == 2) hipLaunchKernelGGL(k_norm_fwd<2>, grid, block, 0, s, x, gamma, beta, y, stats, rows, cols, eps);
-    else hipLaunchKernelGGL(k_norm_fwd<4>, grid, block, 0, s, x, gamma, beta, y, stats, rows, cols, eps);
+    const int at_once = 64 * kWaves / lanes_of(cols);
+    const dim3 grid((rows + at_once - 1) / at_once), block(64 * kWaves);
+#define FWP_FWD(L, V) hipLaunchKernelGGL((k_norm_fwd<L, V>), grid, block, 0, s, x, gamma, beta, y, stats, rows, cols, eps)
+    FWP_BY_COLS(FWP_FWD);
+#undef FWP_FWD
     return (int)hipGetLastError();
 }
 
 int layer_norm_bwd(const float *gy, const float *x, const float *stats, const float *gamma, float *gx,
                    float *ggamma, float *gbeta, float *workspace, int rows, int cols, hipStream_t s) {
-    const int blocks = blocks_of(rows), v = (cols + 255) / 256;
+    const int blocks = blocks_of(rows, cols);
     const dim3 grid(blocks), block(64 * kWaves);
-    if (v == 1) hipLaunchKernelGGL(k_norm_bwd<1>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
-    else if (v == 2) hipLaunchKernelGGL(k_norm_bwd<2>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
-    else hipLaunchKernelGGL(k_norm_bwd<4>, grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols);
-    hipLaunchKernelGGL(k_norm_params, dim3((2 * cols + 15) / 16), dim3(256), 0, s, workspace, ggamma, gbeta, blocks, cols);
+#define FWP_BWD(L, V) hipLaunchKernelGGL((k_norm_bwd<L, V>), grid, block, 0, s, gy, x, stats, gamma, gx, workspace, rows, cols)
+    FWP_BY_COLS(FWP_BWD);
+#undef FWP_BWD
+    hipLaunchKernelGGL(k_norm_params, dim3((2 * cols + 15) / 16), dim3(1024), 0, s, workspace, ggamma, gbeta, blocks, cols);
     return (int)hipGetLastError();
 }
+#undef FWP_BY_COLS
 
 }  // namespace fwp

@@ -38,3 +38,25 @@ def test_rows(layers, T, B, H, D):
     for a, b in list(zip(got, want)) + [(dx, dref)]:
         assert a.shape == b.shape
         assert float((a.double().cpu() - b).norm()) <= 2 ** -20 * float(b.norm())
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 60), (17, 64), (16, 68), (15, 128), (33, 132), (8193, 256), (8, 260), (8191, 64)])
+def test_norm_rows(layers, rows, cols):
+    """LayerNorm where a workgroup's 16 rows of up to 256 columns, a row's last lanes and the workgroups' second turn are cut."""
+    L = importlib.import_module("recurrent-fwp_amd._lib")
+    torch.manual_seed(rows + cols)
+    x, gy = torch.randn(2, rows, cols, device="cuda")
+    g, b = torch.randn(2, cols, device="cuda")
+    ref = [z.double().cpu().requires_grad_() for z in (x, g, b)]
+    want = torch.nn.functional.layer_norm(ref[0], (cols,), ref[1], ref[2], 1e-5)
+    refs = torch.autograd.grad(want, ref, gy.double().cpu())
+    y, gx, stats, gg, gb = torch.empty_like(x), torch.empty_like(x), torch.empty(rows, 2, device="cuda"), torch.empty_like(g), torch.empty_like(b)
+    s = torch.cuda.current_stream().cuda_stream
+    L.check(L.lib().fwp_layer_norm_fwd(x.data_ptr(), g.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr(), rows, cols, 1e-5, s), "fwd")
+    work = torch.empty(L.lib().fwp_layer_norm_workspace(rows, cols), device="cuda")
+    L.check(L.lib().fwp_layer_norm_bwd(gy.data_ptr(), x.data_ptr(), stats.data_ptr(), g.data_ptr(), gx.data_ptr(), gg.data_ptr(), gb.data_ptr(),
+                                       work.data_ptr(), rows, cols, s), "bwd")
+    # about eight roundings an entry (sums of up to 64 lane shares among them): 2^-20 of the result; the column sums add up to rows / 8192
+    # rounded terms a lane and 64 shares one after the other: well below 2^-18
+    for got, ref, bound in ((y, want, 2 ** -20), (gx, refs[0], 2 ** -20), (gg, refs[1], 2 ** -18), (gb, refs[2], 2 ** -18)):
+        assert float((got.double().cpu() - ref).norm()) <= bound * float(ref.norm())
