@@ -319,7 +319,7 @@ int fwp_nll_fwd(const float *x, const float *W, const float *bias, const int64_t
                 float *loss, float *lse, float *workspace, int rows, int vocab, int dim, void *stream);
 
 /* Its adjoint: gloss [rows] to gx [rows,dim], gW [vocab,dim], gbias [vocab] (each may be NULL; gbias comes with gW).
- * workspace: the larger of fwp_matmul_workspace(rows, dim, vocab) and fwp_matmul_workspace(vocab, dim, rows). */
+ * workspace: the larger of fwp_matmul_workspace(rows, dim, vocab) and fwp_matmul_workspace(vocab, dim, rows), or NULL (slower). */
 int fwp_nll_bwd(const float *x, const float *W, const float *logits, const float *lse, const int64_t *target,
                 const float *gloss, float *gx, float *gW, float *gbias, float *workspace, int rows,
                 int vocab, int dim, void *stream);

@@ -523,6 +523,7 @@ struct GemmArgs {
     NllArgs nll;
     // per tile of columns and row: the largest logit and the sum of exp(logit - largest); logits of the targets
     float *part_max, *part_sum, *hit;
+    v4u *image;                  // B split, as k_image leaves it, or NULL
 };
 
 enum { kPlain = 0, kLse = 1, kGrad = 2 };
@@ -758,13 +759,34 @@ __device__ __forceinline__ void add_small(v4f (&acc)[MT][NT], const float (&x)[M
     }
 }
 
+// B split into Bf16x3's numbers: [tile of BN columns][step of k] the step's place in LDS as it is, zeros beyond K.  A workgroup a step.
+template <int BN>
+__global__ __launch_bounds__(2 * BN) void k_image(const float *__restrict__ B, int64_t ldb, int N, int K, v4u *__restrict__ image) {
+    typedef Planes<Bf16x3::kPlanes, BN> Stage;
+    const int k0 = blockIdx.x * kBK, n0 = blockIdx.y * BN;
+    Staged<false, BN, BN / 32> b;
+    typename Staged<false, BN, BN / 32>::Raw x;
+    b.init(threadIdx.x);
+    b.aim(ldb, k0, K);
+    b.load(x, B + n0, ldb, N - n0, k0, K);
+    Stage &to = reinterpret_cast<Stage *>(image)[(int64_t)blockIdx.y * gridDim.x + blockIdx.x];
+#pragma unroll
+    for (int t = 0; t < b.kUnits; t++) {
+        v4u part[Bf16x3::kPlanes];
+#pragma unroll
+        for (int j = 0; j < 4; j++) split_pair<Bf16x3>(x.x[t], j, 1.f, part);
+        b.store(to, t, part);
+    }
+}
+
 // A workgroup of WAVES waves: a wave 16 MT rows and all 16 NT columns; B's rows are staged step by step, in two
-// alternating places, one barrier a step.  What bounds it: 32768 x 256, K = 1024 takes 71 us (one 128 x 128 tile with both
+// alternating places, one barrier a step; IMAGE: they come split.  What bounds it: 32768 x 256, K = 1024 takes 71 us (one 128 x 128 tile with both
 // operands through LDS, Bf16x3: 89): products alone 36 us, the split 10 us, loads 8, LDS 6, the look for small elements 7.
-template <class S, bool AKC, bool BKC, int MT, int NT, int MODE, int WAVES = 4>
+template <class S, bool AKC, bool BKC, int MT, int NT, int MODE, int WAVES = 4, bool IMAGE = false>
 __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
     constexpr int WM = 16 * MT, BM = WAVES * WM, BN = 16 * NT;
     static_assert(WAVES == 4 || !S::kScaled, "four waves' changes of scales");
+    static_assert(!IMAGE || !S::kScaled, "an image of Bf16x3's numbers");
     typedef Direct<AKC, MT, MODE == kGrad> OpA;
     typedef Staged<BKC, BN, WAVES> OpB;
     // the two places of a step's B, and (scaled) behind them its elements in fp32 where some are small; later Bf16x3's places
@@ -821,6 +843,21 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
 #pragma unroll
     for (int t = 0; t < OpB::kUnits; t++) b.s[t].none();
 
+    // IMAGE: a thread's share of a step's B
+    constexpr int kStep = IMAGE ? Bf16x3::kPlanes * kBK / 8 * BN : 0, kShare = IMAGE ? kStep / (64 * WAVES) : 1;
+    v4u share[kShare];
+    const v4u *const image = IMAGE ? g.image + (int64_t)(n0 / BN) * ((g.K + kBK - 1) / kBK) * kStep : nullptr;
+    const auto ask = [&](int k0) {
+        if constexpr (IMAGE) {
+            const v4i rs = buffer_of(reinterpret_cast<const float *>(image + (int64_t)(k0 / kBK) * kStep), k0 < ke ? 4 * kStep : 0);
+#pragma unroll
+            for (int i = 0; i < kShare; i++) share[i] = __builtin_bit_cast(v4u, llvm_raw_buffer_load_v4f32(rs, 16 * tid, i * 1024 * WAVES, 0));
+        }
+    };
+    const auto put = [&](auto &to, int i) {
+        if constexpr (IMAGE) (&to.u[0][0][0])[i * 64 * WAVES + tid] = share[i];
+    };
+
     typename OpA::Raw ra[2];
     typename OpB::Raw rb[2];
     bool far = false;         // results that may not be what fp32 holds
@@ -845,14 +882,14 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
         };
         // Pair q of the 4 (units + MT) pairs of a step's split: B's units first, each to LDS when it is whole, then A's tiles
         v4u part[T::kPlanes];
-        constexpr int kPairs = 4 * (OpB::kUnits + MT);
+        constexpr int kUnits = IMAGE ? 0 : OpB::kUnits, kPairs = 4 * (kUnits + MT);
         const auto split = [&](int q, const typename OpA::Raw &x, const typename OpB::Raw &y, v4u (*f)[T::kPlanes], Stage &to, int k0) {
-            if (q < 4 * OpB::kUnits) {
+            if (q < 4 * kUnits) {
                 split_pair<T>(y.x[q / 4], q % 4, b.s[q / 4].s, part);
                 if (q % 4 == 3) b.store(to, q / 4, part);
                 return;
             }
-            const int j = (q - 4 * OpB::kUnits) / MT, i = q % MT;
+            const int j = (q - 4 * kUnits) / MT, i = q % MT;
             split_a(i, j, x, f, false, k0);
         };
         // once more where split() left something out
@@ -867,7 +904,10 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
         // What a step's split needs: zeros beyond K, and (parity: the step's) scales that its elements fit
         const auto prepare = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0, int parity) __attribute__((always_inline)) {
             a.hand_over(x, lane);
-            if (ke % 4 && k0 + kBK > ke) a.cut(x, k0, ke), b.cut(y, k0, ke);
+            if (ke % 4 && k0 + kBK > ke) {
+                a.cut(x, k0, ke);
+                if constexpr (!IMAGE) b.cut(y, k0, ke);
+            }
             if constexpr (T::kScaled) {
                 float ma[MT], mb[OpB::kUnits];
                 const bool beyond = fmaxf(largest_of(x.x, a.s, ma), largest_of(y.x, b.s, mb)) > kLargest;
@@ -935,10 +975,17 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
             }
             return false;
         };
+        const auto load = [&](typename OpA::Raw &x, typename OpB::Raw &y, int k0) {
+            a.load(x, Ap, g.lda, ml, k0, ke, g.nll, g.K, lane);
+            if constexpr (!IMAGE) b.load(y, Bp, g.ldb, nl, k0, ke);
+        };
+        ask(first);
         aim(first);
         load(ra[0], rb[0], first);
         aim(first + kBK);
         load(ra[1], rb[1], first + kBK);
+#pragma unroll
+        for (int i = 0; i < kShare; i++) put(L[0], i);
         prepare(ra[0], rb[0], first, 0);
 #pragma unroll
         for (int q = 0; q < kPairs; q++) split(q, ra[0], rb[0], fa[0], L[0], first);
@@ -950,6 +997,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
             if (follow(p, ra[p])) return false;
 #pragma unroll
             for (int i = 0; i < MT; i++) csum[i] += part_sum[i];
+            ask(k0 + kBK);
             if (k0 + 3 * kBK > ke) aim(k0 + 2 * kBK);
             load(ra[p], rb[p], k0 + 2 * kBK);
             prepare(ra[p ^ 1], rb[p ^ 1], k0 + kBK, p ^ 1);
@@ -966,6 +1014,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void k_gemm(GemmArgs g) {
                 if (j + 1 < NT) read(j + 1);
 #pragma unroll
                 for (int q = j * kPairs / NT; q < (j + 1) * kPairs / NT; q++) split(q, ra[p ^ 1], rb[p ^ 1], fa[p ^ 1], L[p ^ 1], k0 + kBK);
+                if constexpr (IMAGE)        // in the step's second half
+#pragma unroll
+                    for (int i = max(0, 2 * j - NT) * kShare / NT; i < max(0, 2 * j + 2 - NT) * kShare / NT; i++) put(L[p ^ 1], i);
 #pragma unroll
                 for (int q = 0; q < T::kProducts; q++)
 #pragma unroll
@@ -1602,7 +1653,7 @@ constexpr int kHalfK = 128;
 // The partial results of a range cost a pass over M x N each way, so a range is no shorter than 256 of k; all at once, 129.
 // The loss's gradients (`grad`): 128 x 256 tiles of eight waves, which form an element once for twice the columns, where those divide over the
 // chip as well as 128 x 128 ones, one of them to a CU or two of the others, the latter 1.12 times as long.  dX and dW, tokens = words = 32768: 256 columns
-// 3.09 and 3.36 ms (128-column tiles 3.45, 3.85), 288 (512 tiles, two turns) 5.85 and 6.61 (768 tiles, one and a half: 5.10, 5.94); 8192, in two
+// 3.09 and 3.36 ms (128-column tiles 3.45, 3.85; these and the next before kImage's), 288 (512 tiles, two turns) 5.85 and 6.61 (768 tiles, one and a half: 5.10, 5.94); 8192, in two
 // ranges: 288 columns 0.37 and 0.43 ms (0.38, 0.46); 640 (192 tiles) 0.69 and 0.83 (128 x 64 tiles 0.81, 1.05).
 Plan plan_of(int M, int N, int K, bool may_cut, bool grad) {
     Plan p{};
@@ -1656,7 +1707,16 @@ template <bool AKC, bool BKC, int MODE>
 void launch(GemmArgs g, const Plan &p, hipStream_t s) {
     g.ks = p.ks, g.tm = p.tm, g.tn = p.tn, g.ranges = p.ranges;
     if constexpr (MODE == kGrad) {
-        if (p.bn == 256)
+        if (g.image) {
+            const dim3 steps((unsigned)((g.K + kBK - 1) / kBK), (unsigned)g.tn), grid((unsigned)(g.tm * g.tn * g.ranges));
+            if (p.bn == 256) {
+                hipLaunchKernelGGL(k_image<256>, steps, dim3(512), 0, s, g.B, g.ldb, g.N, g.K, g.image);
+                hipLaunchKernelGGL((k_gemm<Bf16x3, AKC, BKC, 1, 16, MODE, 8, true>), grid, dim3(512), 0, s, g);
+            } else {
+                hipLaunchKernelGGL(k_image<128>, steps, dim3(256), 0, s, g.B, g.ldb, g.N, g.K, g.image);
+                hipLaunchKernelGGL((k_gemm<Bf16x3, AKC, BKC, 2, 8, MODE, 4, true>), grid, dim3(256), 0, s, g);
+            }
+        } else if (p.bn == 256)
             hipLaunchKernelGGL((k_gemm<Bf16x3, AKC, BKC, 1, 16, MODE, 8>), dim3((unsigned)(g.tm * g.tn * g.ranges)), dim3(512), 0, s, g);
         else
             launch_staged<Bf16x3, AKC, BKC, MODE>(g, p, s);
@@ -1687,11 +1747,25 @@ bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 // a partial result, in whole 16-byte groups
 int64_t part_of(int M, int N) { return ((int64_t)M * N + 3) / 4 * 4; }
 
+// The loss's gradients split their second operand (the weights, the tokens) once, for all rows of tiles, where these are many and k is long: each workgroup
+// did it again for its 128 rows, a third of its vector instructions, which bound them as much as the products do (each busy 45 % of the time).
+// Words = tokens = 32768, 256 columns: dX 2.98 -> 2.60 ms, dW 3.19 -> 3.06 ms; 32768 words, 24576 tokens, 128 columns 1.58 -> 1.32 and
+// 1.44 -> 1.25 ms; 4100 tokens, 5001 words, 256 columns 82 -> 75 and 84 -> 83 us; 3000 of both 45 -> 45 and 47 -> 50 us; 1024
+// tokens, 32768 words dX 107 -> 112 us; 32768 tokens, 1024 words dW 114 -> 128 us.  With k of 1024 dX would still gain (100 -> 94 us), but ordinary products of such
+// sizes would ask for the workspace too.
+constexpr int kImage = 4096;
+
+// floats of the partial results and, behind them, of B's image
+int64_t parts_of(const Plan &p, int M, int N) { return p.ranges > 1 ? (p.ranges * (part_of(M, N) + M) + 3) / 4 * 4 : 0; }
+int64_t image_of(const Plan &p, int M, int K) {
+    return p.bm == 128 && p.bn >= 128 && std::min(M, K) >= kImage ? (int64_t)p.tn * ((K + kBK - 1) / kBK) * (Bf16x3::kPlanes * kBK / 2) * p.bn : 0;
+}
+
 }  // namespace
 
 int64_t matmul_workspace(int M, int N, int K) {
-    const int ranges = std::max(plan_of(M, N, K, true, false).ranges, plan_of(M, N, K, true, true).ranges);      // of a product and of a loss's gradient
-    return ranges > 1 ? ranges * (part_of(M, N) + M) : 0;
+    const Plan product = plan_of(M, N, K, true, false), grad = plan_of(M, N, K, true, true);      // of a product and of a loss's gradient
+    return std::max(parts_of(product, M, N), parts_of(grad, M, N) + image_of(grad, M, K));
 }
 
 int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
@@ -1701,6 +1775,7 @@ int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb,
     if (nll) g.nll = NllArgs{nll->lse, nll->stats, nll->gloss, nll->target, nll->vocab};
     const Plan p = plan_of(M, N, K, workspace && ldc == N && aligned(C) && aligned(workspace), nll != nullptr);
     const bool cut = p.ranges > 1;
+    if (nll && workspace && aligned(workspace) && image_of(p, M, K)) g.image = reinterpret_cast<v4u *>(workspace + parts_of(p, M, N));
     g.C = cut ? workspace : C;
     g.ldc = cut ? N : ldc;
     g.part = part_of(M, N);

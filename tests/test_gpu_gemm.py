@@ -434,3 +434,33 @@ def test_layer_norm(fwp, rows, cols):
     for name, got, w in zip(("x", "gamma", "beta"), (gx, gg, gb), wants):
         scale = float(w.abs().max()) + float(gy.abs().max())
         assert float((got.double() - w).abs().max()) <= (rows / 8 + cols / 8 + 64) * EPS * scale * float(rms.max()), name
+
+
+# tiles of 256 columns and of 128 in one range of k, with a rest of k and of columns; an infinity in an operand
+@pytest.mark.parametrize("rows,vocab,dim", [(4100, 4133, 1408), (5501, 5500, 1406)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_gradients_from_an_operand_split_once(fwp, rows, vocab, dim, odd):
+    """With a workspace the loss's gradients read their second operand split beforehand, without one they split it: the same numbers."""
+    L = fwp._lib
+    x, W, b = randn(rows, dim, seed=1) * 0.1, randn(vocab, dim, seed=2) * 0.3, randn(vocab, seed=3)
+    target = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
+    gloss = randn(rows, seed=5)
+    logits, loss, stats = torch.empty(rows, vocab, device="cuda"), torch.empty(rows, device="cuda"), torch.empty(rows, 2, device="cuda")
+    work = torch.empty(L.lib().fwp_nll_workspace(rows, vocab), device="cuda")
+    s = L.stream_of(x)
+    assert L.lib().fwp_nll_stats_fwd(x.data_ptr(), W.data_ptr(), b.data_ptr(), target.data_ptr(), logits.data_ptr(), loss.data_ptr(),
+                                     stats.data_ptr(), work.data_ptr(), rows, vocab, dim, s) == 0
+    if odd:
+        x[rows - 1, 3] = W[70, dim - 1] = float("inf")
+    n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
+    assert n > 3 * dim * rows // 2
+    work = torch.full((n + 64,), 7.0, device="cuda")
+    results = []
+    for w in (work.data_ptr(), None):
+        out = [torch.full_like(t, 5.0) for t in (x, W, b)]
+        assert L.lib().fwp_nll_stats_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), stats.data_ptr(), target.data_ptr(),
+                                         gloss.data_ptr(), *(t.data_ptr() for t in out), w, rows, vocab, dim, s) == 0
+        results.append(out)
+    assert bool((work[n:] == 7).all())
+    for a, c in zip(*results):
+        assert bool(((a == c) | (a.isnan() & c.isnan())).all()) and bool(a.isfinite().all()) != (odd and a is not results[0][2])
