@@ -10,7 +10,7 @@
 // Bound by HBM: 2 (forward) and 3 (adjoint) passes over rows x cols floats, 5.9 and 5.5 TB/s at 32768 x 256.  Four rows to a wave have
 // four times the bytes in flight, and a sum is four moves instead of six shuffles one after the other through the LDS's crossbar; one
 // wave per row took 13.3 us forward and 26.0 us backward there against 11.3 and 21.9 now, 8.9 and 19.2 against 6.0 and 11.9 at 24576 x
-// 128, as much up to 2400 rows, where a pass is as long as its launches.  For the adjoint, 1024 workgroups instead of 512 took 2 us more, 256 of eight waves
+// 128.  For the adjoint, as long as before up to 2400 rows, 1024 workgroups instead of 512 took 2 us more, 256 of eight waves
 // 0.2 us less there and 1.4 us more at 2384 rows; loads a turn ahead nothing.
 #include "fwp_common.hpp"
 #include "fwp_wave.hpp"
@@ -19,6 +19,9 @@ namespace fwp {
 namespace {
 
 constexpr int kWaves = 4, kBlocks = 512;
+// Up to here the forward pass takes 64 lanes for any row: with 16 there are too few waves for a pass of one load each.  Within a model, 2381 x 256 3.2 us
+// against 4.2; other data each time 8192 x 256 5.7 (5.9), 12288 x 256 7.7 (7.7), 16384 x 256 8.9 (8.6), 12288 x 128 6.0 (5.1).
+constexpr int kFew = 8192;
 
 // The sum over the four 16-lane rows of the wave, in all of them
 __device__ __forceinline__ float rows_sum(float x) {
@@ -167,11 +170,11 @@ __global__ __launch_bounds__(1024) void k_norm_params(const float *__restrict__ 
     (col < cols ? ggamma : gbeta)[col < cols ? col : col - cols] = s;
 }
 
-// Lanes to a row
-int lanes_of(int cols) { return cols <= 256 ? 16 : 64; }
+// Rows of a workgroup at once, with 16 or 64 lanes to a row
+int rows_of(int cols, bool few = false) { return 64 * kWaves / (cols <= 256 && !few ? 16 : 64); }
 
 int blocks_of(int rows, int cols) {
-    const int at_once = 64 * kWaves / lanes_of(cols);
+    const int at_once = rows_of(cols);
     return (int)std::min<int64_t>(((int64_t)rows + at_once - 1) / at_once, kBlocks);
 }
 
@@ -189,10 +192,12 @@ int64_t layer_norm_workspace(int rows, int cols) { return (int64_t)blocks_of(row
 
 int layer_norm_fwd(const float *x, const float *gamma, const float *beta, float *y, float *stats, int rows, int cols,
                    float eps, hipStream_t s) {
-    const int at_once = 64 * kWaves / lanes_of(cols);
+    const bool few = rows <= kFew;
+    const int at_once = rows_of(cols, few);
     const dim3 grid((rows + at_once - 1) / at_once), block(64 * kWaves);
 #define FWP_FWD(L, V) hipLaunchKernelGGL((k_norm_fwd<L, V>), grid, block, 0, s, x, gamma, beta, y, stats, rows, cols, eps)
-    FWP_BY_COLS(FWP_FWD);
+    if (few && cols <= 256) FWP_FWD(64, 1);
+    else FWP_BY_COLS(FWP_FWD);
 #undef FWP_FWD
     return (int)hipGetLastError();
 }
