@@ -5,7 +5,7 @@ sources (a development aid for the kernels that are bound by instruction issue o
     hipcc --offload-arch=gfx950 -O3 -std=c++17 -Xclang -target-feature -Xclang -packed-fp32-ops \\
           -I include -I recurrent-fwp_amd/csrc -mllvm -amdgpu-mfma-vgpr-form -S --cuda-device-only \\
           recurrent-fwp_amd/csrc/fwp_rec_reg.hip -o rec.s
-    python3 recurrent-fwp_amd/csrc/isa_budget.py rec.s 'k_rec_fwd_regILi32ELi2ELi1ELi2E' 16
+    python3 recurrent-fwp_amd/csrc/isa_budget.py rec.s 'k_rec_fwd_pairILi2E' 8
 
 The third argument is the number of time steps one iteration of the loops covers (the tile length: the tile
 loops are unrolled).  Every loop that does not overlap a larger one is listed, largest first: a kernel whose
