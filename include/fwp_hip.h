@@ -280,6 +280,10 @@ int fwp_lstm_bwd(const fwp_view *k, const fwp_view *beta, const float *vdiff,
 int fwp_deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *beta,
                           int T, int B, int H, int D, float q_scale, void *stream);
 
+/* The same, and zeros to state [B,H,D,D] (contiguous), from which the operator that follows starts. */
+int fwp_deltanet_prep_start(const float *qkvb, float *q, float *k, float *v, float *beta, float *state,
+                            int T, int B, int H, int D, float q_scale, void *stream);
+
 /* Adjoint of fwp_deltanet_prep_fwd: gradients of q, k, v, beta ([B,H,T,.] contiguous) to the
  * gradient of qkvb [T,B,H,3D+1] (every element written). */
 int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,

@@ -48,6 +48,7 @@ _SIGNATURES = {
     "fwp_lstm_fwd": [_VP] * 4 + [_P] * 8 + [_I] * 5 + [_P],
     "fwp_lstm_bwd": [_VP] * 2 + [_P] * 6 + [_V] + [_P] * 5 + [_I] * 5 + [_P],
     "fwp_deltanet_prep_fwd": [_P] * 5 + [_I] * 4 + [ctypes.c_float, _P],
+    "fwp_deltanet_prep_start": [_P] * 6 + [_I] * 4 + [ctypes.c_float, _P],
     "fwp_deltanet_prep_bwd": [_P] * 6 + [_I] * 4 + [ctypes.c_float, _P],
     "fwp_delta_fwd_strided": [_V] * 4 + [_P, OutView] + [_P] * 2 + [_I] * 6 + [_P],
     "fwp_delta_fwd_segments": [_V] * 4 + [_P, OutView] + [_P] * 3 + [_I] * 6 + [_P],

@@ -400,7 +400,14 @@ int fwp_deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float
                           int H, int D, float q_scale, void *stream) {
     if (!qkvb || !q || !k || !v || !beta) return FWP_E_NULL;
     if (T < 1 || B < 1 || H < 1 || !prep_supported(D)) return FWP_E_SHAPE;
-    return deltanet_prep_fwd(qkvb, q, k, v, beta, T, B, H, D, q_scale, (hipStream_t)stream);
+    return deltanet_prep_fwd(qkvb, q, k, v, beta, nullptr, T, B, H, D, q_scale, (hipStream_t)stream);
+}
+
+int fwp_deltanet_prep_start(const float *qkvb, float *q, float *k, float *v, float *beta, float *state, int T, int B,
+                            int H, int D, float q_scale, void *stream) {
+    if (!qkvb || !q || !k || !v || !beta || !state) return FWP_E_NULL;
+    if (T < 1 || B < 1 || H < 1 || !prep_supported(D)) return FWP_E_SHAPE;
+    return deltanet_prep_fwd(qkvb, q, k, v, beta, state, T, B, H, D, q_scale, (hipStream_t)stream);
 }
 
 int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,

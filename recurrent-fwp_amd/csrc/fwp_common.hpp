@@ -185,7 +185,7 @@ int step_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float
 
 // Fused pre-step of the Delta-Net layer and its adjoint (D in {16, 32, 64}).
 bool prep_supported(int D);
-int deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *beta, int T, int B, int H,
+int deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float *beta, float *state, int T, int B, int H,
                       int D, float q_scale, hipStream_t s);
 int deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,
                       const float *gbeta, float *gqkvb, int T, int B, int H, int D, float q_scale, hipStream_t s);

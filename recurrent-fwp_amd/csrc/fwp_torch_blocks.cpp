@@ -233,9 +233,9 @@ struct DeltaReadOutFn : torch::autograd::Function<DeltaReadOutFn> {
 };
 
 struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
-    // x [T,B,d]; Wqkvb [H (3D+1), d]; Wo [d, H D]; state [B,H,D,D] in/out
+    // x [T,B,d]; Wqkvb [H (3D+1), d]; Wo [d, H D]; state [B,H,D,D] in/out (fresh: out, from zeros)
     static at::Tensor forward(AutogradContext *ctx, const at::Tensor &x_in, const at::Tensor &Wqkvb, const at::Tensor &Wo,
-                              const at::Tensor &state, int64_t H, int64_t D, double scale, bool residual) {
+                              const at::Tensor &state, int64_t H, int64_t D, double scale, bool residual, bool fresh) {
         require_device(x_in);
         same_device(x_in, {Wqkvb, Wo, state});
         require(x_in.dim() == 3, "expected [len, bsz, d_model]");
@@ -251,8 +251,12 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
         Parts parts({rows * H * D, rows * H * D, rows * H * D, rows * H}, opts);
         const at::Tensor q = parts.take(B, H, T, D), k = parts.take(B, H, T, D), v = parts.take(B, H, T, D),
                          beta = parts.take(B, H, T, 1);
-        check(fwp_deltanet_prep_fwd(ptr(qkvb), ptr(q), ptr(k), ptr(v), ptr(beta), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
-              "fwp_deltanet_prep_fwd");
+        if (fresh)
+            check(fwp_deltanet_prep_start(ptr(qkvb), ptr(q), ptr(k), ptr(v), ptr(beta), ptr(state), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
+                  "fwp_deltanet_prep_start");
+        else
+            check(fwp_deltanet_prep_fwd(ptr(qkvb), ptr(q), ptr(k), ptr(v), ptr(beta), (int)T, (int)B, (int)H, (int)D, (float)scale, s),
+                  "fwp_deltanet_prep_fwd");
         const at::Tensor out = at::empty({T, B, H, D}, opts);
         const fwp_out_view ov = {ptr(out), H * D, D, B * H * D};
         const int chunk = fwp_query(FWP_Q_DEFAULT_CHUNK);
@@ -281,7 +285,7 @@ struct DeltaBlockFn : torch::autograd::Function<DeltaBlockFn> {
         return y;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
-        variable_list res(8);
+        variable_list res(9);
         if (!grads[0].defined()) return res;
         const auto saved = ctx->get_saved_variables();
         const at::Tensor x = plain(saved[0]), g = plain(grads[0]), &Wqkvb = saved[1], &Wo = saved[2], &qkvb = saved[3],
@@ -545,10 +549,10 @@ at::Tensor feed_forward(const at::Tensor &x, const at::Tensor &W1, const at::Ten
 }
 
 at::Tensor delta_block(const at::Tensor &x, const at::Tensor &Wqkvb, const at::Tensor &Wo, const at::Tensor &state, int64_t n_head,
-                       int64_t d_head, double scale, bool residual) {
-    if (records({&x, &Wqkvb, &Wo})) return DeltaBlockFn::apply(x, Wqkvb, Wo, state, n_head, d_head, scale, residual);
+                       int64_t d_head, double scale, bool residual, bool fresh) {
+    if (records({&x, &Wqkvb, &Wo})) return DeltaBlockFn::apply(x, Wqkvb, Wo, state, n_head, d_head, scale, residual, fresh);
     at::AutoDispatchBelowADInplaceOrView below;
-    return DeltaBlockFn::forward(nullptr, x, Wqkvb, Wo, state, n_head, d_head, scale, residual);
+    return DeltaBlockFn::forward(nullptr, x, Wqkvb, Wo, state, n_head, d_head, scale, residual, fresh);
 }
 
 at::Tensor layer_norm(const at::Tensor &x, const at::Tensor &gamma, const at::Tensor &beta, double eps) {
@@ -658,5 +662,7 @@ void bind_blocks(py::module_ &m) {
     m.def("embed", &embed, "the model's input from token ids; records nothing");
     m.def("layer_norm", &layer_norm, "LayerNorm over the last axis (a multiple of 4 up to 1024)");
     m.def("nll", &nll, "per-row negative log-likelihood of the targets under softmax(x W^T + bias); a target of -100 counts 0");
-    m.def("delta_block", &delta_block, "the Delta-Net layer between its input and its LayerNorm; the state is updated in place");
+    m.def("delta_block", &delta_block, py::arg("x"), py::arg("Wqkvb"), py::arg("Wo"), py::arg("state"), py::arg("n_head"), py::arg("d_head"),
+          py::arg("scale"), py::arg("residual"), py::arg("fresh") = false,
+          "the Delta-Net layer between its input and its LayerNorm; the state is updated in place, from zeros whatever it holds if it is fresh");
 }

@@ -269,9 +269,12 @@ class DeltaNetLayer(nn.Module):
                 and self.qkvb_net.bias is None and self.o_net.bias is None and _untouched(self.drop, nn.Dropout)):
             blocks = _blocks("takes_delta_block", x, self.qkvb_net.weight, self.o_net.weight, H, D)
         if blocks is not None:
-            W = self._state(mems, carry_over_fast_weight, bsz, h, torch.float32)
+            # the block fills a state that starts at zero itself, beside its pre-step
+            fresh = mems is None and getattr(self._state, "__func__", None) is DeltaNetLayer._state
+            W = (torch.empty(bsz, H, D, D, device=h.device, dtype=torch.float32) if fresh
+                 else self._state(mems, carry_over_fast_weight, bsz, h, torch.float32))
             drops = _drops(self.drop)
-            out = blocks.delta_block(x, self.qkvb_net.weight, self.o_net.weight, W, H, D, self.scale, not drops)
+            out = blocks.delta_block(x, self.qkvb_net.weight, self.o_net.weight, W, H, D, self.scale, not drops, fresh)
             if drops:
                 out = residual + self.drop(out)
             if not self.pre_lnorm:

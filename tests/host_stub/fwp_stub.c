@@ -231,6 +231,11 @@ int fwp_deltanet_prep_fwd(const float *qkvb, float *q, float *k, float *v, float
     fill(beta, R, s);
     return 0;
 }
+int fwp_deltanet_prep_start(const float *qkvb, float *q, float *k, float *v, float *beta, float *state, int T, int B,
+                            int H, int D, float q_scale, void *stream) {
+    fill(state, (long long)B * H * D * D, 0);
+    return fwp_deltanet_prep_fwd(qkvb, q, k, v, beta, T, B, H, D, q_scale, stream);
+}
 int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, const float *gv,
                           const float *gbeta, float *gqkvb, int T, int B, int H, int D, float q_scale,
                           void *stream) {

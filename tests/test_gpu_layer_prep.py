@@ -60,3 +60,18 @@ def test_norm_rows(layers, rows, cols):
     # rounded terms a lane and 64 shares one after the other: well below 2^-18
     for got, ref, bound in ((y, want, 2 ** -20), (gx, refs[0], 2 ** -20), (gg, refs[1], 2 ** -18), (gb, refs[2], 2 ** -18)):
         assert float((got.double().cpu() - ref).norm()) <= bound * float(ref.norm())
+
+
+@pytest.mark.parametrize("T,B,D", [(1, 3, 16), (5, 2, 64), (40, 9, 32)])
+def test_a_fresh_state_starts_at_zero(layers, T, B, D):
+    """Fewer lanes than the state has groups, and more; whatever the state's memory held."""
+    L = importlib.import_module("recurrent-fwp_amd._lib")
+    H = 3
+    x = torch.randn(T, B, H * (3 * D + 1), device="cuda")
+    state = torch.full((B * H * D * D + 8,), float("nan"), device="cuda")
+    a, b = ([torch.empty(B, H, T, n, device="cuda") for n in (D, D, D, 1)] for _ in range(2))
+    s = torch.cuda.current_stream().cuda_stream
+    L.check(L.lib().fwp_deltanet_prep_start(x.data_ptr(), *(t.data_ptr() for t in a), state.data_ptr(), T, B, H, D, 0.5, s), "start")
+    L.check(L.lib().fwp_deltanet_prep_fwd(x.data_ptr(), *(t.data_ptr() for t in b), T, B, H, D, 0.5, s), "fwd")
+    assert not bool(state[:-8].any()) and bool(state[-8:].isnan().all())
+    assert all(torch.equal(p, q) for p, q in zip(a, b))
