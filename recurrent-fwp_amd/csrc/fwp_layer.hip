@@ -27,15 +27,24 @@ struct __attribute__((packed, aligned(4))) Any4 { v4f x; };
 __device__ __forceinline__ v4f load(const float *p) { return reinterpret_cast<const Any4 *>(p)->x; }
 __device__ __forceinline__ void store(float *p, v4f x) { reinterpret_cast<Any4 *>(p)->x = x; }
 
-// The sum over the D/4 lanes of a row, in all of them
+// The sum over the D/4 lanes of a row, in all of them: columns D/2 apart first, then D/4 ... 1, the order in which one lane to a column would
+// exchange them.  (Another order rounds as well, but where the results lie close to zero a rectifier behind may turn.)
 template <int D>
 __device__ __forceinline__ float row_sum(v4f y) {
-    float x = (y.x + y.y) + (y.z + y.w);
-    x += dpp<kQuadXor1>(x);
-    x += dpp<kQuadXor2>(x);
-    if constexpr (D >= 32) x += dpp<0x141>(x);      // row_half_mirror
-    if constexpr (D >= 64) x += dpp<0x140>(x);      // row_mirror
-    return x;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        y[i] += dpp<kQuadXor1>(y[i]);
+        y[i] += dpp<kQuadXor2>(y[i]);
+        if constexpr (D >= 32) y[i] += dpp<0x141>(y[i]);      // row_half_mirror: the quads' lanes are alike by now
+        if constexpr (D >= 64) y[i] += dpp<0x140>(y[i]);      // row_mirror
+    }
+    return (y.x + y.z) + (y.y + y.w);
+}
+
+// The first of lane l's four columns: the bits of l the other way round, as row_sum wants them
+template <int D>
+__device__ __forceinline__ int column_of(int l) {
+    return D == 16 ? (l & 1) * 8 + (l >> 1) * 4 : D == 32 ? (l & 1) * 16 + (l & 2) * 4 + (l >> 2) * 4 : (l & 1) * 32 + (l & 2) * 8 + (l & 4) * 2 + (l >> 3) * 4;
 }
 
 __device__ __forceinline__ float feature(float x) { return x > 0.f ? x + 1.f : __expf(x); }   // elu(x) + 1
@@ -58,7 +67,7 @@ struct Row {
         const int h = (int)((blockIdx.x % nh) << a.h) + (i & ((1 << a.h) - 1));
         const int t = (int)((w % nt) << a.t) + (i >> a.h & ((1 << a.t) - 1));
         const int b = (int)((w / nt) << a.b) + (i >> (a.h + a.t));
-        return {((int64_t)t * a.B + b) * a.H + h, ((int64_t)b * a.H + h) * a.T + t, (int)(4 * (threadIdx.x % lanes)),
+        return {((int64_t)t * a.B + b) * a.H + h, ((int64_t)b * a.H + h) * a.T + t, column_of<D>(threadIdx.x % lanes),
                 t < a.T && b < a.B && h < a.H};
     }
 };

@@ -26,20 +26,28 @@ constexpr int kFew = 8192;
 // The sum over the four 16-lane rows of the wave, in all of them
 __device__ __forceinline__ float rows_sum(float x) {
     float y = x;
-    swap16(x, y);
-    x += y, y = x;
     swap32(x, y);
+    x += y, y = x;
+    swap16(x, y);
     return x + y;
 }
 
-// The sum over the L lanes of a row, in all of them
-template <int L>
-__device__ __forceinline__ float row_sum(float x) {
-    x += dpp<kQuadXor1>(x);
+// The sum over the L lanes of a row of their sums over each 64 (L = 16) or all of their columns, in all of them: in the same order for either L, the
+// columns furthest apart first, so that a row's numbers do not depend on how many rows there are.
+template <int L, int V>
+__device__ __forceinline__ float row_sum(const float (&y)[V]) {
+    float x = y[0];
+    if constexpr (L == 64) {
+#pragma unroll
+        for (int i = 1; i < V; i++) x += y[i];
+        x = rows_sum(x);
+    } else if constexpr (V == 4) x = (y[0] + y[2]) + (y[1] + y[3]);
+    else if constexpr (V == 2) x = y[0] + y[1];
+    x += dpp<kRowRor8>(x);
+    x += dpp<kRowRor4>(x);          // the halves are alike by now
     x += dpp<kQuadXor2>(x);
-    x += dpp<0x141>(x);             // row_half_mirror
-    x += dpp<0x140>(x);             // row_mirror
-    return L == 64 ? rows_sum(x) : x;
+    x += dpp<kQuadXor1>(x);
+    return x;
 }
 
 __device__ __forceinline__ float4 load4(const float *p, bool ok) {
@@ -54,22 +62,20 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_fwd(const float *__restric
     if (row >= rows) return;        // all lanes of a row together
     const float *src = x + (int64_t)row * cols;
     float4 v[V];
-    float s = 0.f;
+    float s[V];
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const int c = 4 * (lane + L * i);
         v[i] = load4(src + c, c < cols);
     }
 #pragma unroll
-    for (int i = 0; i < V; i++) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    for (int i = 0; i < V; i++) s[i] = (v[i].x + v[i].y) + (v[i].z + v[i].w);
     const float mean = row_sum<L>(s) / cols;
-    s = 0.f;
 #pragma unroll
-    for (int i = 0; i < V; i++)
-        if (4 * (lane + L * i) < cols) {
-            const float a = v[i].x - mean, b = v[i].y - mean, c = v[i].z - mean, d = v[i].w - mean;
-            s += (a * a + b * b) + (c * c + d * d);
-        }
+    for (int i = 0; i < V; i++) {
+        const float a = v[i].x - mean, b = v[i].y - mean, c = v[i].z - mean, d = v[i].w - mean;
+        s[i] = 4 * (lane + L * i) < cols ? fmaf(a, a, b * b) + fmaf(c, c, d * d) : 0.f;
+    }
     const float rstd = 1.f / sqrtf(row_sum<L>(s) / cols + eps);
 #pragma unroll
     for (int i = 0; i < V; i++) {
@@ -103,7 +109,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restric
         const int64_t at = row * cols;
         const float2 st = *reinterpret_cast<const float2 *>(stats + 2 * row);
         float4 g[V], xh[V];
-        float s = 0.f, t = 0.f;
+        float sums[V], products[V];
 #pragma unroll
         for (int i = 0; i < V; i++) {
             const int c = 4 * (lane + L * i);
@@ -116,11 +122,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_norm_bwd(const float *__restric
             sb[i].x += d.x, sb[i].y += d.y, sb[i].z += d.z, sb[i].w += d.w;
             sg[i].x += d.x * xh[i].x, sg[i].y += d.y * xh[i].y, sg[i].z += d.z * xh[i].z, sg[i].w += d.w * xh[i].w;
             g[i] = make_float4(d.x * gam[i].x, d.y * gam[i].y, d.z * gam[i].z, d.w * gam[i].w);
-            s += (g[i].x + g[i].y) + (g[i].z + g[i].w);
-            t += (g[i].x * xh[i].x + g[i].y * xh[i].y) + (g[i].z * xh[i].z + g[i].w * xh[i].w);
+            sums[i] = (g[i].x + g[i].y) + (g[i].z + g[i].w);
+            products[i] = (g[i].x * xh[i].x + g[i].y * xh[i].y) + (g[i].z * xh[i].z + g[i].w * xh[i].w);
         }
-        s = row_sum<L>(s) / cols;
-        t = row_sum<L>(t) / cols;
+        const float s = row_sum<L>(sums) / cols, t = row_sum<L>(products) / cols;
 #pragma unroll
         for (int i = 0; i < V; i++) {
             const int c = 4 * (lane + L * i);
