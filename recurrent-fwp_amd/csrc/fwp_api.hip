@@ -2,6 +2,7 @@
 // the register-state kernels (E = M in {16, 32}, 16-byte aligned rows) and the
 // LDS-state kernels (everything else).
 #include "fwp_common.hpp"
+#include "fwp_gemm_plan.hpp"
 
 #include <atomic>
 #include <initializer_list>

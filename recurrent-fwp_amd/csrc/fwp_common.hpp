@@ -198,7 +198,6 @@ struct NllView {
     const int64_t *target;
     int vocab;
 };
-int64_t matmul_workspace(int M, int N, int K);
 int matmul(int layout, const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, int M, int N,
            int K, const fwp_mm_epilogue &epi, float *workspace, const NllView *nll, hipStream_t s);
 int64_t nll_workspace(int rows, int vocab);

@@ -464,3 +464,29 @@ def test_gradients_from_an_operand_split_once(fwp, rows, vocab, dim, odd):
     assert bool((work[n:] == 7).all())
     for a, c in zip(*results):
         assert bool(((a == c) | (a.isnan() & c.isnan())).all()) and bool(a.isfinite().all()) != (odd and a is not results[0][2])
+
+
+def test_gradients_off_a_16_byte_boundary_leave_the_rest_of_the_workspace(fwp):
+    """Such results get another plan than the one the workspace's size comes from: nothing behind that size is written, and the numbers are those
+    of a call without a workspace."""
+    L = fwp._lib
+    rows, vocab, dim = 10142, 35166, 258
+    x, W, b = randn(rows, dim, seed=1) * 0.1, randn(vocab, dim, seed=2) * 0.3, randn(vocab, seed=3)
+    target = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(4)).cuda()
+    gloss = randn(rows, seed=5)
+    logits, loss, stats = torch.empty(rows, vocab, device="cuda"), torch.empty(rows, device="cuda"), torch.empty(rows, 2, device="cuda")
+    work = torch.empty(L.lib().fwp_nll_workspace(rows, vocab), device="cuda")
+    s = L.stream_of(x)
+    assert L.lib().fwp_nll_stats_fwd(x.data_ptr(), W.data_ptr(), b.data_ptr(), target.data_ptr(), logits.data_ptr(), loss.data_ptr(),
+                                     stats.data_ptr(), work.data_ptr(), rows, vocab, dim, s) == 0
+    n = max(L.lib().fwp_matmul_workspace(rows, dim, vocab), L.lib().fwp_matmul_workspace(vocab, dim, rows))
+    work = torch.full((n + (8 << 20),), 7.0, device="cuda")
+    results = []
+    for w in (work.data_ptr(), None):
+        out = [torch.full((t.numel() + 1,), 5.0, device="cuda") for t in (x, W, b)]
+        assert L.lib().fwp_nll_stats_bwd(x.data_ptr(), W.data_ptr(), logits.data_ptr(), stats.data_ptr(), target.data_ptr(),
+                                         gloss.data_ptr(), *(t.data_ptr() + 4 for t in out), w, rows, vocab, dim, s) == 0
+        assert all(float(t[0]) == 5.0 for t in out)
+        results.append(out)
+    assert bool((work[n:] == 7).all())
+    assert all(torch.equal(a, c) for a, c in zip(*results))
