@@ -6,7 +6,8 @@
 // activated q and k "grouped" (every lane of group m holds entry m), periodic operands through ds_bpermute, the softmax
 // maxima/sums, the beta logit and the softmax-Jacobian dot products as wave-wide reductions.  32 x 32: vectors in half and
 // pair form (fwp_reg.hpp), two waves to a sequence forward and four backward.  512 sequences of 256 steps, against the
-// former's kernels for 32 x 32: forward 144 -> 120 us, backward with its sum over the sequences 197 -> 128 us.
+// former's kernels for 32 x 32: forward 144 -> 120 us, backward with its sum over the sequences 197 -> 131 us.  Matrices come and go by way of LDS (see
+// forms::Matrix): of 20 steps, 512 / 1024 / 2048 sequences, forward 19.3 / 30.1 / 52.6 -> 12.9 / 15.2 / 23.4 us, backward 23.9 / 41.1 / 75.0 -> 23.1 / 39.5 / 71.8.
 #include "fwp_reg.hpp"
 #include "fwp_mfma.hpp"
 
@@ -209,6 +210,7 @@ struct RecFwdTile {
     float ba[kFwdTile];                                    // beta
 };
 typedef RecFwdTile RecFwdLds[2];
+static_assert(sizeof(RecFwdTile) >= 4096, "a matrix on its way");
 
 struct RecFwdArgs {
     fwp_view qx, kx, vx, bx;
@@ -226,13 +228,29 @@ __device__ __forceinline__ void rec_fwd_steps(RecFwdLds &M, const RecFwdArgs &g,
     constexpr float kFar = 20.f;
     const int half = forms::half(lane), pair = forms::pair(lane), hd = (int)(seq % g.H), L = g.L;
     float W[16], Rq[16], Rk[16], Rv[16], far = 0.f, far_k = 0.f;
+    {
+        // through the second tile's place, which the other wave fills from its first step on
+        float *const stage = reinterpret_cast<float *>(&M[1]);
+        const int64_t R = (int64_t)hd * 1024;
+        Matrix a, b;
+        a.fetch(g.Rq + R, lane), b.fetch(g.Rk + R, lane);
+        a.put(stage, lane);
 #pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const int64_t at = ((int64_t)hd * 32 + terms_of_half(lane, j)) * 32 + half;
-        Rq[j] = g.Rq[at], Rk[j] = g.Rk[at], Rv[j] = g.Rv[at];
-        W[j] = g.W[(seq * 32 + terms_of_pair(lane, j)) * 32 + pair];
-        far += fabsf(Rq[j]), far_k += fabsf(Rk[j]);
+        for (int j = 0; j < 16; j++) Rq[j] = stage[terms_of_half(lane, j) * 32 + half];
+        a.fetch(g.Rv + R, lane);
+        b.put(stage, lane);
+#pragma unroll
+        for (int j = 0; j < 16; j++) Rk[j] = stage[terms_of_half(lane, j) * 32 + half];
+        b.fetch(g.W + seq * 1024, lane);
+        a.put(stage, lane);
+#pragma unroll
+        for (int j = 0; j < 16; j++) Rv[j] = stage[terms_of_half(lane, j) * 32 + half];
+        b.put(stage, lane);
+#pragma unroll
+        for (int j = 0; j < 16; j++) W[j] = stage[terms_of_pair(lane, j) * 32 + pair];
     }
+#pragma unroll
+    for (int j = 0; j < 16; j++) far += fabsf(Rq[j]), far_k += fabsf(Rk[j]);
     const bool near = !__any(!(sum_to_half(far) <= kFar) || !(sum_to_half(far_k) <= kFar));
     const float rb = g.rb[hd * 32 + pair];
     float h = g.h[seq * 32 + pair];
@@ -304,15 +322,21 @@ __device__ __forceinline__ void rec_fwd_steps(RecFwdLds &M, const RecFwdArgs &g,
             }
         }
         const int t_end = it * kFwdTile + nst;
-        if (g.ckpt && (t_end % g.chunk == 0 || t_end == L)) {
-            float *c = g.ckpt + (seq * g.nchunk + (t_end - 1) / g.chunk) * 1024;
+        if (g.ckpt && t_end % g.chunk == 0 && t_end < L) {
+            float *c = g.ckpt + (seq * g.nchunk + t_end / g.chunk - 1) * 1024;
 #pragma unroll
             for (int j = 0; j < 16; j++) c[terms_of_pair(lane, j) * 32 + pair] = W[j];
         }
         lds_barrier();
     }
+    // through the last tile but one's place, which the other wave has read
+    float *const stage = reinterpret_cast<float *>(&M[ntile & 1]);
+    Matrix last;
 #pragma unroll
-    for (int j = 0; j < 16; j++) g.W[(seq * 32 + terms_of_pair(lane, j)) * 32 + pair] = W[j];
+    for (int j = 0; j < 16; j++) stage[terms_of_pair(lane, j) * 32 + pair] = W[j];
+    last.take(stage, lane);
+    last.store(g.W + seq * 1024, lane);
+    if (g.ckpt) last.store(g.ckpt + (seq * g.nchunk + g.nchunk - 1) * 1024, lane);
     if (first) g.h[seq * 32 + pair] = h;
 }
 
@@ -762,13 +786,25 @@ __device__ __forceinline__ void rec_bwd_x(RecBwdLds &M, const RecBwdArgs &g, int
     using namespace forms;
     const int half = forms::half(lane), pair = forms::pair(lane), hd = (int)(seq % g.H), L = g.L;
     float W[16], Wnext[16], R0[16], R1[16], Rv[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
+    {
+        // through where this wave's results of a tile are kept
+        static_assert(sizeof(M.tile[0].gqk) == 4096, "a matrix on its way");
+        float *const stage = M.tile[0].gqk;
+        const int64_t R = (int64_t)hd * 1024;
         // a row of lanes holds half of one vector of (grad_qx, grad_kx): entries lane % 16 and 16 + lane % 16 of the results
-        const float *R = (lane < 32 ? g.Rq : g.Rk) + (int64_t)hd * 1024 + terms_of_pair(lane, j);
-        R0[j] = R[lane % 16 * 32], R1[j] = R[(16 + lane % 16) * 32];
-        Rv[j] = g.Rv[(int64_t)hd * 1024 + half * 32 + terms_of_half(lane, j)];
-        W[j] = 0.f;
+        const auto read = [&] {
+#pragma unroll
+            for (int j = 0; j < 16; j++) R0[j] = stage[lane % 16 * 32 + terms_of_pair(lane, j)], R1[j] = stage[(16 + lane % 16) * 32 + terms_of_pair(lane, j)];
+        };
+        Matrix a, b, c;
+        a.fetch(g.Rq + R, lane), b.fetch(g.Rk + R, lane), c.fetch(g.Rv + R, lane);
+        a.put(stage, lane);
+        if (lane < 32) read();
+        b.put(stage, lane);
+        if (lane >= 32) read();
+        c.put(stage, lane);
+#pragma unroll
+        for (int j = 0; j < 16; j++) Rv[j] = stage[half * 32 + terms_of_half(lane, j)], W[j] = 0.f;
     }
     const float rb = g.rb[hd * 32 + pair];
     float dh = 0.f;
@@ -818,8 +854,9 @@ __device__ __forceinline__ void rec_bwd_x(RecBwdLds &M, const RecBwdArgs &g, int
         gqk_at[tt * 64] = gqk, gv_at[tt * 32] = gv, gb_at[tt] = gb;
     };
     const int ntile = (L + kTile - 1) / kTile;
-    rec_state_rows(Wnext, g, seq, g.nchunk - 1, lane);
     lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 16; j++) Wnext[j] = M.tile[1].gqk[half * 32 + terms_of_half(lane, j)];      // the last state, from wave C
     for (int it = ntile - 1; it >= 0; it--) {
         const int t0 = it * kTile, nst = min(kTile, L - t0);
         RecBwdTile &T = M.tile[it & 1];
@@ -859,9 +896,12 @@ __device__ __forceinline__ void rec_bwd_c(RecBwdLds &M, const RecBwdArgs &g, int
     using namespace forms;
     const int half = forms::half(lane), pair = forms::pair(lane), L = g.L, ntile = (L + kTile - 1) / kTile;
     float W[16], Wnext[16], G[16], P = 0.f;
-    rec_state_rows(W, g, seq, g.nchunk - 1, lane);
+    float *const stage = M.tile[1].gqk;      // wave X reads it too, before it keeps results there
+    Matrix last;
+    last.fetch(g.ckpt + (seq * g.nchunk + g.nchunk - 1) * 1024, lane);
+    last.put(stage, lane);
 #pragma unroll
-    for (int j = 0; j < 16; j++) G[j] = Wnext[j] = 0.f;
+    for (int j = 0; j < 16; j++) W[j] = stage[half * 32 + terms_of_half(lane, j)], G[j] = Wnext[j] = 0.f;
     M.P[0][half] = M.P[1][half] = 0.f;
     M.Q[0][lane] = M.Q[1][lane] = M.WP[0][lane] = M.WP[1][lane] = 0.f;
     M.Pd[0] = M.Pd[1] = 0.f;
@@ -1184,12 +1224,12 @@ int reg_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float 
             constexpr int NS = decltype(ns)::value;
             hipLaunchKernelGGL(k_rec_fwd_pair<NS>, dim3((nseq + NS - 1) / NS), dim3(2 * NS * kWave), 0, s, g);
         };
-        // Two sequences to a workgroup while that is one workgroup on each CU, four up to 1024 sequences (two-wave shares of a CU are placed
-        // unevenly on its SIMDs once there is more than one), six workgroups of two beside each other up to 1536, then eight. 256 steps,
-        // workgroups of 2 / 4 / 8: 768 sequences 180 / 123 / 191 us, 1536 184 / 241 / 196, 2048 249 / 247 / 202.
+        // Two sequences to a workgroup while that is one workgroup on each CU, and from 1025 to 1536 sequences, three workgroups on a CU; else four (two-wave shares
+        // of a CU are placed unevenly on its SIMDs once there is more than one).  20, 60 and 256 steps, workgroups of 2 / 4 / 8: 512 sequences
+        // 13.0 / 13.5 / 19.6, 32.5 / 33.2 / 48.9 and 122 / 124 / 186 us, 1024 19.5 / 15.2 / 20.9, 47.8 / 34.8 / 49.6 and 181 / 131 / 191, 1536 20.5 / 21.1 / 21.6,
+        // 49.4 / 50.1 / 50.8 and 187 / 193 / 197, 2048 23.9 / 23.4 / 24.6, 55.1 / 51.4 / 52.6 and 209 / 199 / 205.
         if (nseq <= 512 || (nseq > 1024 && nseq <= 1536)) go(std::integral_constant<int, 2>());
-        else if (nseq <= 1024) go(std::integral_constant<int, 4>());
-        else go(std::integral_constant<int, 8>());
+        else go(std::integral_constant<int, 4>());
     }
     return (int)hipGetLastError();
 }

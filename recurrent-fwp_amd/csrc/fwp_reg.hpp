@@ -272,6 +272,31 @@ __device__ __forceinline__ int pair(int lane) { return lane / 32 * 16 + lane % 1
 __device__ __forceinline__ int terms_of_half(int lane, int j) { return lane / 32 * 16 + ((lane - j) & 15); }
 __device__ __forceinline__ int terms_of_pair(int lane, int j) { return lane / 16 % 2 * 16 + ((lane - j) & 15); }
 
+// A 32 x 32 matrix between memory and a wave's registers by way of 4 KB of LDS: in memory a lane has 16 bytes of a row at any address of a
+// float, in LDS the registers' entries are read and written one by one.  Straight from memory each of a matrix's 16 loads, or stores, touches 32 lines
+// of which it needs two entries, which with four sequences on a CU took longer than 20 steps.
+struct Matrix {
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    struct __attribute__((packed, aligned(4))) Any4 { v4f x; };
+    v4f r[4];
+    __device__ __forceinline__ void fetch(const float *from, int lane) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = reinterpret_cast<const Any4 *>(from + 4 * (lane + kWave * i))->x;
+    }
+    __device__ __forceinline__ void put(float *lds, int lane) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++) *reinterpret_cast<v4f *>(lds + 4 * (lane + kWave * i)) = r[i];
+    }
+    __device__ __forceinline__ void take(const float *lds, int lane) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = *reinterpret_cast<const v4f *>(lds + 4 * (lane + kWave * i));
+    }
+    __device__ __forceinline__ void store(float *to, int lane) const {
+#pragma unroll
+        for (int i = 0; i < 4; i++) reinterpret_cast<Any4 *>(to + 4 * (lane + kWave * i))->x = r[i];
+    }
+};
+
 // x is about to be rotated by an asm statement below: the wait states between a vector instruction that wrote it and a DPP
 // read of it, which the compiler cannot see there.
 __device__ __forceinline__ float ready(float x) {

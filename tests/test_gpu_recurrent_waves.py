@@ -96,6 +96,28 @@ def test_rec_where_a_step_looks_for_its_largest_entry(fwp):
         check("grad " + name, t.grad, g, 3, sums=100)
 
 
+def test_rec_matrices_at_any_address(fwp):
+    """The state and the slow weights are read and written 16 bytes at a time from addresses of any float; the floats around the state stay."""
+    x = rec_inputs(8, 3, 2, 21, 32, w0=True)
+
+    def off(a):
+        a = np.asarray(a, np.float32)
+        t = torch.full((a.size + 9,), 7.0, device="cuda")
+        t[5:-4] = torch.from_numpy(a.ravel()).cuda()
+        return t, t[5:-4].view(a.shape)
+
+    ts = [dev(a, True) for a in x[:4]] + [off(a)[1].requires_grad_() for a in x[4:8]]
+    (around, W), (_, h) = off(x[8]), off(x[9])
+    out = fwp.rec_update_fwm_tanh(*ts, W, h)
+    out.backward(dev(x[10]))
+    x64 = [np.asarray(a, np.float32).astype(np.float64) for a in x]
+    for name, a, b in zip(("out", "W", "h"), (out, W, h), oracle.rec_fwd(*x64[:-1])):
+        check(name, a, b, 21)
+    assert bool((around[:5] == 7).all()) and bool((around[-4:] == 7).all())
+    for name, t, g in zip("qx kx vx bx R_q R_k R_v r_b".split(), ts, oracle.rec_bwd(*x64)):
+        check("grad " + name, t.grad, g, 21)
+
+
 def test_rec_masked_and_undefined_entries(fwp):
     """-infinity in a row of the logits is a probability of 0; a row of nothing else, NaN or +infinity make that step and what follows NaN."""
     x = rec_inputs(7, 2, 1, 12, 32, w0=True)
