@@ -1249,6 +1249,10 @@ int reg_rec_bwd(const float *q_act, const float *k_act, const float *beta_act, c
                            nchunk, nseq);
         return (int)hipGetLastError();
     };
+    // D = 32: the two-wave kernel has 1024 sequences on the chip at once, the four-wave one 512.  Where it needs half as many turns and the steps are few, what a turn
+    // costs once weighs more than a step: two waves / four, 1024 sequences of 20, 60, 128, 160, 200 and 256 steps 36 / 39, 70 / 77, 132 / 136, 163 / 165, 204 / 201 and
+    // 260 / 251 us; 2048 of 20, 128, 160 and 256 63 / 72, 265 / 269, 337 / 329 and 522 / 495; 771 of 20 and 200 34 / 39 and 197 / 198.
+    if (D == 32 && L <= 160 && nseq > 768 && (nseq - 1) / 512 % 2 == 1) return launch(k_rec_bwd_pair<32, 4>, 4, 4 * sizeof(RecPairLds<32>));
     if (D == 32) {
         const RecBwdArgs g{q_act, k_act, beta_act, vdiff, out, h_init, go, Rq, Rk, Rv, rb, ckpt, gqx, gkx, gvx, gbx, workspace, H, L, chunk, nchunk};
         const auto run = [&](auto ns) {

@@ -38,9 +38,9 @@ def check(name, got, want, steps, sums=1):
 LENGTHS = (2, 7, 8, 9, 15, 16, 17, 31, 33, 63, 64, 65, 130, 193)
 
 
-@pytest.mark.parametrize("N,H,L", [(1, 3, L) for L in LENGTHS] + [(171, 3, 18), (257, 3, 18), (257, 4, 17), (386, 4, 9)])
+@pytest.mark.parametrize("N,H,L", [(1, 3, L) for L in LENGTHS] + [(171, 3, 18), (257, 3, 18), (257, 4, 17), (386, 4, 9), (257, 3, 160), (257, 3, 161)])
 def test_rec_tiles_and_workgroups(fwp, N, H, L):
-    """513 to 768, more than 768, 1024 and 1536 sequences: each division into workgroups, with spare waves in the last one."""
+    """513 to 768, more than 768, 1024 and 1536 sequences: each division into workgroups, with spare waves in the last one; up to 160 steps and more."""
     x = rec_inputs(L + N, N, H, L, 32, w0=True)
     x, go = x[:-1], x[-1]
     x32 = [np.asarray(a, np.float32) for a in x]
