@@ -40,9 +40,11 @@ def test_rows(layers, T, B, H, D):
         assert float((a.double().cpu() - b).norm()) <= 2 ** -20 * float(b.norm())
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 60), (17, 64), (16, 68), (15, 128), (33, 132), (8193, 256), (8, 260), (8191, 64)])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 60), (17, 64), (16, 68), (15, 128), (33, 132), (8193, 256), (8, 260), (8191, 64),
+                                       (9001, 4), (20001, 60), (1025, 68), (2003, 96), (1030, 128), (8197, 132), (10243, 188), (16389, 252)])
 def test_norm_rows(layers, rows, cols):
-    """LayerNorm where a workgroup's 16 rows of up to 256 columns, a row's last lanes and the workgroups' second turn are cut."""
+    """LayerNorm where a workgroup's rows (4, or 16 of up to 256 columns), a row's last lanes and the workgroups' second turn are cut; with few rows, and with
+    those from which on 16 lanes take a row, forward and in the adjoint."""
     L = importlib.import_module("recurrent-fwp_amd._lib")
     torch.manual_seed(rows + cols)
     x, gy = torch.randn(2, rows, cols, device="cuda")
@@ -60,6 +62,26 @@ def test_norm_rows(layers, rows, cols):
     # rounded terms a lane and 64 shares one after the other: well below 2^-18
     for got, ref, bound in ((y, want, 2 ** -20), (gx, refs[0], 2 ** -20), (gg, refs[1], 2 ** -18), (gb, refs[2], 2 ** -18)):
         assert float((got.double().cpu() - ref).norm()) <= bound * float(ref.norm())
+
+
+@pytest.mark.parametrize("cols", [60, 64, 68, 128, 132, 192, 252, 256])
+def test_norm_of_a_row_does_not_depend_on_the_number_of_rows(layers, cols):
+    """More rows take 16 lanes each instead of 64: every number is the same to the last bit, results and gradients of x."""
+    L = importlib.import_module("recurrent-fwp_amd._lib")
+    torch.manual_seed(cols)
+    rows, few = 16400, 100
+    x, gy = torch.randn(2, rows, cols, device="cuda")
+    g, b = torch.randn(2, cols, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    got = []
+    for n in (rows, few):
+        y, gx, stats, gg, gb = torch.empty_like(x[:n]), torch.empty_like(x[:n]), torch.empty(n, 2, device="cuda"), torch.empty_like(g), torch.empty_like(b)
+        L.check(L.lib().fwp_layer_norm_fwd(x.data_ptr(), g.data_ptr(), b.data_ptr(), y.data_ptr(), stats.data_ptr(), n, cols, 1e-5, s), "fwd")
+        work = torch.empty(L.lib().fwp_layer_norm_workspace(n, cols), device="cuda")
+        L.check(L.lib().fwp_layer_norm_bwd(gy.data_ptr(), x.data_ptr(), stats.data_ptr(), g.data_ptr(), gx.data_ptr(), gg.data_ptr(), gb.data_ptr(),
+                                           work.data_ptr(), n, cols, s), "bwd")
+        got.append((y[:few], stats[:few], gx[:few]))
+    assert all(torch.equal(a, c) for a, c in zip(*got))
 
 
 @pytest.mark.parametrize("T,B,D", [(1, 3, 16), (5, 2, 64), (40, 9, 32)])
