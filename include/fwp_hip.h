@@ -300,7 +300,8 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
  *   FWP_MM_TN: C = A^T B, A [K,M], B [K,N]      row-major, rows lda, ldb, ldc floats apart
  * epi (NULL: none): C = relu(C + bias) + residual, 0 where gate <= 0, each part optional (a NaN passes relu and gate, as in
  * PyTorch); residual and gate are laid out like C.  colsum (FWP_MM_TN): [M], the sums of A's columns (a bias gradient).
- * workspace: fwp_matmul_workspace(M, N, K) floats (16-byte aligned), or NULL (a product with few tiles and a long K then runs on fewer CUs).
+ * workspace: fwp_product_workspace(M, N, K) floats (16-byte aligned), or NULL (a product with few tiles and a long K then runs on fewer CUs);
+ * fwp_matmul_workspace(M, N, K), which the gradients of fwp_nll_bwd need, is no less.
  */
 enum { FWP_MM_NT = 0, FWP_MM_NN = 1, FWP_MM_TN = 2 };
 typedef struct fwp_mm_epilogue {
@@ -308,6 +309,7 @@ typedef struct fwp_mm_epilogue {
     float *colsum;
     int relu;
 } fwp_mm_epilogue;
+long long fwp_product_workspace(int M, int N, int K);
 long long fwp_matmul_workspace(int M, int N, int K);
 int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C,
                long long ldc, int M, int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream);

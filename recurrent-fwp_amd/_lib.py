@@ -71,7 +71,7 @@ _MODEL_SIGNATURES = {
     "fwp_deltanet_step": [_P] * 4 + [_I] * 3 + [ctypes.c_float, _P],
     "fwp_embed": [_P] * 4 + [_I] * 3 + [_L, ctypes.c_float, ctypes.c_float, _P],
 }
-_WORKSPACES = {"fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
+_WORKSPACES = {"fwp_product_workspace": 3, "fwp_matmul_workspace": 3, "fwp_nll_workspace": 2, "fwp_layer_norm_workspace": 2}
 EXPORTS = sorted(list(_SIGNATURES) + list(_MODEL_SIGNATURES) + list(_WORKSPACES) + ["fwp_strerror", "fwp_query", "fwp_check_device", "fwp_config",
                                        "fwp_delta_ckpt_floats", "fwp_delta_segment_floats", "fwp_delta_bwd_segment_floats", "fwp_delta_kind", "fwp_delta_fwd_kind"])
 KIND_LDS, KIND_SCAN, KIND_CHUNKED, KIND_SPLIT, KIND_PHASE, KIND_STEP = 0, 1, 2, 3, 4, 5

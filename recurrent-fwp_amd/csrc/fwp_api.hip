@@ -419,6 +419,10 @@ int fwp_deltanet_prep_bwd(const float *qkvb, const float *gq, const float *gk, c
     return deltanet_prep_bwd(qkvb, gq, gk, gv, gbeta, gqkvb, T, B, H, D, q_scale, (hipStream_t)stream);
 }
 
+long long fwp_product_workspace(int M, int N, int K) {
+    return M < 1 || N < 1 || K < 1 ? FWP_E_SHAPE : product_workspace(M, N, K);
+}
+
 long long fwp_matmul_workspace(int M, int N, int K) {
     return M < 1 || N < 1 || K < 1 ? FWP_E_SHAPE : matmul_workspace(M, N, K);
 }

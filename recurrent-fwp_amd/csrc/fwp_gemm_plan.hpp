@@ -79,8 +79,7 @@ inline int64_t part_of(int M, int N) { return ((int64_t)M * N + 3) / 4 * 4; }
 // did it again for its 128 rows, a third of its vector instructions, which bound them as much as the products do (each busy 45 % of the time).
 // Words = tokens = 32768, 256 columns: dX 2.98 -> 2.60 ms, dW 3.19 -> 3.06 ms; 32768 words, 24576 tokens, 128 columns 1.58 -> 1.32 and
 // 1.44 -> 1.25 ms; 4100 tokens, 5001 words, 256 columns 82 -> 75 and 84 -> 83 us; 3000 of both 45 -> 45 and 47 -> 50 us; 1024
-// tokens, 32768 words dX 107 -> 112 us; 32768 tokens, 1024 words dW 114 -> 128 us.  With k of 1024 dX would still gain (100 -> 94 us), but ordinary products of such
-// sizes would ask for the workspace too.
+// tokens, 32768 words dX 107 -> 112 us; 32768 tokens, 1024 words dW 114 -> 128 us.  With k of 1024 dX would still gain (100 -> 94 us), dW not.
 constexpr int kImage = 4096;
 
 // floats of the partial results and, behind them, of B's image
@@ -100,10 +99,13 @@ inline Scratch scratch_of(int M, int N, int K, bool may_cut, bool grad) {
     return {p, parts_of(p, M, N), grad && may_cut ? image_of(p, M, K) : 0};
 }
 
+// what a product uses (no image: 4096 x 1024 over 32768 tokens 34 MB, with the room for one 235)
+inline int64_t product_workspace(int M, int N, int K) { return scratch_of(M, N, K, true, false).parts; }
+
 // enough for a product and for a loss's gradient
 inline int64_t matmul_workspace(int M, int N, int K) {
-    const Scratch product = scratch_of(M, N, K, true, false), grad = scratch_of(M, N, K, true, true);
-    return std::max(product.parts, grad.parts + grad.image);
+    const Scratch grad = scratch_of(M, N, K, true, true);
+    return std::max(product_workspace(M, N, K), grad.parts + grad.image);
 }
 
 }  // namespace fwp

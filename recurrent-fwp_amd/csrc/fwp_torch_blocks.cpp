@@ -37,7 +37,7 @@ bool ends_in(const at::Tensor &x, int64_t n) { return x.dim() > 0 && x.size(-1) 
 at::Tensor matmul(int layout, const at::Tensor &A, const at::Tensor &B, int64_t M, int64_t N, int64_t K, at::IntArrayRef shape,
                   const fwp_mm_epilogue &epi = {}) {
     at::Tensor C = at::empty(shape, A.options()), work;
-    const int64_t n = fwp_matmul_workspace((int)M, (int)N, (int)K);
+    const int64_t n = fwp_product_workspace((int)M, (int)N, (int)K);
     if (n > 0) work = at::empty({n}, A.options());
     check(fwp_matmul(layout, ptr(A), layout == FWP_MM_TN ? M : K, ptr(B), layout == FWP_MM_NT ? K : N, ptr(C), N, (int)M,
                      (int)N, (int)K, &epi, ptr(work), stream_of(A)),

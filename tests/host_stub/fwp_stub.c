@@ -313,13 +313,14 @@ int fwp_rec_bwd_static(const float *q_act, const float *k_act, const float *beta
 
 /* ---- the language model's kernels, computed */
 
+long long fwp_product_workspace(int M, int N, int K) { (void)M; (void)N; return K >= 64 ? 8 : 0; }
 long long fwp_matmul_workspace(int M, int N, int K) { (void)M; (void)N; return K >= 64 ? 8 : 0; }
 int fwp_matmul(int layout, const float *A, long long lda, const float *B, long long ldb, float *C, long long ldc, int M,
                int N, int K, const fwp_mm_epilogue *epi, float *workspace, void *stream) {
     (void)stream;
     g_calls++;
     const fwp_mm_epilogue none = {0}, e = epi ? *epi : none;
-    if (workspace) fill(workspace, fwp_matmul_workspace(M, N, K), 0);
+    if (workspace) fill(workspace, fwp_product_workspace(M, N, K), 0);
     for (int m = 0; m < M; m++)
         for (int n = 0; n < N; n++) {
             double s = 0;

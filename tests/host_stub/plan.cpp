@@ -19,5 +19,5 @@ int64_t plan_product_used(int M, int N, int K, int aligned) {
     return s.parts + s.image;
 }
 
-int64_t plan_product_workspace(int M, int N, int K) { return matmul_workspace(M, N, K); }
+int64_t plan_product_workspace(int M, int N, int K) { return product_workspace(M, N, K); }
 }

@@ -40,4 +40,10 @@ def test_products_stay_within_their_workspace(plan):
     for M, N, K in list(sizes(20000, 1, 65536, 3)):
         for m, n, k in ((M, K, N), (M, N, K), (K, M, N)):
             have = plan.plan_product_workspace(m, n, k)
-            assert plan.plan_product_used(m, n, k, 1) <= have and plan.plan_product_used(m, n, k, 0) == 0, (m, n, k)
+            assert plan.plan_product_used(m, n, k, 1) == have and plan.plan_product_used(m, n, k, 0) == 0, (m, n, k)
+
+
+def test_a_product_asks_for_no_image_of_its_operand(plan):
+    """A weight gradient of a wide layer: its partial results, a few copies of it, and nothing of the size of the 32768 tokens."""
+    assert plan.plan_product_workspace(4096, 1024, 32768) <= 4 * 4096 * (1024 + 1)
+    assert plan.plan_product_workspace(8192, 2048, 32768) == 0

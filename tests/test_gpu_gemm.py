@@ -490,3 +490,19 @@ def test_gradients_off_a_16_byte_boundary_leave_the_rest_of_the_workspace(fwp):
         results.append(out)
     assert bool((work[n:] == 7).all())
     assert all(torch.equal(a, c) for a, c in zip(*results))
+
+
+@pytest.mark.parametrize("layout,M,N,K", [(NT, 16, 256, 4096), (TN, 776, 256, 3001), (NN, 257, 36, 1000), (TN, 130, 70, 9000), (TN, 4100, 256, 4100)])
+def test_a_product_stays_within_its_own_workspace(fwp, layout, M, N, K):
+    """Its size leaves out what only the loss's gradients use; the partial sums are those of a call with room for both."""
+    L = fwp._lib
+    A, B = randn(*((K, M) if layout == TN else (M, K)), seed=1), randn(*((N, K) if layout == NT else (K, N)), seed=2)
+    n = L.lib().fwp_product_workspace(M, N, K)
+    assert 0 <= n <= L.lib().fwp_matmul_workspace(M, N, K)
+    work, C = torch.full((n + 4096,), 7.0, device="cuda"), torch.empty(M, N, device="cuda")
+    colsum = torch.empty(M, device="cuda")
+    e = L.Epilogue(None, None, None, colsum.data_ptr() if layout == TN else None, 0)
+    assert L.lib().fwp_matmul(layout, A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), C.data_ptr(), N, M, N, K, ctypes.byref(e),
+                              work.data_ptr(), L.stream_of(A)) == 0
+    assert bool((work[n:] == 7).all())
+    assert torch.equal(C, matmul(L, layout, A, B))
