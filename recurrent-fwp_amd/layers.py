@@ -270,7 +270,7 @@ class DeltaNetLayer(nn.Module):
             blocks = _blocks("takes_delta_block", x, self.qkvb_net.weight, self.o_net.weight, H, D)
         if blocks is not None:
             # the block fills a state that starts at zero itself, beside its pre-step
-            fresh = mems is None and getattr(self._state, "__func__", None) is DeltaNetLayer._state
+            fresh = mems is None and getattr(self._state, "__func__", None) is _zeros_or_carried
             W = (torch.empty(bsz, H, D, D, device=h.device, dtype=torch.float32) if fresh
                  else self._state(mems, carry_over_fast_weight, bsz, h, torch.float32))
             drops = _drops(self.drop)
@@ -310,6 +310,9 @@ class DeltaNetLayer(nn.Module):
         if carry_over_fast_weight:
             return out, (W.detach(), None)
         return out
+
+
+_zeros_or_carried = DeltaNetLayer._state      # as it is here, whatever replaces it later
 
 
 class DeltaNetDecoderLayer(nn.Module):

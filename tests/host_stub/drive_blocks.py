@@ -332,6 +332,38 @@ def states_of_their_own(m):
         assert W.untyped_storage().nbytes() == W.numel() * 4 and W.is_contiguous()
 
 
+def replaced_states(m):
+    """What a layer starts from comes from its _state, replaced on the instance, in a subclass or on the class."""
+    pkg, rec = package(m)
+    cls = pkg.layers.DeltaNetLayer
+    H, D, x = 2, 16, rnd(5, 3, 32)
+    layer = cls(H, 32, D)
+    with torch.no_grad():
+        zero = layer(x, carry_over_fast_weight=True)[1][0]
+
+    def other(self, mems, carry_over_fast_weight, bsz, h, dtype):
+        return torch.full((bsz, H, D, D), 0.5, dtype=dtype)
+
+    class Sub(cls):
+        _state = other
+
+    sub = Sub(H, 32, D)
+    sub.load_state_dict(layer.state_dict())
+    here = cls(H, 32, D)
+    here.load_state_dict(layer.state_dict())
+    here._state = lambda *a: other(None, *a)
+    own = cls._state
+    try:
+        for mod in (sub, here, layer):
+            if mod is layer:
+                cls._state = other
+            with torch.no_grad():
+                calls, (_, (W, _)) = rec.of(lambda: mod(x, carry_over_fast_weight=True))
+            assert calls.count("delta_block") == 1 and float((W - zero).abs().max()) > 0.1, type(mod)
+    finally:
+        cls._state = own
+
+
 def beyond_the_kernels(m):
     """Matrices wider than the kernels' offsets reach (2^21) and inputs of more rows than a launch takes go to PyTorch."""
     pkg, rec = package(m)

@@ -46,7 +46,7 @@ def test_host_side_of_every_operator_against_the_stand_in_library(build, functio
 # the language model's blocks: tests/host_stub/drive_blocks.py says what each looks at
 BLOCK_CHECKS = ["results", "misfits", "misfitting_modules", "states_left_out",
                 "unusual_parameters", "wrapped_modules", "replaced_dropouts", "own_scales",
-                "states_of_their_own", "beyond_the_kernels", "traced_and_watched"]
+                "states_of_their_own", "replaced_states", "beyond_the_kernels", "traced_and_watched"]
 
 
 @pytest.mark.parametrize("check", BLOCK_CHECKS)
