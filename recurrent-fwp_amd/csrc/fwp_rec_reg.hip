@@ -23,12 +23,11 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 
 // ------------------------------------------------------------------ forward
 
-template <int D>
 struct RecFwdOps {
     float qx, kx, vx, bx;
 };
 
-template <int D, int RING, int PF, int WPB>
+template <int RING, int PF, int WPB>
 __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
     fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float *__restrict__ Rq,
     const float *__restrict__ Rk, const float *__restrict__ Rv, const float *__restrict__ rb,
@@ -36,6 +35,7 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
     float *__restrict__ q_act, float *__restrict__ k_act, float *__restrict__ beta_act,
     float *__restrict__ vdiff, float *__restrict__ ckpt, int H, int L, int chunk, int nchunk,
     int nseq) {
+    constexpr int D = 16;
     using G = Geo<D>;
     constexpr int S = G::S, R = G::R, NP = G::NP;
     static_assert(kTile % RING == 0 && PF < RING, "ring must divide the tile");
@@ -97,9 +97,7 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
         sb[buf][per] = pb;
     };
 
-    // S = 4: one LDS write per step, s = 0..3 -> out, vdiff, q, k.  S = 2: two writes.
-    float *stage1 = sout[sl] + col;                      // s=0 -> out, s=1 -> vdiff (S=4: s=2 -> q, s=3 -> k)
-    float *stage2 = sout[2 + (sl & 1)] + col;            // S=2 only: s=0 -> q, s=1 -> k
+    float *stage = sout[sl] + col;                       // one LDS write per step: s = 0..3 -> out, vdiff, q, k
     const bool save = vdiff != nullptr;
     float *out_rows = out + seq * L * D;
     auto flush = [&](int t0) {
@@ -113,13 +111,13 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
         }
     };
 
-    auto load_ops = [&](RecFwdOps<D> &o, int buf, int tt) {
+    auto load_ops = [&](RecFwdOps &o, int buf, int tt) {
         o.qx = sq[buf][tt * D + col];
         o.kx = sk[buf][tt * D + col];
         o.vx = sv[buf][tt * D + col];
         o.bx = sb[buf][tt];
     };
-    auto compute = [&](const RecFwdOps<D> &o, int tt) {
+    auto compute = [&](const RecFwdOps &o, int tt) {
         const float y_m = fast_tanh(hcur);
         float y[NP], kp[NP], qp[NP];
         to_periodic<D>(y_m, y, lane);
@@ -142,12 +140,7 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
         hcur = group_sum<S>(dot_rot<D>(Wc, qp)) * rq;
         hcur = pinned(hcur);
         const float o_d = pinned(d), o_q = pinned(eq * rq), o_k = pinned(ek * rk);
-        if constexpr (S == 4) {
-            stage1[tt * D] = sl == 0 ? hcur : (sl == 1 ? o_d : (sl == 2 ? o_q : o_k));
-        } else {
-            stage1[tt * D] = sl == 0 ? hcur : o_d;
-            stage2[tt * D] = sl == 0 ? o_q : o_k;
-        }
+        stage[tt * D] = sl == 0 ? hcur : (sl == 1 ? o_d : (sl == 2 ? o_q : o_k));
         sba[tt] = b;
     };
 
@@ -155,7 +148,7 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
     fetch(0);
     commit(0);
     if (ntile > 1) fetch(kTile);
-    RecFwdOps<D> ring[RING];
+    RecFwdOps ring[RING];
 #pragma unroll
     for (int p = 0; p < PF; p++) load_ops(ring[p], 0, p);
 
@@ -175,7 +168,7 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
             }
         } else {  // ragged last tile: not pipelined
             for (int tt = 0; tt < nst; tt++) {
-                RecFwdOps<D> o;
+                RecFwdOps o;
                 load_ops(o, buf, tt);
                 compute(o, tt);
             }
@@ -1217,7 +1210,7 @@ int reg_rec_fwd(fwp_view qx, fwp_view kx, fwp_view vx, fwp_view bx, const float 
         hipLaunchKernelGGL(kernel, dim3((nseq + wpb - 1) / wpb), dim3(kWave * wpb), 0, s, qx, kx, vx, bx, Rq, Rk, Rv,
                            rb, W, h, out, q_act, k_act, beta_act, vdiff, ckpt, H, L, chunk, nchunk, nseq);
     };
-    if (D == 16) launch(k_rec_fwd_reg<16, 2, 1, 4>, 4);
+    if (D == 16) launch(k_rec_fwd_reg<2, 1, 4>, 4);
     else {
         const RecFwdArgs g{qx, kx, vx, bx, Rq, Rk, Rv, rb, W, h, out, q_act, k_act, beta_act, vdiff, ckpt, H, L, chunk, nchunk, nseq};
         const auto go = [&](auto ns) {

@@ -677,7 +677,7 @@ __global__ __launch_bounds__(kWave * 2 * NS) void k_rnn_bwd_pair(
         rnn_bwd_pair_y<D>(M, ckpt, gk, L, chunk, nchunk, seq, lane);
 }
 
-// ------------------------------------------- backward, three waves per sequence
+// ------------------------------------------- 16 x 16 states, backward: three waves per sequence
 //
 // The same division taken one step further, for when there are SIMDs to spare: wave X keeps only the
 // sequential part (the gradient of h through W and the softmax; grad_z); wave A, one tile behind,
@@ -685,8 +685,8 @@ __global__ __launch_bounds__(kWave * 2 * NS) void k_rnn_bwd_pair(
 // computes grad_k as before.  X loads the tiles into a ring of four slots (it fills the slot of tile
 // it - 1 while X, A and Y work on tiles it, it + 1 and it + 2).  A workgroup holds two sequences, six
 // waves on the four SIMDs of a CU.
-template <int D>
 struct RnnTriLds {
+    static constexpr int D = 16;
     float k[4][kTile * D], u[4][kTile * D], s[4][kTile * D], d[4][kTile * D];
     float b[4][kTile];
     float go[2][kTile * D];
@@ -696,14 +696,12 @@ struct RnnTriLds {
     float gk[kTile * D];
 };
 
-template <int D>
 struct RnnBwdOpsT {   // X of the three
-    float u[Geo<D>::NP];
+    float u[1];
     float go_i, s_i, k_i;
 };
-template <int D>
 struct RnnBwdOpsA {
-    float s[Geo<D>::NP], k[Geo<D>::NP];
+    float s[1], k[1];
     float g_i, d_i, b;
 };
 
@@ -718,13 +716,13 @@ __device__ __forceinline__ void tri_rounds(int ntile, F &&work) {
     }
 }
 
-template <int D>
-__device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_view beta,
+__device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds &M, fwp_view k, fwp_view beta,
                                               const float *__restrict__ vdiff,
                                               const float *__restrict__ out,
                                               const float *__restrict__ h_init, fwp_view go,
                                               const float *__restrict__ ckpt, float *__restrict__ gz, int H,
                                               int L, int chunk, int nchunk, int64_t seq, int lane) {
+    constexpr int D = RnnTriLds::D;
     using G = Geo<D>;
     constexpr int S = G::S, R = G::R, NP = G::NP, NV4 = G::NV4;
     const int i = lane / S, per = lane % 16;
@@ -789,7 +787,7 @@ __device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_v
         for (int jj = 0; jj < R; jj++) Wnext[jj] = src[reg_index<D>(lane, jj)];
     };
     float *gz_rows = gz + seq * L * D;
-    auto load_ops = [&](RnnBwdOpsT<D> &o, int it, int tt) {
+    auto load_ops = [&](RnnBwdOpsT &o, int it, int tt) {
         const int slot = it & 3, off = tt * D;
 #pragma unroll
         for (int p = 0; p < NP; p++) o.u[p] = M.u[slot][off + 16 * p + per];
@@ -797,7 +795,7 @@ __device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_v
         o.s_i = M.s[slot][off + i];
         o.k_i = M.k[slot][off + i];
     };
-    auto compute = [&](const RnnBwdOpsT<D> &o, float *hand, int tt) {
+    auto compute = [&](const RnnBwdOpsT &o, float *hand, int tt) {
         const float g_i = dh_i + o.go_i;                      // gradient of h_t = grad_z
         float g[NP];
         to_periodic<D>(g_i, g, lane);
@@ -829,7 +827,7 @@ __device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_v
         if (it >= 2) fetch(t0 - 2 * kTile);
         float *hand = M.g[it % 3];
         if (nst == kTile) {
-            RnnBwdOpsT<D> ring[2];
+            RnnBwdOpsT ring[2];
             load_ops(ring[(kTile - 1) & 1], it, kTile - 1);
 #pragma unroll
             for (int tt = kTile - 1; tt >= 0; tt--) {
@@ -838,7 +836,7 @@ __device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_v
             }
         } else {  // ragged last tile (first in reverse): not pipelined
             for (int tt = nst - 1; tt >= 0; tt--) {
-                RnnBwdOpsT<D> o;
+                RnnBwdOpsT o;
                 load_ops(o, it, tt);
                 compute(o, hand, tt);
             }
@@ -847,9 +845,9 @@ __device__ __forceinline__ void rnn_bwd_tri_x(RnnTriLds<D> &M, fwp_view k, fwp_v
     flush_tile<D>(M.g[0], gz_rows, 0, L, lane);
 }
 
-template <int D>
-__device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict__ gv,
+__device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds &M, float *__restrict__ gv,
                                               float *__restrict__ gbeta, int L, int64_t seq, int lane) {
+    constexpr int D = RnnTriLds::D;
     using G = Geo<D>;
     constexpr int S = G::S, R = G::R, NP = G::NP, NV4 = G::NV4;
     const int i = lane / S, per = lane % 16;
@@ -877,7 +875,7 @@ __device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict
         acc = group_sum<4>(acc);
         if (tt < nst) gbeta[seq * L + t0 + tt] = acc;
     };
-    auto load_ops = [&](RnnBwdOpsA<D> &o, int ty, int tt) {
+    auto load_ops = [&](RnnBwdOpsA &o, int ty, int tt) {
         const int slot = ty & 3, off = tt * D;
 #pragma unroll
         for (int p = 0; p < NP; p++) {
@@ -888,7 +886,7 @@ __device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict
         o.d_i = M.d[slot][off + i];
         o.b = M.b[slot][tt];
     };
-    auto compute = [&](const RnnBwdOpsA<D> &o, float *hand, int tt) {
+    auto compute = [&](const RnnBwdOpsA &o, float *hand, int tt) {
         // G' = G + s (x) g;  r = G'^T k
         rank1_rot<D>(Gc, o.s, o.g_i);
         const float r_i = group_sum<S>(dot_rot<D>(Gc, o.k));
@@ -904,7 +902,7 @@ __device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict
         if (ty + 1 < ntile) flush(ty + 1);
         float *hand = M.a[ty & 1];
         if (nst == kTile) {
-            RnnBwdOpsA<D> ring[2];
+            RnnBwdOpsA ring[2];
             load_ops(ring[(kTile - 1) & 1], ty, kTile - 1);
 #pragma unroll
             for (int tt = kTile - 1; tt >= 0; tt--) {
@@ -913,7 +911,7 @@ __device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict
             }
         } else {
             for (int tt = nst - 1; tt >= 0; tt--) {
-                RnnBwdOpsA<D> o;
+                RnnBwdOpsA o;
                 load_ops(o, ty, tt);
                 compute(o, hand, tt);
             }
@@ -922,10 +920,10 @@ __device__ __forceinline__ void rnn_bwd_tri_a(RnnTriLds<D> &M, float *__restrict
     flush(0);
 }
 
-template <int D>
-__device__ __forceinline__ void rnn_bwd_tri_y(RnnTriLds<D> &M, const float *__restrict__ ckpt,
+__device__ __forceinline__ void rnn_bwd_tri_y(RnnTriLds &M, const float *__restrict__ ckpt,
                                               float *__restrict__ gk, int L, int chunk, int nchunk,
                                               int64_t seq, int lane) {
+    constexpr int D = RnnTriLds::D;
     using G = Geo<D>;
     constexpr int S = G::S, R = G::R, NP = G::NP;
     const int i = lane / S, per = lane % 16;
@@ -992,7 +990,6 @@ __device__ __forceinline__ void rnn_bwd_tri_y(RnnTriLds<D> &M, const float *__re
 
 // Waves 0..5 of a workgroup, which holds two sequences: X, X, Y, Y, A, A; the two A waves are the
 // fifth and sixth and share SIMDs with the two X waves (the lighter roles), each Y has one to itself.
-template <int D>
 __global__ __launch_bounds__(kWave * 6) void k_rnn_bwd_tri(
     fwp_view k, fwp_view beta, const float *__restrict__ vdiff, const float *__restrict__ out,
     const float *__restrict__ h_init, fwp_view go, const float *__restrict__ ckpt,
@@ -1004,15 +1001,15 @@ __global__ __launch_bounds__(kWave * 6) void k_rnn_bwd_tri(
     const int role = wave >> 1;                                   // 0: X, 1: Y, 2: A
     const int which = role == 2 ? 1 - (wave & 1) : wave & 1;      // A of the other X's sequence
     const int64_t seq = (int64_t)blockIdx.x * 2 + which;
-    RnnTriLds<D> &M = reinterpret_cast<RnnTriLds<D> *>(tri_lds)[which];
+    RnnTriLds &M = reinterpret_cast<RnnTriLds *>(tri_lds)[which];
     if (seq >= nseq) {   // odd number of sequences: the spare waves only keep the barriers' count
         const int ntile = (L + kTile - 1) / kTile;
         for (int j = 0; j < ntile + 3; j++) __syncthreads();
         return;
     }
-    if (role == 0) rnn_bwd_tri_x<D>(M, k, beta, vdiff, out, h_init, go, ckpt, gz, H, L, chunk, nchunk, seq, lane);
-    else if (role == 1) rnn_bwd_tri_y<D>(M, ckpt, gk, L, chunk, nchunk, seq, lane);
-    else rnn_bwd_tri_a<D>(M, gv, gbeta, L, seq, lane);
+    if (role == 0) rnn_bwd_tri_x(M, k, beta, vdiff, out, h_init, go, ckpt, gz, H, L, chunk, nchunk, seq, lane);
+    else if (role == 1) rnn_bwd_tri_y(M, ckpt, gk, L, chunk, nchunk, seq, lane);
+    else rnn_bwd_tri_a(M, gv, gbeta, L, seq, lane);
 }
 
 // ------------------------------------------- 32 x 32 states, backward: four waves per sequence
@@ -1345,7 +1342,7 @@ int reg_rnn_bwd(fwp_view k, fwp_view beta, const float *vdiff, const float *out,
                            go, ckpt, gz, gk, gv, gbeta, H, L, chunk, nchunk, nseq);
         return (int)hipGetLastError();
     };
-    if (nseq <= kQuadMaxSeq) return launch_on(k_rnn_bwd_tri<16>, 6, 2 * sizeof(RnnTriLds<16>));
+    if (nseq <= kQuadMaxSeq) return launch_on(k_rnn_bwd_tri, 6, 2 * sizeof(RnnTriLds));
     return D == 16 ? launch_on(k_rnn_bwd_pair<16, 4>, 8, 4 * sizeof(RnnPairLds<16>), 4)
                    : launch_on(k_rnn_bwd_pair<32, 4>, 8, 4 * sizeof(RnnPairLds<32>), 4);
 }
