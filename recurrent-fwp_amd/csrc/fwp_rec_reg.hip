@@ -5,7 +5,7 @@
 // cores and written out once per sequence.  16 x 16: a step on one wave, the fed-back vector tanh(out_{t-1}) and the
 // activated q and k "grouped" (every lane of group m holds entry m), periodic operands through ds_bpermute, the softmax
 // maxima/sums, the beta logit and the softmax-Jacobian dot products as wave-wide reductions.  32 x 32: vectors in half and
-// pair form (fwp_reg.hpp), two waves to a sequence forward and four backward.  512 sequences of 256 steps, against the
+// pair form (fwp_reg.hpp), two waves to a sequence forward and four backward (few steps of many sequences: two, as 16 x 16).  512 sequences of 256 steps, against the
 // former's kernels for 32 x 32: forward 144 -> 120 us, backward with its sum over the sequences 197 -> 131 us.  Matrices come and go by way of LDS (see
 // forms::Matrix): of 20 steps, 512 / 1024 / 2048 sequences, forward 19.3 / 30.1 / 52.6 -> 12.9 / 15.2 / 23.4 us, backward 23.9 / 41.1 / 75.0 -> 23.1 / 39.5 / 71.8.
 #include "fwp_reg.hpp"
@@ -191,7 +191,8 @@ __global__ __launch_bounds__(kWave * WPB) void k_rec_fwd_reg(
 // Wave S carries the steps; wave T, one tile ahead and behind, loads the inputs and stores the results, a tenth of the
 // instructions that were the sequential wave's.  No product needs a conversion of its operand: R_q and R_k take tanh(h) in pair form and
 // give q and k in half form, one in each half of the wave (one exponential, one sum for both softmaxes), which the state takes to give
-// v_old and h in pair form.  What bounds it: the wave's own instructions, 195 a step in 1100 cycles.
+// v_old and h in pair form.  What bounds it: the wave's own instructions, about 160 vector ones of 220 a step, 30 of
+// them wait states, in 1070 cycles.
 // The softmaxes' shift costs no step anything: T takes a row's largest entry off qx and kx, and what R adds to it is below the sum of a
 // column of |R| (|tanh| <= 1).  Where that is beyond kFar the largest of the sums is looked for in each step.
 // Steps to a tile: 8 take 15 KB a sequence, so that eight fit a CU
@@ -734,7 +735,7 @@ __global__ __launch_bounds__(kWave * 2 * NS) void k_rec_bwd_pair(
 // so of the matrices only W and R meet the step's own vectors.  Wave X carries that; wave C keeps G by columns and a state of its own
 // and prepares P, P.d and W P of the next step, wave D keeps G by rows and prepares its Q, each from the g that X hands over right at the
 // start of a step: one barrier a step.  Wave Y loads and stores, a sixteenth of a tile's work in each step, and sums the
-// gradients of R on the matrix cores.  X is what bounds it: 160 instructions a step, where one wave that forms everything in turn takes 230, most of
+// gradients of R on the matrix cores.  X is what bounds it: 180 instructions a step (134 vector ones, 22 wait states), where one wave that forms everything in turn takes about 200, most of
 // them one behind the other.
 // No product's operand is converted (see forms): g and P in pair form, q and k in half form, of which X holds q in one half of
 // the wave and k in the other for both softmaxes at once; the two products with R_q and R_k are one of 64 terms.

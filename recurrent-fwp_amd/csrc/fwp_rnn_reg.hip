@@ -1018,7 +1018,7 @@ __global__ __launch_bounds__(kWave * 6) void k_rnn_bwd_tri(
 // no wave converts an operand: wave X carries the gradient of h through W and the softmax; one tile behind, wave A keeps G by columns and
 // forms r = G^T k, grad_v, a and grad_beta's terms; two tiles behind, wave D keeps G by rows and forms G u, and wave E forms W a, loads and
 // stores.  256 steps, 8 / 256 / 512 sequences: 54 / 57 / 71 us where three waves take 72 / 76 / 79.  Bound by X's chain while a sequence has a CU
-// to itself, beyond by issue: 70 to 80 instructions a step of each wave, two waves to a SIMD.
+// to itself, beyond by issue: 75 to 84 instructions a step of each wave, two waves to a SIMD.
 typedef float rnn_v4f __attribute__((ext_vector_type(4)));
 constexpr int kRnnTile = 16;                // steps to a tile (8: 59 / 73 us)
 constexpr int kRnnRows = kRnnTile / 8;      // of eight rows each: a wave's 16-byte accesses to a tile
