@@ -1257,8 +1257,8 @@ int reg_rec_bwd(const float *q_act, const float *k_act, const float *beta_act, c
             hipLaunchKernelGGL(k_rec_bwd_quad<NS>, dim3((nseq + NS - 1) / NS), dim3(4 * NS * kWave), NS * sizeof(RecBwdLds), s, g, nseq);
             return (int)hipGetLastError();
         };
-        // Two sequences to a workgroup are 512 at a time; three (with spills) 768: 256 steps, 768 sequences 188 us where
-        // workgroups of two take 248, 1024 372 and 255.
+        // Two sequences to a workgroup are 512 at a time; three (with spills) 768: 768 sequences of 20, 60 and 256 steps 31, 57 and 192 us where
+        // workgroups of two take 39, 73 and 247, 1024 50, 102 and 370 and 39, 76 and 250.
         if (nseq > 512 && nseq <= 768) return run(std::integral_constant<int, 3>());
         return run(std::integral_constant<int, 2>());
     }

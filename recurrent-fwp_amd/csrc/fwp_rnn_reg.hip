@@ -1285,8 +1285,8 @@ constexpr int kFwdPairMaxSeq = 1024;
 
 // Up to this many sequences the backward pass puts four waves on each (16 x 16: three), one sequence to a workgroup while that is
 // one for each CU, then two, and beyond it two waves, four sequences to a workgroup (32 x 32 over 256 steps, 512 sequences:
-// one wave 131 us, two 98, three 79, four 71; 768: one 130, two 113, four 117; 1024: one 143, two 117, four 132;
-// 2048: one 270, two 240, four 264).
+// one wave 131 us, two 98, three 79, four 69; 768: one 130, two 113, four 118; 1024: one 143, two 117, four 132;
+// 2048: one 270, two 240, four 264; over 20 and 60 steps, 512: three 14.2 and 26.5, four 11.8 and 23.3, 768: two 15.0 and 34.2, four 22.3 and 43.8).
 constexpr int kQuadMaxSeq = 512;
 bool reg_rnn_supported(int D) { return D == 16 || D == 32; }
 
